@@ -68,7 +68,7 @@ void free_buffers(clotho_ctx* c) {
                     B.bottom,     B.n_events,  B.events,    B.var_part,   B.fix_part,
                     B.word_cnt,   B.word_bsum, B.cum_local, B.cum_block,  B.fit_stats,
                     B.cdf_rho,    B.cdf_mu,    B.state,     B.by_parent,  B.parent_cnt,
-                    B.parent_bsum, B.prank,    B.given_parents};
+                    B.parent_bsum, B.prank,    B.given_parents, B.trait_part};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     std::memset(&B, 0, sizeof(B));
@@ -166,7 +166,7 @@ int enqueue_generation(clotho_ctx* c, std::vector<hipEvent_t>* marks) {
     HIP_TRY(c, mark(1));
     HIP_TRY(c, launch_recombine(c));
     HIP_TRY(c, mark(2));
-    HIP_TRY(c, launch_traits(c));
+    HIP_TRY(c, launch_traits_pieces(c));
     HIP_TRY(c, mark(3));
     HIP_TRY(c, launch_free_reduce(c));
     HIP_TRY(c, mark(4));
@@ -234,8 +234,8 @@ int clotho_create(const clotho_config* cfg, int device, clotho_ctx** out) {
     if (!(cfg->neutral_p >= 0.0 && cfg->neutral_p <= 1.0)) return CLOTHO_ERR_ARG;
     if (cfg->fitness_kind > CLOTHO_FIT_MV_STABILIZING) return CLOTHO_ERR_ARG;
     if (cfg->effect_quantum_log2 > 0 || cfg->effect_quantum_log2 < -60) return CLOTHO_ERR_ARG;
-    // the exact traits accumulate balanced int8 digits (|d| <= 128) over a whole
-    // row in int32: at most 2^24 slots keep every partial sum in range
+    // the exact traits sum balanced digits (|d| <= 16) of a row segment at a time;
+    // slots are limited to 2^24
     if (cfg->max_alleles == 0 || cfg->max_alleles > kMaxAlleleSlots) return CLOTHO_ERR_ARG;
     if ((cfg->fitness_kind == CLOTHO_FIT_GAUSSIAN || cfg->fitness_kind == CLOTHO_FIT_QUADRATIC) &&
         !(cfg->mu > 0.0))
@@ -329,7 +329,8 @@ int clotho_create(const clotho_config* cfg, int device, clotho_ctx** out) {
     rc |= dalloc(c, &B.sorted, table_elems(P.w_cap));
     rc |= dalloc(c, &B.pm, prefix_elems(P.w_cap));
     rc |= dalloc(c, &B.bucket, table_elems(P.w_cap));
-    rc |= dalloc(c, &B.digits, i8_packed_elems(std::max<uint32_t>(1, P.traits), P.w_cap));
+    rc |= dalloc(c, &B.digits, trait_digit_elems(std::max<uint32_t>(1, P.traits), P.w_cap));
+    rc |= dalloc(c, &B.trait_part, P.traits ? trait_piece_elems(P.traits, h_cap, P.w_cap, c->trait_round) : 1);
     rc |= dalloc(c, &B.mut_count, h_cap);
     rc |= dalloc(c, &B.mut_local, h_cap);
     rc |= dalloc(c, &B.mut_bsum, mut_blocks_cap);
@@ -417,6 +418,7 @@ int clotho_set_population(clotho_ctx* c, const uint64_t* rows, uint32_t words,
         return fail(c, CLOTHO_ERR_ARG, "set_population: null buffer");
     std::vector<uint32_t> keys(P.s_cap, 0);
     std::vector<int32_t> eq((size_t)P.s_cap * std::max<uint32_t>(1, P.traits), 0);
+    uint32_t eff_max = 0;
     for (uint32_t j = 0; j < alleles; ++j) {
         const double x = positions[j];
         const double k = x * 4294967296.0;
@@ -429,6 +431,7 @@ int clotho_set_population(clotho_ctx* c, const uint64_t* rows, uint32_t words,
                 return fail(c, CLOTHO_ERR_ARG,
                             "set_population: effects must be integer multiples of 2^q");
             eq[(size_t)j * P.traits + t] = (int32_t)w;
+            eff_max = std::max(eff_max, (uint32_t)std::fabs(w));
         }
     }
     // the bit of a slot >= alleles must be clear in every row
@@ -462,6 +465,7 @@ int clotho_set_population(clotho_ctx* c, const uint64_t* rows, uint32_t words,
     HIP_TRY(c, hipMemset(B.traits[cur], 0, sizeof(int64_t) * P.h * std::max<uint32_t>(1, P.traits)));
     st.alleles = alleles;
     st.all_size = alleles;
+    st.eff_max = eff_max;
     st.wc = words;
     st.wp = words;
     st.m = 0;
@@ -484,6 +488,7 @@ int clotho_set_synthetic_population(clotho_ctx* c, uint32_t alleles, const doubl
         return fail(c, CLOTHO_ERR_ARG, "synthetic population: null buffer");
     std::vector<uint32_t> keys(P.s_cap, 0), thr(std::max<uint32_t>(alleles, 1), 0);
     std::vector<int32_t> eq((size_t)P.s_cap * std::max<uint32_t>(1, P.traits), 0);
+    uint32_t eff_max = 0;
     for (uint32_t j = 0; j < alleles; ++j) {
         const double x = positions[j], k = x * 4294967296.0;
         if (!(x >= 0.0 && x < 1.0) || k != std::floor(k))
@@ -496,6 +501,7 @@ int clotho_set_synthetic_population(clotho_ctx* c, uint32_t alleles, const doubl
             if (w != std::floor(w) || std::fabs(w) > kEffectLimit)
                 return fail(c, CLOTHO_ERR_ARG, "effects must be integer multiples of 2^q");
             eq[(size_t)j * P.traits + t] = (int32_t)w;
+            eff_max = std::max(eff_max, (uint32_t)std::fabs(w));
         }
     }
     GenState st;
@@ -518,6 +524,7 @@ int clotho_set_synthetic_population(clotho_ctx* c, uint32_t alleles, const doubl
                          sizeof(int64_t) * P.h * std::max<uint32_t>(1, P.traits)));
     st.alleles = alleles;
     st.all_size = alleles;
+    st.eff_max = eff_max;
     st.wc = words;
     st.wp = words;
     st.m = 0;
@@ -844,6 +851,7 @@ int clotho_add_mutations(clotho_ctx* c, const uint32_t* rows, const double* posi
     const uint32_t T = P.traits;
     std::vector<uint32_t> keys(n);
     std::vector<int32_t> eq((size_t)n * std::max<uint32_t>(1, T), 0);
+    uint32_t eff_max = 0;
     for (uint32_t k = 0; k < n; ++k) {
         if (rows[k] >= P.h) return fail(c, CLOTHO_ERR_ARG, "add_mutations: row out of range");
         const double x = positions[k], kk = x * 4294967296.0;
@@ -856,6 +864,7 @@ int clotho_add_mutations(clotho_ctx* c, const uint32_t* rows, const double* posi
                 return fail(c, CLOTHO_ERR_ARG,
                             "add_mutations: effects must be integer multiples of 2^q");
             eq[(size_t)k * T + t] = (int32_t)w;
+            eff_max = std::max(eff_max, (uint32_t)std::fabs(w));
         }
     }
     GenState st;
@@ -917,6 +926,7 @@ int clotho_add_mutations(clotho_ctx* c, const uint32_t* rows, const double* posi
     if (e != hipSuccess) return fail(c, CLOTHO_ERR_HIP, hipGetErrorString(e));
     // traits and free space of the new population
     st.alleles = st.all_size = (uint32_t)A1;
+    st.eff_max = std::max(st.eff_max, eff_max);
     st.wc = st.wp = W1;
     st.m = n;
     rc = analyse_upload(c, st);

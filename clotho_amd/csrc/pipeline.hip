@@ -17,7 +17,7 @@
 #include "device_common.hpp"
 #include "pipeline.hpp"
 #include "traits.hpp"
-#include "traits_i8.hpp"
+#include "traits_f6.hpp"
 
 namespace clotho {
 namespace {
@@ -287,6 +287,7 @@ struct MutAttrs {
         if (!c) return;
         const uint32_t gen = st->gen, F = st->free_count, A = st->alleles, fb = st->free_base;
         const uint32_t k0 = local[o] + boff[o / kBlock];
+        uint32_t most = 0;  // largest |effect| drawn here
         for (uint32_t k = k0; k < k0 + c; ++k) {
             const uint32_t slot = k < F ? free_list[fb + k] : A + (k - F);
             if (slot >= P.s_cap) continue;
@@ -304,8 +305,13 @@ struct MutAttrs {
                     q = (int32_t)n;
                 }
                 effects[(size_t)slot * P.traits + t] = q;
+                most = max(most, (uint32_t)(q < 0 ? -q : q));
             }
         }
+        // the population's bound only grows, so after the first generations
+        // almost every thread stops at the read
+        if (most > __hip_atomic_load(&st->eff_max, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+            __hip_atomic_fetch_max(&st->eff_max, most, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 };
 
@@ -483,8 +489,8 @@ struct GametesOp {
         const auto ev = events + (size_t)o * P.ev_cap;
         for (uint32_t e = 0; e < ne; e += 4) {
             const Draw4 d = philox_draw(P.seed, gen, S_GAMETE, P.replicate, o, 1 + e / 4);
-            *(__attribute__((address_space(1))) i8::u32x4*)(ev + e) =
-                i8::u32x4{d.x[0], d.x[1], d.x[2], d.x[3]};
+            *(__attribute__((address_space(1))) f6::u32x4*)(ev + e) =
+                f6::u32x4{d.x[0], d.x[1], d.x[2], d.x[3]};
         }
         if (ranked) gbl(B.prank)[o] = rank;
     }
@@ -577,8 +583,8 @@ struct ParentScatterOp {
         const uint32_t k0 = gbl(B.mut_local)[o] + gbl(B.mut_bsum)[o / kBlock];
         const uint32_t nx = gbl(B.n_events)[o] | (gbl(B.mut_count)[o] << 8);
         if (pos < P.h)
-            *(__attribute__((address_space(1))) i8::u32x4*)(B.by_parent + pos) =
-                i8::u32x4{o, top, nx, k0};
+            *(__attribute__((address_space(1))) f6::u32x4*)(B.by_parent + pos) =
+                f6::u32x4{o, top, nx, k0};
     }
 };
 
@@ -698,8 +704,8 @@ __device__ __forceinline__ void load_word_tables(const Buffers& B, uint32_t bx, 
                                                  uint32_t fw, uint32_t* s_bucket,
                                                  uint32_t* s_sorted, uint64_t* s_pm) {
     static_assert(kRecBlock == 1024, "one 16-byte table piece per thread");
-    using i8::u32x4;
-    using i8::g_u32x4;
+    using f6::u32x4;
+    using f6::g_u32x4;
     uint32_t t = threadIdx.x;
     // opaque here, so the per-lane table offsets are computed per call: hoisted
     // out of a persistent block's loop they outlive it and spill to scratch
@@ -972,7 +978,7 @@ struct Recombine {
         const auto boff = gbl(B.mut_bsum);
         const auto var_part = gbl(B.var_part);
         const auto fix_part = gbl(B.fix_part);
-        const auto by_parent = (const __attribute__((address_space(1))) i8::u32x4*)B.by_parent;
+        const auto by_parent = (const __attribute__((address_space(1))) f6::u32x4*)B.by_parent;
         const bool ordered = B.by_parent != nullptr;
         const uint32_t bx = blk % P.tiles, by = blk / P.tiles;
         __shared__ __align__(16) uint32_t s_bucket[64 * 64];
@@ -1031,7 +1037,7 @@ struct Recombine {
             const uint32_t pos = first + stride * (j0 + min(lane, nb - 1));
             uint32_t g_row, g_top, g_nx, g_k0;
             if (ordered) {
-                const i8::u32x4 r = by_parent[pos];
+                const f6::u32x4 r = by_parent[pos];
                 g_row = r.x;
                 g_top = r.y;
                 g_nx = r.z;
@@ -1869,7 +1875,7 @@ __global__ void __launch_bounds__(64 * kStatWaves) k_allele_counts(
     // unconditional (rows past the wave's range re-read its first row and are
     // zeroed when counted)
     const uint32_t half_rows = (rw1 - rw0 + 1) / 2;
-    auto load8 = [&](uint32_t i0, i8::u32x4 (&x)[8]) {
+    auto load8 = [&](uint32_t i0, f6::u32x4 (&x)[8]) {
         uint32_t r[8];
 #pragma unroll
         for (int t = 0; t < 8; ++t) {
@@ -1879,17 +1885,17 @@ __global__ void __launch_bounds__(64 * kStatWaves) k_allele_counts(
         }
 #pragma unroll
         for (int t = 0; t < 8; ++t)
-            x[t] = *(const __attribute__((address_space(1))) i8::u32x4*)(rows + (size_t)r[t] * W +
+            x[t] = *(const __attribute__((address_space(1))) f6::u32x4*)(rows + (size_t)r[t] * W +
                                                                          wsrc);
     };
-    i8::u32x4 x[8];
+    f6::u32x4 x[8];
     if (half_rows) load8(0, x);
     for (uint32_t i0 = 0; i0 < half_rows; i0 += 8) {
-        i8::u32x4 xn[8];
+        f6::u32x4 xn[8];
         if (i0 + 8 < half_rows) load8(i0 + 8, xn);
 #pragma unroll
         for (int t = 0; t < 8; ++t)
-            if (!(rw0 + 2 * (i0 + t) + h < rw1 && wok)) x[t] = i8::u32x4{0, 0, 0, 0};
+            if (!(rw0 + 2 * (i0 + t) + h < rw1 && wok)) x[t] = f6::u32x4{0, 0, 0, 0};
         // row margins: popcounts of the lane's two words, summed over the half
         uint32_t v[8];
 #pragma unroll
@@ -2118,57 +2124,60 @@ __global__ void __launch_bounds__(kBlock) k_any_nonzero(const int32_t* effects, 
     if (threadIdx.x == 0) flag_out[blockIdx.x] = s[0];
 }
 
-// Exact genome traits of population `sel` (i8::traits_i8_block); the effect
-// digit planes are packed first (i8::pack_i8_block).
-struct PackI8 {
+// Exact genome traits of population `sel` (f6::traits_block); the effect
+// digit planes are packed first (f6::pack_block).
+struct PackDigits {
     static constexpr int kThreads = 256;
-    __host__ __device__ static uint32_t ng_cap(const Params& P) {
-        return (P.w_cap + i8::kGroupWords - 1) / i8::kGroupWords;
-    }
     __host__ __device__ static uint32_t blocks(const Params& P) {
-        return P.traits ? i8::kernel_tiles(P.traits) * ng_cap(P) * 4 : 0u;  // 1024 items per (nt, G)
+        return P.traits ? f6::pack_blocks(P.traits, f6::kMaxPlanes, P.w_cap) : 0u;
     }
     __device__ static __forceinline__ void run(const Params& P, const Buffers& B, uint32_t,
                                                uint32_t blk) {
-        i8::pack_i8_block(B.effects, P.traits, i8::kernel_tiles(P.traits), &B.state->wc,
-                          &B.state->all_size, ng_cap(P), B.digits, blk);
+        const auto st = gbl(B.state);
+        f6::pack_block(B.effects, P.traits, uniform_read(&st->wc), uniform_read(&st->all_size),
+                       uniform_read(&st->eff_max), B.digits, blk);
     }
 };
 
-// Up to RT row tiles of 16 rows per wave.  kEven: P.trait_blocks blocks
-// share the row tiles evenly (i8::wave_tiles_even), the grid a multiple of
-// the compute-unit count, and a wave one tile short runs the RT - 1 body;
-// otherwise RT tiles per wave in block order, the grid following from Params
-// alone (as the batched launches need).
-template <int RT, int NT, bool kEven>
-struct TraitsI8 {
+// RT row tiles (f6::tile_rows) per wave.  kBalanced: P.trait_blocks blocks, one
+// round of resident ones, share the work evenly (f6::Balance) and TraitReduce
+// sums the pieces of the row blocks that were cut; otherwise one row block per
+// block, the grid following from Params alone (as the batched launches need).
+template <int RT, int CLS, bool kBalanced>
+struct Traits {
+    using Block = f6::TraitsBlock<RT, CLS>;
     static constexpr int kThreads = 256;
-    static constexpr uint32_t kRowTiles = RT;
     __host__ __device__ static uint32_t blocks(const Params& P) {
         if (!P.traits) return 0u;
-        return kEven ? P.trait_blocks : (P.h + 64 * RT - 1) / (64 * RT);
+        return kBalanced ? P.trait_blocks : (P.h + Block::kBlockRows - 1) / Block::kBlockRows;
     }
     __device__ static __forceinline__ void run(const Params& P, const Buffers& B, uint32_t sel,
                                                uint32_t blk) {
-        const uint32_t wave = threadIdx.x >> 6;
-        const i8::WaveTiles wt = kEven ? i8::wave_tiles_even(blk, wave, P.h, P.trait_blocks)
-                                       : i8::wave_tiles_fixed(blk, wave, RT);
-        i8::traits_i8_block<RT, NT, kEven>(B.rows[sel], P.h, &B.state->wc, P.traits, B.digits,
-                                           B.traits[sel], wt);
+        const auto st = gbl(B.state);
+        Block::run(B.rows[sel], P.h, uniform_read(&st->wc), uniform_read(&st->eff_max), P.traits,
+                   B.digits, B.traits[sel], B.trait_part, blk, kBalanced ? P.trait_blocks : 0u);
     }
 };
 
-// Grid of an even traits launch over h rows: the fewest blocks that keep
-// every wave at RT tiles or fewer, rounded up to a multiple of the compute
-// units once there are more blocks than units; 0 when that grid exceeds one
-// round of `resident` blocks per unit (the fixed-tile kernel is used then).
-uint32_t even_trait_blocks(uint32_t h, uint32_t rt, uint32_t cus, uint32_t resident) {
-    const uint32_t tiles = (h + 15u) / 16u;
-    const uint32_t bmin = (tiles + 4u * rt - 1u) / (4u * rt);
-    if (bmin <= cus) return bmin;
-    const uint32_t b = (bmin + cus - 1u) / cus * cus;
-    return b <= resident * cus ? b : 0u;
-}
+// Sums of the balanced traits launch's pieces (none after another launch).
+template <int kBlockThreads>
+struct TraitReduceOp {
+    static constexpr int kThreads = kBlockThreads;
+    __host__ __device__ static uint32_t blocks(const Params& P) {
+        if (!P.trait_blocks) return 0u;
+        const uint32_t rows = f6::balanced_block_rows(f6::trait_class(P.traits));
+        const f6::Balance bal(P.h, rows, P.trait_blocks);
+        const uint64_t n = (uint64_t)(P.h - bal.full * bal.B * rows) * P.traits;
+        return bal.R ? (uint32_t)((n + kThreads - 1) / kThreads) : 0u;
+    }
+    __device__ static __forceinline__ void run(const Params& P, const Buffers& B, uint32_t sel,
+                                               uint32_t blk) {
+        const uint32_t rows = f6::balanced_block_rows(f6::trait_class(P.traits));
+        f6::reduce_pieces(B.trait_part, P.h, uniform_read(&gbl(B.state)->wc), P.traits,
+                          f6::Balance(P.h, rows, P.trait_blocks), rows,
+                          (uint64_t)blk * kThreads + threadIdx.x, B.traits[sel]);
+    }
+};
 
 // Two independent ops in one launch: blocks [0, A::blocks) run A, the rest
 // run Bo (neither reads what the other writes).  One launch instead of two
@@ -2205,11 +2214,9 @@ template <bool W, int K>
 struct MinWaves<Recombine<W, K>> {
     static constexpr int value = 8;
 };
-// four traits waves per SIMD (<= 128 registers): the batched launch at 136
-// registers held three 256-thread blocks per CU where its LDS allows four
-template <>
-struct MinWaves<TraitsI8<4, 1, false>> {
-    static constexpr int value = 4;
+template <int RT, int CLS, bool E>
+struct MinWaves<Traits<RT, CLS, E>> {
+    static constexpr int value = f6::min_waves(RT, CLS);
 };
 
 #define CLOTHO_SINGLE(name, Op)                                                                 \
@@ -2253,25 +2260,36 @@ using BatchRecombineWide = Recombine<true, 1>;
 CLOTHO_SINGLE_XCD(k_recombine, RecombineNarrow)
 CLOTHO_SINGLE_XCD(k_recombine_wide, RecombineWide)
 #undef CLOTHO_SINGLE_XCD
-CLOTHO_SINGLE(k_pack_i8_pop, PackI8)
-using Traits4Even = TraitsI8<5, 1, true>;  // T <= 4, grid within one round of resident blocks
-using Traits4 = TraitsI8<4, 1, false>;      // T <= 4
-using Traits4Two = TraitsI8<2, 1, false>;   // T <= 4, two row tiles per wave (autotuner)
-using Traits8Four = TraitsI8<4, 2, false>;  // T <= 8, four row tiles per wave (autotuner)
-using Traits32Two = TraitsI8<2, 8, false>;  // T <= 32, two row tiles per wave (autotuner)
-using Traits8 = TraitsI8<2, 2, false>;      // T <= 8
-using Traits16 = TraitsI8<4, 4, false>;     // T <= 16 (four row tiles: 5% faster than two at H = 1e6)
-using BatchTraits16 = TraitsI8<2, 4, false>;  // batched T <= 16: the rows per block of Traits8
-using Traits32 = TraitsI8<1, 8, false>;     // T <= 32
-CLOTHO_SINGLE(k_traits_i8_pop, Traits4Even)
-CLOTHO_SINGLE(k_traits_i8_pop_fixed, Traits4)
-CLOTHO_SINGLE(k_traits_i8_pop_t8, Traits8)
-CLOTHO_SINGLE(k_traits_i8_pop_t16, Traits16)
-CLOTHO_SINGLE(k_traits_i8_pop_t32, Traits32)
-CLOTHO_SINGLE(k_traits_i8_pop_two, Traits4Two)
-CLOTHO_SINGLE(k_traits_i8_pop_t8_four, Traits8Four)
-CLOTHO_SINGLE(k_traits_i8_pop_t16_two, BatchTraits16)
-CLOTHO_SINGLE(k_traits_i8_pop_t32_two, Traits32Two)
+CLOTHO_SINGLE(k_pack_digits, PackDigits)
+// by trait class (f6::trait_class: T <= 2, 4, 8, 16, 32)
+using Traits2Balanced = Traits<f6::balanced_tiles(0), 0, true>;
+using Traits4Balanced = Traits<f6::balanced_tiles(1), 1, true>;
+using Traits8Balanced = Traits<f6::balanced_tiles(2), 2, true>;
+using Traits16Balanced = Traits<f6::balanced_tiles(3), 3, true>;
+using Traits32Balanced = Traits<f6::balanced_tiles(4), 4, true>;
+CLOTHO_SINGLE(k_traits_t2, Traits2Balanced)
+CLOTHO_SINGLE(k_traits_t4, Traits4Balanced)
+CLOTHO_SINGLE(k_traits_t8, Traits8Balanced)
+CLOTHO_SINGLE(k_traits_t16, Traits16Balanced)
+CLOTHO_SINGLE(k_traits_t32, Traits32Balanced)
+// the fixed shapes of the batched launches, and the autotuner's alternatives
+using Traits2Fixed = Traits<4, 0, false>;
+using Traits2Two = Traits<2, 0, false>;
+using Traits4Fixed = Traits<4, 1, false>;
+using Traits4Two = Traits<2, 1, false>;
+using Traits8Two = Traits<2, 2, false>;
+using Traits16Two = Traits<2, 3, false>;
+using Traits32Fixed = Traits<2, 4, false>;
+using Traits32One = Traits<1, 4, false>;
+CLOTHO_SINGLE(k_traits_t2_fixed, Traits2Fixed)
+CLOTHO_SINGLE(k_traits_t2_two, Traits2Two)
+CLOTHO_SINGLE(k_traits_t4_fixed, Traits4Fixed)
+CLOTHO_SINGLE(k_traits_t4_two, Traits4Two)
+CLOTHO_SINGLE(k_traits_t8_two, Traits8Two)
+CLOTHO_SINGLE(k_traits_t16_two, Traits16Two)
+CLOTHO_SINGLE(k_traits_t32_one, Traits32One)
+using TraitReduce = TraitReduceOp<kBlock>;
+CLOTHO_SINGLE(k_trait_reduce, TraitReduce)
 CLOTHO_SINGLE(k_free_reduce, FreeReduce)
 CLOTHO_SINGLE(k_free_compact, FreeCompact)
 CLOTHO_SINGLE(k_fitness, Fitness)
@@ -2279,9 +2297,12 @@ CLOTHO_SINGLE(k_fitness_current, FitnessCurrent)
 CLOTHO_SINGLE(k_commit, Commit)
 // more shared launches of a single-population generation: the effect digit
 // planes (new effects are final after the draws) with the parent-order counts,
-// and the free-list compaction with the offspring fitness
-using DrawParents = Fused<ParentScan, PackI8>;
+// the free-space reduction with the sums of the cut traits, and the free-list
+// compaction with the offspring fitness
+using DrawParents = Fused<ParentScan, PackDigits>;
 using CompactFitness = Fused<FreeCompact, Fitness>;
+using FreeTraitReduce = Fused<FreeReduce, TraitReduceOp<FreeReduce::kThreads>>;
+CLOTHO_SINGLE(k_free_trait_reduce, FreeTraitReduce)
 CLOTHO_SINGLE(k_draw_parents, DrawParents)
 CLOTHO_SINGLE(k_compact_fitness, CompactFitness)
 #undef CLOTHO_SINGLE
@@ -2322,18 +2343,16 @@ struct LiveBlocks<WordSort> {
     __device__ static uint32_t block(const Params&, uint32_t, uint32_t u) { return u; }
 };
 template <>
-struct LiveBlocks<PackI8> {
-    // four blocks per (trait tile, 16-word group); live groups NG = ceil(wc / 16)
+struct LiveBlocks<PackDigits> {
+    // four fragments per block over the live 16-word groups, at the tile
+    // count of seven digit planes (the blocks past the live planes exit)
     static constexpr int kind = kLivePack;
     __host__ __device__ static uint32_t count(const Params& P, uint32_t wc) {
         if (!P.traits) return 0u;
-        const uint32_t ng = min((wc + i8::kGroupWords - 1) / i8::kGroupWords, PackI8::ng_cap(P));
-        return i8::kernel_tiles(P.traits) * ng * 4u;
+        return min(f6::pack_blocks(P.traits, f6::kMaxPlanes, wc),
+                   PackDigits::blocks(P));
     }
-    __device__ static uint32_t block(const Params& P, uint32_t wc, uint32_t u) {
-        const uint32_t per = ((wc + i8::kGroupWords - 1) / i8::kGroupWords) * 4u;  // >= 4 here
-        return (u / per) * PackI8::ng_cap(P) * 4u + u % per;
-    }
+    __device__ static uint32_t block(const Params&, uint32_t, uint32_t u) { return u; }
 };
 
 // Batched ops whose persistent blocks take virtual blocks round robin: their
@@ -2349,8 +2368,8 @@ template <bool W, int K>
 struct RoundRobin<Recombine<W, K>> {
     static constexpr bool value = true;
 };
-template <int RT, int NT, bool E>
-struct RoundRobin<TraitsI8<RT, NT, E>> {
+template <int RT, int CLS, bool E>
+struct RoundRobin<Traits<RT, CLS, E>> {
     static constexpr bool value = true;
 };
 template <int K>
@@ -2358,7 +2377,7 @@ struct RoundRobin<GametesOp<K>> {
     static constexpr bool value = true;
 };
 template <>
-struct RoundRobin<PackI8> {
+struct RoundRobin<PackDigits> {
     static constexpr bool value = true;
 };
 template <>
@@ -2396,7 +2415,7 @@ __global__ void __launch_bounds__(1024) k_batch_live_offsets(const RepView* __re
                 const uint32_t wc = gbl(rv.B.state)->wc;
                 n = kind == kLiveRecombine ? LiveBlocks<RecombineNarrow>::count(rv.P, wc)
                     : kind == kLiveWordSort ? LiveBlocks<WordSort>::count(rv.P, wc)
-                                            : LiveBlocks<PackI8>::count(rv.P, wc);
+                                            : LiveBlocks<PackDigits>::count(rv.P, wc);
             }
             uint32_t x = n;  // inclusive scan within the wave
             for (uint32_t d = 1; d < 64; d <<= 1) {
@@ -2518,53 +2537,64 @@ hipError_t launch_draw(clotho_ctx* c) {
     const bool scan_apart = parent_blocks(c->p) > kTotalsLds;
     if (scan_apart) TRY_LAUNCH(launch_single<SelBlockscan>(k_sel_blockscan, c, par));
     TRY_LAUNCH(launch_single<DrawGametes>(k_draw_gametes, c, par));
-    if (!c->b.by_parent) return launch_single<PackI8>(k_pack_i8_pop, c, par);
+    if (!c->b.by_parent) return launch_single<PackDigits>(k_pack_digits, c, par);
     TRY_LAUNCH(launch_single<DrawParents>(k_draw_parents, c, par));
     if (scan_apart) TRY_LAUNCH(launch_single<ParentBlockscan>(k_parent_blockscan, c, par));
     return launch_single<ParentScatter>(k_parent_scatter, c, par);
 }
 
-// Exact genome traits of population [which] (width st->wc, alleles st->all_size).
+// Exact genome traits of population [which] (width st->wc, alleles st->all_size),
+// up to the sums of the pieces (TraitReduce).
 static hipError_t launch_traits_of(clotho_ctx* c, int which, bool pack) {
     if (!c->p.traits) return hipSuccess;
     const uint32_t sel = (uint32_t)which;
-    if (pack) TRY_LAUNCH(launch_single<PackI8>(k_pack_i8_pop, c, sel));
-    const uint32_t nt = (c->p.traits + 3) / 4;
+    if (pack) TRY_LAUNCH(launch_single<PackDigits>(k_pack_digits, c, sel));
+    const int cls = f6::trait_class(c->p.traits);
     const uint32_t v = c->trait_variant;  // 0: default shape; the autotuner may pick another
-    if (nt <= 1) {
-        if (v == 2) return launch_single<Traits4>(k_traits_i8_pop_fixed, c, sel);
-        if (v == 3) return launch_single<Traits4Two>(k_traits_i8_pop_two, c, sel);
-        // one round of the even kernel where it fits, else the fixed tiles
-        if (!c->trait_resident) TRY_LAUNCH(query_trait_residency(c));
-        const uint32_t cus = (uint32_t)std::max(1, c->prop.multiProcessorCount);
-        c->p.trait_blocks = even_trait_blocks(c->p.h, Traits4Even::kRowTiles, cus, c->trait_resident);
-        if (c->p.trait_blocks) return launch_single<Traits4Even>(k_traits_i8_pop, c, sel);
-        return launch_single<Traits4>(k_traits_i8_pop_fixed, c, sel);
+    c->p.trait_blocks = 0;
+    if (v == 2 || v == 3) {
+        if (cls <= 1 && v == 2)
+            return cls ? launch_single<Traits4Fixed>(k_traits_t4_fixed, c, sel)
+                       : launch_single<Traits2Fixed>(k_traits_t2_fixed, c, sel);
+        switch (cls) {
+            case 0: return launch_single<Traits2Two>(k_traits_t2_two, c, sel);
+            case 1: return launch_single<Traits4Two>(k_traits_t4_two, c, sel);
+            case 2: return launch_single<Traits8Two>(k_traits_t8_two, c, sel);
+            case 3: return launch_single<Traits16Two>(k_traits_t16_two, c, sel);
+            default: return launch_single<Traits32One>(k_traits_t32_one, c, sel);
+        }
     }
-    if (nt <= 2) {
-        if (v == 2) return launch_single<Traits8Four>(k_traits_i8_pop_t8_four, c, sel);
-        return launch_single<Traits8>(k_traits_i8_pop_t8, c, sel);
+    c->p.trait_blocks = c->trait_round;
+    switch (cls) {
+        case 0: return launch_single<Traits2Balanced>(k_traits_t2, c, sel);
+        case 1: return launch_single<Traits4Balanced>(k_traits_t4, c, sel);
+        case 2: return launch_single<Traits8Balanced>(k_traits_t8, c, sel);
+        case 3: return launch_single<Traits16Balanced>(k_traits_t16, c, sel);
+        default: return launch_single<Traits32Balanced>(k_traits_t32, c, sel);
     }
-    if (nt <= 4) {
-        if (v == 2) return launch_single<BatchTraits16>(k_traits_i8_pop_t16_two, c, sel);
-        return launch_single<Traits16>(k_traits_i8_pop_t16, c, sel);
-    }
-    if (v == 2) return launch_single<Traits32Two>(k_traits_i8_pop_t32_two, c, sel);
-    return launch_single<Traits32>(k_traits_i8_pop_t32, c, sel);
 }
 
 // Launch-shape candidates of the traits pass for the context's trait count
 // (values of clotho_ctx::trait_variant; 1 is the default shape).
-uint32_t trait_variants(const clotho_ctx* c) { return (c->p.traits + 3) / 4 <= 1 ? 3u : 2u; }
+uint32_t trait_variants(const clotho_ctx* c) { return c->p.traits <= 4 ? 3u : 2u; }
 
-hipError_t launch_traits_current(clotho_ctx* c) { return launch_traits_of(c, c->cur, true); }
+static hipError_t launch_whole_traits_of(clotho_ctx* c, int which, bool pack) {
+    TRY_LAUNCH(launch_traits_of(c, which, pack));
+    return launch_single<TraitReduce>(k_trait_reduce, c, (uint32_t)which);
+}
+
+hipError_t launch_traits_current(clotho_ctx* c) { return launch_whole_traits_of(c, c->cur, true); }
 
 hipError_t query_trait_residency(clotho_ctx* c) {
+    void (*const kernels[f6::kClasses])(Params, Buffers, uint32_t) = {
+        k_traits_t2, k_traits_t4, k_traits_t8, k_traits_t16, k_traits_t32};
     int per_cu = 0;
     const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        &per_cu, reinterpret_cast<const void*>(k_traits_i8_pop), Traits4Even::kThreads, 0);
+        &per_cu, reinterpret_cast<const void*>(kernels[f6::trait_class(c->cfg.trait_count)]),
+        Traits2Balanced::kThreads, 0);
     if (e != hipSuccess) return e;
-    c->trait_resident = (uint32_t)std::max(1, per_cu);
+    c->trait_round =
+        (uint32_t)std::max(1, per_cu) * (uint32_t)std::max(1, c->prop.multiProcessorCount);
     return hipSuccess;
 }
 
@@ -2579,7 +2609,8 @@ hipError_t launch_recombine(clotho_ctx* c) {
 }
 
 // the digit planes were packed by the draw phase
-hipError_t launch_traits(clotho_ctx* c) { return launch_traits_of(c, 1 - c->cur, false); }
+hipError_t launch_traits(clotho_ctx* c) { return launch_whole_traits_of(c, 1 - c->cur, false); }
+hipError_t launch_traits_pieces(clotho_ctx* c) { return launch_traits_of(c, 1 - c->cur, false); }
 
 hipError_t launch_free_space(clotho_ctx* c) {
     TRY_LAUNCH(launch_single<FreeReduce>(k_free_reduce, c, 0));
@@ -2587,7 +2618,7 @@ hipError_t launch_free_space(clotho_ctx* c) {
 }
 
 hipError_t launch_free_reduce(clotho_ctx* c) {
-    return launch_single<FreeReduce>(k_free_reduce, c, 0);
+    return launch_single<FreeTraitReduce>(k_free_trait_reduce, c, (uint32_t)(1 - c->cur));
 }
 hipError_t launch_compact_fitness(clotho_ctx* c) {
     return launch_single<CompactFitness>(k_compact_fitness, c, (uint32_t)c->cur);
@@ -2607,7 +2638,7 @@ hipError_t launch_population_analysis(clotho_ctx* c) {
     const Params& P = c->p;
     Buffers& B = c->b;
     const int cur = c->cur;
-    TRY_LAUNCH(launch_traits_of(c, cur, true));
+    TRY_LAUNCH(launch_whole_traits_of(c, cur, true));
     hipLaunchKernelGGL(k_column_reduce, dim3((P.w_cap + kBlock - 1) / kBlock, P.chunks),
                        dim3(kBlock), 0, c->stream, P, B.state, B.rows[cur], B.var_part,
                        B.fix_part);
@@ -2628,11 +2659,13 @@ void batch_op_blocks(const Params& P, uint32_t* out) {
     out[kOpGametes] = Gametes::blocks(P);
     out[kOpWordSort] = WordSort::blocks(P);
     out[kOpRecombine] = RecombineNarrow::blocks(P);
-    out[kOpPackI8] = PackI8::blocks(P);
-    const uint32_t nt = (P.traits + 3) / 4;
-    out[kOpTraits] = nt <= 1 ? Traits4::blocks(P)
-                   : nt <= 4 ? Traits8::blocks(P)  // same rows per block as BatchTraits16
-                             : Traits32::blocks(P);
+    out[kOpPackDigits] = PackDigits::blocks(P);
+    const int cls = f6::trait_class(P.traits);
+    out[kOpTraits] = cls == 0   ? Traits2Fixed::blocks(P)
+                     : cls == 1 ? Traits4Fixed::blocks(P)
+                     : cls == 2 ? Traits8Two::blocks(P)
+                     : cls == 3 ? Traits16Two::blocks(P)
+                                : Traits32Fixed::blocks(P);
     out[kOpFreeReduce] = FreeReduce::blocks(P);
     out[kOpFreeCompact] = FreeCompact::blocks(P);
     out[kOpFitness] = Fitness::blocks(P);
@@ -2686,6 +2719,16 @@ hipError_t launch_batched_recombine(const BatchLaunch& L, uint32_t par, hipStrea
     return launch_batched<BatchRecombineNarrow>(L, kOpRecombine, par, s);
 }
 
+hipError_t launch_batched_traits(const BatchLaunch& L, uint32_t chi, hipStream_t s) {
+    switch (f6::trait_class(L.traits)) {
+        case 0: return launch_batched<Traits2Fixed>(L, kOpTraits, chi, s);
+        case 1: return launch_batched<Traits4Fixed>(L, kOpTraits, chi, s);
+        case 2: return launch_batched<Traits8Two>(L, kOpTraits, chi, s);
+        case 3: return launch_batched<Traits16Two>(L, kOpTraits, chi, s);
+        default: return launch_batched<Traits32Fixed>(L, kOpTraits, chi, s);
+    }
+}
+
 }  // namespace
 
 // The batch's recombination and traits over the last generation's gametes,
@@ -2695,12 +2738,8 @@ hipError_t launch_batch_replay(const BatchLaunch& L, uint32_t par, hipStream_t s
     TRY_LAUNCH(launch_batched_recombine(L, par, s));
     if (!L.traits) return hipSuccess;
     const uint32_t chi = 1 - par;
-    TRY_LAUNCH(launch_batched<PackI8>(L, kOpPackI8, chi, s));
-    const uint32_t nt = (L.traits + 3) / 4;
-    if (nt <= 1) return launch_batched<Traits4>(L, kOpTraits, chi, s);
-    if (nt <= 2) return launch_batched<Traits8>(L, kOpTraits, chi, s);
-    if (nt <= 4) return launch_batched<BatchTraits16>(L, kOpTraits, chi, s);
-    return launch_batched<Traits32>(L, kOpTraits, chi, s);
+    TRY_LAUNCH(launch_batched<PackDigits>(L, kOpPackDigits, chi, s));
+    return launch_batched_traits(L, chi, s);
 }
 
 hipError_t launch_batch_generation(const BatchLaunch& L, uint32_t par, hipStream_t s,
@@ -2721,16 +2760,8 @@ hipError_t launch_batch_generation(const BatchLaunch& L, uint32_t par, hipStream
     TRY_LAUNCH(mark(2));
     if (L.traits) {
         const uint32_t chi = 1 - par;
-        TRY_LAUNCH(launch_batched<PackI8>(L, kOpPackI8, chi, s));
-        const uint32_t nt = (L.traits + 3) / 4;
-        if (nt <= 1)
-            TRY_LAUNCH(launch_batched<Traits4>(L, kOpTraits, chi, s));
-        else if (nt <= 2)
-            TRY_LAUNCH(launch_batched<Traits8>(L, kOpTraits, chi, s));
-        else if (nt <= 4)
-            TRY_LAUNCH(launch_batched<BatchTraits16>(L, kOpTraits, chi, s));
-        else
-            TRY_LAUNCH(launch_batched<Traits32>(L, kOpTraits, chi, s));
+        TRY_LAUNCH(launch_batched<PackDigits>(L, kOpPackDigits, chi, s));
+        TRY_LAUNCH(launch_batched_traits(L, chi, s));
     }
     TRY_LAUNCH(mark(3));
     TRY_LAUNCH(launch_batched<FreeReduce>(L, kOpFreeReduce, par, s));

@@ -17,7 +17,7 @@ constexpr int kMaxTraits = 32;    // trait capacity of the fused paths
 constexpr int kScanBlock = 256;   // items per block of every two-level scan
 // |quantised effect| bound: four balanced base-256 digits represent it exactly
 constexpr double kEffectLimit = 1073741823.0;  // 2^30 - 1
-// allele-slot capacity limit: int8 digit sums over a row stay within int32
+// allele-slot capacity limit: digit sums over a row stay within int32
 constexpr uint32_t kMaxAlleleSlots = 1u << 24;
 // words per column tile of the population-statistics pass (row partials are
 // kept per tile), its waves per block, and the most rows of one of its row
@@ -79,6 +79,7 @@ struct GenState {
     uint32_t free_base;    // free-list entries used by earlier intermediate generations
     uint32_t inter;        // position in the intermediate batch, 0 .. inter_k
     uint32_t given;        // 1: the next draw takes Buffers::given_parents (one generation)
+    uint32_t eff_max;      // bound on the quantised effects' magnitude (never shrinks)
 };
 
 // Kernel-side constants that do not change between generations.
@@ -107,7 +108,7 @@ struct Params {
     uint32_t mut_blocks;   // scan blocks over gametes
     uint32_t word_blocks;  // 64-word free-space blocks at capacity
     uint32_t max_chunks;   // row-chunk capacity of the partial buffers
-    uint32_t trait_blocks; // grid of the single-population traits launch
+    uint32_t trait_blocks; // blocks of the last balanced traits launch (0: another launch)
 };
 
 // Device buffers.  Index [c] is the population that is current after the
@@ -126,7 +127,8 @@ struct Buffers {
     uint32_t* sorted;         // [tiles][64 k][64 w] position keys of each word, ascending
     uint64_t* pm;             // [tiles][65 c][64 w] bits of the c smallest keys of each word
     uint32_t* bucket;         // [tiles][64 q][64 w] per word: #{keys < b<<24}, four b per dword
-    uint4* digits;            // [ceil(T/4)][w_cap][64] int8 digit planes of the effects
+    uint4* digits;            // FP6 digit planes of the effects (trait_digit_elems)
+    int64_t* trait_part;      // [2 blocks][rows][T] pieces of cut row blocks (f6::piece_elems)
     uint32_t* mut_count;      // [h]
     uint32_t* mut_local;      // [h] exclusive scan inside a block
     uint32_t* mut_bsum;       // [mut_blocks] block totals -> exclusive offsets
@@ -174,7 +176,7 @@ enum BatchOp : int {
     kOpGametes,
     kOpWordSort,
     kOpRecombine,
-    kOpPackI8,
+    kOpPackDigits,
     kOpTraits,
     kOpFreeReduce,
     kOpFreeCompact,
@@ -250,7 +252,7 @@ struct clotho_ctx {
     hipDeviceProp_t prop;
     size_t device_bytes = 0;    // sum of the context's device allocations
     uint32_t next_n = 0;        // offspring individuals of following generations (0: keep)
-    uint32_t trait_resident = 0;  // resident blocks per unit of the even traits kernel (0: unknown)
+    uint32_t trait_round = 1;     // blocks of one resident round of the balanced traits kernel
     // launch shapes the autotuner may change (0 / defaults: the built-in choice)
     uint32_t trait_variant = 0;   // traits-pass kernel shape, 1 .. trait_variants()
     uint32_t compact_rows = 8;    // rows per wave step of the column compaction: 4, 8, 16
@@ -263,7 +265,8 @@ namespace clotho {
 hipError_t launch_draw(clotho_ctx* c);       // draws + per-word order statistics
 hipError_t launch_word_sort(clotho_ctx* c);  // order statistics alone (autotuner replays)
 hipError_t launch_recombine(clotho_ctx* c);
-hipError_t launch_traits(clotho_ctx* c);
+hipError_t launch_traits(clotho_ctx* c);         // whole traits
+hipError_t launch_traits_pieces(clotho_ctx* c);  // launch_free_reduce sums the pieces
 hipError_t launch_free_space(clotho_ctx* c);
 hipError_t launch_fitness(clotho_ctx* c);
 // fitness of the current population from its traits (noise of generation gen - 1)
@@ -286,7 +289,8 @@ hipError_t launch_classify_columns(const uint64_t* d_fix, const uint64_t* d_var,
 hipError_t launch_crossover_rows(clotho_ctx* c, const uint64_t* d_top, const uint64_t* d_bottom,
                                  uint32_t w, const uint32_t* d_nev, const uint32_t* d_ev,
                                  uint32_t stride, uint32_t gametes, uint64_t* d_out, uint32_t ow);
-// the generation's late launches: the reduction alone, then the free-list
+// the generation's late launches: the reduction (and the sums of the traits
+// launch's pieces), then the free-list
 // compaction and the offspring fitness in one launch
 hipError_t launch_free_reduce(clotho_ctx* c);
 hipError_t launch_compact_fitness(clotho_ctx* c);
@@ -300,7 +304,7 @@ uint32_t trait_variants(const clotho_ctx* c);
 hipError_t launch_compact_plan(clotho_ctx* c);
 hipError_t launch_compact_rows(clotho_ctx* c, int src);
 uint32_t compact_chunks_of(const clotho_ctx* c);
-hipError_t query_trait_residency(clotho_ctx* c);  // sets c->trait_resident
+hipError_t query_trait_residency(clotho_ctx* c);  // sets c->trait_round
 // Column compaction of population [src] into [1 - src] (fixed and lost
 // columns removed, slots renumbered in order); the caller flips cur.
 hipError_t launch_compact(clotho_ctx* c, int src);

@@ -6,6 +6,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstdlib>
 #include <vector>
 
 #include "../../include/clotho_amd.h"
@@ -21,15 +22,20 @@ hipError_t launch_traits_walk_fp32(const uint64_t* rows, uint32_t h, uint32_t w,
 hipError_t launch_traits_walk_fp64(const uint64_t* rows, uint32_t h, uint32_t w,
                                    const double* eff, uint32_t sites, uint32_t traits, double* z,
                                    hipStream_t s);
-// Exact traits of the pipeline (traits_mfma.hip): int8 digit planes of the
-// quantised effects, int32 MFMA accumulation, int64 recombination.
-uint32_t i8_ntiles(uint32_t traits);  // N tiles of the kernel for `traits` (1, 2, 4, 8)
-size_t i8_packed_elems(uint32_t traits, uint32_t w_cap);  // uint4 elements
-hipError_t launch_pack_i8(const int32_t* eff, uint32_t traits, const uint32_t* p_words,
-                          const uint32_t* p_alleles, uint32_t w_cap, uint4* packed,
-                          hipStream_t s);
-hipError_t launch_traits_i8(const uint64_t* rows, uint32_t h, const uint32_t* p_words,
-                            uint32_t traits, const uint4* packed, int64_t* out, hipStream_t s);
+// Exact traits of the pipeline (traits_mfma.hip): FP6 digit planes of the
+// quantised effects, exact FP32 MFMA accumulation, int64 recombination.
+size_t trait_digit_elems(uint32_t traits, uint32_t w_cap);  // uint4 elements
+// int64 elements for the pieces of a balanced launch of at most `round` blocks
+// over up to h rows of up to w_cap words
+size_t trait_piece_elems(uint32_t traits, uint32_t h, uint32_t w_cap, uint32_t round);
+uint32_t exact_round(uint32_t traits);  // blocks of launch_traits_exact on the current device
+// most: bound on |effect|
+hipError_t launch_pack_digits(const int32_t* eff, uint32_t traits, uint32_t words, uint32_t sites,
+                              uint32_t most, uint4* packed, hipStream_t s);
+// part: trait_piece_elems(traits, h, words, blocks) elements, blocks <= exact_round
+hipError_t launch_traits_exact(const uint64_t* rows, uint32_t h, uint32_t words, uint32_t most,
+                               uint32_t traits, const uint4* packed, int64_t* out, int64_t* part,
+                               uint32_t blocks, hipStream_t s);
 // MFMA contraction (traits_mfma.hip): effects pre-split into `terms` BF16
 // matrices laid out for the kernel; FP64 partials per K chunk reduced in FP64.
 size_t mfma_effect_elems(uint32_t words, int terms);
@@ -71,9 +77,11 @@ struct TraitWorkspace {
     double* d_z64 = nullptr;
     double* d_partial = nullptr;
     int32_t* d_qeff = nullptr;   // EXACT_I8: effects as integers k (effect ~ k 2^-q)
-    uint32_t* d_dims = nullptr;  // EXACT_I8: {words, sites} as the pack kernel reads them
-    uint4* d_packed8 = nullptr;  // EXACT_I8: int8 digit planes
+    uint32_t most = 0;           // EXACT_I8: largest |k|
+    uint4* d_planes = nullptr;   // EXACT_I8: digit planes
     int64_t* d_sum = nullptr;    // EXACT_I8: exact sums of k
+    int64_t* d_part = nullptr;   // EXACT_I8: pieces of the row blocks cut along K
+    uint32_t blocks = 0;         // EXACT_I8: blocks of the contraction's launch
     int q = 0;
 
     int init(const uint64_t* rows, uint32_t h_, uint32_t w_, const double* eff, uint32_t s_,
@@ -102,19 +110,24 @@ struct TraitWorkspace {
             if (i8_quantum_exponent(eff, (size_t)sites * traits, &q) != CLOTHO_OK)
                 return CLOTHO_ERR_ARG;
             std::vector<int32_t> k((size_t)sites * traits);
-            for (size_t i = 0; i < k.size(); ++i) k[i] = (int32_t)std::llround(std::ldexp(eff[i], q));
-            const uint32_t dims[2] = {w, sites};
+            most = 0;
+            for (size_t i = 0; i < k.size(); ++i) {
+                k[i] = (int32_t)std::llround(std::ldexp(eff[i], q));
+                most = std::max(most, (uint32_t)std::abs(k[i]));
+            }
             if (hipMalloc((void**)&d_qeff, 4 * k.size()) != hipSuccess ||
-                hipMalloc((void**)&d_dims, sizeof(dims)) != hipSuccess ||
-                hipMalloc((void**)&d_packed8, sizeof(uint4) * i8_packed_elems(traits, w)) !=
+                hipMalloc((void**)&d_planes, sizeof(uint4) * trait_digit_elems(traits, w)) !=
                     hipSuccess ||
                 hipMalloc((void**)&d_sum, 8 * (size_t)h * traits) != hipSuccess)
                 return CLOTHO_ERR_HIP;
-            if (hipMemcpy(d_qeff, k.data(), 4 * k.size(), hipMemcpyHostToDevice) != hipSuccess ||
-                hipMemcpy(d_dims, dims, sizeof(dims), hipMemcpyHostToDevice) != hipSuccess)
+            blocks = exact_round(traits);
+            if (!blocks || hipMalloc((void**)&d_part, 8 * trait_piece_elems(traits, h, w, blocks)) !=
+                               hipSuccess)
+                return CLOTHO_ERR_HIP;
+            if (hipMemcpy(d_qeff, k.data(), 4 * k.size(), hipMemcpyHostToDevice) != hipSuccess)
                 return CLOTHO_ERR_HIP;
             // the digit planes are built once per effect set, as in a generation
-            if (launch_pack_i8(d_qeff, traits, d_dims, d_dims + 1, w, d_packed8, st) != hipSuccess)
+            if (launch_pack_digits(d_qeff, traits, w, sites, most, d_planes, st) != hipSuccess)
                 return CLOTHO_ERR_HIP;
         } else if (mode == CLOTHO_TRAITS_EXACT_FP64) {
             if (hipMalloc((void**)&d_eff64, 8 * (size_t)sites * traits) != hipSuccess ||
@@ -146,7 +159,7 @@ struct TraitWorkspace {
         if (mode == CLOTHO_TRAITS_EXACT_FP64)
             return launch_traits_walk_fp64(d_rows, h, w, d_eff64, sites, traits, d_z64, st);
         if (mode == CLOTHO_TRAITS_EXACT_I8)
-            return launch_traits_i8(d_rows, h, d_dims, traits, d_packed8, d_sum, st);
+            return launch_traits_exact(d_rows, h, w, most, traits, d_planes, d_sum, d_part, blocks, st);
         return launch_traits_mfma(d_rows, h, w, d_packed, sites, traits, terms, d_partial, d_z64,
                                   st);
     }
@@ -174,7 +187,7 @@ struct TraitWorkspace {
 
     void release() {
         void* ptrs[] = {d_rows, d_eff32, d_eff64, d_packed, d_z32, d_z64, d_partial,
-                        d_qeff, d_dims, d_packed8, d_sum};
+                        d_qeff, d_planes, d_sum, d_part};
         for (void* p : ptrs)
             if (p) (void)hipFree(p);
     }

@@ -4,12 +4,11 @@
 // population-wide common_phenotype_accumulator,
 // include/clotho/data_spaces/phenotype_evaluator/common_phenotype_accumulator_row_block_alignment.hpp:47-66).
 //
-// Exact path (v_mfma_i32_16x16x64_i8): quantised int32 effects are written as
-// four balanced base-256 digits d_p in [-128, 127]; genotype bits expand to
-// int8 0/1; each 16x16x64 product accumulates exactly in int32 and the digit
-// planes recombine in int64, so the sums equal the FP64 sequential sums of
-// the reference bit for bit (effects are multiples of 2^q).  One N tile holds
-// 4 traits x 4 digit planes.
+// Exact path (v_mfma_scale_f32_16x16x128_f8f6f4): quantised int32 effects are
+// written as balanced base-32 digits in FP6, genotype bits as FP4 0/1; every
+// FP32 sum is exact and the digit planes recombine in int64, so the sums equal
+// the FP64 sequential sums of the reference bit for bit (effects are multiples
+// of 2^q).  Kernel bodies: traits_f6.hpp.
 //
 // Split-BF16 path (v_mfma_f32_16x16x32_bf16): bits expand to BF16 0/1 (exact),
 // effects split into 1-3 BF16 terms hi + mid + lo, FP32 accumulation per
@@ -20,17 +19,18 @@
 // accumulator lane l holds column (l % 16), rows 4 * (l / 16) + i.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 
 #include "pipeline.hpp"
 #include "traits.hpp"
-#include "traits_i8.hpp"
+#include "traits_f6.hpp"
 
 namespace clotho {
 namespace {
 
-using i8::kGroupWords;
+using f6::kGroupWords;
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
@@ -43,21 +43,31 @@ __device__ inline uint32_t bits2_bf16(uint32_t two) {
 }
 
 
-// Exact-path kernels: bodies in traits_i8.hpp.
-__global__ void __launch_bounds__(256) k_pack_i8(const int32_t* __restrict__ eff, uint32_t T,
-                                                 uint32_t ntiles, const uint32_t* p_words,
-                                                 const uint32_t* p_alleles, uint32_t ng_cap,
-                                                 uint4* __restrict__ packed) {
-    i8::pack_i8_block(eff, T, ntiles, p_words, p_alleles, ng_cap, packed, blockIdx.x);
+// Exact-path kernels: bodies in traits_f6.hpp.
+__global__ void __launch_bounds__(256) k_pack_digits_of(const int32_t* __restrict__ eff, uint32_t T,
+                                                        uint32_t words, uint32_t sites,
+                                                        uint32_t most,
+                                                        uint4* __restrict__ packed) {
+    f6::pack_block(eff, T, words, sites, most, packed, blockIdx.x);
 }
 
-template <int RT, int NT>
-__global__ void __launch_bounds__(256) k_traits_i8(const uint64_t* __restrict__ rows, uint32_t h,
-                                                   const uint32_t* p_words, uint32_t T,
-                                                   const uint4* __restrict__ packed,
-                                                   int64_t* __restrict__ traits) {
-    i8::traits_i8_block<RT, NT>(rows, h, p_words, T, packed, traits,
-                                i8::wave_tiles_fixed(blockIdx.x, threadIdx.x >> 6, RT));
+template <int CLS>
+__global__ void __launch_bounds__(256)
+    __attribute__((amdgpu_waves_per_eu(f6::min_waves(f6::balanced_tiles(CLS), CLS))))
+    k_traits_exact(const uint64_t* __restrict__ rows, uint32_t h, uint32_t words, uint32_t most,
+                   uint32_t T, const uint4* __restrict__ packed, int64_t* __restrict__ traits,
+                   int64_t* __restrict__ part, uint32_t blocks) {
+    f6::TraitsBlock<f6::balanced_tiles(CLS), CLS>::run(rows, h, words, most, T, packed, traits, part,
+                                                       blockIdx.x, blocks);
+}
+
+__global__ void __launch_bounds__(256) k_exact_reduce(uint32_t h, uint32_t words, uint32_t T,
+                                                      uint32_t blocks,
+                                                      const int64_t* __restrict__ part,
+                                                      int64_t* __restrict__ traits) {
+    const uint32_t rows = f6::balanced_block_rows(f6::trait_class(T));
+    f6::reduce_pieces(part, h, words, T, f6::Balance(h, rows, blocks), rows,
+                      (uint64_t)blockIdx.x * 256 + threadIdx.x, traits);
 }
 
 
@@ -95,8 +105,8 @@ __global__ void __launch_bounds__(256) k_traits_bf16(const uint64_t* __restrict_
     __shared__ uint4 s_b0[FR * 64];
     __shared__ uint4 s_b1[FR * 64];
     __shared__ uint4 s_lut[256];
-    const auto rows = i8::as_global(rows_in);
-    const auto packed = i8::as_global(packed_in);
+    const auto rows = f6::as_global(rows_in);
+    const auto packed = f6::as_global(packed_in);
     const uint32_t NG = (W + 15) / 16;
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const uint32_t m = lane & 15, g = lane >> 4;
@@ -121,17 +131,17 @@ __global__ void __launch_bounds__(256) k_traits_bf16(const uint64_t* __restrict_
         rv[r] = row < h;
         rp[r] = rows + (size_t)(rv[r] ? row : 0) * W;
     }
-    auto load_rows = [&](uint32_t G, i8::u32x4 (&x)[RT][2]) {
+    auto load_rows = [&](uint32_t G, f6::u32x4 (&x)[RT][2]) {
         const uint32_t w = 16 * G + 4 * g;
 #pragma unroll
         for (int r = 0; r < RT; ++r) {
             if (rv[r] && w < W) {
-                const i8::g_u32x4* src = (const i8::g_u32x4*)(rp[r] + w);
+                const f6::g_u32x4* src = (const f6::g_u32x4*)(rp[r] + w);
                 x[r][0] = src[0];
                 x[r][1] = src[1];
             } else {
-                x[r][0] = i8::u32x4{0, 0, 0, 0};
-                x[r][1] = i8::u32x4{0, 0, 0, 0};
+                x[r][0] = f6::u32x4{0, 0, 0, 0};
+                x[r][1] = f6::u32x4{0, 0, 0, 0};
             }
         }
     };
@@ -159,13 +169,13 @@ __global__ void __launch_bounds__(256) k_traits_bf16(const uint64_t* __restrict_
     };
     // vmcnt(0) only: the direct-to-LDS loads and the next group's rows have landed
     auto wait_loads = [] { __builtin_amdgcn_s_waitcnt(0x0F70); };
-    i8::u32x4 x[RT][2];
+    f6::u32x4 x[RT][2];
     if (n_stages) load_rows(G0, x);
     stage_b(0);
     wait_loads();
     __syncthreads();
     for (uint32_t G = G0; G < G1; ++G) {
-        i8::u32x4 xn[RT][2];
+        f6::u32x4 xn[RT][2];
         if (G + 1 < G1) load_rows(G + 1, xn);
 #pragma unroll
         for (uint32_t st = 0; st < SPG; ++st) {
@@ -180,7 +190,7 @@ __global__ void __launch_bounds__(256) k_traits_bf16(const uint64_t* __restrict_
                 v8bf a[RT];
 #pragma unroll
                 for (int r = 0; r < RT; ++r) {
-                    const i8::u32x4 v = x[r][q >> 4];
+                    const f6::u32x4 v = x[r][q >> 4];
                     const uint32_t sel = (q >> 2) & 3;
                     const uint32_t dw = sel == 0 ? v.x : sel == 1 ? v.y : sel == 2 ? v.z : v.w;
                     const uint32_t b8 = (dw >> (8 * (q & 3))) & 0xFFu;
@@ -248,45 +258,72 @@ float bf16_to_f(uint16_t b) {
 
 }  // namespace
 
-// ---- exact int8 path (used by the pipeline) -------------------------------
-uint32_t i8_ntiles(uint32_t traits) { return i8::kernel_tiles(traits); }
-
-size_t i8_packed_elems(uint32_t traits, uint32_t w_cap) {
+// ---- exact path (used by the pipeline) -------------------------------------
+size_t trait_digit_elems(uint32_t traits, uint32_t w_cap) {
     const size_t ng = (w_cap + kGroupWords - 1) / kGroupWords;
-    return (size_t)i8_ntiles(traits) * ng * 16 * 64;
+    return f6::kernel_tiles(traits, f6::kMaxPlanes) * ng *
+           f6::kGroupBlocks * f6::kFragVecs;
 }
 
-hipError_t launch_pack_i8(const int32_t* eff, uint32_t traits, const uint32_t* p_words,
-                          const uint32_t* p_alleles, uint32_t w_cap, uint4* packed,
-                          hipStream_t s) {
-    const uint32_t nt = i8_ntiles(traits);
-    const uint32_t ng_cap = (w_cap + kGroupWords - 1) / kGroupWords;
-    const size_t n = (size_t)nt * ng_cap * 16 * 64;
-    hipLaunchKernelGGL(k_pack_i8, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, s, eff, traits,
-                       nt, p_words, p_alleles, ng_cap, packed);
+hipError_t launch_pack_digits(const int32_t* eff, uint32_t traits, uint32_t words, uint32_t sites,
+                              uint32_t most, uint4* packed, hipStream_t s) {
+    const uint32_t blocks = f6::pack_blocks(traits, f6::digit_planes(most), words);
+    hipLaunchKernelGGL(k_pack_digits_of, dim3(blocks), dim3(256), 0, s, eff, traits, words, sites,
+                       most, packed);
     return hipGetLastError();
 }
 
-hipError_t launch_traits_i8(const uint64_t* rows, uint32_t h, const uint32_t* p_words,
-                            uint32_t traits, const uint4* packed, int64_t* out, hipStream_t s) {
-    const uint32_t nt = i8_ntiles(traits);
-    if (nt <= 1) {
-        const uint32_t blocks = (h + 4 * 64 - 1) / (4 * 64);
-        hipLaunchKernelGGL((k_traits_i8<4, 1>), dim3(blocks), dim3(256), 0, s, rows, h, p_words,
-                           traits, packed, out);
-    } else if (nt <= 2) {
-        const uint32_t blocks = (h + 4 * 32 - 1) / (4 * 32);
-        hipLaunchKernelGGL((k_traits_i8<2, 2>), dim3(blocks), dim3(256), 0, s, rows, h, p_words,
-                           traits, packed, out);
-    } else if (nt <= 4) {  // four row tiles per wave, as the pipeline's 16-trait kernel
-        const uint32_t blocks = (h + 4 * 64 - 1) / (4 * 64);
-        hipLaunchKernelGGL((k_traits_i8<4, 4>), dim3(blocks), dim3(256), 0, s, rows, h, p_words,
-                           traits, packed, out);
-    } else {
-        const uint32_t blocks = (h + 4 * 16 - 1) / (4 * 16);
-        hipLaunchKernelGGL((k_traits_i8<1, 8>), dim3(blocks), dim3(256), 0, s, rows, h, p_words,
-                           traits, packed, out);
-    }
+size_t trait_piece_elems(uint32_t traits, uint32_t h, uint32_t w_cap, uint32_t round) {
+    // a launch cuts fewer than `round` row blocks into units, and no more
+    // blocks than units write pieces
+    const uint32_t rows = f6::balanced_block_rows(f6::trait_class(traits));
+    const uint64_t ng = std::max<uint32_t>(1, (w_cap + kGroupWords - 1) / kGroupWords);
+    const uint64_t rb = std::min<uint64_t>(round, (h + rows - 1) / rows);
+    return f6::piece_elems(traits, (uint32_t)std::min<uint64_t>(round, std::max<uint64_t>(1, rb * ng)));
+}
+
+namespace {
+typedef void (*ExactKernel)(const uint64_t*, uint32_t, uint32_t, uint32_t, uint32_t, const uint4*, int64_t*,
+                            int64_t*, uint32_t);
+ExactKernel exact_kernel(uint32_t traits) {
+    const ExactKernel kernels[f6::kClasses] = {k_traits_exact<0>, k_traits_exact<1>, k_traits_exact<2>,
+                                               k_traits_exact<3>, k_traits_exact<4>};
+    return kernels[f6::trait_class(traits)];
+}
+}  // namespace
+
+uint32_t exact_round(uint32_t traits) {
+    int device = 0, cus = 0, per_cu = 0;
+    if (hipGetDevice(&device) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(
+            &per_cu, reinterpret_cast<const void*>(exact_kernel(traits)), 256, 0) != hipSuccess)
+        return 0;
+    return (uint32_t)std::max(1, cus) * (uint32_t)std::max(1, per_cu);
+}
+
+// The balanced launch needs a second one for the pieces, about 4 us: taken when
+// cutting the last round's R row blocks saves its blocks at least eight groups
+// (about 0.5 us each in a launch that does not fill the chip, more in one that
+// does); else one row block per block.  Measured: 32,584 rows of 5 groups x 4
+// traits 19.9 us direct, 25.4 us cut; 3,824 rows of 12 groups x 7 traits 21.7 us
+// cut (30.1 us with the direct int8 kernel it replaced), 539 rows of 60 groups
+// x 2 traits 20.6 us cut (167 us).
+hipError_t launch_traits_exact(const uint64_t* rows, uint32_t h, uint32_t words, uint32_t most,
+                               uint32_t traits, const uint4* packed, int64_t* out, int64_t* part,
+                               uint32_t blocks, hipStream_t s) {
+    const uint32_t block_rows = f6::balanced_block_rows(f6::trait_class(traits));
+    const f6::Balance bal(h, block_rows, blocks);
+    const uint32_t ng = (words + kGroupWords - 1) / kGroupWords;
+    const uint64_t saved = bal.R && ng ? ng - bal.units(ng) / bal.sharing(ng) : 0;
+    const bool cut = saved >= 8;
+    hipLaunchKernelGGL(exact_kernel(traits), dim3(cut ? blocks : bal.RB), dim3(256), 0, s, rows, h,
+                       words, most, traits, packed, out, part, cut ? blocks : 0u);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess || !cut) return e;
+    const uint64_t n = (uint64_t)(h - bal.full * blocks * block_rows) * traits;
+    hipLaunchKernelGGL(k_exact_reduce, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, s, h, words,
+                       traits, blocks, part, out);
     return hipGetLastError();
 }
 

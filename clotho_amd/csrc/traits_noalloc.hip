@@ -2,57 +2,63 @@
 // allocate device memory (code under HIP graph capture, serving loops,
 // harnesses that forbid hipMalloc).  No counterpart in the reference.
 //
-// The effect digit planes the int8 MFMA path multiplies by (and the two
-// width words its kernels read from device memory) live in `scratch`, a
-// file-scope device array of fixed size.  Each GPU holds its own copy until
-// the process ends; host code reaches it only through the address
-// hipGetSymbolAddress returns for the current device (the array's name on
-// the host is a stand-in, not a device address).  Every call on one GPU
-// shares that GPU's array: calls that overlap on one GPU race, and a call
-// overwrites everything of the previous call that it reads (the width words
-// and every plane its traits kernel multiplies by), so nothing needs to be
-// cleared between calls.
+// The effect digit planes the exact MFMA path multiplies by and the partial
+// sums of the row blocks it cuts along the sites live in `scratch`, a file-scope
+// device array of fixed size.  Each GPU holds its own copy until the process
+// ends; host code reaches it only through the address hipGetSymbolAddress
+// returns for the current device (the array's name on the host is a stand-in,
+// not a device address).  Every call on one GPU shares that GPU's array: calls
+// that overlap on one GPU race, and a call overwrites everything of the
+// previous call that it reads (every plane it multiplies by and every piece it
+// sums), so nothing needs to be cleared between calls.
 #include <hip/hip_runtime.h>
 
 #include <mutex>
 
 #include "../../include/clotho_amd.h"
+#include "pipeline.hpp"
 #include "traits.hpp"
+#include "traits_f6.hpp"
 
 namespace clotho {
 namespace {
 
-constexpr size_t kDimsBytes = 256;  // {words, sites}, padded to the planes' alignment
 constexpr size_t kPlanesBytes =
-    (size_t)((CLOTHO_NOALLOC_MAX_TRAITS + 3) / 4) * (CLOTHO_NOALLOC_MAX_SITES / 64 / 16) * 16 * 64 *
+    (size_t)f6::kernel_tiles(CLOTHO_NOALLOC_MAX_TRAITS, f6::kMaxPlanes) *
+    (CLOTHO_NOALLOC_MAX_SITES / 64 / f6::kGroupWords) * f6::kGroupBlocks * f6::kFragVecs *
     sizeof(uint4);
-constexpr size_t kScratchBytes = kDimsBytes + kPlanesBytes;
+// pieces of the row blocks a launch cuts along K (512 blocks at 16 traits)
+constexpr size_t kPiecesBytes = (size_t)33554432;
+constexpr size_t kScratchBytes = kPlanesBytes + kPiecesBytes;
 static_assert(kScratchBytes == CLOTHO_NOALLOC_SCRATCH_BYTES, "scratch size as declared");
 
 __device__ __align__(256) uint8_t scratch[kScratchBytes];
 
 constexpr int kMaxDevices = 64;
 std::mutex g_lock;
-uint8_t* g_scratch[kMaxDevices] = {};
+struct DeviceEntry {
+    uint8_t* scratch = nullptr;
+    uint32_t round[f6::kClasses] = {};  // resident blocks of each trait class's kernel
+};
+DeviceEntry g_devices[kMaxDevices];
 
-// the device address of `scratch` on `device` (current), looked up once
-int scratch_of(int device, uint8_t** out) {
+// the device address of `scratch` on `device` (current) and the resident
+// round of the kernel for `traits`, each looked up once
+int entry_of(int device, uint32_t traits, uint8_t** out, uint32_t* round) {
     std::lock_guard<std::mutex> guard(g_lock);
-    if (!g_scratch[device]) {
+    DeviceEntry& e = g_devices[device];
+    if (!e.scratch) {
         void* p = nullptr;
         if (hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)) != hipSuccess || !p)
             return CLOTHO_ERR_HIP;
-        g_scratch[device] = static_cast<uint8_t*>(p);
+        e.scratch = static_cast<uint8_t*>(p);
     }
-    *out = g_scratch[device];
+    uint32_t& r = e.round[f6::trait_class(traits)];
+    if (!r) r = exact_round(traits);
+    if (!r) return CLOTHO_ERR_HIP;
+    *out = e.scratch;
+    *round = r;
     return CLOTHO_OK;
-}
-
-__global__ void k_set_dims(uint32_t* dims, uint32_t words, uint32_t sites) {
-    if (threadIdx.x == 0) {
-        dims[0] = words;
-        dims[1] = sites;
-    }
 }
 
 }  // namespace
@@ -74,16 +80,20 @@ extern "C" int clotho_trait_contract_exact_noalloc(const uint64_t* rows, uint32_
     if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= kMaxDevices)
         return CLOTHO_ERR_HIP;
     uint8_t* base = nullptr;
-    const int rc = scratch_of(device, &base);
+    uint32_t blocks = 0;
+    const int rc = entry_of(device, traits, &base, &blocks);
     if (rc != CLOTHO_OK) return rc;
-    uint32_t* dims = reinterpret_cast<uint32_t*>(base);
-    uint4* planes = reinterpret_cast<uint4*>(base + kDimsBytes);
+    const size_t fit = kPiecesBytes / (sizeof(int64_t) * f6::piece_elems(traits, 1));
+    if (blocks > fit) blocks = (uint32_t)fit;
+    uint4* planes = reinterpret_cast<uint4*>(base);
+    int64_t* pieces = reinterpret_cast<int64_t*>(base + kPlanesBytes);
     const hipStream_t s = static_cast<hipStream_t>(stream);
-    hipLaunchKernelGGL(k_set_dims, dim3(1), dim3(64), 0, s, dims, words, sites);
-    if (hipGetLastError() != hipSuccess) return CLOTHO_ERR_HIP;
-    if (launch_pack_i8(effects, traits, dims, dims + 1, words, planes, s) != hipSuccess)
+    // the effects are not read before they are packed: their bound is the API's
+    const uint32_t most = (uint32_t)kEffectLimit;
+    if (launch_pack_digits(effects, traits, words, sites, most, planes, s) != hipSuccess)
         return CLOTHO_ERR_HIP;
-    if (launch_traits_i8(rows, haplotypes, dims, traits, planes, sums, s) != hipSuccess)
+    if (launch_traits_exact(rows, haplotypes, words, most, traits, planes, sums, pieces, blocks, s) !=
+        hipSuccess)
         return CLOTHO_ERR_HIP;
     return CLOTHO_OK;
 }

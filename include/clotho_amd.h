@@ -81,8 +81,8 @@ extern "C" {
 #define CLOTHO_TRAITS_EXACT_FP64 2 /* set-bit walk, FP64 sums                          */
 #define CLOTHO_TRAITS_WALK_FP32 3  /* set-bit walk, FP32 sums                          */
 #define CLOTHO_TRAITS_EXACT_I8 4   /* the pipeline's exact path: effects quantised to   */
-                                   /* k 2^-q (largest q with |k| < 2^30), int8 digit    */
-                                   /* planes on int8 MFMA, exact int64 sums x 2^-q      */
+                                   /* k 2^-q (largest q with |k| < 2^30), FP6 digit     */
+                                   /* planes on FP4 x FP6 MFMA, exact int64 sums x 2^-q */
 
 typedef struct clotho_config {
     uint64_t seed;            /* random_number.seed (Philox key)                         */
@@ -388,13 +388,13 @@ int clotho_trait_contract(const uint64_t* rows, uint32_t haplotypes, uint32_t wo
 /* ---- exact trait contraction without allocation ------------------------ */
 /* No counterpart in the reference.  For callers that cannot allocate device
  * memory (code under HIP graph capture, serving loops, harnesses that forbid
- * hipMalloc): clotho_trait_contract's exact int8 path over caller-owned
+ * hipMalloc): clotho_trait_contract's exact path over caller-owned
  * device buffers, enqueued on `stream` (a hipStream_t; NULL is the default
  * stream) and not waited for.  rows[haplotypes][words] (words a multiple of
  * 8), quantised effects k[sites][traits] (int32, |k| <= 2^30 - 1; the effect
  * is k 2^q for the caller's q) and the output sums[haplotypes][traits]
  * (int64, the exact sum of k over each row's set bits below `sites`) are
- * device pointers.  The effect digit planes live in a fixed device array of
+ * device pointers.  The effect digit planes and partial sums live in a fixed device array of
  * CLOTHO_NOALLOC_SCRATCH_BYTES on each GPU the library runs on, held until
  * the process ends and shared by every call on that GPU: calls that overlap
  * on one GPU race.  words * 64 up to CLOTHO_NOALLOC_MAX_SITES and traits up
@@ -403,7 +403,7 @@ int clotho_trait_contract(const uint64_t* rows, uint32_t haplotypes, uint32_t wo
  * hipFree or allocating routine. */
 #define CLOTHO_NOALLOC_MAX_SITES 131072
 #define CLOTHO_NOALLOC_MAX_TRAITS 16
-#define CLOTHO_NOALLOC_SCRATCH_BYTES (256 + 8388608)
+#define CLOTHO_NOALLOC_SCRATCH_BYTES (11010048 + 33554432)
 int clotho_trait_contract_exact_noalloc(const uint64_t* rows, uint32_t haplotypes,
                                         uint32_t words, const int32_t* effects, uint32_t sites,
                                         uint32_t traits, int64_t* sums, void* stream);
