@@ -66,7 +66,9 @@ int sync_views(clotho_batch* b) {
         // batched recombination blocks take kBatchChunkDiv times the rows of
         // a replicate's own launch: the replicates supply the parallelism,
         // and every block pays a fixed set-up (offset search, tables, partials)
-        v[r].P.chunks = std::max<uint32_t>(1, (v[r].P.chunks + kBatchChunkDiv - 1) / kBatchChunkDiv);
+        v[r].P.chunks = batch_chunks(v[r].P);
+        v[r].P.free_words = 64;
+        v[r].P.word_blocks = (v[r].P.w_cap + 63) / 64;
     }
     if (b->d_views && b->host_views.size() == R &&
         std::memcmp(v.data(), b->host_views.data(), sizeof(RepView) * R) == 0)

@@ -270,7 +270,7 @@ int clotho_create(const clotho_config* cfg, int device, clotho_ctx** out) {
     if (hipGetDeviceProperties(&c->prop, device) != hipSuccess) return bail(CLOTHO_ERR_HIP);
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess)
         return bail(CLOTHO_ERR_HIP);
-    if (query_trait_residency(c) != hipSuccess) return bail(CLOTHO_ERR_HIP);
+    if (query_residency(c) != hipSuccess) return bail(CLOTHO_ERR_HIP);
 
     Params& P = c->p;
     std::memset(&P, 0, sizeof(P));
@@ -298,17 +298,17 @@ int clotho_create(const clotho_config* cfg, int device, clotho_ctx** out) {
     set_fitness_constants(P, *cfg);
     P.tiles = (P.w_cap + 63) / 64;
     {
-        // default launch shape: ~4096 recombination blocks, but at least ~32
-        // rows per wave (a block's order-statistic tables are loaded once per
-        // block); clotho_autotune may pick another row-chunk count up to max_chunks
+        // clotho_autotune may pick another number of row chunks up to max_chunks
+        const uint32_t groups = (h_cap + 63) / 64;
         P.max_chunks = std::max<uint32_t>(1, std::min<uint32_t>(
                                                  (8192 + P.tiles - 1) / P.tiles, h_cap / 8));
-        uint32_t ch = (4096 + P.tiles - 1) / P.tiles;
-        ch = std::min<uint32_t>(ch, std::max<uint32_t>(1, (P.h + 511) / 512));
-        P.chunks = std::min<uint32_t>(P.max_chunks, std::max<uint32_t>(1, ch));
+        P.max_chunks = std::max(P.max_chunks, std::min(groups, 2 * c->recombine_round));
+        P.chunks = recombine_chunks(c, P.h);
+        P.splits = recombine_splits(c, P.chunks);
     }
     P.mut_blocks = (P.h + kScanBlock - 1) / kScanBlock;
-    P.word_blocks = (P.w_cap + 63) / 64;  // 64-word free-space blocks
+    P.free_words = 16;
+    P.word_blocks = (P.w_cap + P.free_words - 1) / P.free_words;
     const uint32_t sel_blocks = (P.n_cap + kScanBlock - 1) / kScanBlock;  // at capacity
     const uint32_t mut_blocks_cap = (h_cap + kScanBlock - 1) / kScanBlock;
     const uint32_t T1 = std::max<uint32_t>(1, P.traits);
@@ -344,7 +344,7 @@ int clotho_create(const clotho_config* cfg, int device, clotho_ctx** out) {
     rc |= dalloc(c, &B.prank, h_cap);
     rc |= dalloc(c, &B.given_parents, h_cap);
     rc |= dalloc(c, &B.var_part, (size_t)(P.max_chunks + 1) * P.w_cap);
-    rc |= dalloc(c, &B.fix_part, (size_t)P.max_chunks * P.w_cap);
+    rc |= dalloc(c, &B.fix_part, (size_t)(P.max_chunks + 1) * P.w_cap);
     rc |= dalloc(c, &B.word_cnt, P.w_cap);
     rc |= dalloc(c, &B.word_bsum, 2 * P.word_blocks);
     rc |= dalloc(c, &B.cum_local, P.n_cap);
@@ -1158,8 +1158,8 @@ int clotho_generation(clotho_ctx* c) { return clotho_run(c, 1, 0); }
 // row-chunk counts and keeps the fastest.  It replays the last generation's
 // gametes (parents, events, mutation counts; zeros before the first
 // generation) against the resident population and writes only buffers the
-// next generation rewrites: the spare row buffer, the column partials and the
-// per-word order statistics.  Visible state is unchanged.
+// next generation rewrites: the spare row buffer and the column partials.
+// Visible state is unchanged.
 int clotho_autotune(clotho_ctx* c, uint32_t* chosen_chunks) {
     if (!c) return CLOTHO_ERR_ARG;
     HIP_TRY(c, hipSetDevice(c->device));
@@ -1176,12 +1176,12 @@ int clotho_autotune(clotho_ctx* c, uint32_t* chosen_chunks) {
         cand.push_back(std::max<uint32_t>(1, base / f));
         cand.push_back(std::min<uint32_t>(c->p.max_chunks, base * f));
     }
-    // grids that fill whole waves of resident blocks (two per CU)
-    const uint32_t resident = 2u * (uint32_t)std::max(1, c->prop.multiProcessorCount);
-    for (uint32_t k = 1; k <= 16; ++k) {
-        const uint32_t ch = (k * resident) / std::max<uint32_t>(1, c->p.tiles);
-        if (ch >= 1 && ch <= c->p.max_chunks) cand.push_back(ch);
-    }
+    // whole groups of 64 gametes per chunk, and rounds of resident blocks
+    const uint32_t groups = (c->p.h + 63) / 64;
+    for (uint32_t k = 1; k <= 8; ++k)
+        cand.push_back(std::min<uint32_t>(c->p.max_chunks, (groups + k - 1) / k));
+    for (uint32_t k : {1u, 2u})
+        cand.push_back(std::min<uint32_t>(c->p.max_chunks, k * c->recombine_round));
     std::sort(cand.begin(), cand.end());
     cand.erase(std::unique(cand.begin(), cand.end()), cand.end());
     // Each timed recombination is followed by the traits pass over its output,
@@ -1193,7 +1193,6 @@ int clotho_autotune(clotho_ctx* c, uint32_t* chosen_chunks) {
     hipEvent_t ev[2 * kReps] = {};
     for (hipEvent_t& e : ev) HIP_TRY(c, events.add(&e));
     int reps = kReps, passes = 2;
-    HIP_TRY(c, launch_word_sort(c));  // order statistics of the resident columns
     {
         HIP_TRY(c, launch_recombine(c));
         HIP_TRY(c, hipEventRecord(ev[0], c->stream));
@@ -1208,6 +1207,7 @@ int clotho_autotune(clotho_ctx* c, uint32_t* chosen_chunks) {
     for (int pass = 0; pass < passes; ++pass) {
         for (size_t i = 0; i < cand.size(); ++i) {
             c->p.chunks = cand[i];
+            c->p.splits = recombine_splits(c, cand[i]);
             HIP_TRY(c, launch_recombine(c));  // warm-up
             HIP_TRY(c, launch_traits(c));
             for (int r = 0; r < reps; ++r) {
@@ -1235,6 +1235,7 @@ int clotho_autotune(clotho_ctx* c, uint32_t* chosen_chunks) {
         }
     }
     c->p.chunks = best_chunks;
+    c->p.splits = recombine_splits(c, best_chunks);
 
     // The traits pass: every kernel shape over the current population (the
     // pass writes the traits it already holds), fastest of two passes.
@@ -1311,6 +1312,7 @@ int clotho_set_launch_shape(clotho_ctx* c, const clotho_launch_shape* in) {
                         ", traits shape 1.." + std::to_string(nv) +
                         ", compaction rows 4/8/16, compaction tile words 48/56/60/64");
     c->p.chunks = in->recombine_chunks;
+    c->p.splits = recombine_splits(c, in->recombine_chunks);
     c->trait_variant = in->traits_variant;
     c->compact_rows = in->compact_rows;
     c->compact_chunks = in->compact_chunks;  // 0: the default

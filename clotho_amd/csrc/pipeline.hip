@@ -17,6 +17,7 @@
 #include "device_common.hpp"
 #include "pipeline.hpp"
 #include "traits.hpp"
+#include "recombine.hpp"
 #include "traits_f6.hpp"
 
 namespace clotho {
@@ -589,13 +590,17 @@ struct ParentScatterOp {
 };
 
 // ---------------------------------------------------------------------------
-// Recombination + mutation (+ free-space partials)
+// Recombination + mutation (+ free-space partials) of replicate batches; a single
+// population takes rec::Recombine.  The batch keeps a lookup per event and row:
+// its rows are mostly narrow (8 to 32 words), and rec's group tables cost as much
+// as a few hundred words of rows.
 // ---------------------------------------------------------------------------
 // Per-word order statistics, once per generation: the 64 position keys of
 // word w sorted ascending (sorted[w][k]), prefix masks pm[w][c] = bits of the
 // c smallest keys, and a 256-bucket table bucket[w][b] = #{k : key_k < b<<24}
-// (four buckets per dword), each stored tile-major (table_at, prefix_at).  For a gamete event e, c(e) = #{k : key_k < e}
-// is bucket[e>>24] plus the few keys of that bucket below e, and
+// (four buckets per dword), each stored tile-major (table_at, prefix_at).  For
+// a gamete event e, c(e) = #{k : key_k < e} is bucket[e>>24] plus the few keys
+// of that bucket below e, and
 // {j in w : key_j >= e} = ~pm[w][c(e)]; the crossover mask of the word,
 // {j : odd #{events e <= key_j}} (block_crossover + region_classifier's
 // upper_bound), is the XOR over events of ~pm[w][c(e)].
@@ -659,18 +664,14 @@ struct WordSort {
 //   child = (t & ~mask) | (b & mask), then XOR of this row's new mutations
 // OR/AND of the child words accumulate in registers (free_space_accumulator).
 //
-// Latency structure: with parent-ordered gamete records a wave owns a
-// contiguous segment of positions (without them, positions c0 + wave +
-// kRecWaves j).  The records of 64 positions (child row, top row, event and
-// mutation counts, mutation offset) are loaded with one vector load, lane q
-// holding position j0 + q, and read back with v_readlane, so the row loop
-// issues no scalar loads.  Runs of positions with one parent individual are
-// cut into items of at most kSibs children: an item loads the parent pair
-// once and the event keys of each child (lane e holds key e).  Items
-// alternate between two register sets: the loads of item k + 2 are issued as
-// soon as item k is done and stay in flight while item k + 1 is classified
-// (no register rotation, hence no wait on loads still in flight; three or
-// four sets measured no faster on the same device).  Events are classified
+// Latency structure: the records of 64 rows (top row, event and mutation
+// counts, mutation offset) are loaded with one vector load per field, lane q
+// holding row q, and read back with v_readlane, so the row loop issues no
+// scalar loads.  Rows alternate between two register sets of parent words and
+// event keys (lane e holds key e): the loads of row k + 2 are issued as soon as
+// row k is done and stay in flight while row k + 1 is classified (no register
+// rotation, hence no wait on loads still in flight; three or four sets
+// measured no faster on the same device).  Events are classified
 // kEventGroup at a time so that their LDS lookups overlap; a group is padded
 // with rank-64 entries (pm[64] is all ones), and since #real + #padding =
 // kEventGroup is even, the XOR of the group's prefix masks equals the XOR of
@@ -680,9 +681,6 @@ constexpr int kRecBlock = 64 * kRecWaves;
 // events classified together; any even size keeps the padding parity
 // argument (#real + #padding even), and 2 pads Poisson(5) counts least
 constexpr int kEventGroup = 2;
-// children of one parent individual produced from one load of its row pair
-// (parent-ordered gametes; the batched launches keep child order and take 1)
-constexpr int kSibsOrdered = 3;
 // dword 3 of a raw (stride 0) buffer resource on gfx9-family parts: 32-bit
 // data format, offsets range-checked against num_records in bytes
 constexpr int kBufferWord3 = 0x00020000;
@@ -958,7 +956,7 @@ __device__ __forceinline__ void recombine_folded(const Params& P, const Buffers&
     }
 }
 
-template <bool kWideEvents, int kSibs>
+template <bool kWideEvents>
 struct Recombine {
     static constexpr int kThreads = kRecBlock;
     __host__ __device__ static uint32_t blocks(const Params& P) { return P.tiles * P.chunks; }
@@ -978,8 +976,6 @@ struct Recombine {
         const auto boff = gbl(B.mut_bsum);
         const auto var_part = gbl(B.var_part);
         const auto fix_part = gbl(B.fix_part);
-        const auto by_parent = (const __attribute__((address_space(1))) f6::u32x4*)B.by_parent;
-        const bool ordered = B.by_parent != nullptr;
         const uint32_t bx = blk % P.tiles, by = blk / P.tiles;
         __shared__ __align__(16) uint32_t s_bucket[64 * 64];
         __shared__ __align__(16) uint32_t s_sorted[68 * 64];
@@ -988,7 +984,7 @@ struct Recombine {
         const uint32_t wc = uniform_read(&st->wc);
         const uint32_t w0 = bx * 64;
         if (w0 >= wc) return;  // uniform for the block
-        if constexpr (kSibs == 1 && !kWideEvents) {
+        if constexpr (!kWideEvents) {
             // narrow rows: several rows per wave (tile 0 is the only live tile)
             if (wc <= 32)
                 return recombine_folded(P, B, sel, by, wc <= 8 ? 3u : wc <= 16 ? 4u : 5u, s_bucket,
@@ -1009,104 +1005,52 @@ struct Recombine {
         const uint64_t keep = inpar ? ~fixed_bits[w] : 0;  // also clears columns >= wp
         __syncthreads();
 
-        // positions [c0, c1) of this row chunk.  With sibling items a wave
-        // takes the contiguous segment [s0, s1), so the children of one parent
-        // meet in one wave; without, the waves interleave (wave w takes
-        // c0 + w + 16 k), so a block writes consecutive child rows together.
+        // rows [c0, c1) of this chunk, interleaved over the waves (wave w takes
+        // c0 + w + 16 k), so a block writes consecutive child rows together
         const uint32_t rows_per_chunk = (P.h + P.chunks - 1) / P.chunks;
         const uint32_t c0 = min(P.h, by * rows_per_chunk);
         const uint32_t c1 = min(P.h, c0 + rows_per_chunk);
-        uint32_t first, stride, npos;
-        if (kSibs > 1) {
-            const uint32_t seg = (c1 - c0 + kRecWaves - 1) / kRecWaves;
-            first = min(c1, c0 + wave * seg);
-            stride = 1;
-            npos = min(c1, first + seg) - first;
-        } else {
-            first = c0 + wave;
-            stride = kRecWaves;
-            npos = c1 > first ? (c1 - first + kRecWaves - 1) / kRecWaves : 0;
-        }
+        const uint32_t first = c0 + wave;
+        const uint32_t npos = c1 > first ? (c1 - first + kRecWaves - 1) / kRecWaves : 0;
         uint64_t acc_or = 0, acc_and = ~(uint64_t)0;
 
         for (uint32_t j0 = 0; j0 < npos; j0 += 64) {
             const uint32_t nb = min(64u, npos - j0);
             // gamete record of position j0 + lane (the last one repeated past
-            // the batch): child row, top row (bottom = top ^ 1), events |
-            // mutations << 8, first mutation
-            const uint32_t pos = first + stride * (j0 + min(lane, nb - 1));
-            uint32_t g_row, g_top, g_nx, g_k0;
-            if (ordered) {
-                const f6::u32x4 r = by_parent[pos];
-                g_row = r.x;
-                g_top = r.y;
-                g_nx = r.z;
-                g_k0 = r.w;
-            } else {
-                g_row = pos;
-                g_top = top_in[pos];
-                g_nx = nev_in[pos] | (count[pos] << 8);
-                g_k0 = local[pos] + boff[pos / kBlock];
-            }
-            // items: runs of at most kSibs consecutive positions whose gametes
-            // share the parent individual; one item loads the parent pair once
-            uint64_t items = 0;
-            if (kSibs > 1) {
-                const uint32_t parent_id = g_top >> 1;
-                const uint32_t prev_id = __shfl_up(parent_id, 1, 64);
-                const uint64_t starts = __ballot(lane == 0 || lane >= nb || parent_id != prev_id);
-                const uint64_t upto = lane == 63 ? ~(uint64_t)0 : (((uint64_t)2 << lane) - 1);
-                const uint32_t run0 = 63u - (uint32_t)__builtin_clzll(starts & upto);
-                items = __ballot(lane < nb && (lane - run0) % kSibs == 0);
-            }
-            uint32_t next_q = 0;  // kSibs == 1: every position is an item
+            // the batch): top row (bottom = top ^ 1), events | mutations << 8,
+            // first mutation
+            const uint32_t row0 = first + kRecWaves * j0;
+            const uint32_t pos = row0 + kRecWaves * min(lane, nb - 1);
+            const uint32_t g_top = top_in[pos];
+            const uint32_t g_nx = nev_in[pos] | (count[pos] << 8);
+            const uint32_t g_k0 = local[pos] + boff[pos / kBlock];
             struct Item {
-                uint32_t q, len;  // first position (lane) and number of children
-                uint64_t t, b;    // parent rows top-of-first-child and its partner
-                uint32_t lo[kSibs], hi[kSibs];
+                uint64_t t, b;  // the row's words of its parent pair
+                uint32_t lo, hi;
             };
-            auto next_item = [&](Item& it) {
-                if (kSibs == 1) {
-                    it.q = next_q < nb ? next_q++ : 64u;
-                    it.len = 1;
-                } else if (items) {
-                    it.q = (uint32_t)__builtin_ctzll(items);
-                    items &= items - 1;
-                    it.len = (items ? (uint32_t)__builtin_ctzll(items) : nb) - it.q;
-                } else {
-                    it.q = 64;
-                    it.len = 0;
-                }
-            };
-            // loads of an item (issued for every item slot, indices clamped in bounds)
-            auto load_item = [&](Item& it) {
-                const uint32_t qq = min(it.q, nb - 1);
+            // loads of row q (clamped: issued for every item slot)
+            auto load_item = [&](uint32_t q, Item& it) {
+                const uint32_t qq = min(q, nb - 1);
                 const uint32_t top = lane_read(g_top, qq);
                 it.t = parent[(size_t)top * wp + col];
                 it.b = parent[(size_t)(top ^ 1u) * wp + col];
-#pragma unroll
-                for (int k = 0; k < kSibs; ++k) {
-                    const auto ev = events + (size_t)lane_read(g_row, min(qq + k, nb - 1)) * ev_cap;
-                    it.lo[k] = ev[min(lane, ev_cap - 1)];
-                    if (kWideEvents) it.hi[k] = ev[min(lane + 64, ev_cap - 1)];
-                }
+                const auto ev = events + (size_t)(row0 + kRecWaves * qq) * ev_cap;
+                it.lo = ev[min(lane, ev_cap - 1)];
+                if (kWideEvents) it.hi = ev[min(lane + 64, ev_cap - 1)];
             };
 
-            // A child whose top row is the item's bottom row takes the
-            // complemented mask: (b & ~m) | (t & m) = (t & ~~m) | (b & ~m).
-            auto child_row = [&](uint32_t q, uint64_t t, uint64_t b, uint32_t lo, uint32_t hi,
-                                 bool flip) {
+            auto child_row = [&](uint32_t q, const Item& it) {
                 const uint32_t nx = lane_read(g_nx, q);
                 const uint32_t ne = nx & 0xFFu;
-                uint64_t m = flip ? ~(uint64_t)0 : 0;
+                uint64_t m = 0;
                 for (uint32_t e = 0; e < ne; e += kEventGroup) {
                     uint32_t key[kEventGroup], p[kEventGroup];
                     bool more[kEventGroup];
 #pragma unroll
                     for (int i = 0; i < kEventGroup; ++i) {
                         const uint32_t x = e + i;
-                        const uint32_t a = lane_read(lo, x & 63);
-                        key[i] = (kWideEvents && x >= 64) ? lane_read(hi, x & 63) : a;
+                        const uint32_t a = lane_read(it.lo, x & 63);
+                        key[i] = (kWideEvents && x >= 64) ? lane_read(it.hi, x & 63) : a;
                     }
                     // byte (key >> 24) & 3 of dword [key >> 26][lane]: one byte read
                     const uint8_t* sb = reinterpret_cast<const uint8_t*>(s_bucket);
@@ -1140,7 +1084,7 @@ struct Recombine {
                     m ^= xm;
                 }
                 // keep clears fixed columns and columns past the parent width in both
-                uint64_t c = ((t & ~m) | (b & m)) & keep;
+                uint64_t c = ((it.t & ~m) | (it.b & m)) & keep;
                 // new mutations of this row (free columns: zero in every parent row)
                 const uint32_t nm = nx >> 8;
                 if (nm) {
@@ -1155,7 +1099,7 @@ struct Recombine {
                     // reads the child rows next runs ~12% faster than after
                     // ordinary write-back stores
                     const __amdgpu_buffer_rsrc_t row = __builtin_amdgcn_make_buffer_rsrc(
-                        child + (size_t)lane_read(g_row, q) * wc, 0, (int)(wc * 8u), kBufferWord3);
+                        child + (size_t)(row0 + kRecWaves * q) * wc, 0, (int)(wc * 8u), kBufferWord3);
                     typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
                     const u32x2 v = {(uint32_t)c, (uint32_t)(c >> 32)};
                     __builtin_amdgcn_raw_buffer_store_b64(v, row, valid ? w * 8u : 0x80000000u, 0,
@@ -1165,32 +1109,15 @@ struct Recombine {
                 acc_and &= c;
             };
 
-            // each child takes the loaded pair in its own strand order
-            auto process_item = [&](const Item& it) {
-                const uint32_t top0 = lane_read(g_top, it.q);
-#pragma unroll
-                for (int k = 0; k < kSibs; ++k) {
-                    if ((uint32_t)k < it.len) {
-                        const uint32_t q = it.q + k;
-                        const bool flip = lane_read(g_top, q) != top0;
-                        child_row(q, it.t, it.b, it.lo[k], kWideEvents ? it.hi[k] : 0u, flip);
-                    }
-                }
-            };
-
             Item iA, iB;
-            next_item(iA);
-            load_item(iA);
-            next_item(iB);
-            load_item(iB);
-            while (iA.q < 64) {
-                process_item(iA);
-                next_item(iA);
-                load_item(iA);
-                if (iB.q >= 64) break;
-                process_item(iB);
-                next_item(iB);
-                load_item(iB);
+            load_item(0, iA);
+            load_item(1, iB);
+            for (uint32_t q = 0; q < nb; q += 2) {
+                child_row(q, iA);
+                load_item(q + 2, iA);
+                if (q + 1 >= nb) break;
+                child_row(q + 1, iB);
+                load_item(q + 3, iB);
             }
         }
         __syncthreads();  // every wave is past its last prefix-mask read
@@ -1214,9 +1141,12 @@ struct Recombine {
 // ---------------------------------------------------------------------------
 // Free space: reduce chunk partials per word, classify, ordered compaction
 // ---------------------------------------------------------------------------
-// 64 words per block; the four waves fold interleaved chunk partials, then
-// wave 0 classifies its word and scans the per-word counts.
-constexpr uint32_t kFreeWords = 64;
+// P.free_words words per block (16 or 64): lane = word, the other threads fold
+// interleaved chunk partials, then the first wave classifies the words and scans
+// the per-word counts.  A single population takes 16: its reduction reads
+// 16 bytes per word and row chunk, which 64-word blocks leave to a dozen compute
+// units (768 chunks x 816 words: 31 -> 14 us).  A batch takes 64:
+// its replicates have few chunks each, and a block costs more than its reads.
 
 struct FreeReduce {
     static constexpr int kThreads = 1024;  // 16 waves share the chunk partials of 64 words
@@ -1237,14 +1167,20 @@ struct FreeReduce {
         __shared__ uint64_t s_or[kRWaves][64];
         __shared__ uint64_t s_and[kRWaves][64];
         const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-        const uint32_t w = blk * kFreeWords + lane;
+        const uint32_t fw = P.free_words;  // a power of two up to 64
+        const uint32_t w = blk * fw + (lane & (fw - 1));
         const uint32_t wc = st->wc, S = st->all_size;
         uint64_t vo = 0, va = ~(uint64_t)0;
         if (w < wc) {
-            for (uint32_t c = wave; c < chunks; c += kRWaves) {
+#pragma unroll 4
+            for (uint32_t c = threadIdx.x / fw; c < chunks; c += kThreads / fw) {
                 vo |= var_part[(size_t)c * P.w_cap + w];
                 va &= fix_part[(size_t)c * P.w_cap + w];
             }
+        }
+        for (uint32_t d = fw; d < 64; d <<= 1) {
+            vo |= (uint64_t)__shfl_xor((long long)vo, (int)d, 64);
+            va &= (uint64_t)__shfl_xor((long long)va, (int)d, 64);
         }
         s_or[wave][lane] = vo;
         s_and[wave][lane] = va;
@@ -1254,8 +1190,9 @@ struct FreeReduce {
             vo |= s_or[q][lane];
             va &= s_and[q][lane];
         }
+        const bool live = w < wc && lane < fw;
         uint32_t cf = 0, cl = 0;
-        if (w < wc) {
+        if (live) {
             const uint32_t lo = w * 64;
             uint64_t validm = 0;
             if (S > lo) validm = (S - lo >= 64) ? ~(uint64_t)0 : (((uint64_t)1 << (S - lo)) - 1);
@@ -1276,7 +1213,7 @@ struct FreeReduce {
                 xl += yl;
             }
         }
-        if (w < wc) word_cnt[w] = ((xf - cf) & 0xFFFFu) | ((xl - cl) << 16);
+        if (live) word_cnt[w] = ((xf - cf) & 0xFFFFu) | ((xl - cl) << 16);
         if (lane == 63) {
             word_bsum[blk] = xf;
             word_bsum[word_blocks + blk] = xl;
@@ -1300,15 +1237,17 @@ struct FreeCompact {
         __shared__ uint32_t s_off[2];
         __shared__ uint32_t s_red[2][kBlock];
         const uint32_t wc = st->wc;
-        const uint32_t nb = (wc + kFreeWords - 1) / kFreeWords;
+        const uint32_t fw = P.free_words;
+        const uint32_t nb = (wc + fw - 1) / fw;
         if (blk >= nb) return;
         // intermediate generation: the free list of the last analysis stays
         if (st->inter != P.inter_k) return;
-        // offsets of this block and the fixed total, from the block totals
-        uint32_t pf = 0, tfix = 0, pl = 0;
+        // offsets of this block and the totals, from the block totals
+        uint32_t pf = 0, tfix = 0, pl = 0, tlost = 0;
         for (uint32_t q = threadIdx.x; q < nb; q += kBlock) {
             const uint32_t a = word_bsum[q], l = word_bsum[word_blocks + q];
             tfix += a;
+            tlost += l;
             if (q < blk) {
                 pf += a;
                 pl += l;
@@ -1330,14 +1269,18 @@ struct FreeCompact {
         }
         __syncthreads();
         s_red[0][threadIdx.x] = tfix;
+        s_red[1][threadIdx.x] = tlost;
         __syncthreads();
         for (int s = kBlock / 2; s > 0; s >>= 1) {
-            if ((int)threadIdx.x < s) s_red[0][threadIdx.x] += s_red[0][threadIdx.x + s];
+            if ((int)threadIdx.x < s) {
+                s_red[0][threadIdx.x] += s_red[0][threadIdx.x + s];
+                s_red[1][threadIdx.x] += s_red[1][threadIdx.x + s];
+            }
             __syncthreads();
         }
         const uint32_t nfixed = s_red[0][0];
-        const uint32_t w = blk * kFreeWords + threadIdx.x;
-        if (threadIdx.x < kFreeWords && w < wc) {
+        const uint32_t w = blk * fw + threadIdx.x;
+        if (threadIdx.x < fw && w < wc) {
             const uint32_t wcnt = word_cnt[w];
             uint32_t pos = s_off[0] + (wcnt & 0xFFFFu);
             uint64_t fx = fixed_bits[w];
@@ -1353,10 +1296,8 @@ struct FreeCompact {
             }
         }
         if (blk == nb - 1 && threadIdx.x == 0) {
-            uint32_t tl = 0;
-            for (uint32_t q = 0; q < nb; ++q) tl += word_bsum[word_blocks + q];
             st->n_fixed = nfixed;
-            st->free_count = nfixed + tl;
+            st->free_count = nfixed + s_red[1][0];
         }
     }
 };
@@ -2210,9 +2151,13 @@ template <class Op>
 struct MinWaves {
     static constexpr int value = 1;
 };
-template <bool W, int K>
-struct MinWaves<Recombine<W, K>> {
+template <bool W>
+struct MinWaves<Recombine<W>> {
     static constexpr int value = 8;
+};
+template <>
+struct MinWaves<rec::Recombine> {
+    static constexpr int value = rec::kMinWaves;
 };
 template <int RT, int CLS, bool E>
 struct MinWaves<Traits<RT, CLS, E>> {
@@ -2231,20 +2176,17 @@ CLOTHO_SINGLE(k_sel_blockscan, SelBlockscan)
 CLOTHO_SINGLE(k_parent_blockscan, ParentBlockscan)
 using ParentScatter = ParentScatterOp<true>;
 CLOTHO_SINGLE(k_parent_scatter, ParentScatter)
-CLOTHO_SINGLE(k_word_sort, WordSort)
 // the draw phase of a single population: counts and fitness statistics, then
 // attributes and selection scan, then gametes and the per-word order
 // statistics, each pair in one launch
 using DrawCounts = Fused<MutCounts, FitnessStats>;
 using DrawAttrs = Fused<MutAttrs, SelScan>;
-using DrawGametes = Fused<GametesOp<kTotalsScan>, WordSort>;
+using DrawGametes = GametesOp<kTotalsScan>;
 CLOTHO_SINGLE(k_draw_counts, DrawCounts)
 CLOTHO_SINGLE(k_draw_attrs, DrawAttrs)
 CLOTHO_SINGLE(k_draw_gametes, DrawGametes)
-using RecombineNarrow = Recombine<false, kSibsOrdered>;  // at most 64 events per gamete
-using RecombineWide = Recombine<true, 2>;  // two sets of 128 event keys stay in registers
-using BatchRecombineNarrow = Recombine<false, 1>;
-using BatchRecombineWide = Recombine<true, 1>;
+using BatchRecombineNarrow = Recombine<false>;  // at most 64 events per gamete
+using BatchRecombineWide = Recombine<true>;
 // The recombination's blocks are numbered so that each XCD runs a contiguous
 // range of (row chunk, column tile) blocks, i.e. whole row chunks one tile
 // after another: the chunk's gamete records and event keys, which every tile
@@ -2257,8 +2199,7 @@ using BatchRecombineWide = Recombine<true, 1>;
         name(Params P, Buffers B, uint32_t sel) {                                               \
         Op::run(P, B, sel, xcd_contiguous(blockIdx.x, gridDim.x));                              \
     }
-CLOTHO_SINGLE_XCD(k_recombine, RecombineNarrow)
-CLOTHO_SINGLE_XCD(k_recombine_wide, RecombineWide)
+CLOTHO_SINGLE_XCD(k_recombine, rec::Recombine)
 #undef CLOTHO_SINGLE_XCD
 CLOTHO_SINGLE(k_pack_digits, PackDigits)
 // by trait class (f6::trait_class: T <= 2, 4, 8, 16, 32)
@@ -2321,8 +2262,8 @@ template <class Op>
 struct LiveBlocks {
     static constexpr int kind = -1;
 };
-template <bool W, int K>
-struct LiveBlocks<Recombine<W, K>> {
+template <bool W>
+struct LiveBlocks<Recombine<W>> {
     // live tiles lt = ceil(wc / 64) x row chunks: u -> tile u mod lt, chunk u / lt
     static constexpr int kind = kLiveRecombine;
     __host__ __device__ static uint32_t count(const Params& P, uint32_t wc) {
@@ -2364,8 +2305,8 @@ template <class Op>
 struct RoundRobin {
     static constexpr bool value = false;
 };
-template <bool W, int K>
-struct RoundRobin<Recombine<W, K>> {
+template <bool W>
+struct RoundRobin<Recombine<W>> {
     static constexpr bool value = true;
 };
 template <int RT, int CLS, bool E>
@@ -2413,7 +2354,7 @@ __global__ void __launch_bounds__(1024) k_batch_live_offsets(const RepView* __re
             if (r < R) {
                 const RepView& rv = views[r];
                 const uint32_t wc = gbl(rv.B.state)->wc;
-                n = kind == kLiveRecombine ? LiveBlocks<RecombineNarrow>::count(rv.P, wc)
+                n = kind == kLiveRecombine ? LiveBlocks<BatchRecombineNarrow>::count(rv.P, wc)
                     : kind == kLiveWordSort ? LiveBlocks<WordSort>::count(rv.P, wc)
                                             : LiveBlocks<PackDigits>::count(rv.P, wc);
             }
@@ -2537,7 +2478,6 @@ hipError_t launch_draw(clotho_ctx* c) {
     const bool scan_apart = parent_blocks(c->p) > kTotalsLds;
     if (scan_apart) TRY_LAUNCH(launch_single<SelBlockscan>(k_sel_blockscan, c, par));
     TRY_LAUNCH(launch_single<DrawGametes>(k_draw_gametes, c, par));
-    if (!c->b.by_parent) return launch_single<PackDigits>(k_pack_digits, c, par);
     TRY_LAUNCH(launch_single<DrawParents>(k_draw_parents, c, par));
     if (scan_apart) TRY_LAUNCH(launch_single<ParentBlockscan>(k_parent_blockscan, c, par));
     return launch_single<ParentScatter>(k_parent_scatter, c, par);
@@ -2585,27 +2525,44 @@ static hipError_t launch_whole_traits_of(clotho_ctx* c, int which, bool pack) {
 
 hipError_t launch_traits_current(clotho_ctx* c) { return launch_whole_traits_of(c, c->cur, true); }
 
-hipError_t query_trait_residency(clotho_ctx* c) {
+hipError_t query_residency(clotho_ctx* c) {
     void (*const kernels[f6::kClasses])(Params, Buffers, uint32_t) = {
         k_traits_t2, k_traits_t4, k_traits_t8, k_traits_t16, k_traits_t32};
+    const uint32_t cus = (uint32_t)std::max(1, c->prop.multiProcessorCount);
     int per_cu = 0;
-    const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
+    hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
         &per_cu, reinterpret_cast<const void*>(kernels[f6::trait_class(c->cfg.trait_count)]),
         Traits2Balanced::kThreads, 0);
     if (e != hipSuccess) return e;
-    c->trait_round =
-        (uint32_t)std::max(1, per_cu) * (uint32_t)std::max(1, c->prop.multiProcessorCount);
+    c->trait_round = (uint32_t)std::max(1, per_cu) * cus;
+    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
+        &per_cu, reinterpret_cast<const void*>(k_recombine), rec::Recombine::kThreads, 0);
+    if (e != hipSuccess) return e;
+    c->recombine_round = (uint32_t)std::max(1, per_cu) * cus;
     return hipSuccess;
 }
 
-hipError_t launch_word_sort(clotho_ctx* c) {
-    return launch_single<WordSort>(k_word_sort, c, (uint32_t)c->cur);
+// Row chunks of the recombination: as many as its groups of 64 gametes, up to
+// one round of resident blocks (N = 100,000, 816 words: 768 chunks 0.539 ms,
+// 512 0.591, 1536 0.563; more chunks also make more column partials).
+uint32_t recombine_chunks(const clotho_ctx* c, uint32_t h) {
+    const uint32_t groups = (h + rec::kGroup - 1) / rec::kGroup;
+    return std::max<uint32_t>(1, std::min(groups, c->recombine_round));
+}
+
+// Column ranges: enough for one resident round where the row chunks are fewer,
+// down to a tile per wave (N = 1000, 496 words, 32 chunks: 8 ranges 16 us, 4 21
+// us).  Two from 2048 words on: finer blocks even out the last groups, and
+// the tables that each range builds weigh less there (N = 250,000, 2072 words: 3.80
+// -> 3.69 ms; 816 words: 0.539 -> 0.57 ms).
+uint32_t recombine_splits(const clotho_ctx* c, uint32_t chunks) {
+    const uint32_t turns = (c->p.w_cap + rec::kTile * rec::kWaves - 1) / (rec::kTile * rec::kWaves);
+    const uint32_t fill = c->recombine_round / std::max<uint32_t>(1, chunks);
+    return std::max<uint32_t>(1, std::min(turns, std::max(fill, turns >= 32 ? 2u : 1u)));
 }
 
 hipError_t launch_recombine(clotho_ctx* c) {
-    const uint32_t par = (uint32_t)c->cur;
-    if (c->p.ev_cap > 64) return launch_single<RecombineWide>(k_recombine_wide, c, par);
-    return launch_single<RecombineNarrow>(k_recombine, c, par);
+    return launch_single<rec::Recombine>(k_recombine, c, (uint32_t)c->cur);
 }
 
 // the digit planes were packed by the draw phase
@@ -2658,7 +2615,7 @@ void batch_op_blocks(const Params& P, uint32_t* out) {
     out[kOpSelBlockscan] = SelBlockscan::blocks(P);
     out[kOpGametes] = Gametes::blocks(P);
     out[kOpWordSort] = WordSort::blocks(P);
-    out[kOpRecombine] = RecombineNarrow::blocks(P);
+    out[kOpRecombine] = BatchRecombineNarrow::blocks(P);
     out[kOpPackDigits] = PackDigits::blocks(P);
     const int cls = f6::trait_class(P.traits);
     out[kOpTraits] = cls == 0   ? Traits2Fixed::blocks(P)

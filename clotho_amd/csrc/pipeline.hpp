@@ -43,7 +43,7 @@ inline uint32_t stat_chunks(uint32_t words, uint32_t n) {
     return chunks < most ? chunks : most;
 }
 
-// The per-word order-statistic tables of the recombination (sorted keys,
+// The per-word order-statistic tables of the batched recombination (sorted keys,
 // bucket counts, prefix masks) are stored tile-major: the table of a 64-word
 // column tile is one contiguous [row][64 words] image, the layout a
 // recombination block keeps in LDS, so a block fills its LDS copy with
@@ -104,9 +104,11 @@ struct Params {
     uint32_t fitness_kind;
     double fit_coeff, fit_inv;
     uint32_t chunks;       // row chunks of the recombination grid
+    uint32_t splits;       // column ranges of the recombination grid
     uint32_t tiles;        // 64-word column tiles at capacity
     uint32_t mut_blocks;   // scan blocks over gametes
-    uint32_t word_blocks;  // 64-word free-space blocks at capacity
+    uint32_t free_words;   // words per free-space block: 16 or 64
+    uint32_t word_blocks;  // free-space blocks at capacity
     uint32_t max_chunks;   // row-chunk capacity of the partial buffers
     uint32_t trait_blocks; // blocks of the last balanced traits launch (0: another launch)
 };
@@ -138,15 +140,15 @@ struct Buffers {
     uint32_t* events;         // [h][ev_cap] event keys
     // Gamete records in parent order (the children of one parent individual
     // adjacent): {child row, top row, n_events | mutations << 8, first
-    // mutation}.  The recombination loads a parent row pair once for up to
-    // kSibs of its children; nullptr = child order (the batched launches).
+    // mutation}: siblings read their parent pair from cache.  nullptr = child
+    // order.
     uint4* by_parent;         // [h]
     uint32_t* parent_cnt;     // [n] children per parent -> exclusive in-block offsets
     uint32_t* prank;          // [h] rank of the gamete among its parent's picks
     uint32_t* parent_bsum;    // [ceil(n/256)] block totals -> exclusive offsets
     uint32_t* given_parents;  // [h] parent individual of each gamete when GenState::given
     uint64_t* var_part;       // [chunks][w_cap] OR partials
-    uint64_t* fix_part;       // [chunks][w_cap] AND partials
+    uint64_t* fix_part;       // [chunks][w_cap] AND partials, then one spare row
     uint32_t* word_cnt;       // [w_cap] (fixed count << 16 | lost count) per word
     uint32_t* word_bsum;      // [2*word_blocks] block totals of fixed / lost counts
                               // (partials are sized for max_chunks rows)
@@ -189,10 +191,16 @@ enum BatchOp : int {
 // generation (live blocks), and their rows of BatchLaunch::live_offs.
 constexpr int kLiveRecombine = 0, kLiveWordSort = 1, kLivePack = 2, kLiveKinds = 3;
 
-// Row chunks of a replicate's batched recombination: its own launch shape's
-// chunk count divided by this (two measured best of 1, 2, 4, 8 on the
-// 256-replicate workload at generation 200: 1.12 against 1.20 ms).
-constexpr uint32_t kBatchChunkDiv = 2;
+// Row chunks of a replicate's batched recombination: 1024 rows each, up to
+// about 2048 blocks (half that size and twice the blocks measured 1.20 against
+// 1.12 ms on the 256-replicate workload at generation 200, a quarter and an
+// eighth of the chunks no better).
+inline uint32_t batch_chunks(const Params& P) {
+    uint32_t ch = (4096 + P.tiles - 1) / P.tiles;
+    const uint32_t rows = (P.h + 511) / 512;
+    ch = ch < rows ? ch : rows;
+    return (ch + 1) / 2 > 1 ? (ch + 1) / 2 : 1;
+}
 
 struct BatchLaunch {
     const RepView* views = nullptr;  // device [R]
@@ -253,6 +261,7 @@ struct clotho_ctx {
     size_t device_bytes = 0;    // sum of the context's device allocations
     uint32_t next_n = 0;        // offspring individuals of following generations (0: keep)
     uint32_t trait_round = 1;     // blocks of one resident round of the balanced traits kernel
+    uint32_t recombine_round = 1; // and of the recombination
     // launch shapes the autotuner may change (0 / defaults: the built-in choice)
     uint32_t trait_variant = 0;   // traits-pass kernel shape, 1 .. trait_variants()
     uint32_t compact_rows = 8;    // rows per wave step of the column compaction: 4, 8, 16
@@ -262,8 +271,7 @@ struct clotho_ctx {
 
 namespace clotho {
 // Launch sequences (pipeline.hip).
-hipError_t launch_draw(clotho_ctx* c);       // draws + per-word order statistics
-hipError_t launch_word_sort(clotho_ctx* c);  // order statistics alone (autotuner replays)
+hipError_t launch_draw(clotho_ctx* c);
 hipError_t launch_recombine(clotho_ctx* c);
 hipError_t launch_traits(clotho_ctx* c);         // whole traits
 hipError_t launch_traits_pieces(clotho_ctx* c);  // launch_free_reduce sums the pieces
@@ -304,7 +312,11 @@ uint32_t trait_variants(const clotho_ctx* c);
 hipError_t launch_compact_plan(clotho_ctx* c);
 hipError_t launch_compact_rows(clotho_ctx* c, int src);
 uint32_t compact_chunks_of(const clotho_ctx* c);
-hipError_t query_trait_residency(clotho_ctx* c);  // sets c->trait_round
+hipError_t query_residency(clotho_ctx* c);  // sets c->trait_round and c->recombine_round
+// launch shape of the recombination: row chunks for h rows, and the column
+// ranges that go with a number of row chunks
+uint32_t recombine_chunks(const clotho_ctx* c, uint32_t h);
+uint32_t recombine_splits(const clotho_ctx* c, uint32_t chunks);
 // Column compaction of population [src] into [1 - src] (fixed and lost
 // columns removed, slots renumbered in order); the caller flips cur.
 hipError_t launch_compact(clotho_ctx* c, int src);
