@@ -72,6 +72,11 @@ void free_buffers(clotho_ctx* c) {
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     std::memset(&B, 0, sizeof(B));
+    if (c->shape_status) (void)hipFree(c->shape_status);
+    if (c->scratch) (void)hipFree(c->scratch);
+    if (c->stage) (void)hipHostFree(c->stage);
+    for (hipEvent_t e : c->scratch_time)
+        if (e) (void)hipEventDestroy(e);
 }
 
 }  // namespace
@@ -87,16 +92,112 @@ void destroy_graphs(clotho_ctx* c) {
     c->graphs.valid = false;
 }
 
-int read_state(clotho_ctx* c, GenState* st) {
-    HIP_TRY(c, hipStreamSynchronize(c->stream));
-    HIP_TRY(c, hipMemcpy(st, c->b.state, sizeof(GenState), hipMemcpyDeviceToHost));
+constexpr size_t kScratchKept = 64u << 20;  // covers 100,000 individuals of 1000 words
+
+constexpr size_t kStageBytes = 32u << 10;
+
+// Up to kStageBytes from the device, after everything on the context's stream,
+// by way of its pinned stage: take(bytes there).  One asynchronous copy and one
+// wait (16 us with a launch before it, where a wait and a pageable copy take 26).
+template <class Take>
+int fetch_small(clotho_ctx* c, const void* src, size_t bytes, Take take) {
+    const std::lock_guard<std::mutex> lock(c->stage_mutex);
+    const hipError_t e =
+        bytes ? hipMemcpyAsync(c->stage, src, bytes, hipMemcpyDeviceToHost, c->stream) : hipSuccess;
+    const hipError_t s = hipStreamSynchronize(c->stream);
+    HIP_TRY(c, e);
+    HIP_TRY(c, s);
+    take(c->stage);
     return CLOTHO_OK;
 }
 
-int write_state(clotho_ctx* c, const GenState& st) {
+// Copies after everything on the context's stream, done when they return.
+int fetch(clotho_ctx* c, void* dst, const void* src, size_t bytes) {
+    if (bytes <= kStageBytes)
+        return fetch_small(c, src, bytes, [&](const char* p) { std::memcpy(dst, p, bytes); });
     HIP_TRY(c, hipStreamSynchronize(c->stream));
-    HIP_TRY(c, hipMemcpy(c->b.state, &st, sizeof(GenState), hipMemcpyHostToDevice));
+    HIP_TRY(c, hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost));
     return CLOTHO_OK;
+}
+int deliver(clotho_ctx* c, void* dst, const void* src, size_t bytes) {
+    if (bytes > kStageBytes) {
+        HIP_TRY(c, hipStreamSynchronize(c->stream));
+        HIP_TRY(c, hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice));
+        return CLOTHO_OK;
+    }
+    const std::lock_guard<std::mutex> lock(c->stage_mutex);
+    if (bytes) std::memcpy(c->stage, src, bytes);
+    const hipError_t e =
+        bytes ? hipMemcpyAsync(dst, c->stage, bytes, hipMemcpyHostToDevice, c->stream) : hipSuccess;
+    const hipError_t s = hipStreamSynchronize(c->stream);
+    HIP_TRY(c, e);
+    HIP_TRY(c, s);
+    return CLOTHO_OK;
+}
+
+// Device memory of one call: the context's scratch, grown when it is too
+// small, or an allocation of its own above kScratchKept.  Calls on one context
+// do not overlap on its stream; a second thread's call waits.
+struct Scratch {
+    clotho_ctx* c;
+    std::unique_lock<std::mutex> lock;
+    char* base = nullptr;
+    char* own = nullptr;
+    explicit Scratch(clotho_ctx* ctx) : c(ctx), lock(ctx->scratch_mutex) {}
+    ~Scratch() {
+        if (own) (void)hipFree(own);
+    }
+    hipError_t get(size_t bytes) {
+        if (bytes > kScratchKept) {
+            const hipError_t e = hipMalloc((void**)&own, bytes);
+            base = own;
+            return e;
+        }
+        if (bytes > c->scratch_bytes) {
+            if (c->scratch) (void)hipFree(c->scratch);  // waits for the device
+            c->scratch = nullptr;
+            c->device_bytes -= c->scratch_bytes;
+            c->scratch_bytes = 0;
+            const hipError_t e = hipMalloc((void**)&c->scratch, bytes);
+            if (e != hipSuccess) return e;
+            c->scratch_bytes = bytes;
+            c->device_bytes += bytes;
+        }
+        base = c->scratch;
+        return hipSuccess;
+    }
+};
+// parts of a scratch allocation, on 256-byte lines
+struct Parts {
+    size_t total = 0;
+    size_t add(size_t bytes) {
+        const size_t at = total;
+        total += (bytes + 255) / 256 * 256;
+        return at;
+    }
+};
+
+// dst[i] = src[i] * scale.  A few values are converted here; more on the device:
+// the copy then goes straight into the caller's pages (200,000 traits: 171 us
+// with the conversion here, 138 there).
+template <class T>
+int fetch_scaled(clotho_ctx* c, double* dst, const T* src, size_t n, double scale) {
+    if (sizeof(T) * n <= kStageBytes)
+        return fetch_small(c, src, sizeof(T) * n, [&](const char* p) {
+            const T* v = reinterpret_cast<const T*>(p);
+            for (size_t i = 0; i < n; ++i) dst[i] = (double)v[i] * scale;
+        });
+    Scratch tmp(c);
+    HIP_TRY(c, tmp.get(8 * n));
+    double* const d = reinterpret_cast<double*>(tmp.base);
+    HIP_TRY(c, launch_scale(src, n, scale, d, c->stream));
+    return fetch(c, dst, d, 8 * n);
+}
+
+int read_state(clotho_ctx* c, GenState* st) { return fetch(c, st, c->b.state, sizeof(GenState)); }
+
+int write_state(clotho_ctx* c, const GenState& st) {
+    return deliver(c, c->b.state, &st, sizeof(GenState));
 }
 
 // Free space of an uploaded population: the analysis runs as at the end of
@@ -104,13 +205,12 @@ int write_state(clotho_ctx* c, const GenState& st) {
 int analyse_upload(clotho_ctx* c, GenState st) {
     st.inter = c->p.inter_k;
     st.free_base = 0;
-    int rc = write_state(c, st);
+    const int rc = write_state(c, st);
     if (rc) return rc;
     HIP_TRY(c, launch_population_analysis(c));
-    rc = read_state(c, &st);
-    if (rc) return rc;
-    st.inter = 0;
-    return write_state(c, st);
+    HIP_TRY(c, launch_end_analysis(c));
+    HIP_TRY(c, hipStreamSynchronize(c->stream));
+    return CLOTHO_OK;
 }
 
 // ifitness_generator::generate(N) (src/clotho/fitness/normal_fitness_generator.cpp:36-52,
@@ -353,7 +453,13 @@ int clotho_create(const clotho_config* cfg, int device, clotho_ctx** out) {
     rc |= dalloc(c, &B.cdf_rho, kMaxCdf);
     rc |= dalloc(c, &B.cdf_mu, kMaxCdf);
     rc |= dalloc(c, &B.state, 1);
+    rc |= dalloc(c, &c->shape_status, 1);
     if (rc != CLOTHO_OK) return bail(rc);
+    if (hipHostMalloc((void**)&c->stage, kStageBytes, hipHostMallocDefault) != hipSuccess)
+        return bail(CLOTHO_ERR_HIP);
+    for (int k = 0; k < 2; ++k)
+        if (hipEventCreate(&c->scratch_time[k]) != hipSuccess)
+            return bail(CLOTHO_ERR_HIP);
 
     // first generation: empty founders, fitness 1.0 (GeneralFitness::resize)
     bool ok = hipMemcpy(B.cdf_rho, cdf_rho, sizeof(double) * nr, hipMemcpyHostToDevice) ==
@@ -537,9 +643,11 @@ int clotho_set_synthetic_population(clotho_ctx* c, uint32_t alleles, const doubl
 
 int clotho_get_shape(clotho_ctx* c, clotho_shape* out) {
     if (!c || !out) return CLOTHO_ERR_ARG;
-    GenState st;
-    int rc = read_state(c, &st);
+    HIP_TRY(c, launch_shape(c));
+    ShapeStatus now;
+    const int rc = fetch(c, &now, c->shape_status, sizeof(now));
     if (rc) return rc;
+    const GenState& st = now.state;
     std::memset(out, 0, sizeof(*out));
     out->generation = st.gen;
     out->n_individuals = c->p.n;
@@ -552,27 +660,13 @@ int clotho_get_shape(clotho_ctx* c, clotho_shape* out) {
     out->free_count = st.free_count;
     out->variable_count = st.all_size - st.free_count;
     out->error = st.error;
-    // all-neutral over the allele table, fitness constancy of the current population
-    uint32_t* d_flags = nullptr;
-    HIP_TRY(c, hipMalloc((void**)&d_flags, 64 * sizeof(uint32_t)));
-    hipError_t e = launch_all_neutral(c, d_flags);
-    uint32_t flags[64] = {0};
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    if (e == hipSuccess) e = hipMemcpy(flags, d_flags, sizeof(flags), hipMemcpyDeviceToHost);
-    (void)hipFree(d_flags);
-    if (e != hipSuccess) return fail(c, CLOTHO_ERR_HIP, hipGetErrorString(e));
-    uint32_t any = 0;
-    for (uint32_t f : flags) any |= f;
-    out->all_neutral = any ? 0 : 1;
-    std::vector<double> fit(c->p.n);
-    HIP_TRY(c, hipMemcpy(fit.data(), c->b.fitness[c->cur], 8 * fit.size(), hipMemcpyDeviceToHost));
-    bool constant = true;
-    for (double f : fit)
-        if (!(f == fit[0])) {
-            constant = false;
-            break;
-        }
-    out->fitness_constant = constant ? 1 : 0;
+    uint32_t effect = 0, varies = 0;
+    for (uint32_t i = 0; i < kShapeBlocks; ++i) {
+        effect |= now.effect[i];
+        varies |= now.varies[i];
+    }
+    out->all_neutral = effect ? 0 : 1;         // over the allele table
+    out->fitness_constant = varies ? 0 : 1;    // of the current population
     return CLOTHO_OK;
 }
 
@@ -596,18 +690,11 @@ int clotho_download_alleles(clotho_ctx* c, double* positions, double* effects, u
     if (rc) return rc;
     const uint32_t A = st.all_size, T = c->p.traits;
     if (cap < A) return fail(c, CLOTHO_ERR_ARG, "download_alleles: buffer too small");
-    if (positions && A) {
-        std::vector<uint32_t> k(A);
-        HIP_TRY(c, hipMemcpy(k.data(), c->b.keys, 4 * A, hipMemcpyDeviceToHost));
-        for (uint32_t j = 0; j < A; ++j) positions[j] = (double)k[j] * 0x1p-32;
-    }
-    if (effects && A && T) {
-        std::vector<int32_t> q((size_t)A * T);
-        HIP_TRY(c, hipMemcpy(q.data(), c->b.effects, 4 * q.size(), hipMemcpyDeviceToHost));
-        for (size_t j = 0; j < q.size(); ++j) effects[j] = (double)q[j] * c->p.eff_quantum;
-    }
-    if (ages && A) HIP_TRY(c, hipMemcpy(ages, c->b.ages, 4 * A, hipMemcpyDeviceToHost));
-    return CLOTHO_OK;
+    if (positions && A && (rc = fetch_scaled(c, positions, c->b.keys, A, 0x1p-32))) return rc;
+    if (effects && A && T &&
+        (rc = fetch_scaled(c, effects, c->b.effects, (size_t)A * T, c->p.eff_quantum)))
+        return rc;
+    return ages && A ? fetch(c, ages, c->b.ages, 4ull * A) : CLOTHO_OK;
 }
 
 int clotho_download_free_space(clotho_ctx* c, uint32_t* fixed, uint32_t* lost, size_t cap) {
@@ -618,29 +705,27 @@ int clotho_download_free_space(clotho_ctx* c, uint32_t* fixed, uint32_t* lost, s
     const uint32_t nf = st.n_fixed, nl = st.free_count - st.n_fixed;
     if (cap < std::max(nf, nl)) return fail(c, CLOTHO_ERR_ARG, "download_free_space: too small");
     const uint32_t* list = c->b.free_list + st.free_base;  // entries not yet handed out
-    if (fixed && nf) HIP_TRY(c, hipMemcpy(fixed, list, 4 * nf, hipMemcpyDeviceToHost));
-    if (lost && nl) HIP_TRY(c, hipMemcpy(lost, list + nf, 4 * nl, hipMemcpyDeviceToHost));
-    return CLOTHO_OK;
+    const size_t cut = 4ull * nf, bytes = cut + 4ull * nl;
+    if (bytes <= kStageBytes)  // the lists adjoin
+        return fetch_small(c, list, bytes, [&](const char* p) {
+            if (fixed && nf) std::memcpy(fixed, p, cut);
+            if (lost && nl) std::memcpy(lost, p + cut, bytes - cut);
+        });
+    if (fixed && nf && (rc = fetch(c, fixed, list, cut))) return rc;
+    return lost && nl ? fetch(c, lost, list + nf, bytes - cut) : CLOTHO_OK;
 }
 
 int clotho_download_traits(clotho_ctx* c, double* out, size_t cap) {
     if (!c || !out) return CLOTHO_ERR_ARG;
     const size_t n = (size_t)c->p.h * c->p.traits;
     if (cap < n) return fail(c, CLOTHO_ERR_ARG, "download_traits: buffer too small");
-    HIP_TRY(c, hipStreamSynchronize(c->stream));
-    if (!n) return CLOTHO_OK;
-    std::vector<int64_t> q(n);
-    HIP_TRY(c, hipMemcpy(q.data(), c->b.traits[c->cur], 8 * n, hipMemcpyDeviceToHost));
-    for (size_t i = 0; i < n; ++i) out[i] = (double)q[i] * c->p.eff_quantum;
-    return CLOTHO_OK;
+    return fetch_scaled(c, out, c->b.traits[c->cur], n, c->p.eff_quantum);
 }
 
 int clotho_download_fitness(clotho_ctx* c, double* out, size_t cap) {
     if (!c || !out) return CLOTHO_ERR_ARG;
     if (cap < c->p.n) return fail(c, CLOTHO_ERR_ARG, "download_fitness: buffer too small");
-    HIP_TRY(c, hipStreamSynchronize(c->stream));
-    HIP_TRY(c, hipMemcpy(out, c->b.fitness[c->cur], 8 * c->p.n, hipMemcpyDeviceToHost));
-    return CLOTHO_OK;
+    return fetch(c, out, c->b.fitness[c->cur], 8ull * c->p.n);
 }
 
 int clotho_download_gametes(clotho_ctx* c, uint32_t* top, uint32_t* bottom, uint32_t* events,
@@ -737,40 +822,26 @@ int clotho_allele_counts(clotho_ctx* c, const uint32_t* rows, uint32_t n_rows,
             if (rows[i] >= H) return fail(c, CLOTHO_ERR_ARG, "allele_counts: row out of range");
     const uint32_t ngroups = stat_word_tiles(W);
     const uint32_t chunks = stat_chunks(W, n);
-    uint32_t *d_sample = nullptr, *d_cols = nullptr, *d_rows = nullptr, *d_cp = nullptr,
-             *d_rp = nullptr;
-    hipEvent_t e0 = nullptr, e1 = nullptr;
-    auto cleanup = [&]() {
-        for (uint32_t* p : {d_sample, d_cols, d_rows, d_cp, d_rp})
-            if (p) (void)hipFree(p);
-        if (e0) (void)hipEventDestroy(e0);
-        if (e1) (void)hipEventDestroy(e1);
-    };
-    hipError_t e = hipSuccess;
-    auto step = [&](hipError_t r) {
-        if (e == hipSuccess) e = r;
-    };
-    if (rows) step(hipMalloc((void**)&d_sample, 4ull * std::max<uint32_t>(n, 1)));
-    step(hipMalloc((void**)&d_cols, 4ull * std::max<uint32_t>(A, 1)));
-    step(hipMalloc((void**)&d_rows, 4ull * std::max<uint32_t>(n, 1)));
-    step(hipMalloc((void**)&d_cp, 4ull * std::max<size_t>((size_t)chunks * W * 64, 1)));
-    step(hipMalloc((void**)&d_rp, 4ull * std::max<size_t>((size_t)ngroups * n, 1)));
-    step(hipEventCreate(&e0));
-    step(hipEventCreate(&e1));
-    if (rows && e == hipSuccess)
-        step(hipMemcpyAsync(d_sample, rows, 4ull * n, hipMemcpyHostToDevice, c->stream));
-    step(hipEventRecord(e0, c->stream));
-    if (e == hipSuccess)
-        step(launch_allele_counts(c, c->b.rows[c->cur], W, A, d_sample, n, d_cols, d_rows, d_cp,
-                                  d_rp, chunks));
-    step(hipEventRecord(e1, c->stream));
-    if (A) step(hipMemcpyAsync(column_counts, d_cols, 4ull * A, hipMemcpyDeviceToHost, c->stream));
-    if (n) step(hipMemcpyAsync(row_counts, d_rows, 4ull * n, hipMemcpyDeviceToHost, c->stream));
-    step(hipStreamSynchronize(c->stream));
+    Parts at;
+    const size_t at_sample = at.add(rows ? 4ull * n : 0), at_cols = at.add(4ull * A),
+                 at_rows = at.add(4ull * n), at_cp = at.add(4ull * chunks * W * 64),
+                 at_rp = at.add(4ull * ngroups * n);
+    Scratch tmp(c);
+    HIP_TRY(c, tmp.get(std::max<size_t>(at.total, 1)));
+    uint32_t* const d_sample = rows ? (uint32_t*)(tmp.base + at_sample) : nullptr;
+    uint32_t *const d_cols = (uint32_t*)(tmp.base + at_cols), *const d_rows = (uint32_t*)(tmp.base + at_rows);
+    if (rows && n && (rc = deliver(c, d_sample, rows, 4ull * n))) return rc;
+    HIP_TRY(c, hipEventRecord(c->scratch_time[0], c->stream));
+    HIP_TRY(c, launch_allele_counts(c, c->b.rows[c->cur], W, A, d_sample, n, d_cols, d_rows,
+                                    (uint32_t*)(tmp.base + at_cp), (uint32_t*)(tmp.base + at_rp),
+                                    chunks));
+    HIP_TRY(c, hipEventRecord(c->scratch_time[1], c->stream));
+    rc = fetch(c, column_counts, d_cols, 4ull * A);
+    if (!rc) rc = fetch(c, row_counts, d_rows, 4ull * n);
+    if (rc) return rc;
     float ms = 0.f;
-    if (e == hipSuccess) step(hipEventElapsedTime(&ms, e0, e1));
-    cleanup();
-    if (e != hipSuccess) return fail(c, CLOTHO_ERR_HIP, hipGetErrorString(e));
+    HIP_TRY(c, hipEventSynchronize(c->scratch_time[1]));
+    HIP_TRY(c, hipEventElapsedTime(&ms, c->scratch_time[0], c->scratch_time[1]));
     if (kernel_ms) *kernel_ms = ms;
     return CLOTHO_OK;
 }
@@ -792,31 +863,18 @@ int clotho_pairwise_differences(clotho_ctx* c, const uint32_t* rows, uint32_t n_
         if (rows[i] >= H) return fail(c, CLOTHO_ERR_ARG, "pairwise_differences: row out of range");
     if (kernel_ms) *kernel_ms = 0.0;
     if (pairs == 0) return CLOTHO_OK;
-    uint32_t *d_sample = nullptr, *d_out = nullptr;
-    hipEvent_t e0 = nullptr, e1 = nullptr;
-    hipError_t e = hipSuccess;
-    auto step = [&](hipError_t r) {
-        if (e == hipSuccess) e = r;
-    };
-    step(hipMalloc((void**)&d_sample, 4ull * n_rows));
-    step(hipMalloc((void**)&d_out, 4ull * pairs));
-    step(hipEventCreate(&e0));
-    step(hipEventCreate(&e1));
-    if (e == hipSuccess)
-        step(hipMemcpyAsync(d_sample, rows, 4ull * n_rows, hipMemcpyHostToDevice, c->stream));
-    if (e == hipSuccess) step(hipEventRecord(e0, c->stream));
-    if (e == hipSuccess) step(launch_pairwise(c, c->b.rows[c->cur], W, d_sample, n_rows, d_out));
-    if (e == hipSuccess) step(hipEventRecord(e1, c->stream));
-    if (e == hipSuccess)
-        step(hipMemcpyAsync(out, d_out, 4ull * pairs, hipMemcpyDeviceToHost, c->stream));
-    step(hipStreamSynchronize(c->stream));
+    Parts at;
+    const size_t at_sample = at.add(4ull * n_rows), at_out = at.add(4ull * pairs);
+    Scratch tmp(c);
+    HIP_TRY(c, tmp.get(at.total));
+    uint32_t *const d_sample = (uint32_t*)(tmp.base + at_sample), *const d_out = (uint32_t*)(tmp.base + at_out);
+    if ((rc = deliver(c, d_sample, rows, 4ull * n_rows))) return rc;
+    HIP_TRY(c, hipEventRecord(c->scratch_time[0], c->stream));
+    HIP_TRY(c, launch_pairwise(c, c->b.rows[c->cur], W, d_sample, n_rows, d_out));
+    HIP_TRY(c, hipEventRecord(c->scratch_time[1], c->stream));
+    if ((rc = fetch(c, out, d_out, 4ull * pairs))) return rc;
     float ms = 0.f;
-    if (e == hipSuccess) step(hipEventElapsedTime(&ms, e0, e1));
-    for (uint32_t* p : {d_sample, d_out})
-        if (p) (void)hipFree(p);
-    if (e0) (void)hipEventDestroy(e0);
-    if (e1) (void)hipEventDestroy(e1);
-    if (e != hipSuccess) return fail(c, CLOTHO_ERR_HIP, hipGetErrorString(e));
+    HIP_TRY(c, hipEventElapsedTime(&ms, c->scratch_time[0], c->scratch_time[1]));
     if (kernel_ms) *kernel_ms = ms;
     return CLOTHO_OK;
 }
@@ -832,12 +890,10 @@ int clotho_set_parents(clotho_ctx* c, const uint32_t* parents, uint32_t gametes)
         if (parents[o] >= c->p.n)
             return fail(c, CLOTHO_ERR_ARG, "set_parents: parent " + std::to_string(parents[o]) +
                                                " outside the current population");
-    GenState st;
-    int rc = read_state(c, &st);
+    const int rc = deliver(c, c->b.given_parents, parents, 4ull * gametes);
     if (rc) return rc;
-    HIP_TRY(c, hipMemcpy(c->b.given_parents, parents, 4ull * gametes, hipMemcpyHostToDevice));
-    st.given = 1;
-    return write_state(c, st);
+    const uint32_t given = 1;
+    return deliver(c, &c->b.state->given, &given, sizeof(given));
 }
 
 int clotho_add_mutations(clotho_ctx* c, const uint32_t* rows, const double* positions,
@@ -877,9 +933,8 @@ int clotho_add_mutations(clotho_ctx* c, const uint32_t* rows, const double* posi
         return fail(c, CLOTHO_ERR_CAPACITY, "add_mutations: allele capacity exceeded");
     std::vector<uint32_t> slots(n);
     const uint32_t reuse = std::min(n, F);
-    if (reuse)
-        HIP_TRY(c, hipMemcpy(slots.data(), c->b.free_list + st.free_base, 4ull * reuse,
-                             hipMemcpyDeviceToHost));
+    if (reuse && (rc = fetch(c, slots.data(), c->b.free_list + st.free_base, 4ull * reuse)))
+        return rc;
     for (uint32_t k = reuse; k < n; ++k) slots[k] = A + (k - F);
     const uint32_t W0 = st.wc, W1 = (uint32_t)(((A1 + 511) / 512) * 8);
     if (W1 > W0) {  // wider rows: re-stride into the other buffer, which becomes current
@@ -891,39 +946,33 @@ int clotho_add_mutations(clotho_ctx* c, const uint32_t* rows, const double* posi
                                   hipMemcpyDeviceToDevice, c->stream));
         c->cur = 1 - c->cur;
     }
-    uint32_t *d_rows = nullptr, *d_slots = nullptr, *d_keys = nullptr;
-    int32_t* d_eff = nullptr;
-    uint64_t* d_mask = nullptr;
-    hipError_t e = hipSuccess;
-    auto step = [&](hipError_t r) {
-        if (e == hipSuccess) e = r;
-    };
-    // reused fixed slots: the allele leaves every row first (removeFixedAlleles)
+    // one copy for the mutations and, for reused fixed slots (the allele leaves
+    // every row first, removeFixedAlleles), the mask of their columns
     const uint32_t n_fixed_reused = std::min(reuse, st.n_fixed);
-    if (n_fixed_reused) {
-        std::vector<uint64_t> mask(W1, 0);
-        for (uint32_t k = 0; k < n_fixed_reused; ++k) mask[slots[k] / 64] |= 1ull << (slots[k] % 64);
-        step(hipMalloc((void**)&d_mask, 8ull * W1));
-        if (e == hipSuccess)
-            step(hipMemcpy(d_mask, mask.data(), 8ull * W1, hipMemcpyHostToDevice));
-        if (e == hipSuccess) step(launch_clear_columns(c, c->cur, W1, d_mask));
+    Parts at;
+    const size_t at_rows = at.add(4ull * n), at_slots = at.add(4ull * n), at_keys = at.add(4ull * n),
+                 at_eff = at.add(4ull * eq.size()), at_mask = at.add(n_fixed_reused ? 8ull * W1 : 0);
+    std::vector<char> in(at.total, 0);
+    std::memcpy(in.data() + at_rows, rows, 4ull * n);
+    std::memcpy(in.data() + at_slots, slots.data(), 4ull * n);
+    std::memcpy(in.data() + at_keys, keys.data(), 4ull * n);
+    std::memcpy(in.data() + at_eff, eq.data(), 4ull * eq.size());
+    uint64_t* const mask = reinterpret_cast<uint64_t*>(in.data() + at_mask);
+    for (uint32_t k = 0; k < n_fixed_reused; ++k) mask[slots[k] / 64] |= 1ull << (slots[k] % 64);
+    {
+        Scratch tmp(c);
+        HIP_TRY(c, tmp.get(at.total));
+        if ((rc = deliver(c, tmp.base, in.data(), at.total))) return rc;
+        if (n_fixed_reused)
+            HIP_TRY(c, launch_clear_columns(c, c->cur, W1, (const uint64_t*)(tmp.base + at_mask)));
+        // the age of the generation that produced the population
+        const uint32_t age = st.gen > 0 ? st.gen - 1 : 0;
+        HIP_TRY(c, launch_add_mutations(
+                       c, c->cur, W1, (const uint32_t*)(tmp.base + at_rows),
+                       (const uint32_t*)(tmp.base + at_slots), (const uint32_t*)(tmp.base + at_keys),
+                       (const int32_t*)(tmp.base + at_eff), n, age));
+        HIP_TRY(c, hipStreamSynchronize(c->stream));
     }
-    step(hipMalloc((void**)&d_rows, 4ull * n));
-    step(hipMalloc((void**)&d_slots, 4ull * n));
-    step(hipMalloc((void**)&d_keys, 4ull * n));
-    step(hipMalloc((void**)&d_eff, 4ull * eq.size()));
-    if (e == hipSuccess) step(hipMemcpy(d_rows, rows, 4ull * n, hipMemcpyHostToDevice));
-    if (e == hipSuccess) step(hipMemcpy(d_slots, slots.data(), 4ull * n, hipMemcpyHostToDevice));
-    if (e == hipSuccess) step(hipMemcpy(d_keys, keys.data(), 4ull * n, hipMemcpyHostToDevice));
-    if (e == hipSuccess) step(hipMemcpy(d_eff, eq.data(), 4ull * eq.size(), hipMemcpyHostToDevice));
-    // the age of the generation that produced the population
-    const uint32_t age = st.gen > 0 ? st.gen - 1 : 0;
-    if (e == hipSuccess)
-        step(launch_add_mutations(c, c->cur, W1, d_rows, d_slots, d_keys, d_eff, n, age));
-    step(hipStreamSynchronize(c->stream));
-    for (void* p : {(void*)d_rows, (void*)d_slots, (void*)d_keys, (void*)d_eff, (void*)d_mask})
-        if (p) (void)hipFree(p);
-    if (e != hipSuccess) return fail(c, CLOTHO_ERR_HIP, hipGetErrorString(e));
     // traits and free space of the new population
     st.alleles = st.all_size = (uint32_t)A1;
     st.eff_max = std::max(st.eff_max, eff_max);

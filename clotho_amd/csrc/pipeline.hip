@@ -2049,21 +2049,33 @@ struct Commit {
     }
 };
 
-__global__ void __launch_bounds__(kBlock) k_any_nonzero(const int32_t* effects, size_t n,
-                                                        uint32_t* flag_out) {
-    __shared__ int s[kBlock];
-    int any = 0;
-    for (size_t i = blockIdx.x * (size_t)kBlock + threadIdx.x; i < n;
-         i += (size_t)gridDim.x * kBlock)
-        any |= effects[i] != 0;
-    s[threadIdx.x] = any;
-    __syncthreads();
-    for (int q = kBlock / 2; q > 0; q >>= 1) {
-        if ((int)threadIdx.x < q) s[threadIdx.x] |= s[threadIdx.x + q];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) flag_out[blockIdx.x] = s[0];
+// What clotho_get_shape reports: is any effect of the table nonzero, does any
+// fitness of the current population differ from the first (a NaN does), and
+// the generation's scalars.
+__global__ void __launch_bounds__(kBlock) k_shape(const GenState* st, const int32_t* effects,
+                                                  size_t n_effects, const double* fitness,
+                                                  uint32_t n, ShapeStatus* out) {
+    const size_t first = blockIdx.x * (size_t)kBlock + threadIdx.x;
+    const size_t step = (size_t)gridDim.x * kBlock;
+    int effect = 0, varies = 0;
+    for (size_t i = first; i < n_effects; i += step) effect |= effects[i] != 0;
+    const double f0 = fitness[0];
+    for (size_t i = first; i < n; i += step) varies |= !(fitness[i] == f0);
+    effect = __syncthreads_or(effect);
+    varies = __syncthreads_or(varies);
+    if (threadIdx.x) return;
+    out->effect[blockIdx.x] = effect != 0;
+    out->varies[blockIdx.x] = varies != 0;
+    if (blockIdx.x == 0) out->state = *st;
 }
+
+template <class T>
+__global__ void __launch_bounds__(kBlock) k_scale(const T* src, size_t n, double scale, double* dst) {
+    for (size_t i = blockIdx.x * (size_t)kBlock + threadIdx.x; i < n; i += (size_t)gridDim.x * kBlock)
+        dst[i] = (double)src[i] * scale;
+}
+
+__global__ void k_end_analysis(GenState* st) { st->inter = 0; }
 
 // Exact genome traits of population `sel` (f6::traits_block); the effect
 // digit planes are packed first (f6::pack_block).
@@ -3037,12 +3049,32 @@ hipError_t launch_crossover_rows(clotho_ctx* c, const uint64_t* d_top, const uin
     return hipGetLastError();
 }
 
-hipError_t launch_all_neutral(clotho_ctx* c, uint32_t* d_flag) {
-    const size_t n = (size_t)c->p.s_cap * c->p.traits;
-    hipLaunchKernelGGL(k_any_nonzero, dim3(64), dim3(kBlock), 0, c->stream, c->b.effects, n,
-                       d_flag);
-    LAUNCH_CHECK();
-    return hipSuccess;
+template <class T>
+static hipError_t launch_scale_of(const T* src, size_t n, double scale, double* dst, hipStream_t s) {
+    const uint32_t nb = (uint32_t)std::min<size_t>(1024, (n + kBlock - 1) / kBlock);
+    hipLaunchKernelGGL(k_scale<T>, dim3(nb), dim3(kBlock), 0, s, src, n, scale, dst);
+    return hipGetLastError();
+}
+hipError_t launch_scale(const int64_t* src, size_t n, double scale, double* dst, hipStream_t s) {
+    return launch_scale_of(src, n, scale, dst, s);
+}
+hipError_t launch_scale(const int32_t* src, size_t n, double scale, double* dst, hipStream_t s) {
+    return launch_scale_of(src, n, scale, dst, s);
+}
+hipError_t launch_scale(const uint32_t* src, size_t n, double scale, double* dst, hipStream_t s) {
+    return launch_scale_of(src, n, scale, dst, s);
+}
+
+hipError_t launch_shape(clotho_ctx* c) {
+    hipLaunchKernelGGL(k_shape, dim3(kShapeBlocks), dim3(kBlock), 0, c->stream, c->b.state,
+                       c->b.effects, (size_t)c->p.s_cap * c->p.traits, c->b.fitness[c->cur], c->p.n,
+                       c->shape_status);
+    return hipGetLastError();
+}
+
+hipError_t launch_end_analysis(clotho_ctx* c) {
+    hipLaunchKernelGGL(k_end_analysis, dim3(1), dim3(1), 0, c->stream, c->b.state);
+    return hipGetLastError();
 }
 
 hipError_t launch_synth_rows(clotho_ctx* c, uint64_t seed, const uint32_t* d_thr, uint32_t alleles,

@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -216,6 +217,15 @@ struct BatchLaunch {
     uint32_t grid_scale_num = 1, grid_scale_den = 1;
 };
 
+// What clotho_get_shape reports, gathered on the device in one launch and
+// copied in one piece.
+constexpr uint32_t kShapeBlocks = 64;
+struct ShapeStatus {
+    GenState state;
+    uint32_t effect[kShapeBlocks];  // per block: a nonzero effect in the allele table
+    uint32_t varies[kShapeBlocks];  // per block: a fitness unlike the first one
+};
+
 struct Timing {
     bool enabled = false;
     double ms[6] = {0, 0, 0, 0, 0, 0};
@@ -258,6 +268,17 @@ struct clotho_ctx {
     clotho::GraphPair graphs;
     std::string err;
     hipDeviceProp_t prop;
+    // Pinned memory that small results and inputs pass through, one call at a time.
+    std::mutex stage_mutex;
+    char* stage = nullptr;
+    clotho::ShapeStatus* shape_status = nullptr;  // device memory
+    // Device memory of the analysis and mutation calls, kept between them up to
+    // kScratchKept bytes, and the events that time their kernels; one call at a
+    // time uses them.
+    std::mutex scratch_mutex;
+    char* scratch = nullptr;
+    size_t scratch_bytes = 0;
+    hipEvent_t scratch_time[2] = {nullptr, nullptr};
     size_t device_bytes = 0;    // sum of the context's device allocations
     uint32_t next_n = 0;        // offspring individuals of following generations (0: keep)
     uint32_t trait_round = 1;     // blocks of one resident round of the balanced traits kernel
@@ -330,7 +351,12 @@ hipError_t launch_allele_counts(clotho_ctx* c, const uint64_t* rows, uint32_t W,
 // (n (n - 1) / 2 values).
 hipError_t launch_pairwise(clotho_ctx* c, const uint64_t* rows, uint32_t W,
                            const uint32_t* d_sample, uint32_t n, uint32_t* d_out);
-hipError_t launch_all_neutral(clotho_ctx* c, uint32_t* d_flag);
+// dst[i] = (double)src[i] * scale
+hipError_t launch_scale(const int64_t* src, size_t n, double scale, double* dst, hipStream_t s);
+hipError_t launch_scale(const int32_t* src, size_t n, double scale, double* dst, hipStream_t s);
+hipError_t launch_scale(const uint32_t* src, size_t n, double scale, double* dst, hipStream_t s);
+hipError_t launch_shape(clotho_ctx* c);  // fills c->shape_status
+hipError_t launch_end_analysis(clotho_ctx* c);  // the next generation starts an intermediate batch
 hipError_t launch_synth_rows(clotho_ctx* c, uint64_t seed, const uint32_t* d_thr, uint32_t alleles,
                              uint32_t words);
 // Context helpers (capi.hip).
