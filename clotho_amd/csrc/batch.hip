@@ -53,20 +53,35 @@ void drop_graphs(clotho_batch* b) {
         }
 }
 
+// Launch shape of a replicate's recombination within a batch of `groups` groups
+// of 64 gametes: chunks of up to 16 groups (a block's offset search, tables and
+// partials are paid per chunk; half and twice as many chunks measured 1.12 and
+// 1.20 ms on the 256-replicate workload at generation 200), fewer where the batch
+// would not give every resident block four chunks, and column ranges where the
+// chunks alone do not give it one.
+void batch_recombine_shape(Params& P, uint64_t groups, uint32_t resident) {
+    const uint32_t own = (P.h + 63) / 64;
+    const uint64_t per = std::min<uint64_t>(16, std::max<uint64_t>(1, groups / (4ull * resident)));
+    P.chunks = std::min<uint32_t>(P.max_chunks, (uint32_t)((own + per - 1) / per));
+    const uint64_t turns = (P.w_cap + 63) / 64;
+    P.splits = (uint32_t)std::max<uint64_t>(1, std::min(turns, resident / std::max<uint64_t>(1, groups)));
+    P.group_words = groups <= (uint64_t)kSmallBatch * resident ? 0 : kWidePerGroup;
+}
+
 // Upload each replicate's Params/Buffers and the per-kernel block offsets
 // when they changed (a replicate's launch shape may have been retuned).
 int sync_views(clotho_batch* b) {
     const uint32_t R = (uint32_t)b->reps.size();
     std::vector<RepView> v(R);
+    uint64_t groups = 0;
+    for (uint32_t r = 0; r < R; ++r) groups += (b->reps[r]->p.h + 63) / 64;
+    const uint32_t resident = b->reps[0]->recombine_round;
     for (uint32_t r = 0; r < R; ++r) {
         std::memset(&v[r], 0, sizeof(RepView));
         v[r].P = b->reps[r]->p;
         v[r].B = b->reps[r]->b;
         v[r].B.by_parent = nullptr;  // replicates recombine in child order
-        // batched recombination blocks take kBatchChunkDiv times the rows of
-        // a replicate's own launch: the replicates supply the parallelism,
-        // and every block pays a fixed set-up (offset search, tables, partials)
-        v[r].P.chunks = batch_chunks(v[r].P);
+        batch_recombine_shape(v[r].P, groups, resident);
         v[r].P.free_words = 64;
         v[r].P.word_blocks = (v[r].P.w_cap + 63) / 64;
     }
@@ -97,6 +112,11 @@ int sync_views(clotho_batch* b) {
     L.R = R;
     for (int k = 0; k < kOpCount; ++k) L.total[k] = offs[(size_t)k * (R + 1) + R];
     L.traits = v[0].P.traits;
+    L.by_group = L.by_event = false;
+    for (const RepView& x : v) {
+        L.by_group = L.by_group || x.P.w_cap > x.P.group_words;
+        L.by_event = L.by_event || x.P.group_words;
+    }
     L.wide_events = false;
     for (const RepView& x : v) L.wide_events = L.wide_events || x.P.ev_cap > 64;
     L.cus = (uint32_t)std::max(1, b->reps[0]->prop.multiProcessorCount);

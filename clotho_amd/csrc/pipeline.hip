@@ -590,10 +590,9 @@ struct ParentScatterOp {
 };
 
 // ---------------------------------------------------------------------------
-// Recombination + mutation (+ free-space partials) of replicate batches; a single
-// population takes rec::Recombine.  The batch keeps a lookup per event and row:
-// its rows are mostly narrow (8 to 32 words), and rec's group tables cost as much
-// as a few hundred words of rows.
+// Recombination + mutation (+ free-space partials) with a lookup per event and
+// row: the replicates of large batches, up to kWidePerGroup words per row.  Single
+// populations, small batches and wider rows take rec::Recombine.
 // ---------------------------------------------------------------------------
 // Per-word order statistics, once per generation: the 64 position keys of
 // word w sorted ascending (sorted[w][k]), prefix masks pm[w][c] = bits of the
@@ -2169,7 +2168,7 @@ struct MinWaves<Recombine<W>> {
 };
 template <>
 struct MinWaves<rec::Recombine> {
-    static constexpr int value = rec::kMinWaves;
+    static constexpr int value = rec::Recombine::kMinWaves;
 };
 template <int RT, int CLS, bool E>
 struct MinWaves<Traits<RT, CLS, E>> {
@@ -2263,7 +2262,12 @@ CLOTHO_SINGLE(k_compact_fitness, CompactFitness)
 // Occupancy floor of a batched kernel: the recombination kernel needs two
 // resident 1024-thread blocks per CU (8 waves per SIMD, <= 64 VGPRs) to keep
 // enough parent loads in flight.
-constexpr uint32_t kBatchOffsLds = 1024;  // replicate offsets kept in LDS up to this R
+// Replicate offsets kept in LDS up to this R: fewer where three blocks of
+// rec::Recombine just fit a compute unit.
+template <class Op>
+constexpr uint32_t kBatchOffsLds = 1024;
+template <>
+constexpr uint32_t kBatchOffsLds<rec::Recombine> = 256;
 
 // Ops whose batched offsets count live blocks only (k_batch_live_offsets).
 // Their block ranges at capacity cover the allele capacity, but the child
@@ -2279,7 +2283,7 @@ struct LiveBlocks<Recombine<W>> {
     // live tiles lt = ceil(wc / 64) x row chunks: u -> tile u mod lt, chunk u / lt
     static constexpr int kind = kLiveRecombine;
     __host__ __device__ static uint32_t count(const Params& P, uint32_t wc) {
-        return min((wc + 63) / 64, P.tiles) * P.chunks;
+        return wc > P.group_words ? 0u : min((wc + 63) / 64, P.tiles) * P.chunks;
     }
     __device__ static uint32_t block(const Params& P, uint32_t wc, uint32_t u) {
         const uint32_t lt = (wc + 63) / 64;  // >= 1 when u exists
@@ -2287,11 +2291,20 @@ struct LiveBlocks<Recombine<W>> {
     }
 };
 template <>
+struct LiveBlocks<rec::Recombine> {
+    // the replicates whose rows are wider than group_words
+    static constexpr int kind = kLiveGroups;
+    __host__ __device__ static uint32_t count(const Params& P, uint32_t wc) {
+        return wc > P.group_words ? rec::Recombine::live(P, wc) : 0u;
+    }
+    __device__ static uint32_t block(const Params&, uint32_t, uint32_t u) { return u; }
+};
+template <>
 struct LiveBlocks<WordSort> {
     // kWaves words per block: the live blocks are the first ceil(wc / kWaves)
     static constexpr int kind = kLiveWordSort;
     __host__ __device__ static uint32_t count(const Params& P, uint32_t wc) {
-        return min((wc + kWaves - 1) / kWaves, WordSort::blocks(P));
+        return wc > P.group_words ? 0u : min((wc + kWaves - 1) / kWaves, WordSort::blocks(P));
     }
     __device__ static uint32_t block(const Params&, uint32_t, uint32_t u) { return u; }
 };
@@ -2325,6 +2338,10 @@ template <int RT, int CLS, bool E>
 struct RoundRobin<Traits<RT, CLS, E>> {
     static constexpr bool value = true;
 };
+template <>
+struct RoundRobin<rec::Recombine> {
+    static constexpr bool value = true;
+};
 template <int K>
 struct RoundRobin<GametesOp<K>> {
     static constexpr bool value = true;
@@ -2346,8 +2363,8 @@ struct RoundRobin<FreeCompact> {
     static constexpr bool value = true;
 };
 
-// Live virtual blocks of the batched recombination, word sort and digit
-// packing (LiveBlocks): one block scans each kind's live block counts over the
+// Live virtual blocks of the batched recombination (both kernels), word sort and
+// digit packing (LiveBlocks): one block scans each kind's live block counts over the
 // replicates into out[kind][0 .. R] (exclusive, out[kind][R] = total) from the
 // child widths the draws set, so the persistent blocks of those ops visit live
 // blocks only.
@@ -2366,7 +2383,8 @@ __global__ void __launch_bounds__(1024) k_batch_live_offsets(const RepView* __re
             if (r < R) {
                 const RepView& rv = views[r];
                 const uint32_t wc = gbl(rv.B.state)->wc;
-                n = kind == kLiveRecombine ? LiveBlocks<BatchRecombineNarrow>::count(rv.P, wc)
+                n = kind == kLiveRecombine  ? LiveBlocks<BatchRecombineNarrow>::count(rv.P, wc)
+                    : kind == kLiveGroups   ? LiveBlocks<rec::Recombine>::count(rv.P, wc)
                     : kind == kLiveWordSort ? LiveBlocks<WordSort>::count(rv.P, wc)
                                             : LiveBlocks<PackDigits>::count(rv.P, wc);
             }
@@ -2403,8 +2421,8 @@ __global__ void __launch_bounds__(Op::kThreads)
                                                           uint32_t R, uint32_t sel) {
     // the replicate offsets in LDS when they fit: every virtual block
     // searches them, and a search in global memory is a chain of dependent loads
-    __shared__ uint32_t s_offs[kBatchOffsLds + 1];
-    const bool in_lds = R <= kBatchOffsLds;
+    __shared__ uint32_t s_offs[kBatchOffsLds<Op> + 1];
+    const bool in_lds = R <= kBatchOffsLds<Op>;
     if (in_lds)
         for (uint32_t i = threadIdx.x; i <= R; i += Op::kThreads) s_offs[i] = offs[i];
     __syncthreads();
@@ -2568,7 +2586,7 @@ uint32_t recombine_chunks(const clotho_ctx* c, uint32_t h) {
 // the tables that each range builds weigh less there (N = 250,000, 2072 words: 3.80
 // -> 3.69 ms; 816 words: 0.539 -> 0.57 ms).
 uint32_t recombine_splits(const clotho_ctx* c, uint32_t chunks) {
-    const uint32_t turns = (c->p.w_cap + rec::kTile * rec::kWaves - 1) / (rec::kTile * rec::kWaves);
+    const uint32_t turns = (c->p.w_cap + rec::Wide::kTile * rec::kWaves - 1) / (rec::Wide::kTile * rec::kWaves);
     const uint32_t fill = c->recombine_round / std::max<uint32_t>(1, chunks);
     return std::max<uint32_t>(1, std::min(turns, std::max(fill, turns >= 32 ? 2u : 1u)));
 }
@@ -2628,6 +2646,7 @@ void batch_op_blocks(const Params& P, uint32_t* out) {
     out[kOpGametes] = Gametes::blocks(P);
     out[kOpWordSort] = WordSort::blocks(P);
     out[kOpRecombine] = BatchRecombineNarrow::blocks(P);
+    out[kOpRecombineGroups] = rec::Recombine::blocks(P);
     out[kOpPackDigits] = PackDigits::blocks(P);
     const int cls = f6::trait_class(P.traits);
     out[kOpTraits] = cls == 0   ? Traits2Fixed::blocks(P)
@@ -2654,7 +2673,7 @@ hipError_t launch_batched(const BatchLaunch& L, int op, uint32_t sel, hipStream_
     // 7% at twice its resident grid, so its grid stays resident.
     uint32_t per_cu = std::max<uint32_t>(
         1u, (Op::kThreads >= 1024 ? 2u : 8u) * L.grid_scale_num / L.grid_scale_den);
-    if constexpr (LiveBlocks<Op>::kind == kLiveRecombine) {
+    if constexpr (LiveBlocks<Op>::kind == kLiveRecombine || LiveBlocks<Op>::kind == kLiveGroups) {
         static const uint32_t resident = [] {
             int n = 0;
             const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
@@ -2683,7 +2702,11 @@ hipError_t launch_live_offsets(const BatchLaunch& L, hipStream_t s) {
     return hipGetLastError();
 }
 
+// The word sort and recombination of the last draws.
 hipError_t launch_batched_recombine(const BatchLaunch& L, uint32_t par, hipStream_t s) {
+    if (L.by_group) TRY_LAUNCH(launch_batched<rec::Recombine>(L, kOpRecombineGroups, par, s));
+    if (!L.by_event) return hipSuccess;
+    TRY_LAUNCH(launch_batched<WordSort>(L, kOpWordSort, par, s));
     if (L.wide_events) return launch_batched<BatchRecombineWide>(L, kOpRecombine, par, s);
     return launch_batched<BatchRecombineNarrow>(L, kOpRecombine, par, s);
 }
@@ -2724,7 +2747,6 @@ hipError_t launch_batch_generation(const BatchLaunch& L, uint32_t par, hipStream
     TRY_LAUNCH(launch_batched<Gametes>(L, kOpGametes, par, s));
     TRY_LAUNCH(mark(1));
     TRY_LAUNCH(launch_live_offsets(L, s));
-    TRY_LAUNCH(launch_batched<WordSort>(L, kOpWordSort, par, s));
     TRY_LAUNCH(launch_batched_recombine(L, par, s));
     TRY_LAUNCH(mark(2));
     if (L.traits) {

@@ -106,6 +106,7 @@ struct Params {
     double fit_coeff, fit_inv;
     uint32_t chunks;       // row chunks of the recombination grid
     uint32_t splits;       // column ranges of the recombination grid
+    uint32_t group_words;  // batches: wider rows recombine by groups of gametes (rec::Recombine)
     uint32_t tiles;        // 64-word column tiles at capacity
     uint32_t mut_blocks;   // scan blocks over gametes
     uint32_t free_words;   // words per free-space block: 16 or 64
@@ -179,6 +180,7 @@ enum BatchOp : int {
     kOpGametes,
     kOpWordSort,
     kOpRecombine,
+    kOpRecombineGroups,
     kOpPackDigits,
     kOpTraits,
     kOpFreeReduce,
@@ -190,26 +192,27 @@ enum BatchOp : int {
 
 // Batched ops whose virtual blocks are counted from the child width each
 // generation (live blocks), and their rows of BatchLaunch::live_offs.
-constexpr int kLiveRecombine = 0, kLiveWordSort = 1, kLivePack = 2, kLiveKinds = 3;
+constexpr int kLiveRecombine = 0, kLiveWordSort = 1, kLivePack = 2, kLiveGroups = 3, kLiveKinds = 4;
 
-// Row chunks of a replicate's batched recombination: 1024 rows each, up to
-// about 2048 blocks (half that size and twice the blocks measured 1.20 against
-// 1.12 ms on the 256-replicate workload at generation 200, a quarter and an
-// eighth of the chunks no better).
-inline uint32_t batch_chunks(const Params& P) {
-    uint32_t ch = (4096 + P.tiles - 1) / P.tiles;
-    const uint32_t rows = (P.h + 511) / 512;
-    ch = ch < rows ? ch : rows;
-    return (ch + 1) / 2 > 1 ? (ch + 1) / 2 : 1;
-}
+// Rows wider than this recombine by groups in every batch (as in a single
+// population: 336 words 39 against 50 us, 816 words and more no slower); narrower
+// ones only in batches of at most kSmallBatch groups of 64 gametes per resident
+// block.  A group's tables cost as much as a few hundred words of its rows, so a
+// batch that fills the chip loses by them (256 replicates of mostly 8 to 72
+// words, 97,000 groups: 1.27 against 1.06 ms), while one that does not gains by its
+// smaller blocks (24 replicates, 800 groups: 51 against 141 us).
+constexpr uint32_t kWidePerGroup = 256;
+constexpr uint32_t kSmallBatch = 16;
 
 struct BatchLaunch {
     const RepView* views = nullptr;  // device [R]
     const uint32_t* offs = nullptr;  // device [kOpCount][R + 1]
-    uint32_t* live_offs = nullptr;   // device [kLiveKinds][R + 1]: live blocks of three ops
+    uint32_t* live_offs = nullptr;   // device [kLiveKinds][R + 1]: live blocks of four ops
     uint32_t R = 0;
     uint32_t total[kOpCount] = {};   // offs[k][R]
     uint32_t traits = 0;             // trait count shared by every replicate
+    bool by_group = false;           // some replicate may take rec::Recombine
+    bool by_event = true;            // and some the lookup per event
     bool wide_events = false;        // some replicate keeps more than 64 events per gamete
     uint32_t cus = 1;                // compute units of the device
     // persistent grid per compute unit: the default (2 blocks of 1024

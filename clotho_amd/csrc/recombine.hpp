@@ -1,5 +1,6 @@
 // recombine.hpp — recombination, mutation and free-space partials of one
-// generation of a single population (device code of pipeline.hip).
+// generation of a single population, and of replicates of small batches or wide
+// rows (device code of pipeline.hip).
 //
 // A child word is a select between the two words of its parent individual by
 // the crossover mask {slots j : odd #{events e <= key_j}} (block_crossover with
@@ -40,36 +41,63 @@ namespace rec {
 constexpr uint32_t kThreads = 256;
 constexpr uint32_t kWaves = kThreads / 64;
 constexpr uint32_t kGroup = 64;  // gametes of a group: one bit each of a mask column
-// Events of a group: a group with more is cut after the gametes that fit (a
-// gamete has at most 127).  At rho = 10 a full group has 640 on average.
-constexpr uint32_t kEvents = 768;
 // Position buckets of the sorted events: 0.16 (rho = 5) and 0.3 (rho = 10)
 // events per bucket, so that three comparisons almost always place a slot.
 constexpr uint32_t kBucketBits = 11, kBuckets = 1u << kBucketBits;
-// New mutations of a group, likewise (a gamete has at most 127).
+// New mutations of a group: one with more is cut after the gametes that fit (a
+// gamete has at most 127).
 constexpr uint32_t kMutations = 192;
-constexpr int kMinWaves = 3;           // three blocks per compute unit (LDS)
-constexpr uint32_t kTile = 16;         // words of a wave's tile: one 128-byte line per row
-constexpr uint32_t kPitch = kTile + 2;  // words per gamete row of the mask tile
-constexpr uint32_t kStepRows = 64 * 2 / kTile;       // rows of a step, two words per lane
-constexpr uint32_t kSteps = kGroup / kStepRows;
 
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint64_t u64x2 __attribute__((ext_vector_type(2)));
 
+// The two forms of a block.  Rows of more than kNarrowWords words: each wave
+// makes and uses mask tiles of its own, kTile words (a 128-byte line) of all 64
+// gametes.  Narrower rows: the waves share one mask tile of whole rows, and each
+// produces a quarter of the group's rows.  kEvents: a group with more is cut, like
+// one with many mutations; at rho = 10 a full group has 640 on average.
+constexpr uint32_t kNarrowWords = 32;
+struct Wide {
+    static constexpr uint32_t kEvents = 768;
+    static constexpr uint32_t kTile = 16;
+    static constexpr uint32_t kPitch = kTile + 2;  // words per gamete row of a mask tile
+    static constexpr uint32_t kMaskTiles = kWaves;
+};
+struct Narrow {
+    static constexpr uint32_t kEvents = 576;
+    static constexpr uint32_t kTile = kNarrowWords;
+    static constexpr uint32_t kPitch = kTile + 2;
+    static constexpr uint32_t kMaskTiles = 1;
+};
+
+template <class Form>
 struct Shared {
-    // each wave's mask tile (mask_at); scratch while a table is built
-    alignas(16) uint64_t mask[kWaves][kGroup * kPitch];
-    uint64_t px[kEvents + 4];      // XOR of the gamete bits of the r smallest events
-    uint32_t sorted[kEvents + 4];  // the group's event keys, ascending
+    // mask tiles (mask_at); scratch while a table is built
+    alignas(16) uint64_t mask[Form::kMaskTiles * kGroup * Form::kPitch];
+    uint64_t px[Form::kEvents + 4];      // XOR of the gamete bits of the r smallest events
+    uint32_t sorted[Form::kEvents + 4];  // the group's event keys, ascending
     uint32_t start[kBuckets / 2];  // first event of each bucket, two 16-bit counts per word
     u64x2 ptr[kGroup];             // addresses of each gamete's parent pair and child row
-    f6::u32x4 rec[kGroup];         // {child row, top row, events | mutations << 8, first mutation}
-    uint32_t ev_off[kGroup + 1];   // first event of each gamete, unsorted
     uint32_t mut_off[kGroup + 1];  // first staged mutation of each gamete
     uint32_t mut[kMutations];      // the group's new mutations: slot | gamete << 24
     uint64_t scan[kWaves];
     uint32_t count;                // gametes of the group
+    uint32_t total;                // their events
+};
+// What the table build keeps in the mask tiles.
+template <class Form>
+struct BuildScratch {
+    uint32_t key_in[Form::kEvents];  // keys by gamete
+    uint32_t rank_g[Form::kEvents];  // rank in the bucket | gamete << 16
+    uint32_t key_b[Form::kEvents];   // keys and gametes in bucket order
+    uint32_t g_b[Form::kEvents];
+    uint64_t bits[Form::kEvents];    // gamete bits in key order
+    f6::u32x4 rec[kGroup];           // {child row, top row, events | mutations << 8, first mutation}
+    uint32_t ev_off[kGroup + 1];     // first event of each gamete in key_in
+    static __device__ __forceinline__ BuildScratch& of(Shared<Form>& S) {
+        static_assert(sizeof(BuildScratch) <= sizeof(S.mask), "scratch of the table build");
+        return *reinterpret_cast<BuildScratch*>(S.mask);
+    }
 };
 
 template <class T>
@@ -147,12 +175,13 @@ __device__ __forceinline__ void transpose(uint32_t (&x)[2][4], uint32_t lane) {
     }
 }
 
-// Dword of the mask tile with half h of word w (mod kTile), gamete g: 16 bytes
+// Dword of a mask tile with half h of its word w, gamete g: 16 bytes
 // hold two words, low halves first (what the two words of a lane read at
 // once).  The pitch and the exchanged pairs spread a store of the transpose (64
 // dwords: eight gametes 8 apart, four words, two halves) over all 64 banks.
+template <class Form>
 __device__ __forceinline__ uint32_t mask_at(uint32_t g, uint32_t w, uint32_t h) {
-    return g * (2 * kPitch) + 4 * ((w >> 1) ^ (((g >> 4) << 1) & (kTile / 2 - 1))) + 2 * h + (w & 1u);
+    return g * (2 * Form::kPitch) + 4 * ((w >> 1) ^ (((g >> 4) & 3u) << 1)) + 2 * h + (w & 1u);
 }
 
 // Inclusive scan of v over the wave.
@@ -167,29 +196,43 @@ __device__ __forceinline__ uint32_t wave_scan(uint32_t v, uint32_t lane) {
 
 // The group's records, positions [p0, p0 + n) of the chunk (n <= 64, at least
 // one), cut to the gametes whose events and mutations fit.  Ends with a block barrier.
-__device__ __forceinline__ void load_records(const Buffers& B, Shared& S, uint32_t sel, uint32_t wc,
-                                             uint32_t wp, uint32_t p0, uint32_t n) {
+template <class Form>
+__device__ __forceinline__ void load_records(const Params& P, const Buffers& B, Shared<Form>& S,
+                                             uint32_t sel, uint32_t wc, uint32_t wp, uint32_t p0,
+                                             uint32_t n) {
+    BuildScratch<Form>& T = BuildScratch<Form>::of(S);
     const uint32_t tid = threadIdx.x;
     if (tid < 64) {
-        const uint32_t pos = p0 + min(tid, n - 1);  // lanes past the end repeat the last gamete
-        f6::u32x4 r = ((const __attribute__((address_space(1))) f6::u32x4*)B.by_parent)[pos];
+        const uint32_t pos = p0 + min(tid, n - 1);
+        f6::u32x4 r;
+        if (B.by_parent) {
+            r = ((const __attribute__((address_space(1))) f6::u32x4*)B.by_parent)[pos];
+        } else {
+            r.x = pos;
+            r.y = gl(B.top)[pos];
+            r.z = gl(B.n_events)[pos] | (gl(B.mut_count)[pos] << 8);
+            r.w = gl(B.mut_local)[pos] + gl(B.mut_bsum)[pos / kScanBlock];
+        }
         const uint32_t ne = tid < n ? r.z & 0xFFu : 0u;
         const uint32_t nm = tid < n ? r.z >> 8 : 0u;
         const uint32_t ei = wave_scan(ne, tid), mi = wave_scan(nm, tid);
-        const uint64_t fits = __ballot(tid < n && ei <= kEvents && mi <= kMutations);
+        const uint64_t fits = __ballot(tid < n && ei <= Form::kEvents && mi <= kMutations);
         const uint32_t count = (uint32_t)__popcll(fits);  // a prefix of the lanes
-        // lanes past the group repeat its last gamete
+        // lanes past the group repeat its last gamete, into a spare row
         const int src = (int)min(tid, count - 1);
         r.x = (uint32_t)__shfl((int)r.x, src, 64);
         r.y = (uint32_t)__shfl((int)r.y, src, 64);
-        S.rec[tid] = r;
-        S.ptr[tid] = u64x2{(uint64_t)(B.rows[sel] + (size_t)(r.y & ~1u) * wp),
-                           (uint64_t)(B.rows[1 - sel] + (size_t)r.x * wc)};
-        S.ev_off[tid + 1] = ei;
+        T.rec[tid] = r;
+        const uint64_t* const spare = B.fix_part + (size_t)P.max_chunks * P.w_cap;
+        S.ptr[tid] =
+            u64x2{(uint64_t)(B.rows[sel] + (size_t)(r.y & ~1u) * wp),
+                  (uint64_t)(tid < count ? B.rows[1 - sel] + (size_t)r.x * wc : spare)};
+        T.ev_off[tid + 1] = ei;
         S.mut_off[tid + 1] = mi;
-        if (tid == 0) {
-            S.ev_off[0] = S.mut_off[0] = 0;
+        if (tid == 0) T.ev_off[0] = S.mut_off[0] = 0;
+        if (tid == count - 1) {
             S.count = count;
+            S.total = ei;
         }
     } else {
         for (uint32_t i = tid - 64; i < kBuckets / 2; i += kThreads - 64) S.start[i] = 0;
@@ -199,31 +242,26 @@ __device__ __forceinline__ void load_records(const Buffers& B, Shared& S, uint32
 
 // The group's sorted events, bucket starts and prefix XORs (px), and the slots
 // of its new mutations.  Needs load_records; ends with a block barrier.
-__device__ __forceinline__ void build_table(const Params& P, const Buffers& B, Shared& S,
+template <class Form>
+__device__ __forceinline__ void build_table(const Params& P, const Buffers& B, Shared<Form>& S,
                                             uint32_t tid) {
+    constexpr uint32_t kEvents = Form::kEvents;
+    BuildScratch<Form>& T = BuildScratch<Form>::of(S);
     asm volatile("" : "+v"(tid));
     const uint32_t lane = tid & 63;
-    const uint32_t nb = uni(S.count), total = uni(S.ev_off[nb]);
-    // scratch in the mask tile: unsorted keys, then the keys and gametes in
-    // bucket order, and the gamete bits in key order
-    uint32_t* const key_in = reinterpret_cast<uint32_t*>(&S.mask[0][0]);
-    uint32_t* const rank_g = key_in + kEvents;   // rank in the bucket | gamete << 16
-    uint32_t* const key_b = rank_g + kEvents;
-    uint32_t* const g_b = key_b + kEvents;
-    uint64_t* const bits = reinterpret_cast<uint64_t*>(g_b + kEvents);
-    static_assert(sizeof(S.mask) >= kEvents * (16 + 8), "scratch of the table build");
+    const uint32_t nb = uni(S.count), total = uni(S.total);
     // 1: kPerG threads per gamete read its events and count them into buckets
     constexpr uint32_t kPerG = kThreads / kGroup;
     const uint32_t g = tid / kPerG;
     if (g < nb) {
-        const f6::u32x4 r = S.rec[g];
-        const uint32_t ne = r.z & 0xFFu, off = S.ev_off[g];
+        const f6::u32x4 r = T.rec[g];
+        const uint32_t ne = r.z & 0xFFu, off = T.ev_off[g];
         const auto ev = gl(B.events) + (size_t)r.x * P.ev_cap;
         for (uint32_t e = tid & (kPerG - 1); e < ne; e += kPerG) {
             const uint32_t key = ev[e], b = key >> (32 - kBucketBits);
             const uint32_t old = atomicAdd(&S.start[b >> 1], 1u << (16 * (b & 1)));
-            key_in[off + e] = key;
-            rank_g[off + e] = ((old >> (16 * (b & 1))) & 0xFFFFu) | (g << 16);
+            T.key_in[off + e] = key;
+            T.rank_g[off + e] = ((old >> (16 * (b & 1))) & 0xFFFFu) | (g << 16);
         }
         const uint32_t nm = r.z >> 8, mo = S.mut_off[g];
         if (nm) {
@@ -264,23 +302,23 @@ __device__ __forceinline__ void build_table(const Params& P, const Buffers& B, S
     // 3: bucket order, then key order within the bucket (a bucket seldom
     // holds more than one)
     for (uint32_t i = tid; i < total; i += kThreads) {
-        const uint32_t key = key_in[i], rg = rank_g[i];
+        const uint32_t key = T.key_in[i], rg = T.rank_g[i];
         const uint32_t at = start[key >> (32 - kBucketBits)] + (rg & 0xFFFFu);
-        key_b[at] = key;
-        g_b[at] = rg >> 16;
+        T.key_b[at] = key;
+        T.g_b[at] = rg >> 16;
     }
     __syncthreads();
     for (uint32_t i = tid; i < total; i += kThreads) {
-        const uint32_t key = key_b[i], b = key >> (32 - kBucketBits);
+        const uint32_t key = T.key_b[i], b = key >> (32 - kBucketBits);
         const uint32_t s0 = start[b], s1 = b + 1 < kBuckets ? start[b + 1] : total;
         uint32_t at = s0;
         for (uint32_t j = s0; j < s1; ++j) {
-            const uint32_t o = key_b[j];
+            const uint32_t o = T.key_b[j];
             at += (o < key || (o == key && j < i)) ? 1u : 0u;
         }
         S.sorted[at] = key;
         // the last gamete stands for the missing ones of a short group, too
-        bits[at] = (g_b[i] + 1 == nb ? ~(uint64_t)0 : (uint64_t)1) << g_b[i];
+        T.bits[at] = (T.g_b[i] + 1 == nb ? ~(uint64_t)0 : (uint64_t)1) << T.g_b[i];
     }
     __syncthreads();
     // 4: prefix XORs, kPer events per thread.  px[0]: the gametes whose top
@@ -292,7 +330,7 @@ __device__ __forceinline__ void build_table(const Params& P, const Buffers& B, S
 #pragma unroll
         for (uint32_t i = 0; i < kPer; ++i) {
             const uint32_t e = kPer * tid + i;
-            run ^= e < total ? bits[e] : 0;
+            run ^= e < total ? T.bits[e] : 0;
             x[i] = run;
         }
         uint32_t lo = (uint32_t)run, hi = (uint32_t)(run >> 32);
@@ -307,7 +345,7 @@ __device__ __forceinline__ void build_table(const Params& P, const Buffers& B, S
         }
         const uint64_t inc = ((uint64_t)hi << 32) | lo;
         if (lane == 63) S.scan[tid >> 6] = inc;
-        const uint64_t swapped = __ballot(S.rec[lane].y & 1u);
+        const uint64_t swapped = __ballot(T.rec[lane].y & 1u);
         __syncthreads();
         uint64_t off = inc ^ run ^ swapped;
         for (uint32_t w = 0; w < (tid >> 6); ++w) off ^= S.scan[w];
@@ -325,15 +363,17 @@ __device__ __forceinline__ void build_table(const Params& P, const Buffers& B, S
     __syncthreads();
 }
 
-// Masks of the tile's words for the group's gametes, four words at a time.  A
-// lookup is a chain of three LDS reads (bucket start, the bucket's first events,
-// prefix mask): the quads go through it staggered, so that the reads of one are
-// in flight while another is compared or transposed.
-__device__ __forceinline__ void tile_masks(const Shared& S, uint32_t* tile,
-                                           const f6::u32x4 (&key)[kTile / 4], uint32_t total,
-                                           uint32_t lane) {
-    constexpr int kQuads = kTile / 4;
+// Masks of kQuads quads of words of a tile for the group's gametes; quad q has
+// the words word(q) .. + 3, and is left out where they are past the tile's
+// words.  A lookup is a chain of three LDS reads (bucket start, the bucket's first
+// events, prefix mask): the quads go through it staggered, so that the reads
+// of one are in flight while another is compared or transposed.
+template <class Form, int kQuads, class Word>
+__device__ __forceinline__ void quad_masks(const Shared<Form>& S, uint32_t* tile,
+                                           const f6::u32x4 (&key)[kQuads], uint32_t words,
+                                           uint32_t lane, Word word) {
     const uint16_t* const start = reinterpret_cast<const uint16_t*>(S.start);
+    const uint32_t total = uni(S.total);
     uint32_t r[kQuads][4], e[kQuads][4][3], x[kQuads][2][4];
     auto find = [&](int q) {
 #pragma unroll
@@ -368,19 +408,19 @@ __device__ __forceinline__ void tile_masks(const Shared& S, uint32_t* tile,
     };
     auto turn = [&](int q) {
         transpose(x[q], lane);
-        const uint32_t at = mask_at((lane & 14u) << 2, 4 * q + (lane >> 4), lane & 1u);
+        const uint32_t at = mask_at<Form>((lane & 14u) << 2, word(q) + (lane >> 4), lane & 1u);
 #pragma unroll
         for (int d = 0; d < 2; ++d)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) tile[at + (4 * d + i) * (2 * kPitch)] = x[q][d][i];
+            for (int i = 0; i < 4; ++i) tile[at + (4 * d + i) * (2 * Form::kPitch)] = x[q][d][i];
     };
 #pragma unroll
     for (int s = 0; s < kQuads + 3; ++s) {
-        if (s < kQuads) find(s);
-        if (s >= 1 && s - 1 < kQuads) read(s - 1);
+        if (s < kQuads && word(s) < words) find(s);
+        if (s >= 1 && s - 1 < kQuads && word(s - 1) < words) read(s - 1);
         __builtin_amdgcn_sched_barrier(0);
-        if (s >= 2 && s - 2 < kQuads) count(s - 2);
-        if (s >= 3) turn(s - 3);
+        if (s >= 2 && s - 2 < kQuads && word(s - 2) < words) count(s - 2);
+        if (s >= 3 && word(s - 3) < words) turn(s - 3);
         __builtin_amdgcn_sched_barrier(0);
     }
 }
@@ -402,172 +442,284 @@ __device__ __forceinline__ uint32_t fold_rows(f6::u32x4 x, Op op) {
     return y;
 }
 
-// Blocks: P.chunks ranges of groups x P.splits ranges of column tiles (more
-// than one where the row chunks alone do not fill the chip; every split builds
-// the tables of its chunk).  The waves of a block share the tables and take
-// column tiles of kTile words in turn, each on its own: no barrier in the tile
-// loop, so that the waves of a compute unit drift apart and the lookups of some
-// overlap the row loads and stores of others.
+// A lane of a row access holds two words: the addresses of the pair (t, b) of a
+// parent individual and of the child.
+typedef __attribute__((address_space(1))) uint64_t g_u64;
+__device__ __forceinline__ void load_pair(uint64_t pair, uint32_t wp, uint32_t col, f6::u32x4& t,
+                                          f6::u32x4& b) {
+    t = *(const f6::g_u32x4*)((const g_u64*)pair + col);
+    b = *(const f6::g_u32x4*)((const g_u64*)pair + (size_t)wp + col);
+}
+// first word of the lane's pair in the parent row: in bounds for words past it
+__device__ __forceinline__ uint32_t parent_column(uint32_t w, uint32_t wp) {
+    return wp ? min(w, wp - 2) : 0u;
+}
+// Words are (low, high) pairs in rows, low and high pairs in masks.
+__device__ __forceinline__ f6::u32x4 child_words(f6::u32x4 m, f6::u32x4 b, f6::u32x4 t,
+                                                 f6::u32x4 keep) {
+    return f6::u32x4{select32(m.x, b.x, t.x), select32(m.z, b.y, t.y), select32(m.y, b.z, t.z),
+                     select32(m.w, b.w, t.w)} &
+           keep;
+}
+__device__ __forceinline__ f6::u32x4 keep_words(const Buffers& B, uint32_t w, uint32_t wp) {
+    const f6::u32x4 fixed = *(const f6::g_u32x4*)(gl(B.fixed_bits) + w);
+    const uint32_t in_parent = w < wp ? ~0u : 0u;
+    return f6::u32x4{~fixed.x & in_parent, ~fixed.y & in_parent, ~fixed.z & in_parent,
+                     ~fixed.w & in_parent};
+}
+__device__ __forceinline__ void store_words(uint64_t row, uint32_t w, f6::u32x4 c) {
+    __builtin_nontemporal_store(c, (f6::g_u32x4*)((g_u64*)row + w));
+}
+// The staged mutations m0 .. m1 - 1 whose word inside(word) takes: the lane that
+// stored the word (owner(gamete, word)) flips the bit there, and every lane that
+// holds it adds the bit to its OR.  The slot was free, so no other row of the
+// population has the bit: the column's AND is zero without it, too.
+template <class Form, class Inside, class Owner>
+__device__ __forceinline__ void flip_mutations(const Shared<Form>& S, uint32_t m0, uint32_t m1,
+                                               uint32_t lane, uint32_t w, f6::u32x4& acc_or,
+                                               Inside inside, Owner owner) {
+    for (uint32_t j = m0; j < m1; j += 64) {
+        const uint32_t e = S.mut[min(j + lane, kMutations - 1)];
+        uint64_t q = __ballot(j + lane < m1 && e != ~0u && inside((e & 0xFFFFFFu) >> 6));
+        for (; q; q &= q - 1) {
+            const uint32_t x = lane_of(e, (uint32_t)__builtin_ctzll(q));
+            const uint32_t g = x >> 24, xw = (x >> 6) & 0x3FFFFu;
+            const uint32_t bit = 1u << (x & 31u), at = (x >> 5) & 3u;
+#pragma unroll
+            for (uint32_t d = 0; d < 4; ++d) acc_or[d] |= w == (xw & ~1u) && at == d ? bit : 0u;
+            if (lane == owner(g, xw))
+                (void)__hip_atomic_fetch_xor((uint64_t*)S.ptr[g].y + xw, (uint64_t)1 << (x & 63),
+                                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+}
+// the lane's 16 bytes of keys for quad words from w on (in bounds past the last word)
+__device__ __forceinline__ f6::u32x4 load_keys(const Params& P, const Buffers& B, uint32_t w,
+                                               uint32_t lane) {
+    const uint32_t at = uni(min(w, P.w_cap - 4)) * 64u;
+    return *(const f6::g_u32x4*)(gl(B.keys) + at + (lane >> 4) * 64 + 4 * chunk_of_lane(lane));
+}
+
+// Positions [c0, c1) of a row chunk: whole groups of gametes but for the last.
+__device__ __forceinline__ void chunk_range(const Params& P, uint32_t chunk, uint32_t& c0,
+                                            uint32_t& c1) {
+    const uint32_t groups = (P.h + kGroup - 1) / kGroup;
+    c0 = kGroup * (uint32_t)((uint64_t)groups * chunk / P.chunks);
+    c1 = min(P.h, kGroup * (uint32_t)((uint64_t)groups * (chunk + 1) / P.chunks));
+}
+__device__ __forceinline__ void neutral_partials(const Params& P, const Buffers& B, uint32_t chunk,
+                                                 uint32_t w0, uint32_t w1) {
+    for (uint32_t w = w0 + threadIdx.x; w < w1; w += kThreads) {
+        gl(B.var_part)[(size_t)chunk * P.w_cap + w] = 0;
+        gl(B.fix_part)[(size_t)chunk * P.w_cap + w] = ~(uint64_t)0;
+    }
+}
+
+// Rows of up to kNarrowWords words.  A row access has FW / 2 lanes per row (FW:
+// the width rounded up to 8, 16 or 32 words), and the wave's kWaveRows rows take
+// FW / 8 steps; their parent words load before the table is built.  The keys of
+// a wave's words are the same for every group.
+__device__ __forceinline__ void narrow_rows(const Params& P, const Buffers& B, Shared<Narrow>& S,
+                                            uint32_t sel, uint32_t chunk, uint32_t wc,
+                                            uint32_t wp) {
+    constexpr uint32_t kWaveRows = kGroup / kWaves, kMaxSteps = kNarrowWords / 8;
+    uint32_t c0, c1;
+    chunk_range(P, chunk, c0, c1);
+    if (c0 >= c1) return neutral_partials(P, B, chunk, 0, wc);
+    uint32_t tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    const uint32_t lane = tid & 63, wave = uni(tid >> 6);
+    const uint32_t lg = wc <= 8 ? 2u : wc <= 16 ? 3u : 4u;  // lanes per row: 4, 8, 16
+    const uint32_t step_rows = 64u >> lg, steps = kWaveRows >> (6 - lg);
+    const uint32_t pair = 2 * (lane & ((1u << lg) - 1)), w = pair < wc ? pair : pair - 8;
+    const uint32_t col = parent_column(w, wp), g0 = wave * kWaveRows + (lane >> lg);
+    uint32_t* const tile = reinterpret_cast<uint32_t*>(S.mask);
+    auto word = [&](int q) { return 4 * (wave + kWaves * (uint32_t)q); };
+    f6::u32x4 key[kMaxSteps / 2];
+#pragma unroll
+    for (int q = 0; q < (int)kMaxSteps / 2; ++q) key[q] = load_keys(P, B, word(q), lane);
+    const f6::u32x4 keep = keep_words(B, w, wp);
+    f6::u32x4 acc_or = {0, 0, 0, 0}, acc_and = {~0u, ~0u, ~0u, ~0u};
+    for (uint32_t p0 = c0; p0 < c1;) {
+        load_records(P, B, S, sel, wc, wp, p0, min(kGroup, c1 - p0));
+        const uint32_t nb = uni(S.count);
+        f6::u32x4 t[kMaxSteps], b[kMaxSteps];
+#pragma unroll
+        for (uint32_t k = 0; k < kMaxSteps; ++k)
+            if (k < steps) load_pair(S.ptr[g0 + step_rows * k].x, wp, col, t[k], b[k]);
+        build_table(P, B, S, tid);
+        quad_masks(S, tile, key, wc, lane, word);
+        __syncthreads();
+#pragma unroll
+        for (uint32_t k = 0; k < kMaxSteps; ++k) {
+            if (k >= steps) break;
+            const uint32_t g = g0 + step_rows * k;
+            const f6::u32x4 m = *(const f6::u32x4*)(tile + mask_at<Narrow>(g, w, 0));
+            const f6::u32x4 c = child_words(m, b[k], t[k], keep);
+            store_words(S.ptr[g].y, w, c);
+            acc_or |= c;
+            acc_and &= c;
+        }
+        const uint32_t r0 = min(nb, wave * kWaveRows), r1 = min(nb, (wave + 1) * kWaveRows);
+        flip_mutations(
+            S, uni(S.mut_off[r0]), uni(S.mut_off[r1]), lane, w, acc_or,
+            [](uint32_t) { return true; },
+            [&](uint32_t g, uint32_t xw) { return ((g & (step_rows - 1)) << lg) | (xw >> 1); });
+        p0 += nb;
+        __syncthreads();  // the tables are free for the next group
+    }
+    // columns over the block's rows
+    uint32_t* const red = tile;  // ORs, then ANDs
+    for (uint32_t i = tid; i < 4 * kNarrowWords; i += kThreads) red[i] = i < 2 * kNarrowWords ? 0u : ~0u;
+    __syncthreads();
+#pragma unroll
+    for (uint32_t d = 0; d < 4; ++d) {
+        atomicOr(&red[2 * w + d], acc_or[d]);
+        atomicAnd(&red[2 * kNarrowWords + 2 * w + d], acc_and[d]);
+    }
+    __syncthreads();
+    if (tid < 2 * wc) {
+        gl((uint32_t*)B.var_part)[2 * (size_t)chunk * P.w_cap + tid] = red[tid];
+        gl((uint32_t*)B.fix_part)[2 * (size_t)chunk * P.w_cap + tid] = red[2 * kNarrowWords + tid];
+    }
+}
+
+// Wider rows, column tiles [t0, t1).  The waves of a block share the tables and
+// take column tiles of kTile words in turn, each on its own: no barrier in the
+// tile loop, so that the waves of a compute unit drift apart and the lookups of
+// some overlap the row loads and stores of others.
 //
 // A tile: the masks of its words go through the wave's LDS tile; then lane =
-// (row, word), kStepRows rows per step, each a full 128-byte line.  The
+// (row, word pair), kStepRows rows per step, each a full 128-byte line.  The
 // parent pairs of a whole tile are in registers: the loads of the next tile are
 // issued as each step's words are consumed and stay in flight while the next
 // tile's masks are made.  Siblings are adjacent: the second load of a pair hits
 // the line of the first.  Every memory operation of the row loop is
 // unconditional (lanes past the row repeat its last eight words, rows past a
-// short group its last row), so that the compiler's wait counts are exact.
+// short group go to a spare row), so that the compiler's wait counts are exact.
+__device__ __forceinline__ void wide_rows(const Params& P, const Buffers& B, Shared<Wide>& S,
+                                          uint32_t sel, uint32_t chunk, uint32_t wc, uint32_t wp,
+                                          uint32_t t0, uint32_t t1) {
+    constexpr uint32_t kTile = Wide::kTile, kQuads = kTile / 4;
+    constexpr uint32_t kStepRows = 128 / kTile, kSteps = kGroup / kStepRows;
+    uint32_t c0, c1;
+    chunk_range(P, chunk, c0, c1);
+    if (c0 >= c1) return neutral_partials(P, B, chunk, kTile * t0, min(wc, kTile * t1));
+    uint32_t tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    const uint32_t lane = tid & 63, wave = uni(tid >> 6);
+    const uint32_t f = lane / (kTile / 2);
+    uint32_t* const tile_mask =
+        reinterpret_cast<uint32_t*>(S.mask) + wave * (2 * kGroup * Wide::kPitch);
+    bool first = true;
+    for (uint32_t p0 = c0; p0 < c1; first = false) {
+        load_records(P, B, S, sel, wc, wp, p0, min(kGroup, c1 - p0));
+        const uint32_t nb = uni(S.count);
+        f6::u32x4 t[kSteps], b[kSteps], key[kQuads];
+        auto tile_keys = [&](uint32_t tile) {
+#pragma unroll
+            for (uint32_t i = 0; i < kQuads; ++i) key[i] = load_keys(P, B, kTile * tile + 4 * i, lane);
+        };
+        // the lane's two words of a tile
+        auto word_of = [&](uint32_t tile) {
+            const uint32_t w = kTile * tile + 2 * (lane & (kTile / 2 - 1));
+            return w < wc ? w : w - 8;
+        };
+        const uint32_t my0 = t0 + wave;
+        {
+            const uint32_t col = parent_column(word_of(min(my0, t1 - 1)), wp);
+#pragma unroll
+            for (uint32_t k = 0; k < kSteps; ++k)
+                load_pair(S.ptr[kStepRows * k + f].x, wp, col, t[k], b[k]);
+            tile_keys(min(my0, t1 - 1));
+        }
+        build_table(P, B, S, tid);
+        const uint32_t nm = uni(S.mut_off[nb]);
+        const uint32_t my_mut = S.mut[min(lane, kMutations - 1)];
+        for (uint32_t tile = my0; tile < t1; tile += kWaves) {
+            uint32_t lane = tid & 63;  // opaque: nothing per lane is hoisted out and held
+            asm volatile("" : "+v"(lane));
+            const uint32_t fold_dword = ((lane >> 3) & 2u) | (lane >> 5);
+            const uint32_t w = word_of(tile);
+            const size_t part = 2 * ((size_t)chunk * P.w_cap + w) + fold_dword;
+            const f6::u32x4 keep = keep_words(B, w, wp);
+            const uint32_t old_or = gl((const uint32_t*)B.var_part)[part];
+            const uint32_t old_and = gl((const uint32_t*)B.fix_part)[part];
+            quad_masks(S, tile_mask, key, kTile, lane, [](int q) { return 4u * (uint32_t)q; });
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            f6::u32x4 acc_or = {0, 0, 0, 0}, acc_and = {~0u, ~0u, ~0u, ~0u};
+            const bool mutated =
+                nm > 64 || __ballot(lane < nm && (my_mut & 0xFFFFFFu) / (64 * kTile) == tile) != 0;
+            // the next tile's loads; after the last tile, one word pair per row
+            const bool next = tile + kWaves < t1;
+            const uint32_t ntile = next ? tile + kWaves : tile;
+            tile_keys(ntile);
+            const uint32_t ncol = next ? parent_column(word_of(ntile), wp) : 0u;
+            f6::u32x4 mask[2];
+            u64x2 ptr[2];
+            auto read_step = [&](uint32_t k) {
+                const uint32_t g = kStepRows * k + f;
+                mask[k & 1] = *(const f6::u32x4*)(tile_mask + mask_at<Wide>(g, w - kTile * tile, 0));
+                ptr[k & 1] = S.ptr[g];
+            };
+            read_step(0);
+#pragma unroll
+            for (uint32_t k = 0; k < kSteps; ++k) {
+                if (k + 1 < kSteps) read_step(k + 1);
+                const u64x2 p = ptr[k & 1];
+                const f6::u32x4 c = child_words(mask[k & 1], b[k], t[k], keep);
+                store_words(p.y, w, c);
+                acc_or |= c;
+                acc_and &= c;
+                load_pair(p.x, wp, ncol, t[k], b[k]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (mutated)
+                flip_mutations(
+                    S, 0, nm, lane, w, acc_or, [&](uint32_t xw) { return xw / kTile == tile; },
+                    [](uint32_t g, uint32_t xw) {
+                        return (g % kStepRows) * (kTile / 2) + (xw % kTile) / 2;
+                    });
+            // lanes of one dword store the same value
+            const uint32_t col_or = fold_rows(acc_or, [](uint32_t x, uint32_t y) { return x | y; });
+            const uint32_t col_and = fold_rows(acc_and, [](uint32_t x, uint32_t y) { return x & y; });
+            gl((uint32_t*)B.var_part)[part] = first ? col_or : col_or | old_or;
+            gl((uint32_t*)B.fix_part)[part] = first ? col_and : col_and & old_and;
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
+        p0 += nb;
+        __syncthreads();  // the tables are free for the next group
+    }
+}
+
+// Blocks: P.chunks ranges of groups x P.splits ranges of column tiles (more
+// than one where the row chunks alone do not fill the chip; every split builds
+// the tables of its chunk); narrow rows have no column tiles.
 struct Recombine {
     static constexpr int kThreads = (int)rec::kThreads;
+    static constexpr int kMinWaves = 3;  // three blocks per compute unit (LDS)
     __host__ __device__ static uint32_t blocks(const Params& P) { return P.chunks * P.splits; }
+    // blocks with work at a child width of wc words
+    __host__ __device__ static uint32_t live(const Params& P, uint32_t wc) {
+        return !wc ? 0u : wc <= kNarrowWords ? P.chunks : P.chunks * P.splits;
+    }
     __device__ static __forceinline__ void run(const Params& P, const Buffers& B, uint32_t sel,
                                                uint32_t blk) {
-        __shared__ Shared S;
+        static_assert(sizeof(Shared<Wide>) >= sizeof(Shared<Narrow>), "one allocation for both");
+        __shared__ alignas(16) char memory[sizeof(Shared<Wide>)];
         const auto st = gl(B.state);
         const uint32_t wc = uni(st->wc), wp = uni(st->wp);  // multiples of eight
-        if (!wc) return;
+        if (blk >= live(P, wc)) return;
+        if (wc <= kNarrowWords)
+            return narrow_rows(P, B, *reinterpret_cast<Shared<Narrow>*>(memory), sel, uni(blk), wc,
+                               wp);
         const uint32_t chunk = uni(blk / P.splits), split = uni(blk % P.splits);
-        const uint32_t tiles = (wc + kTile - 1) / kTile;
+        const uint32_t tiles = (wc + Wide::kTile - 1) / Wide::kTile;
         const uint32_t t0 = split * tiles / P.splits, t1 = (split + 1) * tiles / P.splits;
-        if (t0 == t1) return;
-        uint32_t tid = threadIdx.x;
-        asm volatile("" : "+v"(tid));
-        const uint32_t lane = tid & 63, wave = uni(tid >> 6);
-        // positions [c0, c1): whole groups of gametes but for the last
-        const uint32_t groups = (P.h + kGroup - 1) / kGroup;
-        const uint32_t c0 = kGroup * (uint32_t)((uint64_t)groups * chunk / P.chunks);
-        const uint32_t c1 =
-            min(P.h, kGroup * (uint32_t)((uint64_t)groups * (chunk + 1) / P.chunks));
-        if (c0 >= c1) {  // no rows: neutral partials
-            for (uint32_t w = kTile * t0 + tid; w < min(wc, kTile * t1); w += kThreads) {
-                gl(B.var_part)[(size_t)chunk * P.w_cap + w] = 0;
-                gl(B.fix_part)[(size_t)chunk * P.w_cap + w] = ~(uint64_t)0;
-            }
-            return;
-        }
-        const auto keys = gl(B.keys);
-        const uint32_t f = lane / (kTile / 2);
-        uint32_t* const tile_mask = reinterpret_cast<uint32_t*>(S.mask[wave]);
-        bool first = true;
-        for (uint32_t p0 = c0; p0 < c1; first = false) {
-            load_records(B, S, sel, wc, wp, p0, min(kGroup, c1 - p0));
-            const uint32_t nb = uni(S.count), total = uni(S.ev_off[nb]);
-            f6::u32x4 t[kSteps], b[kSteps], key[kTile / 4];
-            const uint32_t lane_key = (lane >> 4) * 64 + 4 * chunk_of_lane(lane);
-            auto load_keys = [&](uint32_t tile) {
-#pragma unroll
-                for (uint32_t i = 0; i < kTile / 4; ++i) {
-                    const uint32_t w = uni(min(kTile * tile + 4 * i, P.w_cap - 4));
-                    key[i] = *(const f6::g_u32x4*)(keys + w * 64u + lane_key);
-                }
-            };
-            // the lane's two words of a tile
-            auto word_of = [&](uint32_t tile) {
-                const uint32_t w = kTile * tile + 2 * (lane & (kTile / 2 - 1));
-                return w < wc ? w : w - 8;
-            };
-            auto load_pair = [&](uint32_t k, uint64_t pair, uint32_t col) {
-                const auto row = (const __attribute__((address_space(1))) uint64_t*)pair;
-                t[k] = *(const f6::g_u32x4*)(row + col);
-                b[k] = *(const f6::g_u32x4*)(row + (size_t)wp + col);
-            };
-            auto column = [&](uint32_t w) { return wp ? min(w, wp - 2) : 0u; };
-            const uint32_t my0 = t0 + wave;
-            {
-                const uint32_t col = column(word_of(min(my0, t1 - 1)));
-#pragma unroll
-                for (uint32_t k = 0; k < kSteps; ++k) load_pair(k, S.ptr[kStepRows * k + f].x, col);
-                load_keys(min(my0, t1 - 1));
-            }
-            build_table(P, B, S, tid);
-            const uint32_t nm = uni(S.mut_off[nb]);
-            const uint32_t my_mut = S.mut[min(lane, kMutations - 1)];
-            for (uint32_t tile = my0; tile < t1; tile += kWaves) {
-                uint32_t lane = tid & 63;  // opaque: nothing per lane is hoisted out and held
-                asm volatile("" : "+v"(lane));
-                const uint32_t fold_dword = ((lane >> 3) & 2u) | (lane >> 5);
-                const uint32_t w = word_of(tile);
-                const size_t part = (size_t)chunk * P.w_cap + w;
-                const f6::u32x4 fixed = *(const f6::g_u32x4*)(gl(B.fixed_bits) + w);
-                const uint32_t old_or = gl((const uint32_t*)B.var_part)[2 * part + fold_dword];
-                const uint32_t old_and = gl((const uint32_t*)B.fix_part)[2 * part + fold_dword];
-                tile_masks(S, tile_mask, key, total, lane);
-                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                const uint32_t in_parent = w < wp ? ~0u : 0u;
-                f6::u32x4 keep, acc_or = {0, 0, 0, 0}, acc_and = {~0u, ~0u, ~0u, ~0u};
-#pragma unroll
-                for (int e = 0; e < 4; ++e) keep[e] = ~fixed[e] & in_parent;
-                const bool mutated =
-                    nm > 64 ||
-                    __ballot(lane < nm && (my_mut & 0xFFFFFFu) / (64 * kTile) == tile) != 0;
-                // the next tile's loads; after the last tile, one word pair per row
-                const bool next = tile + kWaves < t1;
-                const uint32_t ntile = next ? tile + kWaves : tile;
-                load_keys(ntile);
-                const uint32_t ncol = next ? column(word_of(ntile)) : 0u;
-                f6::u32x4 mask[2];
-                u64x2 ptr[2];
-                auto read_step = [&](uint32_t k) {
-                    const uint32_t g = kStepRows * k + f;
-                    mask[k & 1] = *(const f6::u32x4*)(tile_mask + mask_at(g, w - kTile * tile, 0));
-                    ptr[k & 1] = S.ptr[g];
-                };
-                read_step(0);
-#pragma unroll
-                for (uint32_t k = 0; k < kSteps; ++k) {
-                    if (k + 1 < kSteps) read_step(k + 1);
-                    const f6::u32x4 m = mask[k & 1];
-                    const u64x2 p = ptr[k & 1];
-                    // words are (low, high) pairs in rows, low and high pairs in masks
-                    f6::u32x4 c = {select32(m.x, b[k].x, t[k].x), select32(m.z, b[k].y, t[k].y),
-                                   select32(m.y, b[k].z, t[k].z), select32(m.w, b[k].w, t[k].w)};
-                    c &= keep;
-                    __builtin_nontemporal_store(
-                        c, (f6::g_u32x4*)((__attribute__((address_space(1))) uint64_t*)p.y + w));
-                    acc_or |= c;
-                    acc_and &= c;
-                    load_pair(k, p.x, ncol);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-                // New mutations of the tile (few): the lane that stored the word
-                // flips the bit there.  The slot was free, so no other row of the
-                // population has the bit: the column's AND is zero without it, too.
-                if (mutated) {
-                    // rows of a short group were stored by several lanes: vmcnt(0)
-                    if (nb < kGroup) __builtin_amdgcn_s_waitcnt(0x0F70);
-                    for (uint32_t j = 0; j < nm; j += 64) {
-                        const uint32_t e = S.mut[min(j + lane, kMutations - 1)];
-                        uint64_t q = __ballot(j + lane < nm && e != ~0u &&
-                                              (e & 0xFFFFFFu) / (64 * kTile) == tile);
-                        for (; q; q &= q - 1) {
-                            const uint32_t x = lane_of(e, (uint32_t)__builtin_ctzll(q));
-                            const uint32_t g = x >> 24, xw = (x >> 6) & 0x3FFFFu;
-                            const uint32_t bit = 1u << (x & 31u), at = (x >> 5) & 3u;
-#pragma unroll
-                            for (uint32_t e4 = 0; e4 < 4; ++e4)
-                                acc_or[e4] |= w == (xw & ~1u) && at == e4 ? bit : 0u;
-                            if (lane == (g % kStepRows) * (kTile / 2) + (xw % kTile) / 2)
-                                (void)__hip_atomic_fetch_xor((uint64_t*)S.ptr[g].y + xw,
-                                                             (uint64_t)1 << (x & 63),
-                                                             __ATOMIC_RELAXED,
-                                                             __HIP_MEMORY_SCOPE_AGENT);
-                        }
-                    }
-                }
-                // lanes of one dword store the same value
-                const uint32_t col_or = fold_rows(acc_or, [](uint32_t x, uint32_t y) { return x | y; });
-                const uint32_t col_and =
-                    fold_rows(acc_and, [](uint32_t x, uint32_t y) { return x & y; });
-                gl((uint32_t*)B.var_part)[2 * part + fold_dword] = first ? col_or : col_or | old_or;
-                gl((uint32_t*)B.fix_part)[2 * part + fold_dword] =
-                    first ? col_and : col_and & old_and;
-                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-            }
-            p0 += nb;
-            __syncthreads();  // the tables are free for the next group
-        }
+        if (t0 < t1)
+            wide_rows(P, B, *reinterpret_cast<Shared<Wide>*>(memory), sel, chunk, wc, wp, t0, t1);
     }
 };
 

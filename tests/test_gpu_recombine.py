@@ -43,3 +43,33 @@ def test_groups_and_tiles(n, alleles, mu, rho):
         orc.step()
         compare_gametes(sim, orc, f"generation {g + 1}, {chunks} chunks")
         compare_state(sim, orc, f"generation {g + 1}, {chunks} chunks")
+
+
+@pytest.mark.parametrize("large", [False, True])
+def test_batch_kernels(large):
+    # a batch of few groups recombines by groups throughout; in one of more
+    # than 16 groups per resident block the rows up to 256 words take a
+    # lookup per event: every replicate equals a lone context
+    specs = [(60, 100, 4.0), (33, 1600, 60.0), (50, 2100, 5.0), (40, 16384, 3.0), (41, 16500, 3.0)]
+    if large:
+        specs.append((420_000, 500, 2.0))  # 13,125 groups
+    cfgs, pops = [], []
+    for r, (n, alleles, rho) in enumerate(specs):
+        cfgs.append(api.make_config(n, 20.0 / n, rho, seed=r, replicate=r, traits=1, neutral_p=0.2,
+                                    sigma=0.1, fitness=api.FIT_GAUSSIAN_FIXED, env_sigma=1.0,
+                                    max_alleles=alleles + 2048))
+        rows, pos, eff = _population(min(n, 100), alleles, r)
+        pops.append((rows[np.arange(2 * n) % len(rows)], pos, eff))
+    batch = api.Batch(cfgs)
+    for r, pop in enumerate(pops):
+        batch.replicate(r).set_population(*pop)
+    batch.run(2, mode="graph")
+    batch.run(1, mode="eager")
+    for r, cfg in enumerate(cfgs):
+        lone = api.Simulation(cfg)
+        lone.set_population(*pops[r])
+        lone.run(3)
+        compare_gametes(batch.replicate(r), lone, f"replicate {r}")
+        compare_state(batch.replicate(r), lone, f"replicate {r}")
+        lone.close()
+    batch.close()
