@@ -2369,8 +2369,8 @@ struct RoundRobin<FreeCompact> {
 // replicates into out[kind][0 .. R] (exclusive, out[kind][R] = total) from the
 // child widths the draws set, so the persistent blocks of those ops visit live
 // blocks only.
-__global__ void __launch_bounds__(1024) k_batch_live_offsets(const RepView* __restrict__ views,
-                                                             uint32_t R, uint32_t* __restrict__ out) {
+__device__ __forceinline__ void live_offsets(const RepView* __restrict__ views, uint32_t R,
+                                             uint32_t* __restrict__ out) {
     __shared__ uint32_t s_wave[16];
     __shared__ uint32_t s_carry;
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -2415,11 +2415,26 @@ __global__ void __launch_bounds__(1024) k_batch_live_offsets(const RepView* __re
     }
 }
 
+__global__ void __launch_bounds__(1024) k_batch_live_offsets(const RepView* __restrict__ views,
+                                                             uint32_t R, uint32_t* __restrict__ out) {
+    live_offsets(views, R, out);
+}
+
+// live: the launch's last block makes the live offsets (the selection's block
+// scan only: both follow the draws' counts and attributes and precede the gametes).
 template <class Op>
 __global__ void __launch_bounds__(Op::kThreads)
     __attribute__((amdgpu_waves_per_eu(MinWaves<Op>::value))) k_batched(const RepView* __restrict__ views,
                                                           const uint32_t* __restrict__ offs,
-                                                          uint32_t R, uint32_t sel) {
+                                                          uint32_t R, uint32_t sel,
+                                                          uint32_t* __restrict__ live) {
+    uint32_t grid = gridDim.x;
+    if constexpr (Op::kThreads == 1024 && LiveBlocks<Op>::kind < 0) {
+        if (live) {
+            if (blockIdx.x + 1 == grid) return live_offsets(views, R, live);
+            --grid;
+        }
+    }
     // the replicate offsets in LDS when they fit: every virtual block
     // searches them, and a search in global memory is a chain of dependent loads
     __shared__ uint32_t s_offs[kBatchOffsLds<Op> + 1];
@@ -2434,9 +2449,9 @@ __global__ void __launch_bounds__(Op::kThreads)
     // blocks then mostly belong to one replicate, so the replicate index
     // advances by a step or two and the replicate's descriptor and state
     // reads hit the caches.
-    uint32_t v = blockIdx.x, vend = total, step = gridDim.x;
+    uint32_t v = blockIdx.x, vend = total, step = grid;
     if constexpr (!RoundRobin<Op>::value) {
-        const uint32_t per = (total + gridDim.x - 1) / gridDim.x;
+        const uint32_t per = (total + grid - 1) / grid;
         v = min(total, blockIdx.x * per);
         vend = min(total, v + per);
         step = 1;
@@ -2640,9 +2655,11 @@ hipError_t launch_population_analysis(clotho_ctx* c) {
 void batch_op_blocks(const Params& P, uint32_t* out) {
     out[kOpMutCounts] = MutCounts::blocks(P);
     out[kOpFitnessStats] = FitnessStats::blocks(P);
+    out[kOpDrawCounts] = DrawCounts::blocks(P);
     out[kOpPrepare] = Prepare::blocks(P);
     out[kOpMutAttrs] = MutAttrs::blocks(P);
     out[kOpSelScan] = SelScan::blocks(P);
+    out[kOpDrawAttrs] = DrawAttrs::blocks(P);
     out[kOpSelBlockscan] = SelBlockscan::blocks(P);
     out[kOpGametes] = Gametes::blocks(P);
     out[kOpWordSort] = WordSort::blocks(P);
@@ -2658,15 +2675,16 @@ void batch_op_blocks(const Params& P, uint32_t* out) {
     out[kOpFreeReduce] = FreeReduce::blocks(P);
     out[kOpFreeCompact] = FreeCompact::blocks(P);
     out[kOpFitness] = Fitness::blocks(P);
+    out[kOpCompactFitness] = CompactFitness::blocks(P);
     out[kOpCommit] = Commit::blocks(P);
 }
 
 namespace {
 
 template <class Op>
-hipError_t launch_batched(const BatchLaunch& L, int op, uint32_t sel, hipStream_t s) {
+uint32_t batched_grid(const BatchLaunch& L, int op) {
     const uint32_t total = L.total[op];  // at capacity: the most live blocks
-    if (!total) return hipSuccess;
+    if (!total) return 0;
     // blocks per compute unit.  A grid past residency starts its last blocks
     // late: for the traits blocks (four resident per CU) that measured faster
     // than a resident grid, since the late blocks take the virtual blocks
@@ -2689,17 +2707,47 @@ hipError_t launch_batched(const BatchLaunch& L, int op, uint32_t sel, hipStream_
     // every tile-0 block to the same quarter of the grid.
     uint32_t grid = std::min<uint32_t>(total, per_cu * L.cus);
     if (grid > 1 && !(grid & 1u)) --grid;
+    return grid;
+}
+
+template <class Op>
+hipError_t launch_batched(const BatchLaunch& L, int op, uint32_t sel, hipStream_t s) {
+    const uint32_t grid = batched_grid<Op>(L, op);
+    if (!grid) return hipSuccess;
     const uint32_t* offs = LiveBlocks<Op>::kind >= 0
                                ? L.live_offs + (size_t)LiveBlocks<Op>::kind * (L.R + 1)
                                : L.offs + (size_t)op * (L.R + 1);
-    hipLaunchKernelGGL(k_batched<Op>, dim3(grid), dim3(Op::kThreads), 0, s, L.views, offs, L.R, sel);
+    hipLaunchKernelGGL(k_batched<Op>, dim3(grid), dim3(Op::kThreads), 0, s, L.views, offs, L.R, sel,
+                       (uint32_t*)nullptr);
     return hipGetLastError();
 }
 
-// The live-block offsets of this generation (child widths are set by the
-// draws' Prepare launch), for the word sort, recombination and digit packing.
+// The live-block offsets of the last draws (child widths are set by their
+// Prepare launch), for the word sort, recombination and digit packing.
 hipError_t launch_live_offsets(const BatchLaunch& L, hipStream_t s) {
     hipLaunchKernelGGL(k_batch_live_offsets, dim3(1), dim3(1024), 0, s, L.views, L.R, L.live_offs);
+    return hipGetLastError();
+}
+
+// Two independent ops of 256 threads: one launch where one pass of the grid covers
+// both (24 replicates: 139 -> 125 us per generation with the three pairs in one
+// launch each), otherwise two, whose persistent blocks get even shares of
+// one kind of work (256 replicates: draws 0.38 ms, 0.42 in pairs).
+bool one_pass(const BatchLaunch& L, int op) { return L.total[op] <= 8 * L.cus; }
+template <class A, class C>
+hipError_t launch_batched_pair(const BatchLaunch& L, int op_a, int op_c, int both, uint32_t sel,
+                               hipStream_t s) {
+    if (one_pass(L, both)) return launch_batched<Fused<A, C>>(L, both, sel, s);
+    TRY_LAUNCH(launch_batched<A>(L, op_a, sel, s));
+    return launch_batched<C>(L, op_c, sel, s);
+}
+
+// The selection's block scan and the live-block offsets of this generation, in
+// one launch.
+hipError_t launch_blockscan_offsets(const BatchLaunch& L, uint32_t sel, hipStream_t s) {
+    const uint32_t grid = batched_grid<SelBlockscan>(L, kOpSelBlockscan);
+    hipLaunchKernelGGL(k_batched<SelBlockscan>, dim3(grid + 1), dim3(1024), 0, s, L.views,
+                       L.offs + (size_t)kOpSelBlockscan * (L.R + 1), L.R, sel, L.live_offs);
     return hipGetLastError();
 }
 
@@ -2739,15 +2787,20 @@ hipError_t launch_batch_generation(const BatchLaunch& L, uint32_t par, hipStream
                                    hipEvent_t* marks) {
     auto mark = [&](int i) { return marks ? hipEventRecord(marks[i], s) : hipSuccess; };
     TRY_LAUNCH(mark(0));
-    TRY_LAUNCH(launch_batched<MutCounts>(L, kOpMutCounts, par, s));
-    TRY_LAUNCH(launch_batched<FitnessStats>(L, kOpFitnessStats, par, s));
+    TRY_LAUNCH((launch_batched_pair<MutCounts, FitnessStats>(L, kOpMutCounts, kOpFitnessStats,
+                                                             kOpDrawCounts, par, s)));
     TRY_LAUNCH(launch_batched<Prepare>(L, kOpPrepare, par, s));
-    TRY_LAUNCH(launch_batched<MutAttrs>(L, kOpMutAttrs, par, s));
-    TRY_LAUNCH(launch_batched<SelScan>(L, kOpSelScan, par, s));
-    TRY_LAUNCH(launch_batched<SelBlockscan>(L, kOpSelBlockscan, par, s));
+    TRY_LAUNCH((launch_batched_pair<MutAttrs, SelScan>(L, kOpMutAttrs, kOpSelScan, kOpDrawAttrs,
+                                                       par, s)));
+    // in a large batch the one block of offsets would outlast the scan
+    const bool small = one_pass(L, kOpDrawCounts);
+    if (small)
+        TRY_LAUNCH(launch_blockscan_offsets(L, par, s));
+    else
+        TRY_LAUNCH(launch_batched<SelBlockscan>(L, kOpSelBlockscan, par, s));
     TRY_LAUNCH(launch_batched<Gametes>(L, kOpGametes, par, s));
     TRY_LAUNCH(mark(1));
-    TRY_LAUNCH(launch_live_offsets(L, s));
+    if (!small) TRY_LAUNCH(launch_live_offsets(L, s));
     TRY_LAUNCH(launch_batched_recombine(L, par, s));
     TRY_LAUNCH(mark(2));
     if (L.traits) {
@@ -2757,9 +2810,9 @@ hipError_t launch_batch_generation(const BatchLaunch& L, uint32_t par, hipStream
     }
     TRY_LAUNCH(mark(3));
     TRY_LAUNCH(launch_batched<FreeReduce>(L, kOpFreeReduce, par, s));
-    TRY_LAUNCH(launch_batched<FreeCompact>(L, kOpFreeCompact, par, s));
     TRY_LAUNCH(mark(4));
-    TRY_LAUNCH(launch_batched<Fitness>(L, kOpFitness, par, s));
+    TRY_LAUNCH((launch_batched_pair<FreeCompact, Fitness>(L, kOpFreeCompact, kOpFitness,
+                                                          kOpCompactFitness, par, s)));
     TRY_LAUNCH(launch_batched<Commit>(L, kOpCommit, par, s));
     TRY_LAUNCH(mark(5));
     return hipSuccess;

@@ -173,9 +173,11 @@ struct RepView {
 enum BatchOp : int {
     kOpMutCounts,
     kOpFitnessStats,
+    kOpDrawCounts,  // the two in one launch (small batches)
     kOpPrepare,
     kOpMutAttrs,
     kOpSelScan,
+    kOpDrawAttrs,  // likewise
     kOpSelBlockscan,
     kOpGametes,
     kOpWordSort,
@@ -186,6 +188,7 @@ enum BatchOp : int {
     kOpFreeReduce,
     kOpFreeCompact,
     kOpFitness,
+    kOpCompactFitness,  // likewise
     kOpCommit,
     kOpCount
 };
