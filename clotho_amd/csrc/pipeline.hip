@@ -2910,40 +2910,94 @@ hipError_t launch_allele_counts(clotho_ctx* c, const uint64_t* rows, uint32_t W,
 // rows i < j (pairwise_difference<association_matrix>::eval with the
 // row-grouped evaluator,
 // include/clotho/data_spaces/analysis/pairwise_difference/association_matrix_pairwise_difference.hpp:78-102,
-// row_grouped_pairwise_difference.hpp:25-55).  Block = a 16 x 16 tile of pairs
-// (tiles on or above the diagonal, enumerated row by row), one pair per
-// thread; 64-word chunks of the tile's 16 + 16 rows are staged in LDS with a
-// 65-word row pitch, so the 16 rows a wave reads per word fall in distinct banks.
-constexpr uint32_t kPairTile = 16;
-constexpr uint32_t kPairChunk = 64;
+// row_grouped_pairwise_difference.hpp:25-55).  Block = a 64 x 64 tile of pairs
+// (tiles on or above the diagonal, enumerated row by row) over a range of the
+// words, 4 x 4 pairs per thread: a word pair costs four instructions (two XORs, two
+// counting adds) and half an LDS read, where one pair per thread took two reads
+// and was bound by them (1000 rows of 784 words: 128 -> 79 us; the instructions
+// alone are 45 us).  32-word chunks of the tile's 64 + 64 rows are staged in LDS
+// with a 33-word row pitch, so the 16 rows a wave reads per word fall in
+// distinct banks; the next chunk's loads are in flight meanwhile.  The word
+// ranges fill the chip where the tiles do not; their counts add up in `out`.
+constexpr uint32_t kPairTile = 64;
+constexpr uint32_t kPairChunk = 32;
+constexpr uint32_t kPairBlocks = 1024;  // four per compute unit (LDS)
 
-__global__ void __launch_bounds__(256) k_pairwise(const uint64_t* __restrict__ rows_in, uint32_t W,
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k_pairwise(const uint64_t* __restrict__ rows_in, uint32_t W,
                                                   const uint32_t* __restrict__ sample, uint32_t n,
-                                                  uint32_t tiles, uint32_t* __restrict__ out) {
+                                                  uint32_t tiles, uint32_t splits,
+                                                  uint32_t* __restrict__ out) {
+    constexpr uint32_t kPerThread = 2 * kPairTile * kPairChunk / 256;
     const auto rows = gbl(rows_in);
-    __shared__ uint64_t sa[kPairTile][kPairChunk + 1], sb[kPairTile][kPairChunk + 1];
-    uint32_t t = blockIdx.x, bi = 0;
+    __shared__ uint64_t s_row[2 * kPairTile][kPairChunk + 1];
+    __shared__ size_t s_first[2 * kPairTile];  // first word of each row of the tile
+    uint32_t t = blockIdx.x / splits, bi = 0;
+    const uint32_t split = blockIdx.x % splits;
     while (t >= tiles - bi) {  // uniform: at most `tiles` steps
         t -= tiles - bi;
         ++bi;
     }
     const uint32_t bj = bi + t;
-    const uint32_t ti = threadIdx.x / kPairTile, tj = threadIdx.x % kPairTile;
-    const uint32_t i = bi * kPairTile + ti, j = bj * kPairTile + tj;
-    uint32_t acc = 0;
-    for (uint32_t w0 = 0; w0 < W; w0 += kPairChunk) {
-        for (uint32_t e = threadIdx.x; e < kPairTile * kPairChunk; e += 256) {
-            const uint32_t r = e / kPairChunk, c = e % kPairChunk, w = w0 + c;
-            const uint32_t ia = bi * kPairTile + r, ib = bj * kPairTile + r;
-            sa[r][c] = (ia < n && w < W) ? rows[(size_t)sample[ia] * W + w] : 0;
-            sb[r][c] = (ib < n && w < W) ? rows[(size_t)sample[ib] * W + w] : 0;
+    const uint32_t chunks = (W + kPairChunk - 1) / kPairChunk;
+    const uint32_t c0 = split * chunks / splits, c1 = (split + 1) * chunks / splits;
+    const uint32_t ti = threadIdx.x / 16, tj = threadIdx.x % 16;
+    // rows of the first set, then of the second; rows past the sample read its last
+    if (threadIdx.x < 2 * kPairTile) {
+        const uint32_t r = threadIdx.x;
+        const uint32_t i = r < kPairTile ? bi * kPairTile + r : bj * kPairTile + (r - kPairTile);
+        s_first[r] = (size_t)sample[min(i, n - 1)] * W;
+    }
+    __syncthreads();
+    // the thread's staged words: word lw of rows lr, lr + 8, ...
+    const uint32_t lw = threadIdx.x % kPairChunk, lr = threadIdx.x / kPairChunk;
+    constexpr uint32_t kRowStep = 256 / kPairChunk;
+    uint64_t x[kPerThread];
+    auto load = [&](uint32_t c) {
+        const uint32_t w = c * kPairChunk + lw;
+#pragma unroll
+        for (uint32_t k = 0; k < kPerThread; ++k)
+            x[k] = w < W ? rows[s_first[lr + k * kRowStep] + w] : 0;
+    };
+    uint32_t acc[4][4] = {};
+    if (c0 < c1) load(c0);
+    for (uint32_t c = c0; c < c1; ++c) {
+#pragma unroll
+        for (uint32_t k = 0; k < kPerThread; ++k) s_row[lr + k * kRowStep][lw] = x[k];
+        __syncthreads();
+        if (c + 1 < c1) load(c + 1);
+#pragma unroll 2
+        for (uint32_t q = 0; q < kPairChunk; ++q) {
+            uint64_t a[4], b[4];
+#pragma unroll
+            for (uint32_t i = 0; i < 4; ++i) {
+                a[i] = s_row[ti + 16 * i][q];
+                b[i] = s_row[kPairTile + tj + 16 * i][q];
+            }
+#pragma unroll
+            for (uint32_t i = 0; i < 4; ++i)
+#pragma unroll
+                for (uint32_t j = 0; j < 4; ++j) acc[i][j] += (uint32_t)__popcll(a[i] ^ b[j]);
         }
         __syncthreads();
-#pragma unroll 8
-        for (uint32_t c = 0; c < kPairChunk; ++c) acc += (uint32_t)__popcll(sa[ti][c] ^ sb[tj][c]);
-        __syncthreads();
     }
-    if (i < j && j < n) out[(size_t)i * n - (size_t)i * (i + 1) / 2 + (j - i - 1)] = acc;
+#pragma unroll
+    for (uint32_t p = 0; p < 4; ++p)
+#pragma unroll
+        for (uint32_t q = 0; q < 4; ++q) {
+            const uint32_t i = bi * kPairTile + ti + 16 * p, j = bj * kPairTile + tj + 16 * q;
+            if (i < j && j < n) {
+                uint32_t* const at = out + (size_t)i * n - (size_t)i * (i + 1) / 2 + (j - i - 1);
+                if (splits == 1)
+                    *at = acc[p][q];
+                else
+                    atomicAdd(at, acc[p][q]);
+            }
+        }
+}
+
+__global__ void __launch_bounds__(kBlock) k_zero(uint32_t* out, size_t n) {
+    for (size_t i = blockIdx.x * (size_t)kBlock + threadIdx.x; i < n; i += (size_t)gridDim.x * kBlock)
+        out[i] = 0;
 }
 
 hipError_t launch_pairwise(clotho_ctx* c, const uint64_t* rows, uint32_t W,
@@ -2951,8 +3005,16 @@ hipError_t launch_pairwise(clotho_ctx* c, const uint64_t* rows, uint32_t W,
     const uint32_t tiles = (n + kPairTile - 1) / kPairTile;
     const uint32_t blocks = tiles * (tiles + 1) / 2;
     if (!blocks) return hipSuccess;
-    hipLaunchKernelGGL(k_pairwise, dim3(blocks), dim3(256), 0, c->stream, rows, W, d_sample, n,
-                       tiles, d_out);
+    const uint32_t chunks = (W + kPairChunk - 1) / kPairChunk;
+    const uint32_t splits = std::max(1u, std::min(chunks, kPairBlocks / blocks));
+    const size_t pairs = (size_t)n * (n - 1) / 2;
+    if (splits > 1 && pairs) {
+        hipLaunchKernelGGL(k_zero, dim3((uint32_t)std::min<size_t>(1024, (pairs + kBlock - 1) / kBlock)),
+                           dim3(kBlock), 0, c->stream, d_out, pairs);
+        TRY_LAUNCH(hipGetLastError());
+    }
+    hipLaunchKernelGGL(k_pairwise, dim3(blocks * splits), dim3(256), 0, c->stream, rows, W, d_sample,
+                       n, tiles, splits, d_out);
     return hipGetLastError();
 }
 
