@@ -4,8 +4,8 @@ x 65,536 sites x 16 traits, genotype bits Bernoulli(f_j) with f_j ~ U(0,1)
 variances and pairwise correlation 0.3 (seed 43).
 
 Reports kernel time of the plain FP32 set-bit walk, the FP64 walk, the
-pipeline's exact int8 path (effects quantised to k 2^-q, int8 digit planes
-on int8 MFMA, exact integer sums) and the split-BF16 MFMA contraction (1, 2,
+pipeline's exact path (effects quantised to k 2^-q, base-32 digit planes on
+FP4 x FP6 MFMA, exact sums) and the split-BF16 MFMA contraction (1, 2,
 3 BF16 terms, FP32 accumulation per K chunk, FP64 chunk reduction), the MFMA/plain speedup, and per-trait error
 against an FP64 reference: normwise max_i |z_i - z*_i| / max_i |z*_i| and the
 median elementwise relative error.  "plain" is the dense bit x effect FP32
@@ -89,8 +89,8 @@ def main():
     out["exact_i8_speedup_vs_plain"] = ms32 / msi
     out["exact_i8_err_normwise_max"] = float(ni.max())
     out["exact_i8_err_median_rel_max"] = float(mi.max())
-    # four int8 digit planes per trait: 2 H S (4 T) integer operations executed
-    out["exact_i8_exec_tops"] = 2.0 * h * s * 4 * t / (msi * 1e-3) / 1e12
+    # seven digit planes per trait: 2 H S (7 T) operations executed
+    out["exact_i8_exec_tops"] = 2.0 * h * s * 7 * t / (msi * 1e-3) / 1e12
     out["exact_i8_row_gbps"] = h * (((s + 511) // 512) * 64) / (msi * 1e-3) / 1e9
     for terms in (1, 2, 3):
         zm, msm = api.trait_contract_synthetic(h, freqs, eff, api.TRAITS_MFMA_BF16, seed=42,
