@@ -403,7 +403,8 @@ int clotho_create(const clotho_config* cfg, int device, clotho_ctx** out) {
         P.max_chunks = std::max<uint32_t>(1, std::min<uint32_t>(
                                                  (8192 + P.tiles - 1) / P.tiles, h_cap / 8));
         P.max_chunks = std::max(P.max_chunks, std::min(groups, 2 * c->recombine_round));
-        P.chunks = recombine_chunks(c, P.h);
+        c->by_event = recombine_by_event(P, cfg->rho);
+        P.chunks = std::min(P.max_chunks, recombine_chunks(c, P.h));
         P.splits = recombine_splits(c, P.chunks);
     }
     P.mut_blocks = (P.h + kScanBlock - 1) / kScanBlock;
@@ -1227,9 +1228,12 @@ int clotho_autotune(clotho_ctx* c, uint32_t* chosen_chunks) {
     }
     // whole groups of 64 gametes per chunk, and rounds of resident blocks
     const uint32_t groups = (c->p.h + 63) / 64;
-    for (uint32_t k = 1; k <= 8; ++k)
+    if (c->by_event)  // whole waves of two resident blocks per compute unit
+        for (uint32_t k = 1, two = 2u * (uint32_t)std::max(1, c->prop.multiProcessorCount); k <= 16; ++k)
+            cand.push_back(std::min(c->p.max_chunks, std::max<uint32_t>(1, k * two / c->p.tiles)));
+    for (uint32_t k = 1; k <= 8 && !c->by_event; ++k)
         cand.push_back(std::min<uint32_t>(c->p.max_chunks, (groups + k - 1) / k));
-    for (uint32_t k : {1u, 2u})
+    for (uint32_t k = 1; k <= 2 && !c->by_event; ++k)
         cand.push_back(std::min<uint32_t>(c->p.max_chunks, k * c->recombine_round));
     std::sort(cand.begin(), cand.end());
     cand.erase(std::unique(cand.begin(), cand.end()), cand.end());
@@ -1242,6 +1246,7 @@ int clotho_autotune(clotho_ctx* c, uint32_t* chosen_chunks) {
     hipEvent_t ev[2 * kReps] = {};
     for (hipEvent_t& e : ev) HIP_TRY(c, events.add(&e));
     int reps = kReps, passes = 2;
+    HIP_TRY(c, launch_word_sort(c));
     {
         HIP_TRY(c, launch_recombine(c));
         HIP_TRY(c, hipEventRecord(ev[0], c->stream));

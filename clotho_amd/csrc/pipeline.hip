@@ -591,8 +591,9 @@ struct ParentScatterOp {
 
 // ---------------------------------------------------------------------------
 // Recombination + mutation (+ free-space partials) with a lookup per event and
-// row: the replicates of large batches, up to kWidePerGroup words per row.  Single
-// populations, small batches and wider rows take rec::Recombine.
+// row: the replicates of large batches, up to kWidePerGroup words per row, and
+// large single populations with few events per gamete (recombine_by_event).  The
+// others take rec::Recombine.
 // ---------------------------------------------------------------------------
 // Per-word order statistics, once per generation: the 64 position keys of
 // word w sorted ascending (sorted[w][k]), prefix masks pm[w][c] = bits of the
@@ -663,14 +664,18 @@ struct WordSort {
 //   child = (t & ~mask) | (b & mask), then XOR of this row's new mutations
 // OR/AND of the child words accumulate in registers (free_space_accumulator).
 //
-// Latency structure: the records of 64 rows (top row, event and mutation
-// counts, mutation offset) are loaded with one vector load per field, lane q
-// holding row q, and read back with v_readlane, so the row loop issues no
-// scalar loads.  Rows alternate between two register sets of parent words and
-// event keys (lane e holds key e): the loads of row k + 2 are issued as soon as
-// row k is done and stay in flight while row k + 1 is classified (no register
-// rotation, hence no wait on loads still in flight; three or four sets
-// measured no faster on the same device).  Events are classified
+// Latency structure: with parent-ordered gamete records a wave owns a
+// contiguous segment of positions (without them, positions c0 + wave +
+// kRecWaves j).  The records of 64 positions (child row, top row, event and
+// mutation counts, mutation offset) are loaded with one vector load, lane q
+// holding position j0 + q, and read back with v_readlane, so the row loop
+// issues no scalar loads.  Runs of positions with one parent individual are
+// cut into items of at most kSibs children: an item loads the parent pair
+// once and the event keys of each child (lane e holds key e).  Items
+// alternate between two register sets: the loads of item k + 2 are issued as
+// soon as item k is done and stay in flight while item k + 1 is classified
+// (no register rotation, hence no wait on loads still in flight; three or
+// four sets measured no faster on the same device).  Events are classified
 // kEventGroup at a time so that their LDS lookups overlap; a group is padded
 // with rank-64 entries (pm[64] is all ones), and since #real + #padding =
 // kEventGroup is even, the XOR of the group's prefix masks equals the XOR of
@@ -680,6 +685,9 @@ constexpr int kRecBlock = 64 * kRecWaves;
 // events classified together; any even size keeps the padding parity
 // argument (#real + #padding even), and 2 pads Poisson(5) counts least
 constexpr int kEventGroup = 2;
+// children of one parent individual produced from one load of its row pair
+// (parent-ordered gametes; the batched launches keep child order and take 1)
+constexpr int kSibsOrdered = 3;
 // dword 3 of a raw (stride 0) buffer resource on gfx9-family parts: 32-bit
 // data format, offsets range-checked against num_records in bytes
 constexpr int kBufferWord3 = 0x00020000;
@@ -955,7 +963,7 @@ __device__ __forceinline__ void recombine_folded(const Params& P, const Buffers&
     }
 }
 
-template <bool kWideEvents>
+template <bool kWideEvents, int kSibs>
 struct Recombine {
     static constexpr int kThreads = kRecBlock;
     __host__ __device__ static uint32_t blocks(const Params& P) { return P.tiles * P.chunks; }
@@ -975,6 +983,8 @@ struct Recombine {
         const auto boff = gbl(B.mut_bsum);
         const auto var_part = gbl(B.var_part);
         const auto fix_part = gbl(B.fix_part);
+        const auto by_parent = (const __attribute__((address_space(1))) f6::u32x4*)B.by_parent;
+        const bool ordered = B.by_parent != nullptr;
         const uint32_t bx = blk % P.tiles, by = blk / P.tiles;
         __shared__ __align__(16) uint32_t s_bucket[64 * 64];
         __shared__ __align__(16) uint32_t s_sorted[68 * 64];
@@ -983,7 +993,7 @@ struct Recombine {
         const uint32_t wc = uniform_read(&st->wc);
         const uint32_t w0 = bx * 64;
         if (w0 >= wc) return;  // uniform for the block
-        if constexpr (!kWideEvents) {
+        if constexpr (kSibs == 1 && !kWideEvents) {
             // narrow rows: several rows per wave (tile 0 is the only live tile)
             if (wc <= 32)
                 return recombine_folded(P, B, sel, by, wc <= 8 ? 3u : wc <= 16 ? 4u : 5u, s_bucket,
@@ -1004,52 +1014,104 @@ struct Recombine {
         const uint64_t keep = inpar ? ~fixed_bits[w] : 0;  // also clears columns >= wp
         __syncthreads();
 
-        // rows [c0, c1) of this chunk, interleaved over the waves (wave w takes
-        // c0 + w + 16 k), so a block writes consecutive child rows together
+        // positions [c0, c1) of this row chunk.  With sibling items a wave
+        // takes the contiguous segment [s0, s1), so the children of one parent
+        // meet in one wave; without, the waves interleave (wave w takes
+        // c0 + w + 16 k), so a block writes consecutive child rows together.
         const uint32_t rows_per_chunk = (P.h + P.chunks - 1) / P.chunks;
         const uint32_t c0 = min(P.h, by * rows_per_chunk);
         const uint32_t c1 = min(P.h, c0 + rows_per_chunk);
-        const uint32_t first = c0 + wave;
-        const uint32_t npos = c1 > first ? (c1 - first + kRecWaves - 1) / kRecWaves : 0;
+        uint32_t first, stride, npos;
+        if (kSibs > 1) {
+            const uint32_t seg = (c1 - c0 + kRecWaves - 1) / kRecWaves;
+            first = min(c1, c0 + wave * seg);
+            stride = 1;
+            npos = min(c1, first + seg) - first;
+        } else {
+            first = c0 + wave;
+            stride = kRecWaves;
+            npos = c1 > first ? (c1 - first + kRecWaves - 1) / kRecWaves : 0;
+        }
         uint64_t acc_or = 0, acc_and = ~(uint64_t)0;
 
         for (uint32_t j0 = 0; j0 < npos; j0 += 64) {
             const uint32_t nb = min(64u, npos - j0);
             // gamete record of position j0 + lane (the last one repeated past
-            // the batch): top row (bottom = top ^ 1), events | mutations << 8,
-            // first mutation
-            const uint32_t row0 = first + kRecWaves * j0;
-            const uint32_t pos = row0 + kRecWaves * min(lane, nb - 1);
-            const uint32_t g_top = top_in[pos];
-            const uint32_t g_nx = nev_in[pos] | (count[pos] << 8);
-            const uint32_t g_k0 = local[pos] + boff[pos / kBlock];
+            // the batch): child row, top row (bottom = top ^ 1), events |
+            // mutations << 8, first mutation
+            const uint32_t pos = first + stride * (j0 + min(lane, nb - 1));
+            uint32_t g_row, g_top, g_nx, g_k0;
+            if (ordered) {
+                const f6::u32x4 r = by_parent[pos];
+                g_row = r.x;
+                g_top = r.y;
+                g_nx = r.z;
+                g_k0 = r.w;
+            } else {
+                g_row = pos;
+                g_top = top_in[pos];
+                g_nx = nev_in[pos] | (count[pos] << 8);
+                g_k0 = local[pos] + boff[pos / kBlock];
+            }
+            // items: runs of at most kSibs consecutive positions whose gametes
+            // share the parent individual; one item loads the parent pair once
+            uint64_t items = 0;
+            if (kSibs > 1) {
+                const uint32_t parent_id = g_top >> 1;
+                const uint32_t prev_id = __shfl_up(parent_id, 1, 64);
+                const uint64_t starts = __ballot(lane == 0 || lane >= nb || parent_id != prev_id);
+                const uint64_t upto = lane == 63 ? ~(uint64_t)0 : (((uint64_t)2 << lane) - 1);
+                const uint32_t run0 = 63u - (uint32_t)__builtin_clzll(starts & upto);
+                items = __ballot(lane < nb && (lane - run0) % kSibs == 0);
+            }
+            uint32_t next_q = 0;  // kSibs == 1: every position is an item
             struct Item {
-                uint64_t t, b;  // the row's words of its parent pair
-                uint32_t lo, hi;
+                uint32_t q, len;  // first position (lane) and number of children
+                uint64_t t, b;    // parent rows top-of-first-child and its partner
+                uint32_t lo[kSibs], hi[kSibs];
             };
-            // loads of row q (clamped: issued for every item slot)
-            auto load_item = [&](uint32_t q, Item& it) {
-                const uint32_t qq = min(q, nb - 1);
+            auto next_item = [&](Item& it) {
+                if (kSibs == 1) {
+                    it.q = next_q < nb ? next_q++ : 64u;
+                    it.len = 1;
+                } else if (items) {
+                    it.q = (uint32_t)__builtin_ctzll(items);
+                    items &= items - 1;
+                    it.len = (items ? (uint32_t)__builtin_ctzll(items) : nb) - it.q;
+                } else {
+                    it.q = 64;
+                    it.len = 0;
+                }
+            };
+            // loads of an item (issued for every item slot, indices clamped in bounds)
+            auto load_item = [&](Item& it) {
+                const uint32_t qq = min(it.q, nb - 1);
                 const uint32_t top = lane_read(g_top, qq);
                 it.t = parent[(size_t)top * wp + col];
                 it.b = parent[(size_t)(top ^ 1u) * wp + col];
-                const auto ev = events + (size_t)(row0 + kRecWaves * qq) * ev_cap;
-                it.lo = ev[min(lane, ev_cap - 1)];
-                if (kWideEvents) it.hi = ev[min(lane + 64, ev_cap - 1)];
+#pragma unroll
+                for (int k = 0; k < kSibs; ++k) {
+                    const auto ev = events + (size_t)lane_read(g_row, min(qq + k, nb - 1)) * ev_cap;
+                    it.lo[k] = ev[min(lane, ev_cap - 1)];
+                    if (kWideEvents) it.hi[k] = ev[min(lane + 64, ev_cap - 1)];
+                }
             };
 
-            auto child_row = [&](uint32_t q, const Item& it) {
+            // A child whose top row is the item's bottom row takes the
+            // complemented mask: (b & ~m) | (t & m) = (t & ~~m) | (b & ~m).
+            auto child_row = [&](uint32_t q, uint64_t t, uint64_t b, uint32_t lo, uint32_t hi,
+                                 bool flip) {
                 const uint32_t nx = lane_read(g_nx, q);
                 const uint32_t ne = nx & 0xFFu;
-                uint64_t m = 0;
+                uint64_t m = flip ? ~(uint64_t)0 : 0;
                 for (uint32_t e = 0; e < ne; e += kEventGroup) {
                     uint32_t key[kEventGroup], p[kEventGroup];
                     bool more[kEventGroup];
 #pragma unroll
                     for (int i = 0; i < kEventGroup; ++i) {
                         const uint32_t x = e + i;
-                        const uint32_t a = lane_read(it.lo, x & 63);
-                        key[i] = (kWideEvents && x >= 64) ? lane_read(it.hi, x & 63) : a;
+                        const uint32_t a = lane_read(lo, x & 63);
+                        key[i] = (kWideEvents && x >= 64) ? lane_read(hi, x & 63) : a;
                     }
                     // byte (key >> 24) & 3 of dword [key >> 26][lane]: one byte read
                     const uint8_t* sb = reinterpret_cast<const uint8_t*>(s_bucket);
@@ -1083,7 +1145,7 @@ struct Recombine {
                     m ^= xm;
                 }
                 // keep clears fixed columns and columns past the parent width in both
-                uint64_t c = ((it.t & ~m) | (it.b & m)) & keep;
+                uint64_t c = ((t & ~m) | (b & m)) & keep;
                 // new mutations of this row (free columns: zero in every parent row)
                 const uint32_t nm = nx >> 8;
                 if (nm) {
@@ -1098,7 +1160,7 @@ struct Recombine {
                     // reads the child rows next runs ~12% faster than after
                     // ordinary write-back stores
                     const __amdgpu_buffer_rsrc_t row = __builtin_amdgcn_make_buffer_rsrc(
-                        child + (size_t)(row0 + kRecWaves * q) * wc, 0, (int)(wc * 8u), kBufferWord3);
+                        child + (size_t)lane_read(g_row, q) * wc, 0, (int)(wc * 8u), kBufferWord3);
                     typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
                     const u32x2 v = {(uint32_t)c, (uint32_t)(c >> 32)};
                     __builtin_amdgcn_raw_buffer_store_b64(v, row, valid ? w * 8u : 0x80000000u, 0,
@@ -1108,15 +1170,32 @@ struct Recombine {
                 acc_and &= c;
             };
 
+            // each child takes the loaded pair in its own strand order
+            auto process_item = [&](const Item& it) {
+                const uint32_t top0 = lane_read(g_top, it.q);
+#pragma unroll
+                for (int k = 0; k < kSibs; ++k) {
+                    if ((uint32_t)k < it.len) {
+                        const uint32_t q = it.q + k;
+                        const bool flip = lane_read(g_top, q) != top0;
+                        child_row(q, it.t, it.b, it.lo[k], kWideEvents ? it.hi[k] : 0u, flip);
+                    }
+                }
+            };
+
             Item iA, iB;
-            load_item(0, iA);
-            load_item(1, iB);
-            for (uint32_t q = 0; q < nb; q += 2) {
-                child_row(q, iA);
-                load_item(q + 2, iA);
-                if (q + 1 >= nb) break;
-                child_row(q + 1, iB);
-                load_item(q + 3, iB);
+            next_item(iA);
+            load_item(iA);
+            next_item(iB);
+            load_item(iB);
+            while (iA.q < 64) {
+                process_item(iA);
+                next_item(iA);
+                load_item(iA);
+                if (iB.q >= 64) break;
+                process_item(iB);
+                next_item(iB);
+                load_item(iB);
             }
         }
         __syncthreads();  // every wave is past its last prefix-mask read
@@ -2163,8 +2242,8 @@ template <class Op>
 struct MinWaves {
     static constexpr int value = 1;
 };
-template <bool W>
-struct MinWaves<Recombine<W>> {
+template <bool W, int K>
+struct MinWaves<Recombine<W, K>> {
     static constexpr int value = 8;
 };
 template <>
@@ -2194,11 +2273,15 @@ CLOTHO_SINGLE(k_parent_scatter, ParentScatter)
 using DrawCounts = Fused<MutCounts, FitnessStats>;
 using DrawAttrs = Fused<MutAttrs, SelScan>;
 using DrawGametes = GametesOp<kTotalsScan>;
+using DrawGametesSort = Fused<DrawGametes, WordSort>;  // recombination by event
 CLOTHO_SINGLE(k_draw_counts, DrawCounts)
 CLOTHO_SINGLE(k_draw_attrs, DrawAttrs)
 CLOTHO_SINGLE(k_draw_gametes, DrawGametes)
-using BatchRecombineNarrow = Recombine<false>;  // at most 64 events per gamete
-using BatchRecombineWide = Recombine<true>;
+CLOTHO_SINGLE(k_draw_gametes_sort, DrawGametesSort)
+CLOTHO_SINGLE(k_word_sort, WordSort)
+using BatchRecombineNarrow = Recombine<false, 1>;  // at most 64 events per gamete
+using BatchRecombineWide = Recombine<true, 1>;
+using RecombineEvents = Recombine<false, kSibsOrdered>;
 // The recombination's blocks are numbered so that each XCD runs a contiguous
 // range of (row chunk, column tile) blocks, i.e. whole row chunks one tile
 // after another: the chunk's gamete records and event keys, which every tile
@@ -2212,6 +2295,7 @@ using BatchRecombineWide = Recombine<true>;
         Op::run(P, B, sel, xcd_contiguous(blockIdx.x, gridDim.x));                              \
     }
 CLOTHO_SINGLE_XCD(k_recombine, rec::Recombine)
+CLOTHO_SINGLE_XCD(k_recombine_events, RecombineEvents)
 #undef CLOTHO_SINGLE_XCD
 CLOTHO_SINGLE(k_pack_digits, PackDigits)
 // by trait class (f6::trait_class: T <= 2, 4, 8, 16, 32)
@@ -2279,8 +2363,8 @@ template <class Op>
 struct LiveBlocks {
     static constexpr int kind = -1;
 };
-template <bool W>
-struct LiveBlocks<Recombine<W>> {
+template <bool W, int K>
+struct LiveBlocks<Recombine<W, K>> {
     // live tiles lt = ceil(wc / 64) x row chunks: u -> tile u mod lt, chunk u / lt
     static constexpr int kind = kLiveRecombine;
     __host__ __device__ static uint32_t count(const Params& P, uint32_t wc) {
@@ -2331,8 +2415,8 @@ template <class Op>
 struct RoundRobin {
     static constexpr bool value = false;
 };
-template <bool W>
-struct RoundRobin<Recombine<W>> {
+template <bool W, int K>
+struct RoundRobin<Recombine<W, K>> {
     static constexpr bool value = true;
 };
 template <int RT, int CLS, bool E>
@@ -2523,7 +2607,10 @@ hipError_t launch_draw(clotho_ctx* c) {
     // themselves; beyond, a one-block scan runs first
     const bool scan_apart = parent_blocks(c->p) > kTotalsLds;
     if (scan_apart) TRY_LAUNCH(launch_single<SelBlockscan>(k_sel_blockscan, c, par));
-    TRY_LAUNCH(launch_single<DrawGametes>(k_draw_gametes, c, par));
+    if (c->by_event)
+        TRY_LAUNCH(launch_single<DrawGametesSort>(k_draw_gametes_sort, c, par));
+    else
+        TRY_LAUNCH(launch_single<DrawGametes>(k_draw_gametes, c, par));
     TRY_LAUNCH(launch_single<DrawParents>(k_draw_parents, c, par));
     if (scan_apart) TRY_LAUNCH(launch_single<ParentBlockscan>(k_parent_blockscan, c, par));
     return launch_single<ParentScatter>(k_parent_scatter, c, par);
@@ -2588,10 +2675,30 @@ hipError_t query_residency(clotho_ctx* c) {
     return hipSuccess;
 }
 
+// A lookup per event and row where the two populations (at capacity) exceed the
+// Infinity Cache and a gamete has few events: its rows are wider (512 bytes per
+// access), it reads a parent pair once for three siblings, and its blocks are
+// smaller, which is worth up to a quarter while the lookups are few.  Measured,
+// generation by event against by groups: N = 12,345, 984 words: 212 against 244
+// us at rho = 0.3, 229 against 241 at 4; N = 40,000, 816 words: 400 against 427 at
+// 0.3, 444 against 434 at 4; N = 100,000, 816 words: 834 against 874 at 0.3, 890
+// against 873 at 3; in the cache (N = 12,345, 328 words) 120 against 123 at 0.3,
+// 131 against 124 at 2; N = 100,000, 40 words: 162 against 153 at 1.
+bool recombine_by_event(const Params& P, double rho) {
+    const double bytes = 2.0 * 8.0 * P.h * P.w_cap;
+    return bytes > 384.0 * (1 << 20) && rho * rho * P.n < 4e5 && P.ev_cap <= 64;
+}
+
 // Row chunks of the recombination: as many as its groups of 64 gametes, up to
 // one round of resident blocks (N = 100,000, 816 words: 768 chunks 0.539 ms,
 // 512 0.591, 1536 0.563; more chunks also make more column partials).
 uint32_t recombine_chunks(const clotho_ctx* c, uint32_t h) {
+    if (c->by_event) {
+        // about 4096 blocks of a column tile each, but at least 32 rows per wave
+        // (a block's order-statistic tables are loaded once per block)
+        const uint32_t tiles = c->p.tiles;
+        return std::max<uint32_t>(1, std::min((4096 + tiles - 1) / tiles, (h + 511) / 512));
+    }
     const uint32_t groups = (h + rec::kGroup - 1) / rec::kGroup;
     return std::max<uint32_t>(1, std::min(groups, c->recombine_round));
 }
@@ -2607,7 +2714,14 @@ uint32_t recombine_splits(const clotho_ctx* c, uint32_t chunks) {
     return std::max<uint32_t>(1, std::min(turns, std::max(fill, turns >= 32 ? 2u : 1u)));
 }
 
+hipError_t launch_word_sort(clotho_ctx* c) {
+    if (!c->by_event) return hipSuccess;
+    return launch_single<WordSort>(k_word_sort, c, (uint32_t)c->cur);
+}
+
 hipError_t launch_recombine(clotho_ctx* c) {
+    if (c->by_event)
+        return launch_single<RecombineEvents>(k_recombine_events, c, (uint32_t)c->cur);
     return launch_single<rec::Recombine>(k_recombine, c, (uint32_t)c->cur);
 }
 

@@ -288,7 +288,8 @@ struct clotho_ctx {
     size_t device_bytes = 0;    // sum of the context's device allocations
     uint32_t next_n = 0;        // offspring individuals of following generations (0: keep)
     uint32_t trait_round = 1;     // blocks of one resident round of the balanced traits kernel
-    uint32_t recombine_round = 1; // and of the recombination
+    uint32_t recombine_round = 1; // and of the recombination by groups
+    bool by_event = false;        // recombination by event (recombine_by_event)
     // launch shapes the autotuner may change (0 / defaults: the built-in choice)
     uint32_t trait_variant = 0;   // traits-pass kernel shape, 1 .. trait_variants()
     uint32_t compact_rows = 8;    // rows per wave step of the column compaction: 4, 8, 16
@@ -299,6 +300,7 @@ struct clotho_ctx {
 namespace clotho {
 // Launch sequences (pipeline.hip).
 hipError_t launch_draw(clotho_ctx* c);
+hipError_t launch_word_sort(clotho_ctx* c);  // order statistics alone, where the recombination reads them
 hipError_t launch_recombine(clotho_ctx* c);
 hipError_t launch_traits(clotho_ctx* c);         // whole traits
 hipError_t launch_traits_pieces(clotho_ctx* c);  // launch_free_reduce sums the pieces
@@ -342,6 +344,7 @@ uint32_t compact_chunks_of(const clotho_ctx* c);
 hipError_t query_residency(clotho_ctx* c);  // sets c->trait_round and c->recombine_round
 // launch shape of the recombination: row chunks for h rows, and the column
 // ranges that go with a number of row chunks
+bool recombine_by_event(const Params& P, double rho);
 uint32_t recombine_chunks(const clotho_ctx* c, uint32_t h);
 uint32_t recombine_splits(const clotho_ctx* c, uint32_t chunks);
 // Column compaction of population [src] into [1 - src] (fixed and lost

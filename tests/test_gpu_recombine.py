@@ -73,3 +73,24 @@ def test_batch_kernels(large):
         compare_state(batch.replicate(r), lone, f"replicate {r}")
         lone.close()
     batch.close()
+
+
+@pytest.mark.parametrize("alleles", [60, 1000, 4700])
+@pytest.mark.parametrize("n,rho", [(20_000, 4.4), (20_000, 4.5), (13_001, 0.5)])
+def test_large_capacity_few_events(n, rho, alleles):
+    # two populations of 131,072 slots exceed the cache: up to rho^2 n = 4e5
+    # (rho = 4.47 at n = 20,000) recombination takes a lookup per event and row
+    cfg = api.make_config(n, 0.01, rho, seed=alleles, traits=1, neutral_p=0.3, sigma=0.1,
+                          fitness=api.FIT_GAUSSIAN_FIXED, env_sigma=1.0, max_alleles=1 << 17)
+    sim, orc = api.Simulation(cfg), oracle.OracleSim(cfg)
+    rows, pos, eff = _population(100, alleles, alleles)
+    rows = rows[np.arange(2 * n) % len(rows)]
+    for x in (sim, orc):
+        x.set_population(rows, pos, eff)
+    for g in range(3):
+        sim.run(1, graph=g == 2)
+        orc.step()
+        if g == 1:
+            sim.autotune()
+    compare_gametes(sim, orc, "generation 3")
+    compare_state(sim, orc, "generation 3")
