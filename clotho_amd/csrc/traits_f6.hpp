@@ -204,20 +204,22 @@ constexpr uint32_t kSegGroups = 512;
 // loads in flight; the clamped last pieces are moved twice, with the same
 // bytes).  As buffer loads: the compiler counts a global (FLAT) load to LDS as
 // an access to either memory, and while one is in flight turns every wait for
-// an LDS read or a row into a wait for everything.
+// an LDS read or a row into a wait for everything.  The buffer starts at the
+// segment's first fragment: the planes of a contraction's rows may take more
+// than the 4 GB that an offset reaches, those of a segment take 88 MB at most.
 template <int VECS>
 struct Stager {
     static constexpr int kPieces = (VECS + 63) / 64;
     static constexpr int kPerWave = (kPieces + 3) / 4;
     __amdgpu_buffer_rsrc_t planes;
-    uint32_t first, wave, lane;
+    uint32_t wave, lane;
     __device__ Stager(const uint4* packed, uint32_t first_stage, uint32_t w, uint32_t l)
-        : planes(__builtin_amdgcn_make_buffer_rsrc((void*)packed, 0, -1, kRawBuffer)),
-          first(first_stage),
+        : planes(__builtin_amdgcn_make_buffer_rsrc((void*)(packed + (size_t)first_stage * VECS), 0, -1,
+                                                   kRawBuffer)),
           wave(w),
           lane(l) {}
     __device__ __forceinline__ void operator()(uint32_t k, u32x4* buf) const {
-        const uint32_t src = (first + k) * (VECS * 16u);
+        const uint32_t src = k * (VECS * 16u);
 #pragma unroll
         for (int j = 0; j < kPerWave; ++j) {
             const uint32_t at = min((wave + 4 * j) * 64, (uint32_t)(VECS - 64));
