@@ -2177,7 +2177,7 @@ struct PackDigits {
 // block, the grid following from Params alone (as the batched launches need).
 template <int RT, int CLS, bool kBalanced>
 struct Traits {
-    using Block = f6::TraitsBlock<RT, CLS>;
+    using Block = f6::TraitsBlock<RT, CLS, kBalanced>;
     static constexpr int kThreads = 256;
     __host__ __device__ static uint32_t blocks(const Params& P) {
         if (!P.traits) return 0u;

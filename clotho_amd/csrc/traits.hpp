@@ -28,14 +28,20 @@ size_t trait_digit_elems(uint32_t traits, uint32_t w_cap);  // uint4 elements
 // int64 elements for the pieces of a balanced launch of at most `round` blocks
 // over up to h rows of up to w_cap words
 size_t trait_piece_elems(uint32_t traits, uint32_t h, uint32_t w_cap, uint32_t round);
-uint32_t exact_round(uint32_t traits);  // blocks of launch_traits_exact on the current device
+// One resident round of the contraction's balanced kernel on the current device
+// (blocks 0: the device could not be asked)
+struct ExactRound {
+    uint32_t blocks = 0, cus = 0;
+};
+ExactRound exact_round(uint32_t traits);
 // most: bound on |effect|
 hipError_t launch_pack_digits(const int32_t* eff, uint32_t traits, uint32_t words, uint32_t sites,
                               uint32_t most, uint4* packed, hipStream_t s);
-// part: trait_piece_elems(traits, h, words, blocks) elements, blocks <= exact_round
+// part: trait_piece_elems(traits, h, words, round.blocks) elements; round: exact_round,
+// or fewer blocks; at most 16 traits
 hipError_t launch_traits_exact(const uint64_t* rows, uint32_t h, uint32_t words, uint32_t most,
                                uint32_t traits, const uint4* packed, int64_t* out, int64_t* part,
-                               uint32_t blocks, hipStream_t s);
+                               const ExactRound& round, hipStream_t s);
 // MFMA contraction (traits_mfma.hip): effects pre-split into `terms` BF16
 // matrices laid out for the kernel; FP64 partials per K chunk reduced in FP64.
 size_t mfma_effect_elems(uint32_t words, int terms);
@@ -81,7 +87,7 @@ struct TraitWorkspace {
     uint4* d_planes = nullptr;   // EXACT_I8: digit planes
     int64_t* d_sum = nullptr;    // EXACT_I8: exact sums of k
     int64_t* d_part = nullptr;   // EXACT_I8: pieces of the row blocks cut along K
-    uint32_t blocks = 0;         // EXACT_I8: blocks of the contraction's launch
+    ExactRound round;            // EXACT_I8
     int q = 0;
 
     int init(const uint64_t* rows, uint32_t h_, uint32_t w_, const double* eff, uint32_t s_,
@@ -120,9 +126,10 @@ struct TraitWorkspace {
                     hipSuccess ||
                 hipMalloc((void**)&d_sum, 8 * (size_t)h * traits) != hipSuccess)
                 return CLOTHO_ERR_HIP;
-            blocks = exact_round(traits);
-            if (!blocks || hipMalloc((void**)&d_part, 8 * trait_piece_elems(traits, h, w, blocks)) !=
-                               hipSuccess)
+            round = exact_round(traits);
+            if (!round.blocks ||
+                hipMalloc((void**)&d_part, 8 * trait_piece_elems(traits, h, w, round.blocks)) !=
+                    hipSuccess)
                 return CLOTHO_ERR_HIP;
             if (hipMemcpy(d_qeff, k.data(), 4 * k.size(), hipMemcpyHostToDevice) != hipSuccess)
                 return CLOTHO_ERR_HIP;
@@ -159,7 +166,7 @@ struct TraitWorkspace {
         if (mode == CLOTHO_TRAITS_EXACT_FP64)
             return launch_traits_walk_fp64(d_rows, h, w, d_eff64, sites, traits, d_z64, st);
         if (mode == CLOTHO_TRAITS_EXACT_I8)
-            return launch_traits_exact(d_rows, h, w, most, traits, d_planes, d_sum, d_part, blocks, st);
+            return launch_traits_exact(d_rows, h, w, most, traits, d_planes, d_sum, d_part, round, st);
         return launch_traits_mfma(d_rows, h, w, d_packed, sites, traits, terms, d_partial, d_z64,
                                   st);
     }

@@ -113,7 +113,9 @@ __device__ inline uint32_t digit_code(int32_t d, bool odd) {
 
 // B fragments: fragment (G * K blocks + q) * NT + nt, column c of the lane
 // (trait c / stride, plane c % stride), for rows of W words, A alleles and
-// effects of at most `most`.  A block packs four fragments, one per wave.
+// effects of at most `most`.  A block packs four fragments, one per wave.  Bound
+// by the latency of its gathers: 32 at once, 12,288 sites x 2 traits 8.1 -> 7.0 us,
+// 4,000 x 16 7.2 -> 5.9.
 __device__ __forceinline__ void pack_block(const int32_t* __restrict__ eff_in, uint32_t T, uint32_t W,
                                            uint32_t A, uint32_t most,
                                            uint4* __restrict__ packed_in, uint32_t block) {
@@ -129,14 +131,19 @@ __device__ __forceinline__ void pack_block(const int32_t* __restrict__ eff_in, u
     const uint32_t c = 16 * nt + (lane & 15);
     const uint32_t t = c / stride, p = c % stride;
     const bool live = t < T && p < P;
+    // every load unconditional and ahead of its use, so that all are in flight
+    int32_t v[32];
+    const auto column = eff + min(t, T - 1);
+#pragma unroll
+    for (uint32_t i = 0; i < 32; ++i)
+        v[i] = A ? column[(size_t)min(site_of(G, q, lane, i), A - 1) * T] : 0;
     // digit p of k: bits 5 p .. 5 p + 4 of k + 16 (32^7 - 1) / 31, less 16 (a
     // balanced digit does not depend on how many planes lie above it)
     uint32_t d[6] = {0, 0, 0, 0, 0, 0};
 #pragma unroll
     for (uint32_t i = 0; i < 32; ++i) {
-        const uint32_t s = site_of(G, q, lane, i);
-        const int32_t v = (live && s < A) ? eff[(size_t)s * T + t] : 0;
-        const uint64_t u = (uint64_t)((int64_t)v + 16ll * (((1ll << 35) - 1) / 31));
+        const int32_t k = site_of(G, q, lane, i) < A ? v[i] : 0;
+        const uint64_t u = (uint64_t)((int64_t)k + 16ll * (((1ll << 35) - 1) / 31));
         const int32_t dg = (int32_t)((u >> (5 * p)) & 31u) - 16;
         const uint32_t code = live ? digit_code(dg, (i >> 3) & 1) : 0u;
         constexpr uint32_t kBits = 6;
@@ -392,9 +399,12 @@ constexpr int stage_in_flight(int s) {
 // in place once its registers were free saved registers, but four traits'
 // rows took 0.37 instead of 0.29 ms).  Fragments are read from LDS two steps
 // ahead of their products, across the stage barriers too: every barrier waits
-// for one stage more than the next.  The last group loads its rows and the
-// last stages once more instead of having a body of its own, which would
-// spill accumulators.
+// for one stage more than the next.  Up to two row tiles the last group is a
+// body of its own, which loads nothing further and has nothing to wait for at its
+// end (with the digit sums' reads in flight at once, 3,000 rows x 1,024 sites x 8
+// traits: two row tiles 12.3 -> 11.3 us, one 10.5 -> 10.2).  With four row
+// tiles that body would spill accumulators, and the last group loads its rows and
+// the last stages once more.
 template <int RT, int NT>
 __device__ __forceinline__ void wave_wide(const uint64_t* __restrict__ rows_in, uint32_t h,
                                           uint32_t W, uint32_t T, uint32_t P,
@@ -448,22 +458,24 @@ __device__ __forceinline__ void wave_wide(const uint64_t* __restrict__ rows_in, 
     u32x2 f1[3];
     read(0, 0, f0[0], f1[0]);
     read(0, 1, f0[1], f1[1]);
-    for (uint32_t G = Ga; G < Gb; ++G) {
+    auto group = [&](uint32_t G, auto is_last) __attribute__((always_inline)) {
+        constexpr bool last = decltype(is_last)::value != 0;
         Rows xn;
 #pragma unroll
         for (int s = 0; s < SPG; ++s) {
             const uint32_t k = (G - Ga) * SPG + s;
             // three stages ahead, into the buffer of the stage before this
             // one, which every wave is done with
-            stage_b(min(k + NB - 1, n_stages - 1), s_b[(s + NB - 1) % NB]);
+            if (!last || s + NB - 1 < SPG)
+                stage_b(min(k + NB - 1, n_stages - 1), s_b[(s + NB - 1) % NB]);
             asm volatile("" ::: "memory");
-            if (s == 0) load_rows(min(G + 1, Gb - 1), xn);
+            if (!last && s == 0) load_rows(min(G + 1, Gb - 1), xn);
             asm volatile("" ::: "memory");
             i32x8 a[RT];
 #pragma unroll
             for (int j = 0; j < STEPS; ++j) {
                 const int q = s * QS + j / NT, nt = j % NT, at = s * STEPS + j;
-                read(s, j + 2, f0[(at + 2) % 3], f1[(at + 2) % 3]);
+                if (!last || at + 2 < SPG * STEPS) read(s, j + 2, f0[(at + 2) % 3], f1[(at + 2) % 3]);
                 if (nt == 0) {
 #pragma unroll
                     for (int r = 0; r < RT; ++r) a[r] = expand_bits(x[r][q >> 2][q & 3]);
@@ -475,35 +487,56 @@ __device__ __forceinline__ void wave_wide(const uint64_t* __restrict__ rows_in, 
                         a[r], b, acc[r][nt], kFp4, kFp6, 0, kScaleOne, 0, kScaleOne);
                 step_barrier();
             }
-            switch (s) {
-                case 0: stage_barrier<stage_in_flight<SPG, RT, Stage::kPerWave>(0), false>(); break;
-                case 1: stage_barrier<stage_in_flight<SPG, RT, Stage::kPerWave>(1), false>(); break;
-                default: stage_barrier<stage_in_flight<SPG, RT, Stage::kPerWave>(2), false>(); break;
+            if constexpr (last) {
+                // the stage after the next complete, where there is one
+                if (s + NB - 1 < SPG)
+                    stage_barrier<Stage::kPerWave, false>();
+                else if (s + 2 < SPG)
+                    stage_barrier<0, false>();
+            } else {
+                switch (s) {
+                    case 0: stage_barrier<stage_in_flight<SPG, RT, Stage::kPerWave>(0), false>(); break;
+                    case 1: stage_barrier<stage_in_flight<SPG, RT, Stage::kPerWave>(1), false>(); break;
+                    default: stage_barrier<stage_in_flight<SPG, RT, Stage::kPerWave>(2), false>(); break;
+                }
             }
         }
-        // the fragment registers rotate by three: move the two read ahead
-        // back to the front
-        constexpr int off = (SPG * STEPS) % 3;
-        if constexpr (off != 0) {
-            const u32x4 a0 = f0[off], a1 = f0[(off + 1) % 3];
-            const u32x2 c0 = f1[off], c1 = f1[(off + 1) % 3];
-            f0[0] = a0;
-            f0[1] = a1;
-            f1[0] = c0;
-            f1[1] = c1;
-        }
+        if constexpr (!last) {
+            // the fragment registers rotate by three: move the two read ahead
+            // back to the front
+            constexpr int off = (SPG * STEPS) % 3;
+            if constexpr (off != 0) {
+                const u32x4 a0 = f0[off], a1 = f0[(off + 1) % 3];
+                const u32x2 c0 = f1[off], c1 = f1[(off + 1) % 3];
+                f0[0] = a0;
+                f0[1] = a1;
+                f1[0] = c0;
+                f1[1] = c1;
+            }
 #pragma unroll
-        for (int r = 0; r < RT; ++r) {
-            x[r][0] = xn[r][0];
-            x[r][1] = xn[r][1];
+            for (int r = 0; r < RT; ++r) {
+                x[r][0] = xn[r][0];
+                x[r][1] = xn[r][1];
+            }
         }
+    };
+    constexpr bool kOwnLast = RT <= 2;
+    for (uint32_t G = Ga; G + (kOwnLast ? 1 : 0) < Gb; ++G) group(G, Int<0>{});
+    if constexpr (kOwnLast) {
+        group(Gb - 1, Int<1>{});
+        // the products stay where they are written: otherwise they are sunk into
+        // the branch of the row tile that needs them, their operands spilled
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) asm volatile("" : "+v"(acc[r][nt]));
     }
-    stage_barrier<0>();  // the repeated last stages are out of the buffers
+    stage_barrier<0>();  // every wave, and any repeated last stage, is done with the buffers
     // Recombine the digit planes (eighths of integers) through a buffer of the
     // wave's own, sixteen rows at a time: register i of lane (m, g) holds row
     // 4 g + i of column m.  Opaque indices as in wave_narrow.
     u32x4* const s_q = wave == 0 ? s_b[0] : wave == 1 ? s_b[1] : wave == 2 ? s_b[2] : s_b[3];
-    static_assert(VECS * 16 >= 16 * 16 * NT * 4, "a buffer holds a row tile's digit sums");
+    static_assert(VECS * 16 >= 16 * 16 * NT * 4 + 32, "a row tile's digit sums, and reads past the last");
     int32_t* const s_w = reinterpret_cast<int32_t*>(s_q);
     uint32_t ol = lane, ob = base;
     asm volatile("" : "+v"(ol), "+s"(ob));
@@ -524,7 +557,9 @@ __device__ __forceinline__ void wave_wide(const uint64_t* __restrict__ rows_in, 
             const uint32_t lr = e / T, t = e % T;
             const int32_t* const src = s_w + lr * (16 * NT) + t * stride;
             int64_t v = 0;
-            for (uint32_t p = 0; p < P; ++p) v += (int64_t)src[p] << (5 * p);
+#pragma unroll
+            for (uint32_t p = 0; p < kMaxPlanes; ++p)  // all reads in flight at once
+                v += (int64_t)(src[p] & (p < P ? -1 : 0)) << (5 * p);
             if (first + lr < h) {
                 const size_t o = (size_t)(first - row0) * T + e;
                 out[o] = add ? out[o] + v : v;
@@ -556,7 +591,9 @@ __device__ __forceinline__ void wave_rows(const uint64_t* rows, uint32_t h, uint
 // Waves per SIMD that the accumulators, the rows and one step's operands of a
 // kernel leave room for (its register limit).
 constexpr int min_waves(int rt, int cls) {
-    return cls == 0 ? (rt >= 5 ? 3 : 4) : cls == 1 ? 3 : 2;
+    if (cls == 0) return rt >= 5 ? 3 : 4;
+    if (cls == 1) return rt <= 2 ? 4 : 3;
+    return cls <= 3 && rt <= 2 ? 3 : 2;
 }
 
 // The work of a balanced launch of B blocks over h rows: row blocks of
@@ -624,7 +661,8 @@ __device__ __forceinline__ void reduce_pieces(const int64_t* __restrict__ part_i
 }
 
 // A block's shared buffers and the body for the population's tile count.
-template <int RT, int CLS>
+// kBalanced: a block of a balanced launch; else one row block.
+template <int RT, int CLS, bool kBalanced>
 struct TraitsBlock {
     static constexpr uint32_t kWaveRows = RT * kTileRows, kBlockRows = 4 * kWaveRows;
     static constexpr int kVecs = CLS == 0   ? kNarrowBlocks * (int)kFragVecs
@@ -635,8 +673,8 @@ struct TraitsBlock {
     static_assert(stage_vecs(4) >= stage_vecs(5) && stage_vecs(4) >= stage_vecs(7),
                   "the stage buffers hold every body's stage");
 
-    // blocks: 0 for one row block per block, else the balanced launch's count
-    // (W, most: wave-uniform, as given to pack_block)
+    // blocks: the balanced launch's count (W, most: wave-uniform, as given to
+    // pack_block)
     __device__ static __forceinline__ void run(const uint64_t* __restrict__ rows, uint32_t h,
                                                uint32_t W, uint32_t most, uint32_t T,
                                                const uint4* __restrict__ packed,
@@ -653,9 +691,9 @@ struct TraitsBlock {
         const uint32_t NG = (W + kGroupWords - 1) / kGroupWords, NT = kernel_tiles(T, P);
         const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
         if (W == 0) {  // no words: every sum is zero
-            const uint64_t n = (uint64_t)h * T, per = blocks ? blocks : gridDim.x;
-            if (blocks)
-                for (uint64_t e = blk * 256ull + threadIdx.x; e < n; e += per * 256ull)
+            const uint64_t n = (uint64_t)h * T;
+            if constexpr (kBalanced)
+                for (uint64_t e = blk * 256ull + threadIdx.x; e < n; e += blocks * 256ull)
                     as_global(out)[e] = 0;
             else
                 for (uint32_t e = threadIdx.x; e < kBlockRows * T; e += 256)
@@ -687,7 +725,7 @@ struct TraitsBlock {
             }
 #undef CLOTHO_F6_BODY
         };
-        if (!blocks) {
+        if constexpr (!kBalanced) {
             piece(blk, 0, NG, out, 0);
             return;
         }

@@ -57,8 +57,17 @@ __global__ void __launch_bounds__(256)
     k_traits_exact(const uint64_t* __restrict__ rows, uint32_t h, uint32_t words, uint32_t most,
                    uint32_t T, const uint4* __restrict__ packed, int64_t* __restrict__ traits,
                    int64_t* __restrict__ part, uint32_t blocks) {
-    f6::TraitsBlock<f6::balanced_tiles(CLS), CLS>::run(rows, h, words, most, T, packed, traits, part,
-                                                       blockIdx.x, blocks);
+    f6::TraitsBlock<f6::balanced_tiles(CLS), CLS, true>::run(rows, h, words, most, T, packed, traits,
+                                                             part, blockIdx.x, blocks);
+}
+
+// one row block of RT row tiles per wave and block
+template <int RT, int CLS>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(f6::min_waves(RT, CLS))))
+    k_traits_rows(const uint64_t* __restrict__ rows, uint32_t h, uint32_t words, uint32_t most,
+                  uint32_t T, const uint4* __restrict__ packed, int64_t* __restrict__ traits) {
+    f6::TraitsBlock<RT, CLS, false>::run(rows, h, words, most, T, packed, traits, nullptr,
+                                         blockIdx.x, 0);
 }
 
 __global__ void __launch_bounds__(256) k_exact_reduce(uint32_t h, uint32_t words, uint32_t T,
@@ -283,47 +292,98 @@ size_t trait_piece_elems(uint32_t traits, uint32_t h, uint32_t w_cap, uint32_t r
 }
 
 namespace {
+// The contraction takes at most 16 traits: classes 0-3.
 typedef void (*ExactKernel)(const uint64_t*, uint32_t, uint32_t, uint32_t, uint32_t, const uint4*, int64_t*,
                             int64_t*, uint32_t);
-ExactKernel exact_kernel(uint32_t traits) {
-    const ExactKernel kernels[f6::kClasses] = {k_traits_exact<0>, k_traits_exact<1>, k_traits_exact<2>,
-                                               k_traits_exact<3>, k_traits_exact<4>};
-    return kernels[f6::trait_class(traits)];
+typedef void (*RowsKernel)(const uint64_t*, uint32_t, uint32_t, uint32_t, uint32_t, const uint4*, int64_t*);
+ExactKernel exact_kernel(int cls) {
+    const ExactKernel kernels[4] = {k_traits_exact<0>, k_traits_exact<1>, k_traits_exact<2>,
+                                    k_traits_exact<3>};
+    return kernels[cls];
+}
+RowsKernel rows_kernel(int cls, uint32_t row_tiles) {
+    const RowsKernel one[4] = {k_traits_rows<1, 0>, k_traits_rows<1, 1>, k_traits_rows<1, 2>,
+                               k_traits_rows<1, 3>};
+    const RowsKernel two[4] = {k_traits_rows<2, 0>, k_traits_rows<2, 1>, k_traits_rows<2, 2>,
+                               k_traits_rows<2, 3>};
+    return row_tiles == 1 ? one[cls] : two[cls];
+}
+
+// The launch over h rows of ng groups and nt column tiles: row tiles per wave, or 0 and
+// the blocks of the balanced launch; the least expected time past the launch itself, in us.  A launch of one row block per block takes its groups' latency
+// or the rows of its fullest compute unit, whichever is longer: small blocks
+// reach every compute unit and have the shorter latency, larger ones read each
+// fragment from LDS for more rows.  The balanced launch divides rows evenly
+// and pays for its pieces, their sums and a second launch.  Constants fitted to
+// launches of 1 to 16 traits, 500 to 65,536 sites and 500 to 200,000 rows, of which
+// the rule takes the fastest form or one within 3%, with few exceptions.  Measured,
+// int8 kernel of a fixed 64 to 256 rows per block (which this path replaced)
+// against one / two row tiles / balanced, whole calls in us: 3,000 rows x
+// 1,024 sites x 8 traits: 12.8 against 10.2 / 11.3 / -; 20,000 x 5,120 x 8: 19.1
+// against 16.3 / 16.3 / -; 80,000 x 2,048 x 5: 20.0 against 16.8 / 16.0 / -;
+// 200,000 x 1,024 x 8: 24.9 against 25.7 / 23.3 / -; 8,000 x 20,000 x 16: 99.9 against
+// 48.5 / 57.7 / 37.8; 200,000 x 65,536 x 16: 816 against 1103 / 808 / 675.
+// One column tile is bound by memory, and row blocks for most of a round reach its
+// rate without being cut: a balanced launch of as many blocks has no pieces
+// (200,000 x 12,288 x 2: 72 us, cut 77).
+struct ExactShape {
+    uint32_t tiles, blocks;
+};
+ExactShape exact_shape(uint32_t h, uint32_t ng, uint32_t nt, uint32_t traits, const ExactRound& round) {
+    const auto rows = [&](uint32_t tiles, double latency, double per_row) {
+        const uint32_t block = 64 * tiles, blocks = (h + block - 1) / block;
+        const uint32_t most = (blocks + round.cus - 1) / round.cus * block;  // of one compute unit
+        return ng * std::max(latency, most * per_row);
+    };
+    const double one = rows(1, 0.45 + 0.19 * nt, 5.0e-3 + 2.2e-3 * nt);
+    const double two = rows(2, 0.50 + 0.24 * nt, 5.0e-3 + 1.4e-3 * nt);
+    const uint32_t direct = one <= two ? 1 : 2;
+    if (h >> 30) return {0, round.blocks};  // a grid of fewer than 2^32 threads
+    if (ng <= 8) return {direct, 0};        // the balanced launch's own cost is as long
+    const f6::Balance bal(h, f6::balanced_block_rows(f6::trait_class(traits)), round.blocks);
+    const double even = (double)ng * h / round.cus * (5.0e-3 + 1.3e-3 * nt);
+    const double pieces = bal.R ? 7.0 + 0.8 / 512 * traits * bal.sharing(ng) : 0.0;
+    if (even + pieces >= std::min(one, two)) return {direct, 0};
+    if (nt == 1 && bal.RB <= bal.B && 4 * bal.RB >= 3 * bal.B && 0.05 * even < pieces)
+        return {0, bal.RB};
+    return {0, bal.B};
 }
 }  // namespace
 
-uint32_t exact_round(uint32_t traits) {
+ExactRound exact_round(uint32_t traits) {
     int device = 0, cus = 0, per_cu = 0;
     if (hipGetDevice(&device) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
         hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &per_cu, reinterpret_cast<const void*>(exact_kernel(traits)), 256, 0) != hipSuccess)
-        return 0;
-    return (uint32_t)std::max(1, cus) * (uint32_t)std::max(1, per_cu);
+            &per_cu, reinterpret_cast<const void*>(exact_kernel(f6::trait_class(traits))), 256, 0) !=
+            hipSuccess)
+        return {};
+    const uint32_t n = (uint32_t)std::max(1, cus);
+    return {n * (uint32_t)std::max(1, per_cu), n};
 }
 
-// The balanced launch needs a second one for the pieces, about 4 us: taken when
-// cutting the last round's R row blocks saves its blocks at least eight groups
-// (about 0.5 us each in a launch that does not fill the chip, more in one that
-// does); else one row block per block.  Measured: 32,584 rows of 5 groups x 4
-// traits 19.9 us direct, 25.4 us cut; 3,824 rows of 12 groups x 7 traits 21.7 us
-// cut (30.1 us with the direct int8 kernel it replaced), 539 rows of 60 groups
-// x 2 traits 20.6 us cut (167 us).
 hipError_t launch_traits_exact(const uint64_t* rows, uint32_t h, uint32_t words, uint32_t most,
                                uint32_t traits, const uint4* packed, int64_t* out, int64_t* part,
-                               uint32_t blocks, hipStream_t s) {
-    const uint32_t block_rows = f6::balanced_block_rows(f6::trait_class(traits));
-    const f6::Balance bal(h, block_rows, blocks);
+                               const ExactRound& round, hipStream_t s) {
+    const int cls = f6::trait_class(traits);
     const uint32_t ng = (words + kGroupWords - 1) / kGroupWords;
-    const uint64_t saved = bal.R && ng ? ng - bal.units(ng) / bal.sharing(ng) : 0;
-    const bool cut = saved >= 8;
-    hipLaunchKernelGGL(exact_kernel(traits), dim3(cut ? blocks : bal.RB), dim3(256), 0, s, rows, h,
-                       words, most, traits, packed, out, part, cut ? blocks : 0u);
+    const uint32_t nt = f6::kernel_tiles(traits, f6::digit_planes(most));
+    const ExactShape shape = exact_shape(h, ng, nt, traits, round);
+    if (shape.tiles) {
+        const uint32_t block_rows = 64 * shape.tiles;
+        hipLaunchKernelGGL(rows_kernel(cls, shape.tiles), dim3((h + block_rows - 1) / block_rows),
+                           dim3(256), 0, s, rows, h, words, most, traits, packed, out);
+        return hipGetLastError();
+    }
+    hipLaunchKernelGGL(exact_kernel(cls), dim3(shape.blocks), dim3(256), 0, s, rows, h, words, most,
+                       traits, packed, out, part, shape.blocks);
     hipError_t e = hipGetLastError();
-    if (e != hipSuccess || !cut) return e;
-    const uint64_t n = (uint64_t)(h - bal.full * blocks * block_rows) * traits;
+    const uint32_t block_rows = f6::balanced_block_rows(cls);
+    const f6::Balance bal(h, block_rows, shape.blocks);
+    if (e != hipSuccess || !bal.R) return e;
+    const uint64_t n = (uint64_t)(h - bal.full * bal.B * block_rows) * traits;
     hipLaunchKernelGGL(k_exact_reduce, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, s, h, words,
-                       traits, blocks, part, out);
+                       traits, bal.B, part, out);
     return hipGetLastError();
 }
 

@@ -38,13 +38,13 @@ constexpr int kMaxDevices = 64;
 std::mutex g_lock;
 struct DeviceEntry {
     uint8_t* scratch = nullptr;
-    uint32_t round[f6::kClasses] = {};  // resident blocks of each trait class's kernel
+    ExactRound round[f6::kClasses];  // of each trait class's kernel
 };
 DeviceEntry g_devices[kMaxDevices];
 
 // the device address of `scratch` on `device` (current) and the resident
 // round of the kernel for `traits`, each looked up once
-int entry_of(int device, uint32_t traits, uint8_t** out, uint32_t* round) {
+int entry_of(int device, uint32_t traits, uint8_t** out, ExactRound* round) {
     std::lock_guard<std::mutex> guard(g_lock);
     DeviceEntry& e = g_devices[device];
     if (!e.scratch) {
@@ -53,9 +53,9 @@ int entry_of(int device, uint32_t traits, uint8_t** out, uint32_t* round) {
             return CLOTHO_ERR_HIP;
         e.scratch = static_cast<uint8_t*>(p);
     }
-    uint32_t& r = e.round[f6::trait_class(traits)];
-    if (!r) r = exact_round(traits);
-    if (!r) return CLOTHO_ERR_HIP;
+    ExactRound& r = e.round[f6::trait_class(traits)];
+    if (!r.blocks) r = exact_round(traits);
+    if (!r.blocks) return CLOTHO_ERR_HIP;
     *out = e.scratch;
     *round = r;
     return CLOTHO_OK;
@@ -80,11 +80,11 @@ extern "C" int clotho_trait_contract_exact_noalloc(const uint64_t* rows, uint32_
     if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= kMaxDevices)
         return CLOTHO_ERR_HIP;
     uint8_t* base = nullptr;
-    uint32_t blocks = 0;
-    const int rc = entry_of(device, traits, &base, &blocks);
+    ExactRound round;
+    const int rc = entry_of(device, traits, &base, &round);
     if (rc != CLOTHO_OK) return rc;
     const size_t fit = kPiecesBytes / (sizeof(int64_t) * f6::piece_elems(traits, 1));
-    if (blocks > fit) blocks = (uint32_t)fit;
+    if (round.blocks > fit) round.blocks = (uint32_t)fit;
     uint4* planes = reinterpret_cast<uint4*>(base);
     int64_t* pieces = reinterpret_cast<int64_t*>(base + kPlanesBytes);
     const hipStream_t s = static_cast<hipStream_t>(stream);
@@ -92,7 +92,7 @@ extern "C" int clotho_trait_contract_exact_noalloc(const uint64_t* rows, uint32_
     const uint32_t most = (uint32_t)kEffectLimit;
     if (launch_pack_digits(effects, traits, words, sites, most, planes, s) != hipSuccess)
         return CLOTHO_ERR_HIP;
-    if (launch_traits_exact(rows, haplotypes, words, most, traits, planes, sums, pieces, blocks, s) !=
+    if (launch_traits_exact(rows, haplotypes, words, most, traits, planes, sums, pieces, round, s) !=
         hipSuccess)
         return CLOTHO_ERR_HIP;
     return CLOTHO_OK;
