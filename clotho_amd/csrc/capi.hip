@@ -194,7 +194,11 @@ int fetch_scaled(clotho_ctx* c, double* dst, const T* src, size_t n, double scal
     return fetch(c, dst, d, 8 * n);
 }
 
-int read_state(clotho_ctx* c, GenState* st) { return fetch(c, st, c->b.state, sizeof(GenState)); }
+int read_state(clotho_ctx* c, GenState* st) {
+    const int rc = fetch(c, st, c->b.state, sizeof(GenState));
+    if (!rc) c->live_words = st->wc;
+    return rc;
+}
 
 int write_state(clotho_ctx* c, const GenState& st) {
     return deliver(c, c->b.state, &st, sizeof(GenState));
@@ -253,6 +257,14 @@ void begin_generation(clotho_ctx* c) {
 void end_generation(clotho_ctx* c) {
     if (c->p.n_par == c->p.n) return;
     c->p.n_par = c->p.n;
+    destroy_graphs(c);
+}
+
+// Launch shapes that follow the population's width (captured launches bake them in).
+void refresh_shapes(clotho_ctx* c) {
+    const bool brief = short_traits(c);
+    if (brief == c->short_traits) return;
+    c->short_traits = brief;
     destroy_graphs(c);
 }
 
@@ -404,6 +416,7 @@ int clotho_create(const clotho_config* cfg, int device, clotho_ctx** out) {
                                                  (8192 + P.tiles - 1) / P.tiles, h_cap / 8));
         P.max_chunks = std::max(P.max_chunks, std::min(groups, 2 * c->recombine_round));
         c->by_event = recombine_by_event(P, cfg->rho);
+        c->short_traits = short_traits(c);
         P.chunks = std::min(P.max_chunks, recombine_chunks(c, P.h));
         P.splits = recombine_splits(c, P.chunks);
     }
@@ -431,7 +444,7 @@ int clotho_create(const clotho_config* cfg, int device, clotho_ctx** out) {
     rc |= dalloc(c, &B.pm, prefix_elems(P.w_cap));
     rc |= dalloc(c, &B.bucket, table_elems(P.w_cap));
     rc |= dalloc(c, &B.digits, trait_digit_elems(std::max<uint32_t>(1, P.traits), P.w_cap));
-    rc |= dalloc(c, &B.trait_part, P.traits ? trait_piece_elems(P.traits, h_cap, P.w_cap, c->trait_round) : 1);
+    rc |= dalloc(c, &B.trait_part, population_piece_elems(c, h_cap));
     rc |= dalloc(c, &B.mut_count, h_cap);
     rc |= dalloc(c, &B.mut_local, h_cap);
     rc |= dalloc(c, &B.mut_bsum, mut_blocks_cap);
@@ -1136,6 +1149,7 @@ int clotho_run(clotho_ctx* c, uint32_t n, int use_graph) {
     for (double& v : tm.ms) v = 0.0;
     tm.generations = 0;
     std::vector<hipEvent_t> marks;
+    refresh_shapes(c);
     // a generation that changes the population size runs with eager launches
     if (c->next_n && c->next_n != c->p.n) use_graph = 0;
     if (use_graph) {

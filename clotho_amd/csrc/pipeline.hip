@@ -2171,13 +2171,14 @@ struct PackDigits {
     }
 };
 
-// RT row tiles (f6::tile_rows) per wave.  kBalanced: P.trait_blocks blocks, one
+// RT row tiles (f6::kTileRows) per wave.  Balanced: P.trait_blocks blocks, one
 // round of resident ones, share the work evenly (f6::Balance) and TraitReduce
 // sums the pieces of the row blocks that were cut; otherwise one row block per
 // block, the grid following from Params alone (as the batched launches need).
-template <int RT, int CLS, bool kBalanced>
+template <int RT, int CLS, f6::Form kForm>
 struct Traits {
-    using Block = f6::TraitsBlock<RT, CLS, kBalanced>;
+    using Block = f6::TraitsBlock<RT, CLS, kForm>;
+    static constexpr bool kBalanced = kForm != f6::Form::kRowBlock;
     static constexpr int kThreads = 256;
     __host__ __device__ static uint32_t blocks(const Params& P) {
         if (!P.traits) return 0u;
@@ -2195,18 +2196,20 @@ struct Traits {
 template <int kBlockThreads>
 struct TraitReduceOp {
     static constexpr int kThreads = kBlockThreads;
+    __host__ __device__ static f6::Balance balance(const Params& P) {
+        return f6::Balance(P.h, P.trait_rows, P.trait_blocks);
+    }
     __host__ __device__ static uint32_t blocks(const Params& P) {
         if (!P.trait_blocks) return 0u;
-        const uint32_t rows = f6::balanced_block_rows(f6::trait_class(P.traits));
-        const f6::Balance bal(P.h, rows, P.trait_blocks);
-        const uint64_t n = (uint64_t)(P.h - bal.full * bal.B * rows) * P.traits;
+        const f6::Balance bal = balance(P);
+        const uint64_t n = (uint64_t)(P.h - bal.full * bal.B * P.trait_rows) * P.traits;
         return bal.R ? (uint32_t)((n + kThreads - 1) / kThreads) : 0u;
     }
     __device__ static __forceinline__ void run(const Params& P, const Buffers& B, uint32_t sel,
                                                uint32_t blk) {
-        const uint32_t rows = f6::balanced_block_rows(f6::trait_class(P.traits));
-        f6::reduce_pieces(B.trait_part, P.h, uniform_read(&gbl(B.state)->wc), P.traits,
-                          f6::Balance(P.h, rows, P.trait_blocks), rows,
+        const bool whole_few = P.traits <= 16 || P.trait_rows == f6::tile_block_rows(1);
+        f6::reduce_pieces(B.trait_part, P.h, uniform_read(&gbl(B.state)->wc), P.traits, balance(P),
+                          P.trait_rows, whole_few ? f6::kFewGroups : 0u,
                           (uint64_t)blk * kThreads + threadIdx.x, B.traits[sel]);
     }
 };
@@ -2250,8 +2253,8 @@ template <>
 struct MinWaves<rec::Recombine> {
     static constexpr int value = rec::Recombine::kMinWaves;
 };
-template <int RT, int CLS, bool E>
-struct MinWaves<Traits<RT, CLS, E>> {
+template <int RT, int CLS, f6::Form F>
+struct MinWaves<Traits<RT, CLS, F>> {
     static constexpr int value = f6::min_waves(RT, CLS);
 };
 
@@ -2299,25 +2302,26 @@ CLOTHO_SINGLE_XCD(k_recombine_events, RecombineEvents)
 #undef CLOTHO_SINGLE_XCD
 CLOTHO_SINGLE(k_pack_digits, PackDigits)
 // by trait class (f6::trait_class: T <= 2, 4, 8, 16, 32)
-using Traits2Balanced = Traits<f6::balanced_tiles(0), 0, true>;
-using Traits4Balanced = Traits<f6::balanced_tiles(1), 1, true>;
-using Traits8Balanced = Traits<f6::balanced_tiles(2), 2, true>;
-using Traits16Balanced = Traits<f6::balanced_tiles(3), 3, true>;
-using Traits32Balanced = Traits<f6::balanced_tiles(4), 4, true>;
+using Traits2Balanced = Traits<f6::balanced_tiles(0), 0, f6::Form::kBalancedFew>;
+using Traits4Balanced = Traits<f6::balanced_tiles(1), 1, f6::Form::kBalancedFew>;
+using Traits8Balanced = Traits<f6::balanced_tiles(2), 2, f6::Form::kBalancedFew>;
+using Traits16Balanced = Traits<f6::balanced_tiles(3), 3, f6::Form::kBalancedFew>;
+using Traits32Balanced = Traits<f6::balanced_tiles(4), 4, f6::Form::kBalanced>;
+using Traits32Short = Traits<1, 4, f6::Form::kBalancedFew>;  // rows of few words (short_traits)
 CLOTHO_SINGLE(k_traits_t2, Traits2Balanced)
 CLOTHO_SINGLE(k_traits_t4, Traits4Balanced)
 CLOTHO_SINGLE(k_traits_t8, Traits8Balanced)
 CLOTHO_SINGLE(k_traits_t16, Traits16Balanced)
 CLOTHO_SINGLE(k_traits_t32, Traits32Balanced)
+CLOTHO_SINGLE(k_traits_t32_short, Traits32Short)
 // the fixed shapes of the batched launches, and the autotuner's alternatives
-using Traits2Fixed = Traits<4, 0, false>;
-using Traits2Two = Traits<2, 0, false>;
-using Traits4Fixed = Traits<4, 1, false>;
-using Traits4Two = Traits<2, 1, false>;
-using Traits8Two = Traits<2, 2, false>;
-using Traits16Two = Traits<2, 3, false>;
-using Traits32Fixed = Traits<2, 4, false>;
-using Traits32One = Traits<1, 4, false>;
+using Traits2Fixed = Traits<4, 0, f6::Form::kRowBlock>;
+using Traits2Two = Traits<2, 0, f6::Form::kRowBlock>;
+using Traits4Fixed = Traits<4, 1, f6::Form::kRowBlock>;
+using Traits4Two = Traits<2, 1, f6::Form::kRowBlock>;
+using Traits8Two = Traits<2, 2, f6::Form::kRowBlock>;
+using Traits16Two = Traits<2, 3, f6::Form::kRowBlock>;
+using Traits32One = Traits<1, 4, f6::Form::kRowBlock>;
 CLOTHO_SINGLE(k_traits_t2_fixed, Traits2Fixed)
 CLOTHO_SINGLE(k_traits_t2_two, Traits2Two)
 CLOTHO_SINGLE(k_traits_t4_fixed, Traits4Fixed)
@@ -2419,8 +2423,8 @@ template <bool W, int K>
 struct RoundRobin<Recombine<W, K>> {
     static constexpr bool value = true;
 };
-template <int RT, int CLS, bool E>
-struct RoundRobin<Traits<RT, CLS, E>> {
+template <int RT, int CLS, f6::Form F>
+struct RoundRobin<Traits<RT, CLS, F>> {
     static constexpr bool value = true;
 };
 template <>
@@ -2637,7 +2641,10 @@ static hipError_t launch_traits_of(clotho_ctx* c, int which, bool pack) {
             default: return launch_single<Traits32One>(k_traits_t32_one, c, sel);
         }
     }
-    c->p.trait_blocks = c->trait_round;
+    const bool brief = cls == 4 && c->short_traits;
+    c->p.trait_blocks = brief ? c->short_round : c->trait_round;
+    c->p.trait_rows = f6::tile_block_rows(brief ? 1 : f6::balanced_tiles(cls));
+    if (brief) return launch_single<Traits32Short>(k_traits_t32_short, c, sel);
     switch (cls) {
         case 0: return launch_single<Traits2Balanced>(k_traits_t2, c, sel);
         case 1: return launch_single<Traits4Balanced>(k_traits_t4, c, sel);
@@ -2668,11 +2675,40 @@ hipError_t query_residency(clotho_ctx* c) {
         Traits2Balanced::kThreads, 0);
     if (e != hipSuccess) return e;
     c->trait_round = (uint32_t)std::max(1, per_cu) * cus;
+    if (f6::trait_class(c->cfg.trait_count) == 4) {
+        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
+            &per_cu, reinterpret_cast<const void*>(k_traits_t32_short), Traits32Short::kThreads, 0);
+        if (e != hipSuccess) return e;
+        c->short_round = (uint32_t)std::max(1, per_cu) * cus;
+    }
     e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
         &per_cu, reinterpret_cast<const void*>(k_recombine), rec::Recombine::kThreads, 0);
     if (e != hipSuccess) return e;
     c->recombine_round = (uint32_t)std::max(1, per_cu) * cus;
     return hipSuccess;
+}
+
+// More than 16 traits: up to 256 words the balanced launch of one row tile per
+// wave, three blocks per compute unit, wider rows the one of two, which reads
+// each fragment from LDS for twice the rows but is alone on its compute unit.
+// Measured, traits and free space, 24 traits, two row tiles against one and the int8
+// kernel both replaced: 40,000 rows x 16 words 28 / 24 / 23 us; 200,000 x 16 75 / 48 /
+// 62; 200,000 x 80 147 / 134 / 184; 60,000 x 256 116 / 119 / 152; 200,000 x 480 530 /
+// 614 / 773.  By the width that the last run left (the capacity before it), as
+// either is right at any width.
+bool short_traits(const clotho_ctx* c) {
+    return c->p.traits > 16 && (c->live_words ? c->live_words : c->p.w_cap) <= 256;
+}
+
+// int64 elements that the pieces of either balanced launch take
+size_t population_piece_elems(const clotho_ctx* c, uint32_t h_cap) {
+    const Params& P = c->p;
+    if (!P.traits) return 1;
+    const uint32_t rows = f6::balanced_block_rows(f6::trait_class(P.traits));
+    const size_t n = trait_piece_elems(P.traits, rows, h_cap, P.w_cap, c->trait_round);
+    return P.traits <= 16 ? n
+                          : std::max(n, trait_piece_elems(P.traits, f6::tile_block_rows(1), h_cap,
+                                                          P.w_cap, c->short_round));
 }
 
 // A lookup per event and row where the two populations (at capacity) exceed the
@@ -2785,7 +2821,7 @@ void batch_op_blocks(const Params& P, uint32_t* out) {
                      : cls == 1 ? Traits4Fixed::blocks(P)
                      : cls == 2 ? Traits8Two::blocks(P)
                      : cls == 3 ? Traits16Two::blocks(P)
-                                : Traits32Fixed::blocks(P);
+                                : Traits32One::blocks(P);
     out[kOpFreeReduce] = FreeReduce::blocks(P);
     out[kOpFreeCompact] = FreeCompact::blocks(P);
     out[kOpFitness] = Fitness::blocks(P);
@@ -2880,7 +2916,7 @@ hipError_t launch_batched_traits(const BatchLaunch& L, uint32_t chi, hipStream_t
         case 1: return launch_batched<Traits4Fixed>(L, kOpTraits, chi, s);
         case 2: return launch_batched<Traits8Two>(L, kOpTraits, chi, s);
         case 3: return launch_batched<Traits16Two>(L, kOpTraits, chi, s);
-        default: return launch_batched<Traits32Fixed>(L, kOpTraits, chi, s);
+        default: return launch_batched<Traits32One>(L, kOpTraits, chi, s);
     }
 }
 

@@ -113,6 +113,7 @@ struct Params {
     uint32_t word_blocks;  // free-space blocks at capacity
     uint32_t max_chunks;   // row-chunk capacity of the partial buffers
     uint32_t trait_blocks; // blocks of the last balanced traits launch (0: another launch)
+    uint32_t trait_rows;   // and the rows of its row blocks
 };
 
 // Device buffers.  Index [c] is the population that is current after the
@@ -288,6 +289,9 @@ struct clotho_ctx {
     size_t device_bytes = 0;    // sum of the context's device allocations
     uint32_t next_n = 0;        // offspring individuals of following generations (0: keep)
     uint32_t trait_round = 1;     // blocks of one resident round of the balanced traits kernel
+    uint32_t short_round = 1;     // and of the one for rows of few words (more than 16 traits)
+    bool short_traits = false;    // which of the two is launched (short_traits)
+    uint32_t live_words = 0;      // row width at the last look at the device's state
     uint32_t recombine_round = 1; // and of the recombination by groups
     bool by_event = false;        // recombination by event (recombine_by_event)
     // launch shapes the autotuner may change (0 / defaults: the built-in choice)
@@ -341,7 +345,9 @@ uint32_t trait_variants(const clotho_ctx* c);
 hipError_t launch_compact_plan(clotho_ctx* c);
 hipError_t launch_compact_rows(clotho_ctx* c, int src);
 uint32_t compact_chunks_of(const clotho_ctx* c);
-hipError_t query_residency(clotho_ctx* c);  // sets c->trait_round and c->recombine_round
+hipError_t query_residency(clotho_ctx* c);  // sets the resident rounds of the context's kernels
+bool short_traits(const clotho_ctx* c);
+size_t population_piece_elems(const clotho_ctx* c, uint32_t h_cap);
 // launch shape of the recombination: row chunks for h rows, and the column
 // ranges that go with a number of row chunks
 bool recombine_by_event(const Params& P, double rho);

@@ -25,9 +25,11 @@ hipError_t launch_traits_walk_fp64(const uint64_t* rows, uint32_t h, uint32_t w,
 // Exact traits of the pipeline (traits_mfma.hip): FP6 digit planes of the
 // quantised effects, exact FP32 MFMA accumulation, int64 recombination.
 size_t trait_digit_elems(uint32_t traits, uint32_t w_cap);  // uint4 elements
-// int64 elements for the pieces of a balanced launch of at most `round` blocks
-// over up to h rows of up to w_cap words
-size_t trait_piece_elems(uint32_t traits, uint32_t h, uint32_t w_cap, uint32_t round);
+// int64 elements for the pieces of a balanced launch of at most `round` blocks of
+// block_rows rows over up to h rows of up to w_cap words
+size_t trait_piece_elems(uint32_t traits, uint32_t block_rows, uint32_t h, uint32_t w_cap,
+                         uint32_t round);
+uint32_t exact_block_rows(uint32_t traits);  // of the contraction's balanced launch
 // One resident round of the contraction's balanced kernel on the current device
 // (blocks 0: the device could not be asked)
 struct ExactRound {
@@ -37,8 +39,8 @@ ExactRound exact_round(uint32_t traits);
 // most: bound on |effect|
 hipError_t launch_pack_digits(const int32_t* eff, uint32_t traits, uint32_t words, uint32_t sites,
                               uint32_t most, uint4* packed, hipStream_t s);
-// part: trait_piece_elems(traits, h, words, round.blocks) elements; round: exact_round,
-// or fewer blocks; at most 16 traits
+// part: trait_piece_elems(traits, exact_block_rows(traits), h, words, round.blocks)
+// elements; round: exact_round, or fewer blocks; at most 16 traits
 hipError_t launch_traits_exact(const uint64_t* rows, uint32_t h, uint32_t words, uint32_t most,
                                uint32_t traits, const uint4* packed, int64_t* out, int64_t* part,
                                const ExactRound& round, hipStream_t s);
@@ -128,7 +130,8 @@ struct TraitWorkspace {
                 return CLOTHO_ERR_HIP;
             round = exact_round(traits);
             if (!round.blocks ||
-                hipMalloc((void**)&d_part, 8 * trait_piece_elems(traits, h, w, round.blocks)) !=
+                hipMalloc((void**)&d_part, 8 * trait_piece_elems(traits, exact_block_rows(traits), h, w,
+                                                            round.blocks)) !=
                     hipSuccess)
                 return CLOTHO_ERR_HIP;
             if (hipMemcpy(d_qeff, k.data(), 4 * k.size(), hipMemcpyHostToDevice) != hipSuccess)

@@ -394,7 +394,7 @@ constexpr int stage_in_flight(int s) {
 }
 
 // Classes 1-4, one wave's share of groups [Ga, Gb): rows base .. base + 16 RT -
-// 1, NT column tiles.  The next group's rows load into registers of their own
+// 1, NT column tiles, NB stage buffers.  The next group's rows load into registers of their own
 // at the group's first stage (whole lines at a time: loading each half line
 // in place once its registers were free saved registers, but four traits'
 // rows took 0.37 instead of 0.29 ms).  Fragments are read from LDS two steps
@@ -405,15 +405,21 @@ constexpr int stage_in_flight(int s) {
 // traits: two row tiles 12.3 -> 11.3 us, one 10.5 -> 10.2).  With four row
 // tiles that body would spill accumulators, and the last group loads its rows and
 // the last stages once more.
-template <int RT, int NT>
+// With two buffers (class 4, one row tile) a stage's loads have one stage of
+// products to land in and its fragments are read from its own barrier on: three
+// blocks per compute unit hide what four buffers, for which LDS holds one block,
+// hid within the wave.
+template <int RT, int NT, int NB>
 __device__ __forceinline__ void wave_wide(const uint64_t* __restrict__ rows_in, uint32_t h,
                                           uint32_t W, uint32_t T, uint32_t P,
                                           const uint4* __restrict__ packed_in,
                                           int64_t* __restrict__ out_in, uint32_t row0,
                                           uint32_t base, uint32_t Ga, uint32_t Gb,
                                           bool add, u32x4* const (&s_b)[4]) {
-    constexpr int QS = stage_blocks(NT), SPG = 8 / QS, NB = 4, VECS = stage_vecs(NT);
+    constexpr int QS = stage_blocks(NT), SPG = 8 / QS, VECS = stage_vecs(NT);
     static_assert(SPG % NB == 0, "every group starts in buffer 0");
+    static_assert(NB == 4 || (NB == 2 && RT <= 2), "with two buffers the last group has its own body");
+    constexpr bool kAhead = NB == 4;
     const auto rows = as_global(rows_in);
     const auto out = as_global(out_in);
     const uint32_t lane = threadIdx.x & 63;
@@ -456,15 +462,17 @@ __device__ __forceinline__ void wave_wide(const uint64_t* __restrict__ rows_in, 
     };
     u32x4 f0[3];
     u32x2 f1[3];
-    read(0, 0, f0[0], f1[0]);
-    read(0, 1, f0[1], f1[1]);
+    if constexpr (kAhead) {
+        read(0, 0, f0[0], f1[0]);
+        read(0, 1, f0[1], f1[1]);
+    }
     auto group = [&](uint32_t G, auto is_last) __attribute__((always_inline)) {
         constexpr bool last = decltype(is_last)::value != 0;
         Rows xn;
 #pragma unroll
         for (int s = 0; s < SPG; ++s) {
             const uint32_t k = (G - Ga) * SPG + s;
-            // three stages ahead, into the buffer of the stage before this
+            // NB - 1 stages ahead, into the buffer of the stage before this
             // one, which every wave is done with
             if (!last || s + NB - 1 < SPG)
                 stage_b(min(k + NB - 1, n_stages - 1), s_b[(s + NB - 1) % NB]);
@@ -472,10 +480,15 @@ __device__ __forceinline__ void wave_wide(const uint64_t* __restrict__ rows_in, 
             if (!last && s == 0) load_rows(min(G + 1, Gb - 1), xn);
             asm volatile("" ::: "memory");
             i32x8 a[RT];
+            if constexpr (!kAhead) {
+                read(s, 0, f0[0], f1[0]);
+                read(s, 1, f0[1], f1[1]);
+            }
 #pragma unroll
             for (int j = 0; j < STEPS; ++j) {
-                const int q = s * QS + j / NT, nt = j % NT, at = s * STEPS + j;
-                if (!last || at + 2 < SPG * STEPS) read(s, j + 2, f0[(at + 2) % 3], f1[(at + 2) % 3]);
+                const int q = s * QS + j / NT, nt = j % NT, at = kAhead ? s * STEPS + j : j;
+                if (kAhead ? !last || at + 2 < SPG * STEPS : j + 2 < STEPS)
+                    read(s, j + 2, f0[(at + 2) % 3], f1[(at + 2) % 3]);
                 if (nt == 0) {
 #pragma unroll
                     for (int r = 0; r < RT; ++r) a[r] = expand_bits(x[r][q >> 2][q & 3]);
@@ -487,7 +500,13 @@ __device__ __forceinline__ void wave_wide(const uint64_t* __restrict__ rows_in, 
                         a[r], b, acc[r][nt], kFp4, kFp6, 0, kScaleOne, 0, kScaleOne);
                 step_barrier();
             }
-            if constexpr (last) {
+            if constexpr (!kAhead) {
+                // the next stage complete, this one's buffer free
+                if (!last && s == 0)
+                    stage_barrier<2 * RT>();
+                else if (!last || s + 1 < SPG)
+                    stage_barrier<0>();
+            } else if constexpr (last) {
                 // the stage after the next complete, where there is one
                 if (s + NB - 1 < SPG)
                     stage_barrier<Stage::kPerWave, false>();
@@ -504,7 +523,7 @@ __device__ __forceinline__ void wave_wide(const uint64_t* __restrict__ rows_in, 
         if constexpr (!last) {
             // the fragment registers rotate by three: move the two read ahead
             // back to the front
-            constexpr int off = (SPG * STEPS) % 3;
+            constexpr int off = kAhead ? (SPG * STEPS) % 3 : 0;
             if constexpr (off != 0) {
                 const u32x4 a0 = f0[off], a1 = f0[(off + 1) % 3];
                 const u32x2 c0 = f1[off], c1 = f1[(off + 1) % 3];
@@ -532,11 +551,18 @@ __device__ __forceinline__ void wave_wide(const uint64_t* __restrict__ rows_in, 
             for (int nt = 0; nt < NT; ++nt) asm volatile("" : "+v"(acc[r][nt]));
     }
     stage_barrier<0>();  // every wave, and any repeated last stage, is done with the buffers
-    // Recombine the digit planes (eighths of integers) through a buffer of the
-    // wave's own, sixteen rows at a time: register i of lane (m, g) holds row
+    // Recombine the digit planes (eighths of integers) through LDS of the wave's
+    // own, a row tile at a time (with two buffers half of one: rows 4 g and
+    // 4 g + 1, then 4 g + 2 and 4 g + 3): register i of lane (m, g) holds row
     // 4 g + i of column m.  Opaque indices as in wave_narrow.
-    u32x4* const s_q = wave == 0 ? s_b[0] : wave == 1 ? s_b[1] : wave == 2 ? s_b[2] : s_b[3];
-    static_assert(VECS * 16 >= 16 * 16 * NT * 4 + 32, "a row tile's digit sums, and reads past the last");
+    constexpr int PARTS = 4 / NB, REGS = 4 / PARTS;
+    static_assert(VECS * 4 * NB >= 64 * REGS * NT * 4 + 32,
+                  "a wave's share of the buffers holds a part's digit sums, and reads past the last");
+    u32x4* const s_q = NB == 2     ? (wave < 2 ? s_b[0] : s_b[1]) + (wave & 1) * (VECS / 2)
+                       : wave == 0 ? s_b[0]
+                       : wave == 1 ? s_b[1]
+                       : wave == 2 ? s_b[2]
+                                   : s_b[3];
     int32_t* const s_w = reinterpret_cast<int32_t*>(s_q);
     uint32_t ol = lane, ob = base;
     asm volatile("" : "+v"(ol), "+s"(ob));
@@ -545,34 +571,38 @@ __device__ __forceinline__ void wave_wide(const uint64_t* __restrict__ rows_in, 
     for (int r = 0; r < RT; ++r) {
         if (ob + 16 * r >= h) break;
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int part = 0; part < PARTS; ++part) {
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt)
-                s_w[(4 * (ol >> 4) + i) * (16 * NT) + 16 * nt + (ol & 15)] =
-                    (int32_t)(acc[r][nt][i] * 8.0f);
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        const uint32_t first = ob + 16 * r;
-        for (uint32_t e = ol; e < 16 * T; e += 64) {
-            const uint32_t lr = e / T, t = e % T;
-            const int32_t* const src = s_w + lr * (16 * NT) + t * stride;
-            int64_t v = 0;
+            for (int i = 0; i < REGS; ++i)
 #pragma unroll
-            for (uint32_t p = 0; p < kMaxPlanes; ++p)  // all reads in flight at once
-                v += (int64_t)(src[p] & (p < P ? -1 : 0)) << (5 * p);
-            if (first + lr < h) {
-                const size_t o = (size_t)(first - row0) * T + e;
-                out[o] = add ? out[o] + v : v;
+                for (int nt = 0; nt < NT; ++nt)
+                    s_w[(REGS * (ol >> 4) + i) * (16 * NT) + 16 * nt + (ol & 15)] =
+                        (int32_t)(acc[r][nt][REGS * part + i] * 8.0f);
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            const uint32_t first = ob + 16 * r;
+            for (uint32_t e = ol; e < 4 * REGS * T; e += 64) {
+                const uint32_t pr = e / T, t = e % T;  // row of the part, of the tile
+                const uint32_t lr = 4 * (pr / REGS) + REGS * part + pr % REGS;
+                const int32_t* const src = s_w + pr * (16 * NT) + t * stride;
+                int64_t v = 0;
+#pragma unroll
+                for (uint32_t p = 0; p < kMaxPlanes; ++p)  // all reads in flight at once
+                    v += (int64_t)(src[p] & (p < P ? -1 : 0)) << (5 * p);
+                if (first + lr < h) {
+                    const size_t o = (size_t)(first - row0 + lr) * T + t;
+                    out[o] = add ? out[o] + v : v;
+                }
             }
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         }
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     }
 }
 
 // Groups [Ga, Gb) of the wave's rows, kSegGroups at a time: sums of row r into
 // out[r - row0][T].  NT = 0: class 0.
-template <int RT, int NT>
+template <int RT, int NT, int NB>
 __device__ __forceinline__ void wave_rows(const uint64_t* rows, uint32_t h, uint32_t W, uint32_t T,
                                           uint32_t P, const uint4* packed, int64_t* out,
                                           uint32_t row0, uint32_t base, uint32_t Ga,
@@ -583,17 +613,18 @@ __device__ __forceinline__ void wave_rows(const uint64_t* rows, uint32_t h, uint
         if constexpr (NT == 0)
             wave_narrow<RT>(rows, h, W, T, packed, out, row0, base, g0, g1, g0 != Ga, s_b);
         else
-            wave_wide<RT, NT>(rows, h, W, T, P, packed, out, row0, base, g0, g1, g0 != Ga,
+            wave_wide<RT, NT, NB>(rows, h, W, T, P, packed, out, row0, base, g0, g1, g0 != Ga,
                               s_b);
     }
 }
 
 // Waves per SIMD that the accumulators, the rows and one step's operands of a
-// kernel leave room for (its register limit).
+// kernel, and its LDS, leave room for (its register limit).
 constexpr int min_waves(int rt, int cls) {
     if (cls == 0) return rt >= 5 ? 3 : 4;
     if (cls == 1) return rt <= 2 ? 4 : 3;
-    return cls <= 3 && rt <= 2 ? 3 : 2;
+    if (cls == 4) return rt == 1 ? 3 : 1;
+    return rt <= 2 ? 3 : 2;
 }
 
 // The work of a balanced launch of B blocks over h rows: row blocks of
@@ -628,16 +659,23 @@ struct Balance {
     }
 };
 
+// Rows of at most this many groups of a population are not cut: their pieces, sums
+// and second prologues take longer than the units even out, and blocks of two row
+// tiles per wave in turn reach more compute units (traits and free space of
+// a generation, us: 40,000 rows x 48 words x 8 traits 34.9 -> 25.6, 200,000 x 16 x 6
+// 44.3 -> 34.8, 400 x 16 x 4 16.7 -> 13.8).
+constexpr uint32_t kFewGroups = 8;
+
 // The sums of element e = (row, trait) of the rows past the whole rounds,
-// where its row block was cut into pieces.
+// where its row block was cut into pieces (rows of more than `few` groups).
 __device__ __forceinline__ void reduce_pieces(const int64_t* __restrict__ part_in, uint32_t h,
                                               uint32_t W, uint32_t T, const Balance& bal,
-                                              uint32_t block_rows, uint64_t e,
+                                              uint32_t block_rows, uint32_t few, uint64_t e,
                                               int64_t* __restrict__ out_in) {
     const uint32_t NG = (W + kGroupWords - 1) / kGroupWords;
     const uint32_t row0 = bal.full * bal.B * block_rows;
     const uint32_t local = (uint32_t)(e / T), row = row0 + local;
-    if (row >= h || !NG) return;
+    if (row >= h || NG <= few) return;
     const uint32_t rb = local / block_rows;
     const uint32_t b0 = bal.owner((uint64_t)rb * NG, NG);
     const uint32_t b1 = bal.owner((uint64_t)(rb + 1) * NG - 1, NG);
@@ -660,16 +698,22 @@ __device__ __forceinline__ void reduce_pieces(const int64_t* __restrict__ part_i
     as_global(out_in)[(size_t)row * T + (size_t)(e % T)] = v;
 }
 
+// Forms of a launch: one row block per block; a balanced launch; a balanced
+// launch that takes rows of few groups in whole blocks.
+enum class Form { kRowBlock, kBalanced, kBalancedFew };
+
 // A block's shared buffers and the body for the population's tile count.
-// kBalanced: a block of a balanced launch; else one row block.
-template <int RT, int CLS, bool kBalanced>
+template <int RT, int CLS, Form kForm>
 struct TraitsBlock {
     static constexpr uint32_t kWaveRows = RT * kTileRows, kBlockRows = 4 * kWaveRows;
     static constexpr int kVecs = CLS == 0   ? kNarrowBlocks * (int)kFragVecs
                                  : CLS == 1 ? stage_vecs(2)
                                  : CLS <= 3 ? stage_vecs(4)  // the largest of 2 to 7 tiles
                                             : stage_vecs(14);
-    static constexpr bool kRing = CLS >= 1;
+    // stage buffers: two of class 4's leave LDS for three blocks of one row tile
+    // (with two row tiles registers leave one)
+    static constexpr int kBuffers = CLS == 4 && RT == 1 ? 2 : 4;
+    static constexpr bool kRing = CLS >= 1 && kBuffers == 4;
     static_assert(stage_vecs(4) >= stage_vecs(5) && stage_vecs(4) >= stage_vecs(7),
                   "the stage buffers hold every body's stage");
 
@@ -692,7 +736,7 @@ struct TraitsBlock {
         const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
         if (W == 0) {  // no words: every sum is zero
             const uint64_t n = (uint64_t)h * T;
-            if constexpr (kBalanced)
+            if constexpr (kForm != Form::kRowBlock)
                 for (uint64_t e = blk * 256ull + threadIdx.x; e < n; e += blocks * 256ull)
                     as_global(out)[e] = 0;
             else
@@ -701,10 +745,12 @@ struct TraitsBlock {
                         as_global(out)[(size_t)blk * kBlockRows * T + e] = 0;
             return;
         }
-        auto piece = [&](uint32_t rb, uint32_t Ga, uint32_t Gb, int64_t* dst, uint32_t row0) {
-            const uint32_t base = rb * kBlockRows + wave * kWaveRows;
+        // a wave's rows from base on, `tiles` row tiles
+        auto piece = [&](auto tiles, uint32_t base, uint32_t Ga, uint32_t Gb, int64_t* dst,
+                         uint32_t row0) __attribute__((always_inline)) {
+            constexpr int rt = decltype(tiles)::value;
 #define CLOTHO_F6_BODY(n) \
-    wave_rows<RT, n>(rows, h, W, T, P, packed, dst, row0, base, Ga, Gb, s_b)
+    wave_rows<rt, n, kBuffers>(rows, h, W, T, P, packed, dst, row0, base, Ga, Gb, s_b)
             if constexpr (CLS == 0) {
                 CLOTHO_F6_BODY(0);
             } else if constexpr (CLS == 1) {
@@ -725,9 +771,22 @@ struct TraitsBlock {
             }
 #undef CLOTHO_F6_BODY
         };
-        if constexpr (!kBalanced) {
-            piece(blk, 0, NG, out, 0);
+        if constexpr (kForm == Form::kRowBlock) {
+            piece(Int<RT>{}, blk * kBlockRows + wave * kWaveRows, 0, NG, out, 0);
             return;
+        }
+        if constexpr (kForm == Form::kBalancedFew) {
+            if (NG <= kFewGroups) {
+                constexpr int kFewTiles = RT < 2 ? RT : 2;
+                constexpr uint32_t few_rows = 4 * kFewTiles * kTileRows;
+                for (uint64_t row = (uint64_t)blk * few_rows; row < h; row += (uint64_t)blocks * few_rows) {
+                    const uint32_t base = (uint32_t)row + wave * (kFewTiles * kTileRows);
+                    piece(Int<kFewTiles>{}, (uint32_t)__builtin_amdgcn_readfirstlane((int)base), 0, NG,
+                          out, 0);
+                    __syncthreads();  // the stage buffers are free for the next row block
+                }
+                return;
+            }
         }
         // One loop over the block's row blocks, whole ones and then its share
         // of the units, so that the bodies are inlined once.
@@ -756,7 +815,8 @@ struct TraitsBlock {
                 }
                 ++slot;
             }
-            piece((uint32_t)__builtin_amdgcn_readfirstlane((int)rb),
+            piece(Int<RT>{},
+                  (uint32_t)__builtin_amdgcn_readfirstlane((int)(rb * kBlockRows + wave * kWaveRows)),
                   (uint32_t)__builtin_amdgcn_readfirstlane((int)Ga),
                   (uint32_t)__builtin_amdgcn_readfirstlane((int)Gb), dst,
                   (uint32_t)__builtin_amdgcn_readfirstlane((int)row0));
@@ -766,16 +826,17 @@ struct TraitsBlock {
 };
 
 // The balanced launches: row tiles per wave of each class (as many as the
-// registers of the class's resident waves hold) and the int64 elements of
-// piece slots a launch of B blocks needs.
+// registers of the class's resident waves hold) and the int64 elements of piece
+// slots a launch of B blocks of block_rows rows needs.
 __host__ __device__ constexpr int balanced_tiles(int cls) {
     return cls == 0 ? 5 : cls <= 3 ? 4 : 2;
 }
+__host__ __device__ constexpr uint32_t tile_block_rows(int tiles) { return 4u * tiles * kTileRows; }
 __host__ __device__ constexpr uint32_t balanced_block_rows(int cls) {
-    return 4u * balanced_tiles(cls) * kTileRows;
+    return tile_block_rows(balanced_tiles(cls));
 }
-__host__ __device__ inline size_t piece_elems(uint32_t traits, uint32_t blocks) {
-    return 2 * (size_t)blocks * balanced_block_rows(trait_class(traits)) * traits;
+__host__ __device__ inline size_t piece_elems(uint32_t traits, uint32_t block_rows, uint32_t blocks) {
+    return 2 * (size_t)blocks * block_rows * traits;
 }
 
 }  // namespace f6

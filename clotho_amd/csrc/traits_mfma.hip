@@ -57,8 +57,8 @@ __global__ void __launch_bounds__(256)
     k_traits_exact(const uint64_t* __restrict__ rows, uint32_t h, uint32_t words, uint32_t most,
                    uint32_t T, const uint4* __restrict__ packed, int64_t* __restrict__ traits,
                    int64_t* __restrict__ part, uint32_t blocks) {
-    f6::TraitsBlock<f6::balanced_tiles(CLS), CLS, true>::run(rows, h, words, most, T, packed, traits,
-                                                             part, blockIdx.x, blocks);
+    f6::TraitsBlock<f6::balanced_tiles(CLS), CLS, f6::Form::kBalanced>::run(
+        rows, h, words, most, T, packed, traits, part, blockIdx.x, blocks);
 }
 
 // one row block of RT row tiles per wave and block
@@ -66,8 +66,8 @@ template <int RT, int CLS>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(f6::min_waves(RT, CLS))))
     k_traits_rows(const uint64_t* __restrict__ rows, uint32_t h, uint32_t words, uint32_t most,
                   uint32_t T, const uint4* __restrict__ packed, int64_t* __restrict__ traits) {
-    f6::TraitsBlock<RT, CLS, false>::run(rows, h, words, most, T, packed, traits, nullptr,
-                                         blockIdx.x, 0);
+    f6::TraitsBlock<RT, CLS, f6::Form::kRowBlock>::run(rows, h, words, most, T, packed, traits,
+                                                       nullptr, blockIdx.x, 0);
 }
 
 __global__ void __launch_bounds__(256) k_exact_reduce(uint32_t h, uint32_t words, uint32_t T,
@@ -75,7 +75,7 @@ __global__ void __launch_bounds__(256) k_exact_reduce(uint32_t h, uint32_t words
                                                       const int64_t* __restrict__ part,
                                                       int64_t* __restrict__ traits) {
     const uint32_t rows = f6::balanced_block_rows(f6::trait_class(T));
-    f6::reduce_pieces(part, h, words, T, f6::Balance(h, rows, blocks), rows,
+    f6::reduce_pieces(part, h, words, T, f6::Balance(h, rows, blocks), rows, 0,
                       (uint64_t)blockIdx.x * 256 + threadIdx.x, traits);
 }
 
@@ -282,13 +282,14 @@ hipError_t launch_pack_digits(const int32_t* eff, uint32_t traits, uint32_t word
     return hipGetLastError();
 }
 
-size_t trait_piece_elems(uint32_t traits, uint32_t h, uint32_t w_cap, uint32_t round) {
+size_t trait_piece_elems(uint32_t traits, uint32_t block_rows, uint32_t h, uint32_t w_cap,
+                         uint32_t round) {
     // a launch cuts fewer than `round` row blocks into units, and no more
     // blocks than units write pieces
-    const uint32_t rows = f6::balanced_block_rows(f6::trait_class(traits));
     const uint64_t ng = std::max<uint32_t>(1, (w_cap + kGroupWords - 1) / kGroupWords);
-    const uint64_t rb = std::min<uint64_t>(round, (h + rows - 1) / rows);
-    return f6::piece_elems(traits, (uint32_t)std::min<uint64_t>(round, std::max<uint64_t>(1, rb * ng)));
+    const uint64_t rb = std::min<uint64_t>(round, (h + block_rows - 1) / block_rows);
+    return f6::piece_elems(traits, block_rows,
+                           (uint32_t)std::min<uint64_t>(round, std::max<uint64_t>(1, rb * ng)));
 }
 
 namespace {
@@ -349,6 +350,8 @@ ExactShape exact_shape(uint32_t h, uint32_t ng, uint32_t nt, uint32_t traits, co
     return {0, bal.B};
 }
 }  // namespace
+
+uint32_t exact_block_rows(uint32_t traits) { return f6::balanced_block_rows(f6::trait_class(traits)); }
 
 ExactRound exact_round(uint32_t traits) {
     int device = 0, cus = 0, per_cu = 0;

@@ -83,7 +83,7 @@ extern "C" int clotho_trait_contract_exact_noalloc(const uint64_t* rows, uint32_
     ExactRound round;
     const int rc = entry_of(device, traits, &base, &round);
     if (rc != CLOTHO_OK) return rc;
-    const size_t fit = kPiecesBytes / (sizeof(int64_t) * f6::piece_elems(traits, 1));
+    const size_t fit = kPiecesBytes / (sizeof(int64_t) * f6::piece_elems(traits, f6::balanced_block_rows(f6::trait_class(traits)), 1));
     if (round.blocks > fit) round.blocks = (uint32_t)fit;
     uint4* planes = reinterpret_cast<uint4*>(base);
     int64_t* pieces = reinterpret_cast<int64_t*>(base + kPlanesBytes);
