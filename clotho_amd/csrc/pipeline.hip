@@ -2317,7 +2317,7 @@ CLOTHO_SINGLE(k_traits_t32_short, Traits32Short)
 // the fixed shapes of the batched launches, and the autotuner's alternatives
 using Traits2Fixed = Traits<4, 0, f6::Form::kRowBlock>;
 using Traits2Two = Traits<2, 0, f6::Form::kRowBlock>;
-using Traits4Fixed = Traits<4, 1, f6::Form::kRowBlock>;
+using Traits4Fixed = Traits<f6::kBatchTiles, 1, f6::Form::kRowBlock>;
 using Traits4Two = Traits<2, 1, f6::Form::kRowBlock>;
 using Traits8Two = Traits<2, 2, f6::Form::kRowBlock>;
 using Traits16Two = Traits<2, 3, f6::Form::kRowBlock>;

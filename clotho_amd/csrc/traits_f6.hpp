@@ -62,7 +62,8 @@ __host__ __device__ inline uint32_t digit_planes(uint32_t max_abs) {
 // Trait classes: one kernel each, with a body per possible number of
 // 16-column tiles.  Up to two traits (class 0) take eight columns per trait, so
 // that a trait's planes sum over aligned lanes; more traits take P adjacent
-// columns per trait.  Measured against the 32x32x64 instruction (same layout,
+// columns per trait (three and four in eights, where that takes no more tiles: 57
+// -> 61 us at 60,000 rows x 256 words x 4, as an eighth of the lanes store).  Measured against the 32x32x64 instruction (same layout,
 // rows paired by v_permlane16_swap), which alone runs twice as fast: with real
 // operands both are held back by the card's power limit (1.7-1.9 GHz), and its
 // coarser tiles multiply more padding (16 traits, seven planes, 2e5 x 65,536:
@@ -267,7 +268,120 @@ struct Int {
     static constexpr int value = N;
 };
 
-// Class 0 (at most two traits), one wave's share of groups [Ga, Gb) (at least
+// The sum of v over the eight lanes of an aligned group, in each of them: quads,
+// then their mirror images.
+template <int kCtrl>
+__device__ __forceinline__ int64_t add_dpp(int64_t v) {
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)v, kCtrl, 0xF, 0xF, true);
+    const uint32_t hi =
+        (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(v >> 32), kCtrl, 0xF, 0xF, true);
+    return v + (int64_t)(((uint64_t)hi << 32) | lo);
+}
+__device__ __forceinline__ int64_t sum_eight(int64_t v) {
+    v = add_dpp<0xB1>(v);      // quad_perm [1, 0, 3, 2]
+    v = add_dpp<0x4E>(v);      // quad_perm [2, 3, 0, 1]
+    return add_dpp<0x141>(v);  // row_half_mirror
+}
+
+// A wave's sums, of rows base .. base + 16 RT - 1, from its accumulators (eighths
+// of integers): register i of lane (m, g) holds row 4 g + i of column m.
+// Opaque indices: the output addresses of every segment are the same, and hoisted
+// out of the segment loop they would be held, in scratch memory, through the
+// products.
+//
+// Eight columns per trait: shift by 5 p and sum over the lanes (with shuffles by
+// way of LDS, a generation's traits of 256 replicates took 245 us, in row shifts
+// 224).
+template <int RT>
+__device__ __forceinline__ void store_eights(const f32x4 (&acc)[RT][1], uint32_t lane, uint32_t h,
+                                             uint32_t T, int64_t* __restrict__ out_in,
+                                             uint32_t row0, uint32_t base, bool add) {
+    const auto out = as_global(out_in);
+    uint32_t ol = lane, ob = base;
+    asm volatile("" : "+v"(ol), "+s"(ob));
+    const uint32_t om = ol & 15, og = ol >> 4, p = om & 7, t = om >> 3;
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int64_t v = sum_eight((int64_t)(int32_t)(acc[r][0][i] * 8.0f) << (5 * p));
+            const uint32_t row = ob + 16 * r + 4 * og + i;
+            if (p == 0 && row < h && t < T) {
+                const size_t o = (size_t)(row - row0) * T + t;
+                out[o] = add ? out[o] + v : v;
+            }
+        }
+}
+// Adjacent columns: through s_w, LDS of the wave's own, TILES row tiles at a time
+// (in two parts half of one: rows 4 g and 4 g + 1, then 4 g + 2 and 4 g + 3).
+template <int RT, int NT, int PARTS, int TILES>
+__device__ __forceinline__ void store_adjacent(const f32x4 (&acc)[RT][NT], int32_t* s_w,
+                                               uint32_t lane, uint32_t h, uint32_t T, uint32_t P,
+                                               int64_t* __restrict__ out_in, uint32_t row0,
+                                               uint32_t base, bool add) {
+    static_assert(RT % TILES == 0 && (PARTS == 1 || TILES == 1), "whole passes");
+    constexpr int REGS = 4 / PARTS;
+    const auto out = as_global(out_in);
+    uint32_t ol = lane, ob = base;
+    asm volatile("" : "+v"(ol), "+s"(ob));
+#pragma unroll
+    for (int r = 0; r < RT; r += TILES) {
+        const uint32_t first = ob + 16 * r;
+        if (first >= h) break;
+#pragma unroll
+        for (int part = 0; part < PARTS; ++part) {
+#pragma unroll
+            for (int q = 0; q < TILES; ++q)
+#pragma unroll
+                for (int i = 0; i < REGS; ++i)
+#pragma unroll
+                    for (int nt = 0; nt < NT; ++nt)
+                        s_w[(16 * q + REGS * (ol >> 4) + i) * (16 * NT) + 16 * nt + (ol & 15)] =
+                            (int32_t)(acc[r + q][nt][REGS * part + i] * 8.0f);
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            for (uint32_t e = ol; e < 4 * REGS * TILES * T; e += 64) {
+                const uint32_t pr = e / T, t = e % T;  // row of the part, of the pass
+                const uint32_t lr = PARTS == 1 ? pr : 4 * (pr / REGS) + REGS * part + pr % REGS;
+                const int32_t* const src = s_w + pr * (16 * NT) + t * P;
+                int64_t v = 0;
+#pragma unroll
+                for (uint32_t p = 0; p < kMaxPlanes; ++p)  // all reads in flight at once
+                    v += (int64_t)(src[p] & (p < P ? -1 : 0)) << (5 * p);
+                if (first + lr < h) {
+                    const size_t o = (size_t)(first - row0 + lr) * T + t;
+                    out[o] = add ? out[o] + v : v;
+                }
+            }
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        }
+    }
+}
+// int32 elements that a pass takes of a wave's LDS, and `past` more that the last
+// trait's reads past its planes reach
+constexpr int pass_elems(int nt, int parts, int tiles, int past) { return 256 / parts * tiles * nt + past; }
+// row tiles per pass: as many as `share` elements hold
+constexpr int pass_tiles(int rt, int nt, int parts, int past, int share) {
+    int n = parts == 1 ? rt : 1;
+    while (n > 1 && (rt % n != 0 || pass_elems(nt, parts, n, past) > share)) --n;
+    return n;
+}
+
+// The products stay where they are written: otherwise they are sunk into the
+// branch of the row tile that needs them, their operands spilled.
+template <int RT, int NT>
+__device__ __forceinline__ void pin(f32x4 (&acc)[RT][NT]) {
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) asm volatile("" : "+v"(acc[r][nt]));
+}
+
+// One or two column tiles in stages of four K blocks, two buffers (class 0, and class
+// 1 in batches, whose rows are mostly one group: 256 replicates x 3 / 4 traits
+// 290 / 338 us in wave_wide's four stages and four row tiles, 239 / 275 here in three),
+// one wave's share of groups [Ga, Gb) (at least
 // one): rows base .. base + 16 RT - 1 (those below h; base wave-uniform).
 // The next group's rows load into registers of their own at the group's first
 // stage, after the stage's fragment loads, and stay in flight across its
@@ -276,9 +390,9 @@ struct Int {
 // which loads no further rows or fragments, is a body of its own: under a
 // run-time condition the compiler could not count what is in flight and would
 // wait for everything before the first LDS read of a stage.
-template <int RT>
+template <int RT, int NT, bool kEights>
 __device__ __forceinline__ void wave_narrow(const uint64_t* __restrict__ rows_in, uint32_t h,
-                                            uint32_t W, uint32_t T,
+                                            uint32_t W, uint32_t T, uint32_t P,
                                             const uint4* __restrict__ packed_in,
                                             int64_t* __restrict__ out_in, uint32_t row0,
                                             uint32_t base, uint32_t Ga, uint32_t Gb,
@@ -286,14 +400,16 @@ __device__ __forceinline__ void wave_narrow(const uint64_t* __restrict__ rows_in
     constexpr int QS = kNarrowBlocks, SPG = 8 / QS;
     static_assert(SPG == 2, "two stages per group, two buffers");
     const auto rows = as_global(rows_in);
-    const auto out = as_global(out_in);
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const uint32_t m = lane & 15, g = lane >> 4;
-    const Stager<QS * (int)kFragVecs> stage_b(packed_in, Ga * SPG, wave, lane);
-    f32x4 acc[RT];
+    constexpr int VECS = QS * NT * (int)kFragVecs;
+    const Stager<VECS> stage_b(packed_in, Ga * SPG, wave, lane);
+    f32x4 acc[RT][NT];
 #pragma unroll
-    for (int r = 0; r < RT; ++r) acc[r] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) acc[r][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
     const __attribute__((address_space(1))) uint64_t* rp[RT];
 #pragma unroll
     for (int r = 0; r < RT; ++r) {
@@ -326,19 +442,21 @@ __device__ __forceinline__ void wave_narrow(const uint64_t* __restrict__ rows_in
             asm volatile("" ::: "memory");
             u32x4 b0, c0;
             u32x2 b1, c1;
+            i32x8 a[RT];
             read_frag(cur, lane, b0, b1);
 #pragma unroll
-            for (int j = 0; j < QS; ++j) {
-                const int q = s * QS + j;
-                if (j + 1 < QS) read_frag(cur + (j + 1) * (int)kFragVecs, lane, c0, c1);
+            for (int j = 0; j < QS * NT; ++j) {
+                const int q = s * QS + j / NT, nt = j % NT;
+                if (j + 1 < QS * NT) read_frag(cur + (j + 1) * (int)kFragVecs, lane, c0, c1);
                 const i32x8 b = frag_of(b0, b1);
-                i32x8 a[RT];
+                if (nt == 0) {
 #pragma unroll
-                for (int r = 0; r < RT; ++r) a[r] = expand_bits(x[r][q >> 2][q & 3]);
+                    for (int r = 0; r < RT; ++r) a[r] = expand_bits(x[r][q >> 2][q & 3]);
+                }
 #pragma unroll
                 for (int r = 0; r < RT; ++r)
-                    acc[r] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
-                        a[r], b, acc[r], kFp4, kFp6, 0, kScaleOne, 0, kScaleOne);
+                    acc[r][nt] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+                        a[r], b, acc[r][nt], kFp4, kFp6, 0, kScaleOne, 0, kScaleOne);
                 step_barrier();
                 b0 = c0;
                 b1 = c1;
@@ -359,29 +477,17 @@ __device__ __forceinline__ void wave_narrow(const uint64_t* __restrict__ rows_in
     };
     for (uint32_t G = Ga; G + 1 < Gb; ++G) group(G, Int<0>{});
     group(Gb - 1, Int<1>{});
-    // Recombine: column 8 t + p in lane m; shift by 5 p and sum over the eight
-    // lanes of the trait (the accumulators hold eighths of integers).  The
-    // indices are opaque: the output addresses of every segment are the same,
-    // and hoisted out of the segment loop they would be held, in scratch
-    // memory, through the products.
-    uint32_t ol = lane, ob = base;
-    asm volatile("" : "+v"(ol), "+s"(ob));
-    const uint32_t om = ol & 15, og = ol >> 4;
-    const uint32_t p = om & 7, t = om >> 3;
-#pragma unroll
-    for (int r = 0; r < RT; ++r)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            int64_t v = (int64_t)(int32_t)(acc[r][i] * 8.0f) << (5 * p);
-            v += __shfl_xor((long long)v, 1, 64);
-            v += __shfl_xor((long long)v, 2, 64);
-            v += __shfl_xor((long long)v, 4, 64);
-            const uint32_t row = ob + 16 * r + 4 * og + i;
-            if (p == 0 && row < h && t < T) {
-                const size_t o = (size_t)(row - row0) * T + t;
-                out[o] = add ? out[o] + v : v;
-            }
-        }
+    pin(acc);
+    if constexpr (kEights) {
+        store_eights<RT>(acc, lane, h, T, out_in, row0, base, add);
+    } else {
+        // a wave's quarter of the two buffers; up to four traits' reads end within two tiles
+        constexpr int PAST = NT == 2 ? 0 : 8, TILES = pass_tiles(RT, NT, 1, PAST, 2 * VECS);
+        static_assert(2 * VECS >= pass_elems(NT, 1, TILES, PAST), "a pass fits");
+        u32x4* const s_q = (wave < 2 ? s_b[0] : s_b[1]) + (wave & 1) * (VECS / 2);
+        store_adjacent<RT, NT, 1, TILES>(acc, reinterpret_cast<int32_t*>(s_q), lane, h, T, P, out_in,
+                                         row0, base, add);
+    }
 }
 
 // Loads of classes 1-4 that may be in flight at the end of stage s of a group:
@@ -421,7 +527,6 @@ __device__ __forceinline__ void wave_wide(const uint64_t* __restrict__ rows_in, 
     static_assert(NB == 4 || (NB == 2 && RT <= 2), "with two buffers the last group has its own body");
     constexpr bool kAhead = NB == 4;
     const auto rows = as_global(rows_in);
-    const auto out = as_global(out_in);
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const uint32_t m = lane & 15, g = lane >> 4;
@@ -543,66 +648,24 @@ __device__ __forceinline__ void wave_wide(const uint64_t* __restrict__ rows_in, 
     for (uint32_t G = Ga; G + (kOwnLast ? 1 : 0) < Gb; ++G) group(G, Int<0>{});
     if constexpr (kOwnLast) {
         group(Gb - 1, Int<1>{});
-        // the products stay where they are written: otherwise they are sunk into
-        // the branch of the row tile that needs them, their operands spilled
-#pragma unroll
-        for (int r = 0; r < RT; ++r)
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) asm volatile("" : "+v"(acc[r][nt]));
+        pin(acc);
     }
     stage_barrier<0>();  // every wave, and any repeated last stage, is done with the buffers
-    // Recombine the digit planes (eighths of integers) through LDS of the wave's
-    // own, a row tile at a time (with two buffers half of one: rows 4 g and
-    // 4 g + 1, then 4 g + 2 and 4 g + 3): register i of lane (m, g) holds row
-    // 4 g + i of column m.  Opaque indices as in wave_narrow.
-    constexpr int PARTS = 4 / NB, REGS = 4 / PARTS;
-    static_assert(VECS * 4 * NB >= 64 * REGS * NT * 4 + 32,
-                  "a wave's share of the buffers holds a part's digit sums, and reads past the last");
+    constexpr int PARTS = 4 / NB, TILES = pass_tiles(RT, NT, PARTS, 8, VECS * NB);
+    static_assert(VECS * NB >= pass_elems(NT, PARTS, TILES, 8), "a wave's quarter of the buffers holds a pass");
     u32x4* const s_q = NB == 2     ? (wave < 2 ? s_b[0] : s_b[1]) + (wave & 1) * (VECS / 2)
                        : wave == 0 ? s_b[0]
                        : wave == 1 ? s_b[1]
                        : wave == 2 ? s_b[2]
                                    : s_b[3];
-    int32_t* const s_w = reinterpret_cast<int32_t*>(s_q);
-    uint32_t ol = lane, ob = base;
-    asm volatile("" : "+v"(ol), "+s"(ob));
-    const uint32_t stride = column_stride(T, P);
-#pragma unroll
-    for (int r = 0; r < RT; ++r) {
-        if (ob + 16 * r >= h) break;
-#pragma unroll
-        for (int part = 0; part < PARTS; ++part) {
-#pragma unroll
-            for (int i = 0; i < REGS; ++i)
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt)
-                    s_w[(REGS * (ol >> 4) + i) * (16 * NT) + 16 * nt + (ol & 15)] =
-                        (int32_t)(acc[r][nt][REGS * part + i] * 8.0f);
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-            const uint32_t first = ob + 16 * r;
-            for (uint32_t e = ol; e < 4 * REGS * T; e += 64) {
-                const uint32_t pr = e / T, t = e % T;  // row of the part, of the tile
-                const uint32_t lr = 4 * (pr / REGS) + REGS * part + pr % REGS;
-                const int32_t* const src = s_w + pr * (16 * NT) + t * stride;
-                int64_t v = 0;
-#pragma unroll
-                for (uint32_t p = 0; p < kMaxPlanes; ++p)  // all reads in flight at once
-                    v += (int64_t)(src[p] & (p < P ? -1 : 0)) << (5 * p);
-                if (first + lr < h) {
-                    const size_t o = (size_t)(first - row0 + lr) * T + t;
-                    out[o] = add ? out[o] + v : v;
-                }
-            }
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        }
-    }
+    store_adjacent<RT, NT, PARTS, TILES>(acc, reinterpret_cast<int32_t*>(s_q), lane, h, T, P, out_in,
+                                         row0, base, add);
 }
 
 // Groups [Ga, Gb) of the wave's rows, kSegGroups at a time: sums of row r into
-// out[r - row0][T].  NT = 0: class 0.
-template <int RT, int NT, int NB>
+// out[r - row0][T].  NB: wave_wide's stage buffers, 0 for wave_narrow; kEights: eight
+// columns per trait (class 0).
+template <int RT, int NT, int NB, bool kEights>
 __device__ __forceinline__ void wave_rows(const uint64_t* rows, uint32_t h, uint32_t W, uint32_t T,
                                           uint32_t P, const uint4* packed, int64_t* out,
                                           uint32_t row0, uint32_t base, uint32_t Ga,
@@ -610,8 +673,9 @@ __device__ __forceinline__ void wave_rows(const uint64_t* rows, uint32_t h, uint
     for (uint32_t g0 = Ga; g0 < Gb; g0 += kSegGroups) {
         const uint32_t g1 = min(Gb, g0 + kSegGroups);
         if (g0 != Ga) __syncthreads();  // the previous segment's sums are out of the buffers
-        if constexpr (NT == 0)
-            wave_narrow<RT>(rows, h, W, T, packed, out, row0, base, g0, g1, g0 != Ga, s_b);
+        if constexpr (NB == 0)
+            wave_narrow<RT, NT, kEights>(rows, h, W, T, P, packed, out, row0, base, g0, g1, g0 != Ga,
+                                         s_b);
         else
             wave_wide<RT, NT, NB>(rows, h, W, T, P, packed, out, row0, base, g0, g1, g0 != Ga,
                               s_b);
@@ -620,9 +684,10 @@ __device__ __forceinline__ void wave_rows(const uint64_t* rows, uint32_t h, uint
 
 // Waves per SIMD that the accumulators, the rows and one step's operands of a
 // kernel, and its LDS, leave room for (its register limit).
+constexpr int kBatchTiles = 3;  // row tiles of class 1's blocks in batches (wave_narrow)
 constexpr int min_waves(int rt, int cls) {
     if (cls == 0) return rt >= 5 ? 3 : 4;
-    if (cls == 1) return rt <= 2 ? 4 : 3;
+    if (cls == 1) return rt <= kBatchTiles ? 4 : 3;
     if (cls == 4) return rt == 1 ? 3 : 1;
     return rt <= 2 ? 3 : 2;
 }
@@ -706,14 +771,15 @@ enum class Form { kRowBlock, kBalanced, kBalancedFew };
 template <int RT, int CLS, Form kForm>
 struct TraitsBlock {
     static constexpr uint32_t kWaveRows = RT * kTileRows, kBlockRows = 4 * kWaveRows;
-    static constexpr int kVecs = CLS == 0   ? kNarrowBlocks * (int)kFragVecs
+    // stage buffers of wave_wide, 0 for wave_narrow and its two: two of class 4's
+    // leave LDS for three blocks of one row tile (with two row tiles registers leave one)
+    static constexpr bool kNarrow = CLS == 0 || (CLS == 1 && RT == kBatchTiles);
+    static constexpr int kBuffers = kNarrow ? 0 : CLS == 4 && RT == 1 ? 2 : 4;
+    static constexpr int kVecs = kNarrow    ? (CLS + 1) * kNarrowBlocks * (int)kFragVecs
                                  : CLS == 1 ? stage_vecs(2)
                                  : CLS <= 3 ? stage_vecs(4)  // the largest of 2 to 7 tiles
                                             : stage_vecs(14);
-    // stage buffers: two of class 4's leave LDS for three blocks of one row tile
-    // (with two row tiles registers leave one)
-    static constexpr int kBuffers = CLS == 4 && RT == 1 ? 2 : 4;
-    static constexpr bool kRing = CLS >= 1 && kBuffers == 4;
+    static constexpr bool kRing = kBuffers == 4;
     static_assert(stage_vecs(4) >= stage_vecs(5) && stage_vecs(4) >= stage_vecs(7),
                   "the stage buffers hold every body's stage");
 
@@ -750,9 +816,9 @@ struct TraitsBlock {
                          uint32_t row0) __attribute__((always_inline)) {
             constexpr int rt = decltype(tiles)::value;
 #define CLOTHO_F6_BODY(n) \
-    wave_rows<rt, n, kBuffers>(rows, h, W, T, P, packed, dst, row0, base, Ga, Gb, s_b)
+    wave_rows<rt, n, kBuffers, CLS == 0>(rows, h, W, T, P, packed, dst, row0, base, Ga, Gb, s_b)
             if constexpr (CLS == 0) {
-                CLOTHO_F6_BODY(0);
+                CLOTHO_F6_BODY(1);
             } else if constexpr (CLS == 1) {
                 if (NT == 1) CLOTHO_F6_BODY(1);
                 else CLOTHO_F6_BODY(2);
