@@ -201,6 +201,7 @@ int read_state(clotho_ctx* c, GenState* st) {
 }
 
 int write_state(clotho_ctx* c, const GenState& st) {
+    c->live_words = st.wc;
     return deliver(c, c->b.state, &st, sizeof(GenState));
 }
 
@@ -257,14 +258,6 @@ void begin_generation(clotho_ctx* c) {
 void end_generation(clotho_ctx* c) {
     if (c->p.n_par == c->p.n) return;
     c->p.n_par = c->p.n;
-    destroy_graphs(c);
-}
-
-// Launch shapes that follow the population's width (captured launches bake them in).
-void refresh_shapes(clotho_ctx* c) {
-    const bool brief = short_traits(c);
-    if (brief == c->short_traits) return;
-    c->short_traits = brief;
     destroy_graphs(c);
 }
 
@@ -415,10 +408,9 @@ int clotho_create(const clotho_config* cfg, int device, clotho_ctx** out) {
         P.max_chunks = std::max<uint32_t>(1, std::min<uint32_t>(
                                                  (8192 + P.tiles - 1) / P.tiles, h_cap / 8));
         P.max_chunks = std::max(P.max_chunks, std::min(groups, 2 * c->recombine_round));
-        c->by_event = recombine_by_event(P, cfg->rho);
-        c->short_traits = short_traits(c);
         P.chunks = std::min(P.max_chunks, recombine_chunks(c, P.h));
         P.splits = recombine_splits(c, P.chunks);
+        (void)refresh_shapes(c);
     }
     P.mut_blocks = (P.h + kScanBlock - 1) / kScanBlock;
     P.free_words = 16;
@@ -662,6 +654,7 @@ int clotho_get_shape(clotho_ctx* c, clotho_shape* out) {
     const int rc = fetch(c, &now, c->shape_status, sizeof(now));
     if (rc) return rc;
     const GenState& st = now.state;
+    c->live_words = st.wc;
     std::memset(out, 0, sizeof(*out));
     out->generation = st.gen;
     out->n_individuals = c->p.n;
@@ -1149,7 +1142,7 @@ int clotho_run(clotho_ctx* c, uint32_t n, int use_graph) {
     for (double& v : tm.ms) v = 0.0;
     tm.generations = 0;
     std::vector<hipEvent_t> marks;
-    refresh_shapes(c);
+    if (refresh_shapes(c)) destroy_graphs(c);
     // a generation that changes the population size runs with eager launches
     if (c->next_n && c->next_n != c->p.n) use_graph = 0;
     if (use_graph) {
@@ -1304,6 +1297,7 @@ int clotho_autotune(clotho_ctx* c, uint32_t* chosen_chunks) {
     }
     c->p.chunks = best_chunks;
     c->p.splits = recombine_splits(c, best_chunks);
+    c->chunks_set = true;
 
     // The traits pass: every kernel shape over the current population (the
     // pass writes the traits it already holds), fastest of two passes.
@@ -1379,6 +1373,7 @@ int clotho_set_launch_shape(clotho_ctx* c, const clotho_launch_shape* in) {
                     "set_launch_shape: chunks 1.." + std::to_string(c->p.max_chunks) +
                         ", traits shape 1.." + std::to_string(nv) +
                         ", compaction rows 4/8/16, compaction tile words 48/56/60/64");
+    if (in->recombine_chunks != c->p.chunks) c->chunks_set = true;
     c->p.chunks = in->recombine_chunks;
     c->p.splits = recombine_splits(c, in->recombine_chunks);
     c->trait_variant = in->traits_variant;

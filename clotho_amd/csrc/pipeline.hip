@@ -2688,6 +2688,9 @@ hipError_t query_residency(clotho_ctx* c) {
     return hipSuccess;
 }
 
+// The population's width when its state was last looked at, its capacity before.
+static uint32_t width_of(const clotho_ctx* c) { return c->live_words ? c->live_words : c->p.w_cap; }
+
 // More than 16 traits: up to 256 words the balanced launch of one row tile per
 // wave, three blocks per compute unit, wider rows the one of two, which reads
 // each fragment from LDS for twice the rows but is alone on its compute unit.
@@ -2696,9 +2699,7 @@ hipError_t query_residency(clotho_ctx* c) {
 // 62; 200,000 x 80 147 / 134 / 184; 60,000 x 256 116 / 119 / 152; 200,000 x 480 530 /
 // 614 / 773.  By the width that the last run left (the capacity before it), as
 // either is right at any width.
-bool short_traits(const clotho_ctx* c) {
-    return c->p.traits > 16 && (c->live_words ? c->live_words : c->p.w_cap) <= 256;
-}
+bool short_traits(const clotho_ctx* c) { return c->p.traits > 16 && width_of(c) <= 256; }
 
 // int64 elements that the pieces of either balanced launch take
 size_t population_piece_elems(const clotho_ctx* c, uint32_t h_cap) {
@@ -2711,18 +2712,41 @@ size_t population_piece_elems(const clotho_ctx* c, uint32_t h_cap) {
                                                           P.w_cap, c->short_round));
 }
 
-// A lookup per event and row where the two populations (at capacity) exceed the
-// Infinity Cache and a gamete has few events: its rows are wider (512 bytes per
-// access), it reads a parent pair once for three siblings, and its blocks are
-// smaller, which is worth up to a quarter while the lookups are few.  Measured,
-// generation by event against by groups: N = 12,345, 984 words: 212 against 244
-// us at rho = 0.3, 229 against 241 at 4; N = 40,000, 816 words: 400 against 427 at
-// 0.3, 444 against 434 at 4; N = 100,000, 816 words: 834 against 874 at 0.3, 890
-// against 873 at 3; in the cache (N = 12,345, 328 words) 120 against 123 at 0.3,
-// 131 against 124 at 2; N = 100,000, 40 words: 162 against 153 at 1.
-bool recombine_by_event(const Params& P, double rho) {
-    const double bytes = 2.0 * 8.0 * P.h * P.w_cap;
-    return bytes > 384.0 * (1 << 20) && rho * rho * P.n < 4e5 && P.ev_cap <= 64;
+// A lookup per event and row where the two populations outgrow the caches and a
+// gamete has few events: its rows are wider (512 bytes per access), it reads a
+// parent pair once for three siblings, and its blocks are smaller, which is worth up
+// to a quarter while the lookups are few.  Where rows are an odd number of 64-byte
+// halves every second row lies across the lines of a group's 128-byte accesses,
+// which costs it a fifth and moves the limit up (not looked at where every
+// generation is compacted, as its width may change from run to run).  `words` is
+// the population's width.  Measured over N = 2,000 to 250,000, 8 to 1,712 words, rho = 0.3 to 8 (us per
+// generation, by event / by groups / by event before there were groups): N =
+// 60,000, 40 words: 89 / 104 / 95 at rho = 0.3, 110 / 109 / 115 at 4; N = 30,000, 280
+// words: 162 / 188 / 184 at 1, 229 / 196 / 254 at 8; N = 60,000, 1,080 words: 754 / 865 / 762
+// at 4, 900 / 880 / 908 at 8; 1,216 words: 792 / 781 / 824 at 5, 943 / 804 / 979 at 8; N = 2,000,
+// 552 words: 90 / 83 / 190 at 0.3; N = 100,000, 24 words: 110 / 118 / 116 at 0.3, 147 / 126 /
+// 153 at 4; N = 250,000, 272 words: 764 / 783 / 809 at 2, 837 / 779 / 883 at 4.
+static bool recombine_by_event(const Params& P, const clotho_config& cfg, uint32_t words) {
+    const double bytes = 2.0 * 8.0 * P.h * words, rho = cfg.rho;
+    const bool whole_lines = words % 16 == 0 || cfg.compact_every;
+    const double limit = whole_lines ? (P.h > 400000 ? 2.5 : 4.5) : words > 896 ? 6.5 : 5.0;
+    return P.h >= 8192 && rho < limit && bytes > (20.0 + 50.0 * rho) * 1e6 && P.ev_cap <= 64;
+}
+
+// The launch shapes that follow the population's width, decided where a run
+// starts.  Row chunks that were set or tuned stay, with their kernel.
+bool refresh_shapes(clotho_ctx* c) {
+    const bool brief = short_traits(c);
+    const bool by_event =
+        c->chunks_set ? c->by_event : recombine_by_event(c->p, c->cfg, width_of(c));
+    if (brief == c->short_traits && by_event == c->by_event) return false;
+    c->short_traits = brief;
+    if (by_event != c->by_event) {
+        c->by_event = by_event;
+        c->p.chunks = std::min(c->p.max_chunks, recombine_chunks(c, c->p.h));
+        c->p.splits = recombine_splits(c, c->p.chunks);
+    }
+    return true;
 }
 
 // Row chunks of the recombination: as many as its groups of 64 gametes, up to

@@ -294,6 +294,7 @@ struct clotho_ctx {
     uint32_t live_words = 0;      // row width at the last look at the device's state
     uint32_t recombine_round = 1; // and of the recombination by groups
     bool by_event = false;        // recombination by event (recombine_by_event)
+    bool chunks_set = false;      // its row chunks were set or tuned
     // launch shapes the autotuner may change (0 / defaults: the built-in choice)
     uint32_t trait_variant = 0;   // traits-pass kernel shape, 1 .. trait_variants()
     uint32_t compact_rows = 8;    // rows per wave step of the column compaction: 4, 8, 16
@@ -347,10 +348,10 @@ hipError_t launch_compact_rows(clotho_ctx* c, int src);
 uint32_t compact_chunks_of(const clotho_ctx* c);
 hipError_t query_residency(clotho_ctx* c);  // sets the resident rounds of the context's kernels
 bool short_traits(const clotho_ctx* c);
+bool refresh_shapes(clotho_ctx* c);  // true: captured launches have the former shapes
 size_t population_piece_elems(const clotho_ctx* c, uint32_t h_cap);
 // launch shape of the recombination: row chunks for h rows, and the column
 // ranges that go with a number of row chunks
-bool recombine_by_event(const Params& P, double rho);
 uint32_t recombine_chunks(const clotho_ctx* c, uint32_t h);
 uint32_t recombine_splits(const clotho_ctx* c, uint32_t chunks);
 // Column compaction of population [src] into [1 - src] (fixed and lost
