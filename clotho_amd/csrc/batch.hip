@@ -54,18 +54,22 @@ void drop_graphs(clotho_batch* b) {
 }
 
 // Launch shape of a replicate's recombination within a batch of `groups` groups
-// of 64 gametes: chunks of up to 16 groups (a block's offset search, tables and
+// of 64 gametes: chunks of 16 groups (a block's offset search, tables and
 // partials are paid per chunk; half and twice as many chunks measured 1.12 and
-// 1.20 ms on the 256-replicate workload at generation 200), fewer where the batch
-// would not give every resident block four chunks, and column ranges where the
-// chunks alone do not give it one.
-void batch_recombine_shape(Params& P, uint64_t groups, uint32_t resident) {
+// 1.20 ms on the 256-replicate workload at generation 200; eight groups in a batch of
+// 26,000 234 us, 16 210).  A small batch, by groups throughout, takes fewer where
+// that would not give every resident block four chunks, and column ranges where
+// the chunks alone do not give it one.  Row chunks that were set or tuned for a
+// replicate are taken for it, two per block.
+void batch_recombine_shape(Params& P, bool chunks_set, uint64_t groups, uint32_t resident) {
+    const bool small = groups <= (uint64_t)kSmallBatch * resident;
+    P.group_words = small ? 0 : kWidePerGroup;
     const uint32_t own = (P.h + 63) / 64;
-    const uint64_t per = std::min<uint64_t>(16, std::max<uint64_t>(1, groups / (4ull * resident)));
-    P.chunks = std::min<uint32_t>(P.max_chunks, (uint32_t)((own + per - 1) / per));
+    const uint64_t per = small ? std::max<uint64_t>(1, groups / (4ull * resident)) : 16;
+    P.chunks = std::min<uint32_t>(
+        P.max_chunks, chunks_set ? (P.chunks + 1) / 2 : (uint32_t)((own + per - 1) / per));
     const uint64_t turns = (P.w_cap + 63) / 64;
     P.splits = (uint32_t)std::max<uint64_t>(1, std::min(turns, resident / std::max<uint64_t>(1, groups)));
-    P.group_words = groups <= (uint64_t)kSmallBatch * resident ? 0 : kWidePerGroup;
 }
 
 // Upload each replicate's Params/Buffers and the per-kernel block offsets
@@ -81,7 +85,7 @@ int sync_views(clotho_batch* b) {
         v[r].P = b->reps[r]->p;
         v[r].B = b->reps[r]->b;
         v[r].B.by_parent = nullptr;  // replicates recombine in child order
-        batch_recombine_shape(v[r].P, groups, resident);
+        batch_recombine_shape(v[r].P, b->reps[r]->chunks_set, groups, resident);
         v[r].P.free_words = 64;
         v[r].P.word_blocks = (v[r].P.w_cap + 63) / 64;
     }

@@ -310,8 +310,9 @@ struct MutAttrs {
             }
         }
         // the population's bound only grows, so after the first generations
-        // almost every thread stops at the read
-        if (most > __hip_atomic_load(&st->eff_max, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        // almost every thread stops at the read, a cached one (an old value only
+        // costs an atomic more)
+        if (most > __hip_atomic_load(&st->eff_max, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT))
             __hip_atomic_fetch_max(&st->eff_max, most, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 };
