@@ -57,15 +57,23 @@ void drop_graphs(clotho_batch* b) {
 // of 64 gametes: chunks of 16 groups (a block's offset search, tables and
 // partials are paid per chunk; half and twice as many chunks measured 1.12 and
 // 1.20 ms on the 256-replicate workload at generation 200; eight groups in a batch of
-// 26,000 234 us, 16 210).  A small batch, by groups throughout, takes fewer where
-// that would not give every resident block four chunks, and column ranges where
-// the chunks alone do not give it one.  Row chunks that were set or tuned for a
-// replicate are taken for it, two per block.
-void batch_recombine_shape(Params& P, bool chunks_set, uint64_t groups, uint32_t resident) {
-    const bool small = groups <= (uint64_t)kSmallBatch * resident;
-    P.group_words = small ? 0 : kWidePerGroup;
+// 26,000 by event 234 us, 16 210).  A replicate that may recombine by groups takes
+// fewer where that would not give every resident block four chunks (64 x 6,000, 392
+// words, rho = 5: 2334 us, with 16 2699), and column ranges where the chunks alone
+// do not give it one.  Row chunks that were set or tuned for a
+// replicate are taken for it, two per block.  rho, words: events per gamete and row
+// width, mean over the batch's rows.
+void batch_recombine_shape(Params& P, bool chunks_set, uint64_t groups, double rho, double words,
+                           uint32_t resident) {
+    if (groups <= (uint64_t)kGroupBatch * resident)
+        P.group_words = 0;
+    else if (rho <= (words < kEventWords ? kEventRho : kWideEventRho))
+        P.group_words = kNeverPerGroup;
+    else
+        P.group_words = groups <= (uint64_t)kSmallBatch * resident ? 0 : kWidePerGroup;
     const uint32_t own = (P.h + 63) / 64;
-    const uint64_t per = small ? std::max<uint64_t>(1, groups / (4ull * resident)) : 16;
+    const uint64_t fill = std::min<uint64_t>(16, std::max<uint64_t>(1, groups / (4ull * resident)));
+    const uint64_t per = P.w_cap > P.group_words ? fill : 16;
     P.chunks = std::min<uint32_t>(
         P.max_chunks, chunks_set ? (P.chunks + 1) / 2 : (uint32_t)((own + per - 1) / per));
     const uint64_t turns = (P.w_cap + 63) / 64;
@@ -78,16 +86,26 @@ int sync_views(clotho_batch* b) {
     const uint32_t R = (uint32_t)b->reps.size();
     std::vector<RepView> v(R);
     uint64_t groups = 0;
-    for (uint32_t r = 0; r < R; ++r) groups += (b->reps[r]->p.h + 63) / 64;
+    double rho = 0.0, words = 0.0;
+    for (const clotho_ctx* c : b->reps) {
+        const uint32_t own = (c->p.h + 63) / 64;
+        groups += own;
+        rho += own * c->cfg.rho;
+        words += (double)own * width_of(c);
+    }
+    rho /= (double)groups;
+    words /= (double)groups;
     const uint32_t resident = b->reps[0]->recombine_round;
     for (uint32_t r = 0; r < R; ++r) {
         std::memset(&v[r], 0, sizeof(RepView));
         v[r].P = b->reps[r]->p;
         v[r].B = b->reps[r]->b;
         v[r].B.by_parent = nullptr;  // replicates recombine in child order
-        batch_recombine_shape(v[r].P, b->reps[r]->chunks_set, groups, resident);
-        v[r].P.free_words = 64;
-        v[r].P.word_blocks = (v[r].P.w_cap + 63) / 64;
+        batch_recombine_shape(v[r].P, b->reps[r]->chunks_set, groups, rho, words,
+                              resident);
+        // a replicate with many chunks has its partials folded as in a single population
+        v[r].P.free_words = v[r].P.chunks > 64 ? 16 : 64;
+        v[r].P.word_blocks = (v[r].P.w_cap + v[r].P.free_words - 1) / v[r].P.free_words;
     }
     if (b->d_views && b->host_views.size() == R &&
         std::memcmp(v.data(), b->host_views.data(), sizeof(RepView) * R) == 0)

@@ -1224,8 +1224,9 @@ struct Recombine {
 // interleaved chunk partials, then the first wave classifies the words and scans
 // the per-word counts.  A single population takes 16: its reduction reads
 // 16 bytes per word and row chunk, which 64-word blocks leave to a dozen compute
-// units (768 chunks x 816 words: 31 -> 14 us).  A batch takes 64:
-// its replicates have few chunks each, and a block costs more than its reads.
+// units (768 chunks x 816 words: 31 -> 14 us).  A replicate of a batch takes 64 up
+// to 64 chunks, where a block costs more than its reads (8 x 20,000 by groups, 400
+// words: 28 us with 64, 12 with 16).
 
 struct FreeReduce {
     static constexpr int kThreads = 1024;  // 16 waves share the chunk partials of 64 words
@@ -2689,8 +2690,7 @@ hipError_t query_residency(clotho_ctx* c) {
     return hipSuccess;
 }
 
-// The population's width when its state was last looked at, its capacity before.
-static uint32_t width_of(const clotho_ctx* c) { return c->live_words ? c->live_words : c->p.w_cap; }
+uint32_t width_of(const clotho_ctx* c) { return c->live_words ? c->live_words : c->p.w_cap; }
 
 // More than 16 traits: up to 256 words the balanced launch of one row tile per
 // wave, three blocks per compute unit, wider rows the one of two, which reads

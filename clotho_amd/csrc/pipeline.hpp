@@ -198,15 +198,23 @@ enum BatchOp : int {
 // generation (live blocks), and their rows of BatchLaunch::live_offs.
 constexpr int kLiveRecombine = 0, kLiveWordSort = 1, kLivePack = 2, kLiveGroups = 3, kLiveKinds = 4;
 
-// Rows wider than this recombine by groups in every batch (as in a single
-// population: 336 words 39 against 50 us, 816 words and more no slower); narrower
-// ones only in batches of at most kSmallBatch groups of 64 gametes per resident
-// block.  A group's tables cost as much as a few hundred words of its rows, so a
-// batch that fills the chip loses by them (256 replicates of mostly 8 to 72
-// words, 97,000 groups: 1.27 against 1.06 ms), while one that does not gains by its
-// smaller blocks (24 replicates, 800 groups: 51 against 141 us).
-constexpr uint32_t kWidePerGroup = 256;
+// Batches recombine by groups throughout up to kGroupBatch groups of 64 gametes per
+// resident block, where groups gain by their smaller blocks (16 replicates of 2,000,
+// 1,120 groups, 72 words x rho = 2: 157 us per generation against 212 by event). In larger
+// ones by event throughout while gametes have up to kEventRho events on average, as
+// in a single population, rows of kEventWords words on average up to kWideEventRho
+// (4 x 40,000, 5,600 groups: 8 words x rho = 0.5 142 us by
+// event, 196 by groups; 168 words x 2 475 / 559, 5 509 / 565; 32 words x 5 287 / 234; 64 x
+// 6,000, 13,440 groups: 32 words x 0.5 410 / 437, 168 x 2 1171 / 1298, 392 x 5 2394 / 2325).
+// With more events by groups, but beyond kSmallBatch groups per resident block only
+// rows wider than kWidePerGroup words: a group's tables cost as much as a few
+// hundred words of its rows (256 replicates of mostly 8 to 72 words, 97,000 groups: 1.27
+// against 1.06 ms).
+constexpr uint32_t kGroupBatch = 6;
 constexpr uint32_t kSmallBatch = 16;
+constexpr double kEventRho = 3.0, kWideEventRho = 5.0, kEventWords = 100.0;
+constexpr uint32_t kWidePerGroup = 256;
+constexpr uint32_t kNeverPerGroup = 1u << 30;
 
 struct BatchLaunch {
     const RepView* views = nullptr;  // device [R]
@@ -347,6 +355,7 @@ hipError_t launch_compact_plan(clotho_ctx* c);
 hipError_t launch_compact_rows(clotho_ctx* c, int src);
 uint32_t compact_chunks_of(const clotho_ctx* c);
 hipError_t query_residency(clotho_ctx* c);  // sets the resident rounds of the context's kernels
+uint32_t width_of(const clotho_ctx* c);  // row width when last looked at, the capacity before
 bool short_traits(const clotho_ctx* c);
 bool refresh_shapes(clotho_ctx* c);  // true: captured launches have the former shapes
 size_t population_piece_elems(const clotho_ctx* c, uint32_t h_cap);
