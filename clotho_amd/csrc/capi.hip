@@ -73,7 +73,6 @@ void free_buffers(clotho_ctx* c) {
         if (p) (void)hipFree(p);
     std::memset(&B, 0, sizeof(B));
     if (c->shape_status) (void)hipFree(c->shape_status);
-    if (c->scratch) (void)hipFree(c->scratch);
     if (c->stage) (void)hipHostFree(c->stage);
     for (hipEvent_t e : c->scratch_time)
         if (e) (void)hipEventDestroy(e);
@@ -91,8 +90,6 @@ void destroy_graphs(clotho_ctx* c) {
         }
     c->graphs.valid = false;
 }
-
-constexpr size_t kScratchKept = 64u << 20;  // covers 100,000 individuals of 1000 words
 
 constexpr size_t kStageBytes = 32u << 10;
 
@@ -135,36 +132,96 @@ int deliver(clotho_ctx* c, void* dst, const void* src, size_t bytes) {
     return CLOTHO_OK;
 }
 
-// Device memory of one call: the context's scratch, grown when it is too
-// small, or an allocation of its own above kScratchKept.  Calls on one context
-// do not overlap on its stream; a second thread's call waits.
+// The calling thread's current device is the context's for a scope: memory is
+// allocated on the current device, which a caller with contexts on several leaves
+// at another.
+struct OnDevice {
+    int before = -1;
+    explicit OnDevice(int device) {
+        int now = device;
+        if (hipGetDevice(&now) == hipSuccess && now != device) {
+            before = now;
+            (void)hipSetDevice(device);
+        }
+    }
+    ~OnDevice() {
+        if (before >= 0) (void)hipSetDevice(before);
+    }
+};
+
+// Memory that calls on one device's contexts work in, kept between calls while a
+// context is there: at most kScratchKept bytes per device, however many contexts
+// (replicates of a batch, say) it serves.
+constexpr size_t kScratchKept = 64u << 20;  // covers 100,000 individuals of 1000 words
+struct DeviceScratch {
+    std::mutex in_use;  // held by the call that works in it
+    char* base = nullptr;
+    size_t bytes = 0;
+    std::mutex counted;
+    uint32_t contexts = 0;
+};
+constexpr int kMaxDevices = 64;
+DeviceScratch g_scratch[kMaxDevices];
+
+void scratch_join(int device) {
+    if (device < 0 || device >= kMaxDevices) return;
+    DeviceScratch& d = g_scratch[device];
+    const std::lock_guard<std::mutex> lock(d.counted);
+    ++d.contexts;
+}
+void scratch_leave(int device) {
+    if (device < 0 || device >= kMaxDevices) return;
+    DeviceScratch& d = g_scratch[device];
+    const std::lock_guard<std::mutex> lock(d.counted);
+    if (--d.contexts) return;
+    const std::lock_guard<std::mutex> use(d.in_use);
+    if (d.base) (void)hipFree(d.base);
+    d.base = nullptr;
+    d.bytes = 0;
+}
+
+// Device memory of one call: the device's scratch, grown when it is too small,
+// or an allocation of its own above kScratchKept and while another context's call
+// has the scratch.  A second call on the same context waits (the events that time the
+// kernels are the context's).  Whatever path the call returns by, its work on the
+// stream is done before the memory is free for others.
 struct Scratch {
     clotho_ctx* c;
-    std::unique_lock<std::mutex> lock;
+    std::unique_lock<std::mutex> mine, shared;
     char* base = nullptr;
     char* own = nullptr;
-    explicit Scratch(clotho_ctx* ctx) : c(ctx), lock(ctx->scratch_mutex) {}
+    bool finished = false;
+    explicit Scratch(clotho_ctx* ctx) : c(ctx), mine(ctx->scratch_mutex) {}
     ~Scratch() {
+        if (base && !finished) (void)hipStreamSynchronize(c->stream);
         if (own) (void)hipFree(own);
     }
     hipError_t get(size_t bytes) {
-        if (bytes > kScratchKept) {
-            const hipError_t e = hipMalloc((void**)&own, bytes);
-            base = own;
-            return e;
+        const OnDevice here(c->device);
+        if (bytes <= kScratchKept && c->device < kMaxDevices) {
+            DeviceScratch& d = g_scratch[c->device];
+            shared = std::unique_lock<std::mutex>(d.in_use, std::try_to_lock);
+            if (shared && bytes > d.bytes) {
+                if (d.base) (void)hipFree(d.base);  // waits for the device
+                d.base = nullptr;
+                d.bytes = 0;
+                const hipError_t e = hipMalloc((void**)&d.base, bytes);
+                if (e != hipSuccess) return failed(e);
+                d.bytes = bytes;
+            }
+            if (shared) {
+                base = d.base;
+                return hipSuccess;
+            }
         }
-        if (bytes > c->scratch_bytes) {
-            if (c->scratch) (void)hipFree(c->scratch);  // waits for the device
-            c->scratch = nullptr;
-            c->device_bytes -= c->scratch_bytes;
-            c->scratch_bytes = 0;
-            const hipError_t e = hipMalloc((void**)&c->scratch, bytes);
-            if (e != hipSuccess) return e;
-            c->scratch_bytes = bytes;
-            c->device_bytes += bytes;
-        }
-        base = c->scratch;
+        const hipError_t e = hipMalloc((void**)&own, bytes);
+        if (e != hipSuccess) return failed(e);
+        base = own;
         return hipSuccess;
+    }
+    static hipError_t failed(hipError_t e) {
+        (void)hipGetLastError();  // not for the next call to find
+        return e;
     }
 };
 // parts of a scratch allocation, on 256-byte lines
@@ -177,9 +234,10 @@ struct Parts {
     }
 };
 
-// dst[i] = src[i] * scale.  A few values are converted here; more on the device:
-// the copy then goes straight into the caller's pages (200,000 traits: 171 us
-// with the conversion here, 138 there).
+// dst[i] = src[i] * scale.  A few values are converted here; more on the device, as
+// many at a time as the kept scratch holds: the copy then goes straight into the
+// caller's pages (200,000 traits: 171 us with the conversion here, 138 there).
+// Where a full device has no memory for that, they are converted here, too.
 template <class T>
 int fetch_scaled(clotho_ctx* c, double* dst, const T* src, size_t n, double scale) {
     if (sizeof(T) * n <= kStageBytes)
@@ -187,11 +245,26 @@ int fetch_scaled(clotho_ctx* c, double* dst, const T* src, size_t n, double scal
             const T* v = reinterpret_cast<const T*>(p);
             for (size_t i = 0; i < n; ++i) dst[i] = (double)v[i] * scale;
         });
+    const size_t piece = std::min<size_t>(n, kScratchKept / 8);
+    const OnDevice here(c->device);  // for the launches
     Scratch tmp(c);
-    HIP_TRY(c, tmp.get(8 * n));
+    if (tmp.get(8 * piece) != hipSuccess) {
+        std::vector<T> v(piece);
+        for (size_t at = 0; at < n; at += piece) {
+            const size_t m = std::min(piece, n - at);
+            if (const int rc = fetch(c, v.data(), src + at, sizeof(T) * m)) return rc;
+            for (size_t i = 0; i < m; ++i) dst[at + i] = (double)v[i] * scale;
+        }
+        return CLOTHO_OK;
+    }
     double* const d = reinterpret_cast<double*>(tmp.base);
-    HIP_TRY(c, launch_scale(src, n, scale, d, c->stream));
-    return fetch(c, dst, d, 8 * n);
+    for (size_t at = 0; at < n; at += piece) {
+        const size_t m = std::min(piece, n - at);
+        HIP_TRY(c, launch_scale(src + at, m, scale, d, c->stream));
+        if (const int rc = fetch(c, dst + at, d, 8 * m)) return rc;
+    }
+    tmp.finished = true;
+    return CLOTHO_OK;
 }
 
 int read_state(clotho_ctx* c, GenState* st) {
@@ -365,9 +438,11 @@ int clotho_create(const clotho_config* cfg, int device, clotho_ctx** out) {
         delete c;
         return CLOTHO_ERR_ARG;
     }
+    scratch_join(device);
     auto bail = [&](int rc) {
         free_buffers(c);
         if (c->stream) (void)hipStreamDestroy(c->stream);
+        scratch_leave(device);
         delete c;
         return rc;
     };
@@ -516,6 +591,7 @@ void clotho_destroy(clotho_ctx* ctx) {
     destroy_graphs(ctx);
     free_buffers(ctx);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
+    scratch_leave(ctx->device);
     delete ctx;
 }
 
@@ -649,6 +725,7 @@ int clotho_set_synthetic_population(clotho_ctx* c, uint32_t alleles, const doubl
 
 int clotho_get_shape(clotho_ctx* c, clotho_shape* out) {
     if (!c || !out) return CLOTHO_ERR_ARG;
+    const OnDevice here(c->device);
     HIP_TRY(c, launch_shape(c));
     ShapeStatus now;
     const int rc = fetch(c, &now, c->shape_status, sizeof(now));
@@ -848,6 +925,7 @@ int clotho_allele_counts(clotho_ctx* c, const uint32_t* rows, uint32_t n_rows,
     if (rc) return rc;
     float ms = 0.f;
     HIP_TRY(c, hipEventSynchronize(c->scratch_time[1]));
+    tmp.finished = true;
     HIP_TRY(c, hipEventElapsedTime(&ms, c->scratch_time[0], c->scratch_time[1]));
     if (kernel_ms) *kernel_ms = ms;
     return CLOTHO_OK;
@@ -880,6 +958,7 @@ int clotho_pairwise_differences(clotho_ctx* c, const uint32_t* rows, uint32_t n_
     HIP_TRY(c, launch_pairwise(c, c->b.rows[c->cur], W, d_sample, n_rows, d_out));
     HIP_TRY(c, hipEventRecord(c->scratch_time[1], c->stream));
     if ((rc = fetch(c, out, d_out, 4ull * pairs))) return rc;
+    tmp.finished = true;
     float ms = 0.f;
     HIP_TRY(c, hipEventElapsedTime(&ms, c->scratch_time[0], c->scratch_time[1]));
     if (kernel_ms) *kernel_ms = ms;
@@ -979,6 +1058,7 @@ int clotho_add_mutations(clotho_ctx* c, const uint32_t* rows, const double* posi
                        (const uint32_t*)(tmp.base + at_slots), (const uint32_t*)(tmp.base + at_keys),
                        (const int32_t*)(tmp.base + at_eff), n, age));
         HIP_TRY(c, hipStreamSynchronize(c->stream));
+        tmp.finished = true;
     }
     // traits and free space of the new population
     st.alleles = st.all_size = (uint32_t)A1;

@@ -287,12 +287,9 @@ struct clotho_ctx {
     std::mutex stage_mutex;
     char* stage = nullptr;
     clotho::ShapeStatus* shape_status = nullptr;  // device memory
-    // Device memory of the analysis and mutation calls, kept between them up to
-    // kScratchKept bytes, and the events that time their kernels; one call at a
-    // time uses them.
+    // The events that time the analysis calls' kernels; one call at a time uses them
+    // and works in the device's scratch memory.
     std::mutex scratch_mutex;
-    char* scratch = nullptr;
-    size_t scratch_bytes = 0;
     hipEvent_t scratch_time[2] = {nullptr, nullptr};
     size_t device_bytes = 0;    // sum of the context's device allocations
     uint32_t next_n = 0;        // offspring individuals of following generations (0: keep)
