@@ -101,6 +101,7 @@ int sync_views(clotho_batch* b) {
         v[r].P = b->reps[r]->p;
         v[r].B = b->reps[r]->b;
         v[r].B.by_parent = nullptr;  // replicates recombine in child order
+        v[r].B.trait_part = nullptr;  // and sum their traits in whole row blocks
         batch_recombine_shape(v[r].P, b->reps[r]->chunks_set, groups, rho, words,
                               resident);
         // a replicate with many chunks has its partials folded as in a single population
@@ -191,7 +192,7 @@ int clotho_batch_create(const clotho_config* cfgs, uint32_t count, int device,
         return bail(CLOTHO_ERR_HIP);
     for (uint32_t r = 0; r < count; ++r) {
         clotho_ctx* c = nullptr;
-        const int rc = clotho_create(&cfgs[r], device, &c);
+        const int rc = create_context(&cfgs[r], device, true, &c);
         if (rc != CLOTHO_OK) return bail(rc);
         b->reps.push_back(c);
     }

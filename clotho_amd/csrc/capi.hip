@@ -356,11 +356,20 @@ int enqueue_generation(clotho_ctx* c, std::vector<hipEvent_t>* marks) {
     return CLOTHO_OK;
 }
 
+// Memory for the pieces of the context's own balanced traits launches.  A batch makes
+// none, so a replicate gets it with the first launches of its own.
+int ensure_pieces(clotho_ctx* c) {
+    if (c->b.trait_part) return CLOTHO_OK;
+    const OnDevice here(c->device);
+    return dalloc(c, &c->b.trait_part, population_piece_elems(c));
+}
+
 // Population index current after one generation from parent index cur.
 int after_generation(const clotho_ctx* c, int cur) { return c->cfg.compact_every ? cur : 1 - cur; }
 
 int capture_graphs(clotho_ctx* c) {
     if (c->graphs.valid) return CLOTHO_OK;
+    if (const int rc = ensure_pieces(c)) return rc;
     const int saved = c->cur;
     for (int k = 0; k < 2; ++k) {
         c->cur = k;
@@ -388,19 +397,7 @@ int capture_graphs(clotho_ctx* c) {
     return CLOTHO_OK;
 }
 
-}  // namespace clotho
-
-extern "C" {
-
-const char* clotho_version(void) { return "clotho_amd 0.1 (gfx950)"; }
-
-const char* clotho_last_error(const clotho_ctx* ctx) { return ctx ? ctx->err.c_str() : ""; }
-
-int clotho_poisson_table(double lambda, double* cdf, int cap) {
-    return poisson_table(lambda, cdf, cap);
-}
-
-int clotho_create(const clotho_config* cfg, int device, clotho_ctx** out) {
+int create_context(const clotho_config* cfg, int device, bool replicate, clotho_ctx** out) {
     if (!cfg || !out) return CLOTHO_ERR_ARG;
     *out = nullptr;
     if (cfg->n_individuals == 0 || cfg->n_individuals > (1u << 28)) return CLOTHO_ERR_ARG;
@@ -511,7 +508,7 @@ int clotho_create(const clotho_config* cfg, int device, clotho_ctx** out) {
     rc |= dalloc(c, &B.pm, prefix_elems(P.w_cap));
     rc |= dalloc(c, &B.bucket, table_elems(P.w_cap));
     rc |= dalloc(c, &B.digits, trait_digit_elems(std::max<uint32_t>(1, P.traits), P.w_cap));
-    rc |= dalloc(c, &B.trait_part, population_piece_elems(c, h_cap));
+    if (!replicate) rc |= ensure_pieces(c);
     rc |= dalloc(c, &B.mut_count, h_cap);
     rc |= dalloc(c, &B.mut_local, h_cap);
     rc |= dalloc(c, &B.mut_bsum, mut_blocks_cap);
@@ -582,6 +579,22 @@ int clotho_create(const clotho_config* cfg, int device, clotho_ctx** out) {
     c->cur = 0;
     *out = c;
     return CLOTHO_OK;
+}
+
+}  // namespace clotho
+
+extern "C" {
+
+const char* clotho_version(void) { return "clotho_amd 0.1 (gfx950)"; }
+
+const char* clotho_last_error(const clotho_ctx* ctx) { return ctx ? ctx->err.c_str() : ""; }
+
+int clotho_poisson_table(double lambda, double* cdf, int cap) {
+    return poisson_table(lambda, cdf, cap);
+}
+
+int clotho_create(const clotho_config* cfg, int device, clotho_ctx** out) {
+    return create_context(cfg, device, false, out);
 }
 
 void clotho_destroy(clotho_ctx* ctx) {
@@ -1223,6 +1236,7 @@ int clotho_run(clotho_ctx* c, uint32_t n, int use_graph) {
     tm.generations = 0;
     std::vector<hipEvent_t> marks;
     if (refresh_shapes(c)) destroy_graphs(c);
+    if (const int rc = ensure_pieces(c)) return rc;
     // a generation that changes the population size runs with eager launches
     if (c->next_n && c->next_n != c->p.n) use_graph = 0;
     if (use_graph) {

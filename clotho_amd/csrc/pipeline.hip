@@ -2629,7 +2629,8 @@ static hipError_t launch_traits_of(clotho_ctx* c, int which, bool pack) {
     const uint32_t sel = (uint32_t)which;
     if (pack) TRY_LAUNCH(launch_single<PackDigits>(k_pack_digits, c, sel));
     const int cls = f6::trait_class(c->p.traits);
-    const uint32_t v = c->trait_variant;  // 0: default shape; the autotuner may pick another
+    // 0 or 1: default shape; the autotuner may pick another
+    const uint32_t v = !c->b.trait_part && c->trait_variant < 2 ? 2 : c->trait_variant;
     c->p.trait_blocks = 0;
     if (v == 2 || v == 3) {
         if (cls <= 1 && v == 2)
@@ -2703,8 +2704,9 @@ uint32_t width_of(const clotho_ctx* c) { return c->live_words ? c->live_words : 
 bool short_traits(const clotho_ctx* c) { return c->p.traits > 16 && width_of(c) <= 256; }
 
 // int64 elements that the pieces of either balanced launch take
-size_t population_piece_elems(const clotho_ctx* c, uint32_t h_cap) {
+size_t population_piece_elems(const clotho_ctx* c) {
     const Params& P = c->p;
+    const uint32_t h_cap = 2 * P.n_cap;
     if (!P.traits) return 1;
     const uint32_t rows = f6::balanced_block_rows(f6::trait_class(P.traits));
     const size_t n = trait_piece_elems(P.traits, rows, h_cap, P.w_cap, c->trait_round);

@@ -133,7 +133,8 @@ struct Buffers {
     uint64_t* pm;             // [tiles][65 c][64 w] bits of the c smallest keys of each word
     uint32_t* bucket;         // [tiles][64 q][64 w] per word: #{keys < b<<24}, four b per dword
     uint4* digits;            // FP6 digit planes of the effects (trait_digit_elems)
-    int64_t* trait_part;      // [2 blocks][rows][T] pieces of cut row blocks (f6::piece_elems)
+    int64_t* trait_part;      // [2 blocks][rows][T] pieces of cut row blocks (f6::piece_elems); nullptr:
+                              // traits launches take whole row blocks
     uint32_t* mut_count;      // [h]
     uint32_t* mut_local;      // [h] exclusive scan inside a block
     uint32_t* mut_bsum;       // [mut_blocks] block totals -> exclusive offsets
@@ -355,7 +356,7 @@ hipError_t query_residency(clotho_ctx* c);  // sets the resident rounds of the c
 uint32_t width_of(const clotho_ctx* c);  // row width when last looked at, the capacity before
 bool short_traits(const clotho_ctx* c);
 bool refresh_shapes(clotho_ctx* c);  // true: captured launches have the former shapes
-size_t population_piece_elems(const clotho_ctx* c, uint32_t h_cap);
+size_t population_piece_elems(const clotho_ctx* c);
 // launch shape of the recombination: row chunks for h rows, and the column
 // ranges that go with a number of row chunks
 uint32_t recombine_chunks(const clotho_ctx* c, uint32_t h);
@@ -382,6 +383,7 @@ hipError_t launch_end_analysis(clotho_ctx* c);  // the next generation starts an
 hipError_t launch_synth_rows(clotho_ctx* c, uint64_t seed, const uint32_t* d_thr, uint32_t alleles,
                              uint32_t words);
 // Context helpers (capi.hip).
+int create_context(const clotho_config* cfg, int device, bool replicate, clotho_ctx** out);
 void destroy_graphs(clotho_ctx* c);
 int read_state(clotho_ctx* c, GenState* st);
 int write_state(clotho_ctx* c, const GenState& st);

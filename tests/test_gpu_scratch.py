@@ -1,5 +1,6 @@
 """Device memory that calls keep between them: one scratch allocation of at most 64 MiB
-per device for all contexts."""
+per device for all contexts, and none of a replicate's for launches that its batch does
+not make."""
 import threading
 
 import numpy as np
@@ -62,3 +63,29 @@ def test_threads_with_contexts_of_their_own():
     assert not errors
     for s in sims:
         s.close()
+
+
+def test_replicates_hold_no_pieces():
+    # 16 traits: a balanced launch of a replicate's own would keep up to 33 MB for its
+    # pieces, which a batch never makes
+    cfgs = [api.make_config(4000, 0.01, 1.0, seed=1, replicate=r, traits=16, sigma=0.1,
+                            max_alleles=4096) for r in range(8)]
+    batch = api.Batch(cfgs)
+    lone = api.Simulation(cfgs[0])
+    per = [batch.replicate(r).device_bytes() for r in range(8)]
+    assert max(per) < lone.device_bytes() - 3 * MIB
+    rng = np.random.default_rng(2)
+    rows = rng.integers(0, 2**63, (8000, 32), dtype=np.int64).view(np.uint64)
+    eff = rng.integers(-2**20, 2**20, (2048, 16)) * 2.0**-24
+    for s in (lone, *[batch.replicate(r) for r in range(8)]):
+        s.set_population(rows, np.arange(2048) / 2**32, eff)
+    assert max(batch.replicate(r).device_bytes() for r in range(8)) == max(per)
+    assert np.array_equal(batch.replicate(3).traits(), lone.traits())
+    batch.run(2, mode="graph")
+    lone.run(2)
+    assert np.array_equal(batch.replicate(0).traits(), lone.traits())
+    batch.run(2, mode="sequential")  # replicates' own launches
+    lone.run(2)
+    assert np.array_equal(batch.replicate(0).traits(), lone.traits())
+    batch.close()
+    lone.close()
