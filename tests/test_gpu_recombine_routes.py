@@ -74,3 +74,15 @@ def test_tuned_by_event():
     _steps(sim, orc, 1, False, "before")
     sim.autotune()
     _steps(sim, orc, 2, True, "tuned")
+
+
+@pytest.mark.parametrize("chunks", [1, 3, 8, 13])
+def test_blocks_without_work(chunks):
+    # the grid has several blocks per chunk for wide rows; rows of up to 32 words have
+    # work in one of them only
+    sim, orc = _pair(700, 1.5, 1 << 15)
+    sim.set_launch_shape(recombine_chunks=chunks)
+    for alleles, graph in ((300, True), (1900, False), (2400, True), (100, True)):
+        for x in (sim, orc):
+            x.set_population(*_population(700, alleles, alleles))
+        _steps(sim, orc, 2, graph, f"{chunks} chunks, {alleles} alleles")
