@@ -1434,7 +1434,8 @@ int clotho_autotune(clotho_ctx* c, uint32_t* chosen_chunks) {
         c->compact_chunks = 0;
         const uint32_t dflt = compact_chunks_of(c);
         for (uint32_t rows : {4u, 8u, 16u})
-            for (uint32_t ch : {std::max<uint32_t>(1, dflt / 2), dflt, dflt * 2}) {
+            for (uint32_t ch : {std::max<uint32_t>(1, dflt / 2), dflt,
+                                std::min(2 * dflt, compact_chunks_limit(c))}) {
                 c->compact_rows = rows;
                 c->compact_chunks = ch;
                 float ms = 0.f;

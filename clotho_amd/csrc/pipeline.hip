@@ -3020,9 +3020,15 @@ static uint32_t compact_tile_groups_of(const clotho_ctx* c) {
     return (compact_tiles_of(c) + kCompactWaves - 1) / kCompactWaves;
 }
 
+// a launch holds fewer than 2^32 threads (32-row chunks reach that at N = 2^28)
+uint32_t compact_chunks_limit(const clotho_ctx* c) {
+    return 0xFFFFFFFFu / (64 * kCompactWaves) / compact_tile_groups_of(c);
+}
+
 uint32_t compact_chunks_of(const clotho_ctx* c) {
     if (c->compact_chunks) return c->compact_chunks;
-    return std::max<uint32_t>(1, (c->p.h + kCompactChunkRows - 1) / kCompactChunkRows);
+    return std::max<uint32_t>(1, std::min((c->p.h + kCompactChunkRows - 1) / kCompactChunkRows,
+                                          compact_chunks_limit(c)));
 }
 
 hipError_t launch_compact_rows(clotho_ctx* c, int src) {

@@ -352,6 +352,7 @@ uint32_t trait_variants(const clotho_ctx* c);
 hipError_t launch_compact_plan(clotho_ctx* c);
 hipError_t launch_compact_rows(clotho_ctx* c, int src);
 uint32_t compact_chunks_of(const clotho_ctx* c);
+uint32_t compact_chunks_limit(const clotho_ctx* c);
 hipError_t query_residency(clotho_ctx* c);  // sets the resident rounds of the context's kernels
 uint32_t width_of(const clotho_ctx* c);  // row width when last looked at, the capacity before
 bool short_traits(const clotho_ctx* c);
