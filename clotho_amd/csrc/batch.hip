@@ -91,7 +91,7 @@ int sync_views(clotho_batch* b) {
         const uint32_t own = (c->p.h + 63) / 64;
         groups += own;
         rho += own * c->cfg.rho;
-        words += (double)own * width_of(c);
+        words += (double)own * c->live_words;
     }
     rho /= (double)groups;
     words /= (double)groups;
@@ -164,6 +164,24 @@ int capture_batch(clotho_batch* b) {
         if (e3 != hipSuccess) {
             b->err = std::string("batch instantiate: ") + hipGetErrorString(e3);
             return CLOTHO_ERR_HIP;
+        }
+    }
+    return CLOTHO_OK;
+}
+
+// The views and, where the mode replays them, the captured launches, at the
+// replicates' widths when last looked at (replicates one by one, 256 of 8-72 words:
+// 19.8 -> 17.8 ms per generation against the shapes for their capacity).
+int ready_launches(clotho_batch* b, int mode) {
+    int rc = sync_views(b);
+    if (rc == CLOTHO_OK && mode == CLOTHO_BATCH_GRAPH) rc = capture_batch(b);
+    if (rc != CLOTHO_OK || mode != CLOTHO_BATCH_SEQUENTIAL) return rc;
+    for (clotho_ctx* c : b->reps) {
+        if (refresh_shapes(c)) destroy_graphs(c);
+        rc = capture_graphs(c);
+        if (rc != CLOTHO_OK) {
+            b->err = "replicate graph: " + c->err;
+            return rc;
         }
     }
     return CLOTHO_OK;
@@ -287,20 +305,8 @@ int clotho_batch_run(clotho_batch* b, uint32_t n, int mode, double* elapsed_ms) 
         }
         BATCH_TRY(b, hipStreamSynchronize(c->stream));  // uploads done
     }
-    int rc = sync_views(b);
+    int rc = ready_launches(b, mode);
     if (rc != CLOTHO_OK) return rc;
-    if (mode == CLOTHO_BATCH_GRAPH) {
-        rc = capture_batch(b);
-        if (rc != CLOTHO_OK) return rc;
-    } else if (mode == CLOTHO_BATCH_SEQUENTIAL) {
-        for (clotho_ctx* c : b->reps) {
-            rc = capture_graphs(c);
-            if (rc != CLOTHO_OK) {
-                b->err = "replicate graph: " + c->err;
-                return rc;
-            }
-        }
-    }
     Timing& tm = b->timing;
     for (double& v : tm.ms) v = 0.0;
     tm.generations = 0;
@@ -313,6 +319,17 @@ int clotho_batch_run(clotho_batch* b, uint32_t n, int mode, double* elapsed_ms) 
     BATCH_TRY(b, hipEventRecord(e0, b->stream));
     for (uint32_t g = 0; g < n; ++g) {
         const uint32_t par = (uint32_t)b->cur;
+        if (width_due(g)) {
+            BATCH_TRY(b, hipStreamSynchronize(b->stream));
+            for (clotho_ctx* c : b->reps) {
+                GenState seen;
+                if ((rc = read_state(c, &seen)) != CLOTHO_OK) {
+                    b->err = c->err;
+                    return rc;
+                }
+            }
+            if ((rc = ready_launches(b, mode)) != CLOTHO_OK) return rc;
+        }
         if (mode == CLOTHO_BATCH_GRAPH) {
             BATCH_TRY(b, hipGraphLaunch(b->exec[par], b->stream));
         } else if (mode == CLOTHO_BATCH_EAGER) {

@@ -1251,6 +1251,14 @@ int clotho_run(clotho_ctx* c, uint32_t n, int use_graph) {
             HIP_TRY(c, hipEventRecord(e0, c->stream));
         }
         for (uint32_t g = 0; g < n; ++g) {
+            if (width_due(g)) {
+                GenState seen;
+                if (const int rc2 = read_state(c, &seen)) return rc2;
+                if (refresh_shapes(c)) {
+                    destroy_graphs(c);
+                    if (const int rc2 = capture_graphs(c)) return rc2;
+                }
+            }
             HIP_TRY(c, hipGraphLaunch(c->graphs.exec[c->cur], c->stream));
             c->cur = after_generation(c, c->cur);
         }
@@ -1273,6 +1281,11 @@ int clotho_run(clotho_ctx* c, uint32_t n, int use_graph) {
                 mk = &all.back();
             }
             begin_generation(c);
+            if (width_due(g)) {
+                GenState seen;
+                if (const int rc2 = read_state(c, &seen)) return rc2;
+                if (refresh_shapes(c)) destroy_graphs(c);
+            }
             int rc = enqueue_generation(c, mk);
             if (rc) return rc;
             c->cur = after_generation(c, c->cur);

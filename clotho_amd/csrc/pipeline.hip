@@ -2700,17 +2700,14 @@ hipError_t query_residency(clotho_ctx* c) {
     return hipSuccess;
 }
 
-uint32_t width_of(const clotho_ctx* c) { return c->live_words ? c->live_words : c->p.w_cap; }
-
 // More than 16 traits: up to 256 words the balanced launch of one row tile per
 // wave, three blocks per compute unit, wider rows the one of two, which reads
 // each fragment from LDS for twice the rows but is alone on its compute unit.
 // Measured, traits and free space, 24 traits, two row tiles against one and the int8
 // kernel both replaced: 40,000 rows x 16 words 28 / 24 / 23 us; 200,000 x 16 75 / 48 /
 // 62; 200,000 x 80 147 / 134 / 184; 60,000 x 256 116 / 119 / 152; 200,000 x 480 530 /
-// 614 / 773.  By the width that the last run left (the capacity before it), as
-// either is right at any width.
-bool short_traits(const clotho_ctx* c) { return c->p.traits > 16 && width_of(c) <= 256; }
+// 614 / 773.  By the width when last looked at, as either is right at any width.
+bool short_traits(const clotho_ctx* c) { return c->p.traits > 16 && c->live_words <= 256; }
 
 // int64 elements that the pieces of either balanced launch take
 size_t population_piece_elems(const clotho_ctx* c) {
@@ -2745,12 +2742,15 @@ static bool recombine_by_event(const Params& P, const clotho_config& cfg, uint32
     return P.h >= 8192 && rho < limit && bytes > (20.0 + 50.0 * rho) * 1e6 && P.ev_cap <= 64;
 }
 
-// The launch shapes that follow the population's width, decided where a run
-// starts.  Row chunks that were set or tuned stay, with their kernel.
+// The launch shapes that follow the population's width, decided where a run starts
+// and again within it (width_due): a population starts out empty, so the
+// capacity says nothing of its rows (200 generations from none, N = 20,000, capacity
+// 256 words, rho = 1: 68 us each by groups, 90 by event).
+// Row chunks that were set or tuned stay, with their kernel.
 bool refresh_shapes(clotho_ctx* c) {
     const bool brief = short_traits(c);
     const bool by_event =
-        c->chunks_set ? c->by_event : recombine_by_event(c->p, c->cfg, width_of(c));
+        c->chunks_set ? c->by_event : recombine_by_event(c->p, c->cfg, c->live_words);
     if (brief == c->short_traits && by_event == c->by_event) return false;
     c->short_traits = brief;
     if (by_event != c->by_event) {

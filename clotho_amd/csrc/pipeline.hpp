@@ -297,7 +297,7 @@ struct clotho_ctx {
     uint32_t trait_round = 1;     // blocks of one resident round of the balanced traits kernel
     uint32_t short_round = 1;     // and of the one for rows of few words (more than 16 traits)
     bool short_traits = false;    // which of the two is launched (short_traits)
-    uint32_t live_words = 0;      // row width at the last look at the device's state
+    uint32_t live_words = 0;      // row width at the last look at the device's state, 0 before
     uint32_t recombine_round = 1; // and of the recombination by groups
     bool by_event = false;        // recombination by event (recombine_by_event)
     bool chunks_set = false;      // its row chunks were set or tuned
@@ -354,9 +354,10 @@ hipError_t launch_compact_rows(clotho_ctx* c, int src);
 uint32_t compact_chunks_of(const clotho_ctx* c);
 uint32_t compact_chunks_limit(const clotho_ctx* c);
 hipError_t query_residency(clotho_ctx* c);  // sets the resident rounds of the context's kernels
-uint32_t width_of(const clotho_ctx* c);  // row width when last looked at, the capacity before
 bool short_traits(const clotho_ctx* c);
 bool refresh_shapes(clotho_ctx* c);  // true: captured launches have the former shapes
+// generations of a run at which the widths are looked at: 64, 128, 256, ...
+inline bool width_due(uint32_t g) { return g >= 64 && (g & (g - 1)) == 0; }
 size_t population_piece_elems(const clotho_ctx* c);
 // launch shape of the recombination: row chunks for h rows, and the column
 // ranges that go with a number of row chunks

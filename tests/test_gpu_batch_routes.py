@@ -50,3 +50,24 @@ def test_routes(sizes, rho):
         compare_state(batch.replicate(r), lone, f"replicate {r}")
         lone.close()
     batch.close()
+
+
+@pytest.mark.parametrize("mode", ["graph", "eager", "sequential"])
+def test_width_looked_at_within_a_run(mode):
+    # 8 x 12,500 from no alleles to about 110 words, where rho = 4 changes the rule
+    cfgs = [api.make_config(12_500, 0.06, 4.0, seed=9, replicate=r, traits=1, neutral_p=0.3,
+                            sigma=0.1, fitness=api.FIT_GAUSSIAN_FIXED, env_sigma=1.0,
+                            max_alleles=1 << 14) for r in range(8)]
+    batch = api.Batch(cfgs)
+    batch.run(66, mode=mode)
+    batch.run(2, mode=mode)
+    for r in (0, 7):
+        alone = api.Simulation(cfgs[r])
+        for _ in range(17):
+            alone.run(4, graph=True)
+        rep = batch.replicate(r)
+        assert rep.shape().words == alone.shape().words >= 100
+        np.testing.assert_array_equal(rep.rows(), alone.rows())
+        np.testing.assert_array_equal(rep.traits(), alone.traits())
+        for a, b in zip(rep.free_space(), alone.free_space()):
+            np.testing.assert_array_equal(a, b)

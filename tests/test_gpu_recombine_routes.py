@@ -86,3 +86,14 @@ def test_blocks_without_work(chunks):
         for x in (sim, orc):
             x.set_population(*_population(700, alleles, alleles))
         _steps(sim, orc, 2, graph, f"{chunks} chunks, {alleles} alleles")
+
+
+@pytest.mark.parametrize("graph", [True, False])
+def test_width_looked_at_within_a_run(graph):
+    # 0 words at the start, about 270 at generation 64: by event from there on
+    cfg = api.make_config(4200, 0.2, 0.0, seed=5, traits=1, neutral_p=0.3, sigma=0.1,
+                          fitness=api.FIT_GAUSSIAN_FIXED, env_sigma=1.0, max_alleles=1 << 15)
+    sim, orc = api.Simulation(cfg), oracle.OracleSim(cfg)
+    assert sim.launch_shape()["recombine_chunks"] == 132
+    _steps(sim, orc, 67, graph, "from no alleles")
+    assert sim.launch_shape()["recombine_chunks"] == 17
