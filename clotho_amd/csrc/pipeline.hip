@@ -2292,25 +2292,27 @@ using RecombineEvents = Recombine<false, kSibsOrdered>;
 // after another: the chunk's gamete records and event keys, which every tile
 // block of the chunk reads, then stay in that XCD's L2 (with the hardware's
 // round-robin order every tile block of a chunk ran on another XCD and
-// fetched them again).
-#define CLOTHO_SINGLE_XCD(name, Op)                                                             \
-    __global__ void __launch_bounds__(Op::kThreads)                                            \
-        __attribute__((amdgpu_waves_per_eu(MinWaves<Op>::value)))                               \
-        name(Params P, Buffers B, uint32_t sel) {                                               \
-        Op::run(P, B, sel, xcd_contiguous(blockIdx.x, gridDim.x));                              \
-    }
-// By groups only the blocks with work are numbered, and they come first: narrow rows
-// have work in P.chunks blocks, which as the first numbers of the whole grid would lie
-// on a part of the XCDs (N = 100,000, 8 words, 768 of 1,536 blocks: 53 -> 31 us; work in
-// every second block also took 53, with idle blocks between; N = 1,000: 11.1 -> 11.4).
+// fetched them again).  Only the blocks with work are numbered, and they come
+// first.  By groups narrow rows have work in P.chunks blocks, which as the first numbers of
+// the whole grid would lie on a part of the XCDs (N = 100,000, 8 words, 768 of
+// 1,536 blocks: 53 -> 31 us; work in every second block also took 53, with idle
+// blocks between; N = 1,000: 11.1 -> 11.4).  By event the column tiles past the width
+// have none (N = 250,000, 112 words, rho = 3: capacity 1,024 words 398 -> 208 us, 4,096
+// words 632 -> 225; 122 words 213 -> 201).
 __global__ void __launch_bounds__(rec::Recombine::kThreads)
     __attribute__((amdgpu_waves_per_eu(MinWaves<rec::Recombine>::value)))
     k_recombine(Params P, Buffers B, uint32_t sel) {
     const uint32_t live = rec::Recombine::live(P, uniform_read(&gbl(B.state)->wc));
     if (blockIdx.x < live) rec::Recombine::run(P, B, sel, xcd_contiguous(blockIdx.x, live));
 }
-CLOTHO_SINGLE_XCD(k_recombine_events, RecombineEvents)
-#undef CLOTHO_SINGLE_XCD
+__global__ void __launch_bounds__(RecombineEvents::kThreads)
+    __attribute__((amdgpu_waves_per_eu(MinWaves<RecombineEvents>::value)))
+    k_recombine_events(Params P, Buffers B, uint32_t sel) {
+    const uint32_t tiles = min((uniform_read(&gbl(B.state)->wc) + 63) / 64, P.tiles);
+    if (blockIdx.x >= tiles * P.chunks) return;
+    const uint32_t u = xcd_contiguous(blockIdx.x, tiles * P.chunks);
+    RecombineEvents::run(P, B, sel, u / tiles * P.tiles + u % tiles);
+}
 CLOTHO_SINGLE(k_pack_digits, PackDigits)
 // by trait class (f6::trait_class: T <= 2, 4, 8, 16, 32)
 using Traits2Balanced = Traits<f6::balanced_tiles(0), 0, f6::Form::kBalancedFew>;
@@ -2751,13 +2753,19 @@ bool refresh_shapes(clotho_ctx* c) {
     const bool brief = short_traits(c);
     const bool by_event =
         c->chunks_set ? c->by_event : recombine_by_event(c->p, c->cfg, c->live_words);
-    if (brief == c->short_traits && by_event == c->by_event) return false;
-    c->short_traits = brief;
-    if (by_event != c->by_event) {
-        c->by_event = by_event;
-        c->p.chunks = std::min(c->p.max_chunks, recombine_chunks(c, c->p.h));
-        c->p.splits = recombine_splits(c, c->p.chunks);
+    const bool same = by_event == c->by_event;
+    c->by_event = by_event;
+    uint32_t chunks = c->p.chunks;
+    if (!c->chunks_set) {
+        chunks = std::min(c->p.max_chunks, recombine_chunks(c, c->p.h));
+        // not for a column tile more or less from run to run
+        if (same && 4 * chunks < 5 * c->p.chunks && 4 * c->p.chunks < 5 * chunks)
+            chunks = c->p.chunks;
     }
+    if (same && brief == c->short_traits && chunks == c->p.chunks) return false;
+    c->short_traits = brief;
+    c->p.chunks = chunks;
+    c->p.splits = recombine_splits(c, chunks);
     return true;
 }
 
@@ -2767,8 +2775,9 @@ bool refresh_shapes(clotho_ctx* c) {
 uint32_t recombine_chunks(const clotho_ctx* c, uint32_t h) {
     if (c->by_event) {
         // about 4096 blocks of a column tile each, but at least 32 rows per wave
-        // (a block's order-statistic tables are loaded once per block)
-        const uint32_t tiles = c->p.tiles;
+        // (a block's order-statistic tables are loaded once per block); of the
+        // present tiles, as the tiles of the capacity would leave few blocks with work
+        const uint32_t tiles = std::max(1u, (c->live_words + 63) / 64);
         return std::max<uint32_t>(1, std::min((4096 + tiles - 1) / tiles, (h + 511) / 512));
     }
     const uint32_t groups = (h + rec::kGroup - 1) / rec::kGroup;

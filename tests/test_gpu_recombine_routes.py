@@ -97,3 +97,13 @@ def test_width_looked_at_within_a_run(graph):
     assert sim.launch_shape()["recombine_chunks"] == 132
     _steps(sim, orc, 67, graph, "from no alleles")
     assert sim.launch_shape()["recombine_chunks"] == 17
+
+
+@pytest.mark.parametrize("words", [152, 192, 200])
+def test_capacity_beyond_the_width(words):
+    # by event with 3 and 4 live column tiles of 64
+    sim, orc = _pair(4200, 0.0, 1 << 18)
+    for x in (sim, orc):
+        x.set_population(*_population(4200, 64 * words - 100, words))
+    _steps(sim, orc, 2, True, f"{words} words")
+    assert sim.launch_shape()["recombine_chunks"] == 17
