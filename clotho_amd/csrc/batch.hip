@@ -61,13 +61,13 @@ void drop_graphs(clotho_batch* b) {
 // fewer where that would not give every resident block four chunks (64 x 6,000, 392
 // words, rho = 5: 2334 us, with 16 2699), and column ranges where the chunks alone
 // do not give it one.  Row chunks that were set or tuned for a
-// replicate are taken for it, two per block.  rho, words: events per gamete and row
-// width, mean over the batch's rows.
-void batch_recombine_shape(Params& P, bool chunks_set, uint64_t groups, double rho, double words,
+// replicate are taken for it, two per block.  rho: events per gamete, filled: the
+// part of the rows' column tiles of 64 words that they fill, over all rows.
+void batch_recombine_shape(Params& P, bool chunks_set, uint64_t groups, double rho, double filled,
                            uint32_t resident) {
     if (groups <= (uint64_t)kGroupBatch * resident)
         P.group_words = 0;
-    else if (rho <= (words < kEventWords ? kEventRho : kWideEventRho))
+    else if (rho <= (filled < kEventFill ? kEventRho : kWideEventRho))
         P.group_words = kNeverPerGroup;
     else
         P.group_words = groups <= (uint64_t)kSmallBatch * resident ? 0 : kWidePerGroup;
@@ -86,15 +86,16 @@ int sync_views(clotho_batch* b) {
     const uint32_t R = (uint32_t)b->reps.size();
     std::vector<RepView> v(R);
     uint64_t groups = 0;
-    double rho = 0.0, words = 0.0;
+    double rho = 0.0, words = 0.0, tiles = 0.0;
     for (const clotho_ctx* c : b->reps) {
         const uint32_t own = (c->p.h + 63) / 64;
         groups += own;
         rho += own * c->cfg.rho;
         words += (double)own * c->live_words;
+        tiles += (double)own * (64 * ((c->live_words + 63) / 64));
     }
     rho /= (double)groups;
-    words /= (double)groups;
+    const double filled = tiles > 0.0 ? words / tiles : 0.0;
     const uint32_t resident = b->reps[0]->recombine_round;
     for (uint32_t r = 0; r < R; ++r) {
         std::memset(&v[r], 0, sizeof(RepView));
@@ -102,7 +103,7 @@ int sync_views(clotho_batch* b) {
         v[r].B = b->reps[r]->b;
         v[r].B.by_parent = nullptr;  // replicates recombine in child order
         v[r].B.trait_part = nullptr;  // and sum their traits in whole row blocks
-        batch_recombine_shape(v[r].P, b->reps[r]->chunks_set, groups, rho, words,
+        batch_recombine_shape(v[r].P, b->reps[r]->chunks_set, groups, rho, filled,
                               resident);
         // a replicate with many chunks has its partials folded as in a single population
         v[r].P.free_words = v[r].P.chunks > 64 ? 16 : 64;
@@ -319,7 +320,9 @@ int clotho_batch_run(clotho_batch* b, uint32_t n, int mode, double* elapsed_ms) 
     BATCH_TRY(b, hipEventRecord(e0, b->stream));
     for (uint32_t g = 0; g < n; ++g) {
         const uint32_t par = (uint32_t)b->cur;
-        if (width_due(g)) {
+        // Batched launches keep their shapes within a run: reading 256 replicates' widths
+        // takes as long as eight generations of 3,000 individuals.
+        if (mode == CLOTHO_BATCH_SEQUENTIAL && width_due(g)) {
             BATCH_TRY(b, hipStreamSynchronize(b->stream));
             for (clotho_ctx* c : b->reps) {
                 GenState seen;

@@ -203,8 +203,9 @@ constexpr int kLiveRecombine = 0, kLiveWordSort = 1, kLivePack = 2, kLiveGroups 
 // resident block, where groups gain by their smaller blocks (16 replicates of 2,000,
 // 1,120 groups, 72 words x rho = 2: 157 us per generation against 212 by event). In larger
 // ones by event throughout while gametes have up to kEventRho events on average, as
-// in a single population, rows of kEventWords words on average up to kWideEventRho
-// (4 x 40,000, 5,600 groups: 8 words x rho = 0.5 142 us by
+// in a single population, where the rows fill kEventFill of their column tiles of 64
+// words up to kWideEventRho (16 x 12,500, rho = 3.4: 56 words 310 / 316, 72 words
+// 410 / 374, 64 x 6,000: 88 words x 4 706 / 749; 4 x 40,000, 5,600 groups: 8 words x rho = 0.5 142 us by
 // event, 196 by groups; 168 words x 2 475 / 559, 5 509 / 565; 32 words x 5 287 / 234; 64 x
 // 6,000, 13,440 groups: 32 words x 0.5 410 / 437, 168 x 2 1171 / 1298, 392 x 5 2394 / 2325).
 // With more events by groups, but beyond kSmallBatch groups per resident block only
@@ -213,7 +214,7 @@ constexpr int kLiveRecombine = 0, kLiveWordSort = 1, kLivePack = 2, kLiveGroups 
 // against 1.06 ms).
 constexpr uint32_t kGroupBatch = 6;
 constexpr uint32_t kSmallBatch = 16;
-constexpr double kEventRho = 3.0, kWideEventRho = 5.0, kEventWords = 100.0;
+constexpr double kEventRho = 3.0, kWideEventRho = 5.0, kEventFill = 2.0 / 3.0;
 constexpr uint32_t kWidePerGroup = 256;
 constexpr uint32_t kNeverPerGroup = 1u << 30;
 
