@@ -841,6 +841,7 @@ int clotho_download_gametes(clotho_ctx* c, uint32_t* top, uint32_t* bottom, uint
 int clotho_phase_draw(clotho_ctx* c) {
     if (!c) return CLOTHO_ERR_ARG;
     begin_generation(c);
+    if (refresh_shapes(c)) destroy_graphs(c);
     HIP_TRY(c, launch_draw(c));
     return CLOTHO_OK;
 }
@@ -1334,6 +1335,7 @@ int clotho_autotune(clotho_ctx* c, uint32_t* chosen_chunks) {
         if (chosen_chunks) *chosen_chunks = c->p.chunks;
         return CLOTHO_OK;
     }
+    if (refresh_shapes(c)) destroy_graphs(c);
     const uint32_t base = c->p.chunks;
     std::vector<uint32_t> cand;
     for (uint32_t f : {1u, 2u, 4u, 8u}) {
@@ -1344,7 +1346,7 @@ int clotho_autotune(clotho_ctx* c, uint32_t* chosen_chunks) {
     const uint32_t groups = (c->p.h + 63) / 64;
     if (c->by_event)  // whole waves of two resident blocks per compute unit
         for (uint32_t k = 1, two = 2u * (uint32_t)std::max(1, c->prop.multiProcessorCount); k <= 16; ++k)
-            cand.push_back(std::min(c->p.max_chunks, std::max<uint32_t>(1, k * two / c->p.tiles)));
+            cand.push_back(std::min(c->p.max_chunks, std::max<uint32_t>(1, k * two / std::max(1u, (c->live_words + 63) / 64))));
     for (uint32_t k = 1; k <= 8 && !c->by_event; ++k)
         cand.push_back(std::min<uint32_t>(c->p.max_chunks, (groups + k - 1) / k));
     for (uint32_t k = 1; k <= 2 && !c->by_event; ++k)
@@ -1404,7 +1406,7 @@ int clotho_autotune(clotho_ctx* c, uint32_t* chosen_chunks) {
     }
     c->p.chunks = best_chunks;
     c->p.splits = recombine_splits(c, best_chunks);
-    c->chunks_set = true;
+    c->chunks_set = c->kernel_set = true;
 
     // The traits pass: every kernel shape over the current population (the
     // pass writes the traits it already holds), fastest of two passes.
@@ -1481,7 +1483,10 @@ int clotho_set_launch_shape(clotho_ctx* c, const clotho_launch_shape* in) {
                     "set_launch_shape: chunks 1.." + std::to_string(c->p.max_chunks) +
                         ", traits shape 1.." + std::to_string(nv) +
                         ", compaction rows 4/8/16, compaction tile words 48/56/60/64");
-    if (in->recombine_chunks != c->p.chunks) c->chunks_set = true;
+    if (in->recombine_chunks != c->p.chunks) {
+        c->chunks_set = true;
+        c->kernel_set = false;
+    }
     c->p.chunks = in->recombine_chunks;
     c->p.splits = recombine_splits(c, in->recombine_chunks);
     c->trait_variant = in->traits_variant;

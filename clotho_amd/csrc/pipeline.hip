@@ -2748,11 +2748,12 @@ static bool recombine_by_event(const Params& P, const clotho_config& cfg, uint32
 // and again within it (width_due): a population starts out empty, so the
 // capacity says nothing of its rows (200 generations from none, N = 20,000, capacity
 // 256 words, rho = 1: 68 us each by groups, 90 by event).
-// Row chunks that were set or tuned stay, with their kernel.
+// Row chunks that were set or tuned stay; tuned ones with the kernel they were timed
+// for.
 bool refresh_shapes(clotho_ctx* c) {
     const bool brief = short_traits(c);
     const bool by_event =
-        c->chunks_set ? c->by_event : recombine_by_event(c->p, c->cfg, c->live_words);
+        c->kernel_set ? c->by_event : recombine_by_event(c->p, c->cfg, c->live_words);
     const bool same = by_event == c->by_event;
     c->by_event = by_event;
     uint32_t chunks = c->p.chunks;

@@ -302,6 +302,7 @@ struct clotho_ctx {
     uint32_t recombine_round = 1; // and of the recombination by groups
     bool by_event = false;        // recombination by event (recombine_by_event)
     bool chunks_set = false;      // its row chunks were set or tuned
+    bool kernel_set = false;      // tuned: they are for the kernel in use
     // launch shapes the autotuner may change (0 / defaults: the built-in choice)
     uint32_t trait_variant = 0;   // traits-pass kernel shape, 1 .. trait_variants()
     uint32_t compact_rows = 8;    // rows per wave step of the column compaction: 4, 8, 16

@@ -107,3 +107,21 @@ def test_capacity_beyond_the_width(words):
         x.set_population(*_population(4200, 64 * words - 100, words))
     _steps(sim, orc, 2, True, f"{words} words")
     assert sim.launch_shape()["recombine_chunks"] == 17
+
+
+def test_saved_chunks_by_phases():
+    # chunks tuned by event, given to a context that has no population yet; the
+    # phases of a generation called one by one
+    sim, orc = _pair(4200, 0.5, 1 << 15)
+    sim.set_launch_shape(recombine_chunks=17)
+    for alleles in (400, 24_000, 300):
+        for x in (sim, orc):
+            x.set_population(*_population(4200, alleles, alleles))
+        for _ in range(2):
+            for phase in ("draw", "recombine_mutate", "traits", "free_space", "fitness", "commit"):
+                assert getattr(api.lib(), "clotho_phase_" + phase)(sim.ctx) == 0
+            orc.step()
+        compare_gametes(sim, orc, f"{alleles} alleles")
+        compare_state(sim, orc, f"{alleles} alleles")
+        _steps(sim, orc, 1, True, f"{alleles} alleles, a run")
+        assert sim.launch_shape()["recombine_chunks"] == 17
