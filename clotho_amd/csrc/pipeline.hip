@@ -592,9 +592,10 @@ struct ParentScatterOp {
 
 // ---------------------------------------------------------------------------
 // Recombination + mutation (+ free-space partials) with a lookup per event and
-// row: the replicates of large batches, up to kWidePerGroup words per row, and
-// large single populations with few events per gamete (recombine_by_event).  The
-// others take rec::Recombine.
+// row: large single populations with few events per gamete (recombine_by_event),
+// batches of many groups with few events, and the rows of up to kWidePerGroup
+// words of the largest batches (batch_recombine_shape).  The others take
+// rec::Recombine.
 // ---------------------------------------------------------------------------
 // Per-word order statistics, once per generation: the 64 position keys of
 // word w sorted ascending (sorted[w][k]), prefix masks pm[w][c] = bits of the
@@ -2158,7 +2159,7 @@ __global__ void __launch_bounds__(kBlock) k_scale(const T* src, size_t n, double
 
 __global__ void k_end_analysis(GenState* st) { st->inter = 0; }
 
-// Exact genome traits of population `sel` (f6::traits_block); the effect
+// Exact genome traits of population `sel` (f6::TraitsBlock::run); the effect
 // digit planes are packed first (f6::pack_block).
 struct PackDigits {
     static constexpr int kThreads = 256;
@@ -2612,9 +2613,9 @@ hipError_t launch_single(void (*kernel)(Params, Buffers, uint32_t), clotho_ctx* 
 
 }  // namespace
 
-// Draws of the generation, the per-word order statistics of the child columns
-// (which need only the new mutations' keys) and the effect digit planes of
-// the traits pass.
+// Draws of the generation, the effect digit planes of the traits pass and, where
+// the recombination goes by event, the per-word order statistics of the child
+// columns (which need only the new mutations' keys).
 hipError_t launch_draw(clotho_ctx* c) {
     const uint32_t par = (uint32_t)c->cur;  // parent = current population
     TRY_LAUNCH(launch_single<DrawCounts>(k_draw_counts, c, par));

@@ -16,9 +16,10 @@ namespace clotho {
 constexpr int kMaxCdf = 128;      // Poisson inversion table capacity
 constexpr int kMaxTraits = 32;    // trait capacity of the fused paths
 constexpr int kScanBlock = 256;   // items per block of every two-level scan
-// |quantised effect| bound: four balanced base-256 digits represent it exactly
+// |quantised effect| bound: seven balanced base-32 digits represent it exactly
+// (f6::digit_planes)
 constexpr double kEffectLimit = 1073741823.0;  // 2^30 - 1
-// allele-slot capacity limit: digit sums over a row stay within int32
+// allele-slot capacity limit: a group's mutations are kept as slot (24 bits) and gamete (8)
 constexpr uint32_t kMaxAlleleSlots = 1u << 24;
 // words per column tile of the population-statistics pass (row partials are
 // kept per tile), its waves per block, and the most rows of one of its row
@@ -44,7 +45,7 @@ inline uint32_t stat_chunks(uint32_t words, uint32_t n) {
     return chunks < most ? chunks : most;
 }
 
-// The per-word order-statistic tables of the batched recombination (sorted keys,
+// The per-word order-statistic tables of the recombination by event (sorted keys,
 // bucket counts, prefix masks) are stored tile-major: the table of a 64-word
 // column tile is one contiguous [row][64 words] image, the layout a
 // recombination block keeps in LDS, so a block fills its LDS copy with

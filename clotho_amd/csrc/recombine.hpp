@@ -1,6 +1,7 @@
 // recombine.hpp — recombination, mutation and free-space partials of one
-// generation of a single population, and of replicates of small batches or wide
-// rows (device code of pipeline.hip).
+// generation by groups of 64 gametes (device code of pipeline.hip): of single
+// populations and replicates but those with few events in many rows, and narrow
+// rows of the largest batches (recombine_by_event, batch_recombine_shape).
 //
 // A child word is a select between the two words of its parent individual by
 // the crossover mask {slots j : odd #{events e <= key_j}} (block_crossover with

@@ -7,7 +7,8 @@
 // popcount-weighted baseline); EXACT_FP64 does the same walk in FP64;
 // MFMA_BF16 expands bits to BF16 and runs the contraction on matrix cores
 // with effects split into BF16 terms (traits_mfma.hip); EXACT_I8 is the
-// pipeline's exact path (int8 digit planes of quantised effects).
+// pipeline's exact path (FP6 digit planes of quantised effects; its sums take the
+// place of the int8 path that named the mode).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -18,9 +18,9 @@
 // spread every genotype byte to 8 bytes through an LDS table, whose lookups
 // (10 GB of LDS reads at 2e5 x 50,176 sites, with bank conflicts) bounded the
 // one-trait pass.  Measured, int8 against this: one trait at 2e5 x 816 words
-// 281 -> 241 us (5.4 TB/s of rows; copies run at 5.8), 16 traits at 5e5 x 2,136
-// words 3.35 -> 2.34 ms, 16 traits of the full 31-bit range at 2e5 x 65,536
-// sites 862 -> 695 us, 2,000 rows of 496 words 97 -> 12 us (Balance, below).
+// 281 -> 241 us (5.4 TB/s of rows; copies run at 5.8), 16 traits at 5e5 x 2,072
+// words 3.35 -> 2.17 ms, 16 traits of the full 31-bit range at 2e5 x 65,536
+// sites 844 -> 656 us, 2,000 rows of 496 words 97 -> 10 us (Balance, below).
 #pragma once
 
 #include <hip/hip_runtime.h>
