@@ -2212,7 +2212,7 @@ struct TraitReduceOp {
                                                uint32_t blk) {
         const bool whole_few = P.traits <= 16 || P.trait_rows == f6::tile_block_rows(1);
         f6::reduce_pieces(B.trait_part, P.h, uniform_read(&gbl(B.state)->wc), P.traits, balance(P),
-                          P.trait_rows, whole_few ? f6::kFewGroups : 0u,
+                          P.trait_rows, whole_few ? f6::few_groups(P.h, P.traits) : 0u,
                           (uint64_t)blk * kThreads + threadIdx.x, B.traits[sel]);
     }
 };

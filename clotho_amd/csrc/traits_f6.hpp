@@ -728,8 +728,16 @@ struct Balance {
 // and second prologues take longer than the units even out, and blocks of two row
 // tiles per wave in turn reach more compute units (traits and free space of
 // a generation, us: 40,000 rows x 48 words x 8 traits 34.9 -> 25.6, 200,000 x 16 x 6
-// 44.3 -> 34.8, 400 x 16 x 4 16.7 -> 13.8).
-constexpr uint32_t kFewGroups = 8;
+// 44.3 -> 34.8, 400 x 16 x 4 16.7 -> 13.8).  With few row blocks only the shortest
+// rows, as units along K then reach more compute units than row blocks do (3,000
+// rows x 1 trait, 48 / 96 words: cut 17.6 / 17.9, whole 16.3 / 19.1; 40,000 rows
+// 22.4 / 25.5, 19.6 / 25.5; 10,000 rows x 8, 96 words 21.7, 22.1; 200 rows x 20, 64
+// words 17.4, 25.8).
+__host__ __device__ constexpr uint32_t few_groups(uint32_t h, uint32_t traits) {
+    const int cls = trait_class(traits);
+    if (cls == 4) return h > 20480 ? 8u : 1u;
+    return h > 16384 ? 8u : cls == 1 ? 3u : 4u;
+}
 
 // The sums of element e = (row, trait) of the rows past the whole rounds,
 // where its row block was cut into pieces (rows of more than `few` groups).
@@ -842,7 +850,7 @@ struct TraitsBlock {
             return;
         }
         if constexpr (kForm == Form::kBalancedFew) {
-            if (NG <= kFewGroups) {
+            if (NG <= few_groups(h, T)) {
                 constexpr int kFewTiles = RT < 2 ? RT : 2;
                 constexpr uint32_t few_rows = 4 * kFewTiles * kTileRows;
                 for (uint64_t row = (uint64_t)blk * few_rows; row < h; row += (uint64_t)blocks * few_rows) {

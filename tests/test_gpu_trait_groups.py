@@ -77,3 +77,18 @@ def test_batch_many_traits():
     for r in range(3):
         _check(batch.replicate(r), f"replicate {r}")
     batch.close()
+
+
+@pytest.mark.parametrize("traits", [2, 4, 8, 16, 20])
+@pytest.mark.parametrize("n", [150, 8192, 8193, 10_241])
+def test_few_groups(n, traits):
+    # 3, 4, 5 and 8 groups of 16 words, whole or cut by the number of rows
+    rng = np.random.default_rng(n + traits)
+    sim = api.Simulation(api.make_config(n, 2.0 / n, 1.0, seed=3, traits=traits, neutral_p=0.0,
+                                         sigma=0.1, max_alleles=8704))
+    for alleles in (3072, 4096, 4100, 8192):
+        sim.set_population(*_population(rng, n, alleles, traits))
+        _check(sim, f"{alleles} alleles")
+        sim.run(1)
+        _check(sim, f"{alleles} alleles, a generation on")
+    sim.close()
