@@ -150,15 +150,62 @@ struct OnDevice {
 };
 
 // Memory that calls on one device's contexts work in, kept between calls while a
-// context is there: at most kScratchKept bytes per device, however many contexts
-// (replicates of a batch, say) it serves.
+// context is there, in as many buffers of at most kScratchKept bytes as calls were
+// under way at a time, however many contexts (replicates of a batch, say) a device has,
+// and at most kScratchTotal (eight threads that read the margins of 32 replicates:
+// 2.4 ms, with one buffer for all 5.8, as the others allocated and freed theirs).
 constexpr size_t kScratchKept = 64u << 20;  // covers 100,000 individuals of 1000 words
+constexpr size_t kScratchTotal = 512u << 20;
 struct DeviceScratch {
-    std::mutex in_use;  // held by the call that works in it
-    char* base = nullptr;
-    size_t bytes = 0;
-    std::mutex counted;
+    struct Buffer {
+        char* base;
+        size_t bytes;
+        bool used;
+    };
+    std::mutex mutex;
+    std::vector<Buffer> buffers;
+    size_t kept = 0;
     uint32_t contexts = 0;
+
+    // a free buffer of `bytes` or more, the smallest, or a new one; nullptr: there is no
+    // room for that
+    char* take(size_t bytes) {
+        const std::lock_guard<std::mutex> lock(mutex);
+        Buffer* best = nullptr;
+        for (Buffer& f : buffers)
+            if (!f.used && f.bytes >= bytes && (!best || f.bytes < best->bytes)) best = &f;
+        if (best) {
+            best->used = true;
+            return best->base;
+        }
+        for (size_t i = 0; i < buffers.size();)  // those are too small
+            if (buffers[i].used)
+                ++i;
+            else
+                drop(i);
+        size_t step = 256u << 10;  // a quarter more at most, not a size per call
+        while (8 * step <= bytes) step *= 2;
+        const size_t size = std::min(kScratchKept, (bytes + step - 1) / step * step);
+        char* base = nullptr;
+        if (kept + size > kScratchTotal) return nullptr;
+        if (hipMalloc((void**)&base, size) != hipSuccess) {
+            (void)hipGetLastError();  // not for the next call to find
+            return nullptr;
+        }
+        kept += size;
+        buffers.push_back({base, size, true});
+        return base;
+    }
+    void give_back(const char* base) {
+        const std::lock_guard<std::mutex> lock(mutex);
+        for (Buffer& f : buffers)
+            if (f.base == base) f.used = false;
+    }
+    void drop(size_t i) {
+        (void)hipFree(buffers[i].base);
+        kept -= buffers[i].bytes;
+        buffers.erase(buffers.begin() + (ptrdiff_t)i);
+    }
 };
 constexpr int kMaxDevices = 64;
 DeviceScratch g_scratch[kMaxDevices];
@@ -166,61 +213,47 @@ DeviceScratch g_scratch[kMaxDevices];
 void scratch_join(int device) {
     if (device < 0 || device >= kMaxDevices) return;
     DeviceScratch& d = g_scratch[device];
-    const std::lock_guard<std::mutex> lock(d.counted);
+    const std::lock_guard<std::mutex> lock(d.mutex);
     ++d.contexts;
 }
 void scratch_leave(int device) {
     if (device < 0 || device >= kMaxDevices) return;
     DeviceScratch& d = g_scratch[device];
-    const std::lock_guard<std::mutex> lock(d.counted);
+    const std::lock_guard<std::mutex> lock(d.mutex);
     if (--d.contexts) return;
-    const std::lock_guard<std::mutex> use(d.in_use);
-    if (d.base) (void)hipFree(d.base);
-    d.base = nullptr;
-    d.bytes = 0;
+    while (!d.buffers.empty()) d.drop(0);
 }
 
-// Device memory of one call: the device's scratch, grown when it is too small,
-// or an allocation of its own above kScratchKept and while another context's call
-// has the scratch.  A second call on the same context waits (the events that time the
-// kernels are the context's).  Whatever path the call returns by, its work on the
-// stream is done before the memory is free for others.
+// Device memory of one call: a buffer of the device's, or an allocation of its own
+// past those bounds.  A second call on the same context
+// waits (the events that time the kernels are the context's).  Whatever path the call
+// returns by, its work on the stream is done before the memory is free for others.
 struct Scratch {
     clotho_ctx* c;
-    std::unique_lock<std::mutex> mine, shared;
+    std::unique_lock<std::mutex> mine;
     char* base = nullptr;
-    char* own = nullptr;
+    bool kept = false;
     bool finished = false;
     explicit Scratch(clotho_ctx* ctx) : c(ctx), mine(ctx->scratch_mutex) {}
     ~Scratch() {
-        if (base && !finished) (void)hipStreamSynchronize(c->stream);
-        if (own) (void)hipFree(own);
+        if (!base) return;
+        if (!finished) (void)hipStreamSynchronize(c->stream);
+        if (kept)
+            g_scratch[c->device].give_back(base);
+        else
+            (void)hipFree(base);
     }
     hipError_t get(size_t bytes) {
         const OnDevice here(c->device);
-        if (bytes <= kScratchKept && c->device < kMaxDevices) {
-            DeviceScratch& d = g_scratch[c->device];
-            shared = std::unique_lock<std::mutex>(d.in_use, std::try_to_lock);
-            if (shared && bytes > d.bytes) {
-                if (d.base) (void)hipFree(d.base);  // waits for the device
-                d.base = nullptr;
-                d.bytes = 0;
-                const hipError_t e = hipMalloc((void**)&d.base, bytes);
-                if (e != hipSuccess) return failed(e);
-                d.bytes = bytes;
-            }
-            if (shared) {
-                base = d.base;
-                return hipSuccess;
-            }
+        if (bytes <= kScratchKept && c->device < kMaxDevices)
+            base = g_scratch[c->device].take(bytes);
+        kept = base != nullptr;
+        if (kept) return hipSuccess;
+        const hipError_t e = hipMalloc((void**)&base, bytes);
+        if (e != hipSuccess) {
+            base = nullptr;
+            (void)hipGetLastError();
         }
-        const hipError_t e = hipMalloc((void**)&own, bytes);
-        if (e != hipSuccess) return failed(e);
-        base = own;
-        return hipSuccess;
-    }
-    static hipError_t failed(hipError_t e) {
-        (void)hipGetLastError();  // not for the next call to find
         return e;
     }
 };

@@ -1,7 +1,8 @@
-"""Device memory that calls keep between them: one scratch allocation of at most 64 MiB
-per device for all contexts, and none of a replicate's for launches that its batch does
-not make."""
+"""Device memory that calls keep between them: scratch buffers of at most 64 MiB per
+device for all contexts, as many as calls were under way at a time, and none of a
+replicate's for launches that its batch does not make."""
 import threading
+from concurrent.futures import ThreadPoolExecutor
 
 import numpy as np
 import pytest
@@ -37,6 +38,22 @@ def test_contexts_share_scratch():
     assert all(np.array_equal(a, b) for a, b in zip(first, again))
     for s in sims:
         s.close()
+
+
+def test_as_many_buffers_as_threads():
+    start = _used()
+    sims = [_context(20_000, 8192, s) for s in range(12)]
+    want = [s.allele_counts() for s in sims]
+    one = _used()
+    with ThreadPoolExecutor(4) as pool:
+        for _ in range(3):
+            got = list(pool.map(lambda s: s.allele_counts(), sims))
+            for a, b in zip(want, got):
+                assert all(np.array_equal(x, y) for x, y in zip(a, b))
+    assert _used() - one <= 3 * 64 * MIB
+    for s in sims:
+        s.close()
+    assert _used() - start <= 8 * MIB
 
 
 def test_threads_with_contexts_of_their_own():
